@@ -9,7 +9,10 @@
 // the reference's final order is the lexicographic order
 // (tile, depth bits, gaussian id).
 //
-// Single view, with far less sort traffic than a 64-bit key sort:
+// Single view: grids of up to 256 tiles per axis are binned by tile rows
+// (rowbin.hip), of the Gaussians in depth order where they have many pairs
+// each, else in id order with step 5 below after it.  Smaller (one radix pass)
+// and larger grids, and batches:
 //  1. depth_keys_kernel: per Gaussian its depth bits and packed tile
 //     rectangle;
 //  2. emission in Gaussian id order: a reduce-then-scan of the Gaussians'
@@ -19,9 +22,9 @@
 //     max-scan), so neither a Gaussian covering hundreds of tiles nor a run
 //     of large Gaussians serialises a lane or a wave; the expansion also
 //     counts the tile sort's first digit;
-//  3. an LSD radix sort of the pairs on the tile id bits only (2 passes at
-//     1080p/16x16; the first need not be stable, the order inside a tile
-//     being set in step 5);
+//  3. an LSD radix sort of the pairs on the tile id bits only (one pass up to
+//     256 tiles; the first need not be stable, the order inside a tile being
+//     set in step 5);
 //  4. tile_bins_kernel: [start, end) edges from the sorted tile ids, empty
 //     tiles (0, 0);
 //  5. tile_depth_sort_kernel: every tile's run ordered by (depth bits, id)
@@ -915,19 +918,38 @@ struct BinLayout {
     size_t err, total, zero_end;
     size_t tile_sort, tiles, gids, ttmp_k, ttmp_v, tiles_sorted, end;
     EmitLayout emit;
+    // by_rows: its scratch, the runs (8 bytes per pair; then the long runs' ka
+    // and va), the long runs' kv or (by_depth) the depth sort's buffers
+    size_t rows, runs, kv, depth_sort, keys_out, perm, dtmp_k, dtmp_v;
 };
 
 BinLayout layout(const BinPlan& p) {
-    BinLayout L;
+    BinLayout L{};
     size_t o = 0;
     L.err = o;
     L.total = o + 8;
     o += 16;
     L.zero_end = o;
     o = align256(o);
+    const size_t i4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
+    if (p.by_rows) {
+        const size_t n4 = align256(4ull * (p.n > 0 ? p.n : 1));
+        L.rows = o; o = align256(o + p.rows.scratch_bytes);
+        L.runs = o; o += 2 * i4;
+        if (p.by_depth) {
+            L.depth_sort = o; o = align256(o + p.depth_sort.scratch_bytes);
+            L.keys_out = o; o += n4;
+            L.perm = o; o += n4;
+            L.dtmp_k = o; o += n4;
+            L.dtmp_v = o; o += n4;
+        } else {
+            L.kv = o; o += 2 * i4;
+        }
+        L.end = o;
+        return L;
+    }
     L.tile_sort = o; o = align256(o + p.tile_sort.scratch_bytes);
     o = emit_layout(o, p.n, p.isect_cap, false, L.emit);
-    const size_t i4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
     L.tiles = o; o += i4;
     L.gids = o; o += i4;
     L.ttmp_k = o; o += i4;
@@ -939,7 +961,49 @@ BinLayout layout(const BinPlan& p) {
 
 int bitlen(uint32_t v) { return v ? 32 - __builtin_clz(v) : 0; }
 
+// Binning by tile rows: of the Gaussians in depth order (by_depth), whose
+// tiles' lists are then ordered as they are placed, or in id order and every
+// tile's run ordered where it lies.  dkeys: the depth bits.
+hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rects,
+                       int* gids_sorted, int* tiles_sorted, int* tile_bins, void* scratch,
+                       hipStream_t s) {
+    const BinLayout L = layout(p);
+    uint8_t* b = static_cast<uint8_t*>(scratch);
+    auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
+    uint32_t* ids = reinterpret_cast<uint32_t*>(gids_sorted);
+    int2* bins = reinterpret_cast<int2*>(tile_bins);
+    hipError_t e;
+    if (p.by_depth &&
+        (e = sort_pairs(p.depth_sort, dkeys, nullptr, U(L.keys_out), U(L.perm), U(L.dtmp_k),
+                        U(L.dtmp_v), p.n, nullptr, b + L.depth_sort, nullptr, s)) != hipSuccess)
+        return e;
+    // (the depth sort's ping-pong buffers, adjacent, are free again)
+    e = row_bin(p.rows, p.by_depth ? U(L.perm) : nullptr, rects,
+                reinterpret_cast<uint2*>(b + L.dtmp_k), reinterpret_cast<uint2*>(b + L.runs), ids,
+                reinterpret_cast<uint32_t*>(tiles_sorted), bins,
+                reinterpret_cast<unsigned long long*>(b + L.total), U(L.err), b + L.rows, s);
+    if (e != hipSuccess) return e;
+    stage_mark(kMarkBinned, s);
+    if (p.by_depth) return hipSuccess;
+    const size_t i4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
+    return tile_depth_order(bins, p.num_tiles, true, dkeys, ids, U(L.runs), U(L.runs + i4),
+                            reinterpret_cast<uint2*>(b + L.kv), s);
+}
+
 }  // namespace
+
+// Pairs of the capacity per Gaussian from which the lists are ordered by one
+// depth sort of the Gaussians and stable placements, instead of tile by tile:
+// the depth sort costs 40 us + 36 us per 1M Gaussians, the order of the tiles
+// 7.6 us per 1M pairs in runs of up to kSegCap and several times that beyond.
+// Forward of 50k Gaussians with 100 pairs each at 900 x 1600: 232 us by depth,
+// 392 tile by tile; 610k Gaussians with 11 pairs each at 1080p: 664 against
+// 607 us (forward and backward).
+constexpr int kByDepthPairs = 16;
+// Grids of up to this many tiles are one radix pass of the emitted pairs,
+// whose three launches fewer are worth more than the traffic of few pairs
+// (2k Gaussians at 256 x 256: 50 against 61 us of kernels).
+constexpr int kOnePassTiles = 256;
 
 BinPlan bin_plan(const Camera& c, int isect_cap) {
     BinPlan p;
@@ -947,6 +1011,11 @@ BinPlan bin_plan(const Camera& c, int isect_cap) {
     p.isect_cap = isect_cap;
     p.num_tiles = c.tiles_x * c.tiles_y;
     p.tile_bits = bitlen((uint32_t)(p.num_tiles > 1 ? p.num_tiles - 1 : 1));
+    p.by_rows = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
+                p.num_tiles > kOnePassTiles;
+    p.by_depth = p.by_rows && (long long)isect_cap > kByDepthPairs * (long long)p.n;
+    p.rows = row_bin_plan(p.n, c.tiles_x, c.tiles_y, isect_cap);
+    p.depth_sort = sort_plan(p.n, 0, 32);
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
     p.depth_bytes = align256(depth_layout(p).end);
     p.emit_bytes = align256(layout(p).end);
@@ -974,6 +1043,13 @@ hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
                     int* tiles_sorted, int* tile_bins, void* scratch, hipStream_t s) {
     const BinLayout L = layout(p);
     uint8_t* b = static_cast<uint8_t*>(scratch);
+    const DepthLayout D = depth_layout(p);
+    const uint8_t* d = static_cast<const uint8_t*>(depth_ws);
+    const uint32_t* dkeys = reinterpret_cast<const uint32_t*>(d + D.dkeys);
+    const uint2* rect_by_id = reinterpret_cast<const uint2*>(d + D.rect_by_id);
+    if (p.by_rows && p.n > 0)
+        return bin_by_rows(p, dkeys, rect_by_id, gids_sorted, tiles_sorted, tile_bins, scratch,
+                           s);
     hipError_t e = fill_zero(b, L.zero_end, s);
     if (e != hipSuccess) return e;
     e = fill_zero(tile_bins, 8ull * p.num_tiles, s);
@@ -981,10 +1057,6 @@ hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
     if (p.n <= 0) return hipSuccess;
     uint32_t* err = reinterpret_cast<uint32_t*>(b + L.err);
     auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
-    const DepthLayout D = depth_layout(p);
-    const uint8_t* d = static_cast<const uint8_t*>(depth_ws);
-    const uint32_t* dkeys = reinterpret_cast<const uint32_t*>(d + D.dkeys);
-    const uint2* rect_by_id = reinterpret_cast<const uint2*>(d + D.rect_by_id);
     // the sort and the edges cover the slots the emission wrote, min(total,
     // capacity), read on the device: a count given too large (an inconsistent
     // cum_tiles_hit) then never sorts unwritten slots, and one too small is
@@ -1036,6 +1108,9 @@ hipError_t bin_rects(const BinPlan& p, const Camera& c, const float* depths,
         if ((e = fill_zero(b, L.zero_end, s)) != hipSuccess) return e;
         return fill_zero(tile_bins, 8ull * p.num_tiles, s);
     }
+    if (p.by_rows)
+        return bin_by_rows(p, reinterpret_cast<const uint32_t*>(depths), rects, gids_sorted,
+                           tiles_sorted, tile_bins, scratch, s);
     uint32_t* err = reinterpret_cast<uint32_t*>(b + L.err);
     auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
     int* written = reinterpret_cast<int*>(b + L.emit.info);

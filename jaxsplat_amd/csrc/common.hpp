@@ -150,16 +150,17 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, int bits, uint64_t v
 
 // Exclusive scan of one value per thread over a 256-thread block (s_tmp: 4
 // words of LDS; two barriers).
-__device__ __forceinline__ uint32_t block_exclusive_scan256(uint32_t v, uint32_t* s_tmp) {
+template <typename T>
+__device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
     const int tid = threadIdx.x;
     const int lane = lane_id();
     const int wave = tid >> 6;
-    const uint32_t incl = wave_inclusive_sum(v);
+    const T incl = wave_inclusive_sum(v);
     if (lane == 63) s_tmp[wave] = incl;
     __syncthreads();
-    uint32_t off = 0;
+    T off = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) off += (w < wave) ? s_tmp[w] : 0u;
+    for (int w = 0; w < 4; ++w) off += (w < wave) ? s_tmp[w] : T(0);
     __syncthreads();
     return off + incl - v;
 }
@@ -608,13 +609,44 @@ hipError_t sort_pairs(const SortPlan& p, const uint32_t* keys_in, const uint32_t
                       uint32_t* err, hipStream_t s, bool counted = false,
                       bool unstable_first = false);
 
+// Exclusive scan over the partitions of each column counts[c * parts + 0..parts)
+// in place, c < columns, and the columns' sums totals[c].
+hipError_t column_scan(uint32_t* counts, int parts, uint32_t* totals, int columns, hipStream_t s);
+
+// ---- binning by tile rows (rowbin.hip) ----
+constexpr int kRowBinAxis = 256;    // tiles per axis, at most
+struct RowBinPlan {
+    int n, tiles_x, tiles_y, cap;
+    int parts;              // partitions of the Gaussians
+    int max_col_parts;      // partitions of the runs, at most
+    size_t row_len, row_counts, part_tot, tile_first, desc, col_counts;  // offsets in the scratch
+    size_t scratch_bytes;
+};
+RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap);
+// The tiles' lists of the packed rectangles rects (tile counts up to
+// kRowBinAxis per axis): bins (cleared first; empty tiles stay (0, 0)) and
+// ids, at most p.cap of them (the pairs past it are dropped and bit 8 of *err
+// set; *err is cleared first), *total the exact pair total.  With perm (n
+// Gaussian ids, each once) every tile's list is in perm's order; without, its
+// order is arbitrary.  in_order (with perm): n rectangles of scratch; runs: 8
+// bytes per pair of the capacity.  tiles_sorted (optional): every entry's tile
+// id.
+hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects,
+                   uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
+                   int2* bins, unsigned long long* total, uint32_t* err, void* scratch,
+                   hipStream_t s);
+
 // ---- binning ----
 struct BinPlan {
     int n;              // Gaussians
     int isect_cap;      // intersection capacity
     int num_tiles;
     int tile_bits;
-    SortPlan tile_sort;
+    bool by_rows;           // rowbin.hip (tile grids up to kRowBinAxis per axis)
+    bool by_depth;          // by_rows, from the Gaussians in depth order
+    RowBinPlan rows;
+    SortPlan depth_sort;    // by_depth
+    SortPlan tile_sort;     // not by_rows
     size_t depth_bytes;     // depth stage workspace (depends on n only)
     size_t emit_bytes;      // emission stage workspace
     size_t scratch_bytes;   // both, for bin_and_sort: emission region first

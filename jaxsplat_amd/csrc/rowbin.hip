@@ -1,0 +1,625 @@
+// Binning of packed tile rectangles by tile rows, for gfx950.
+//
+// A rectangle of w x h tiles is h runs of w consecutive tiles.  Instead of
+// emitting its w h (tile, id) pairs and radix sorting them, the rectangles are
+// split in two steps, each one a counting sort of intervals:
+//  1. every Gaussian's row interval [y0, y0 + h) puts one 8-byte run
+//     (id, x0 | w << 16) into the segment of each of its tile rows;
+//  2. within a row segment every run's column interval [x0, x0 + w) puts the
+//     id into the list of each of its tiles.
+// A step counts with differences (+1 at the interval's begin, -1 at its end,
+// one prefix sum per partition), so counting costs two LDS atomics per
+// interval, however long it is, and the pairs themselves exist only as the
+// final ids: per pair 4 bytes are written, per run 8 are written and read
+// twice.  The pair sort this replaces moved 52 bytes per pair (8 written by
+// the emission, 16 by each pass, 4 read by a counting pass and by the edges,
+// 4 read again): at 1M Gaussians and 1080p (6.6M pairs, 1.9M runs) its kernels
+// took 126 us and these take 62; at 3M large Gaussians 1540 us, and 445 in the
+// stable form, after a depth sort of 150, which also replaces 3440 us of
+// ordering the tiles' runs.  What bounds the placements is LDS (the
+// per-pair accesses and their bank conflicts) and its latency: the arrays are
+// sized for six workgroups per CU.
+//
+// Stable form (STABLE): the intervals of a partition are placed in their
+// order, by 64-lane column masks in LDS (an interval's rank in a column is the
+// population count of the mask below its lane), so that Gaussians given in
+// depth order leave every tile's list in depth order.  Otherwise one returning
+// LDS atomic per pair places it (about half of the LDS work), and the order
+// inside a tile is the caller's to set.
+//
+// A partition is 1024 intervals (512 took 31 us instead of 25 at 1M Gaussians:
+// half as long runs of stores).  Its values are staged in LDS in column
+// order (stable: half a partition at a time), so that each column's values are
+// stored contiguously; with more values than the stage holds (long intervals,
+// whose columns then hold many values anyway) they are stored directly.
+#include "common.hpp"
+
+namespace jsa {
+namespace {
+
+constexpr int kRbThreads = 256;
+constexpr int kRbWaves = kRbThreads / kWave;
+constexpr int kRbPart = 1024;                       // intervals per partition
+constexpr int kRbPer = kRbPart / kRbThreads;        // and per lane
+static_assert(kRowBinAxis == kRbThreads, "one thread per column");
+
+// Columns (rows) that the LDS arrays hold: 128 up to 128 tiles, which leaves
+// room for more workgroups per CU, else 256.
+inline bool narrow(int tiles) { return tiles <= 128; }
+
+struct Interval {
+    int lo, len;        // columns [lo, lo + len) (len = 0: none)
+};
+
+__device__ __forceinline__ void add_differences(int* v, int ncols, Interval iv) {
+    if (iv.len <= 0) return;
+    atomicAdd(&v[iv.lo], 1);
+    if (iv.lo + iv.len < ncols) atomicAdd(&v[iv.lo + iv.len], -1);
+}
+
+// LDS of one round of a placement: values V, staged up to CAP of them.
+template <typename V, int COLS, int CAP, bool STABLE>
+struct PlaceShared {
+    // per wave and column: differences, then counts, then the next position
+    // (relative to the round's first value in column order)
+    alignas(16) int cnt[kRbWaves][COLS];
+    // STABLE: the lanes (low, high word) that cover a column; two arrays, so
+    // that the columns of a wave spread over all banks
+    uint32_t lo[STABLE ? kRbWaves : 1][STABLE ? COLS : 1];
+    uint32_t hi[STABLE ? kRbWaves : 1][STABLE ? COLS : 1];
+    int first[COLS + 1];            // column c's values are first[c] .. first[c + 1]
+    int delta[COLS];                // and go to delta[c] + position
+    V out[CAP];
+    uint32_t tmp[kRbWaves];
+};
+
+// Per-column counts of a wave's own intervals: v[c] holds the differences on
+// entry and the counts on return; COLS / 64 columns per lane.
+template <int COLS>
+__device__ __forceinline__ void wave_counts(int* v, int lane) {
+    if constexpr (COLS == 256) {
+        int4* q = reinterpret_cast<int4*>(v) + lane;
+        int4 d = *q;
+        d.y += d.x;
+        d.z += d.y;
+        d.w += d.z;
+        const int before = wave_inclusive_sum(d.w) - d.w;
+        *q = make_int4(d.x + before, d.y + before, d.z + before, d.w + before);
+    } else {
+        static_assert(COLS == 128, "2 or 4 columns per lane");
+        int2* q = reinterpret_cast<int2*>(v) + lane;
+        int2 d = *q;
+        d.y += d.x;
+        const int before = wave_inclusive_sum(d.y) - d.y;
+        *q = make_int2(d.x + before, d.y + before);
+    }
+}
+
+template <typename V, int COLS, int CAP, bool STABLE>
+__device__ __forceinline__ void clear_place(PlaceShared<V, COLS, CAP, STABLE>& sh) {
+    if ((int)threadIdx.x < COLS) {
+#pragma unroll
+        for (int w = 0; w < kRbWaves; ++w) {
+            sh.cnt[w][threadIdx.x] = 0;
+            if (STABLE) {
+                sh.lo[w][threadIdx.x] = 0u;
+                sh.hi[w][threadIdx.x] = 0u;
+            }
+        }
+    }
+}
+
+// One round of a placement: val[k] of interval iv[k] (k-th 64-lane block of
+// the wave's PER * 64 intervals) into every column of the interval.  Column c's
+// values go to out_g[column_base(thread c) ..) in interval order (STABLE) or
+// any order.  Nothing is written at or past cap.  Returns the number of the
+// thread's column's values.  Called by the whole workgroup with cleared LDS;
+// ends with a barrier.
+template <int PER, typename V, int COLS, int CAP, bool STABLE>
+__device__ __forceinline__ int place(PlaceShared<V, COLS, CAP, STABLE>& sh, const Interval* iv,
+                                     const V* val, int ncols, int column_base, V* out_g,
+                                     int cap) {
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) add_differences(sh.cnt[wave], COLS, iv[k]);
+    wave_lds_sync();
+    wave_counts<COLS>(sh.cnt[wave], lane);
+    __syncthreads();
+    int total = 0, before[kRbWaves];
+#pragma unroll
+    for (int w = 0; w < kRbWaves; ++w) {
+        before[w] = total;
+        total += tid < COLS ? sh.cnt[w][tid] : 0;
+    }
+    const int first = (int)block_exclusive_scan256((uint32_t)total, sh.tmp);
+    if (tid < COLS) {
+#pragma unroll
+        for (int w = 0; w < kRbWaves; ++w) sh.cnt[w][tid] = first + before[w];
+        sh.first[tid] = first;
+        sh.delta[tid] = column_base - first;
+    }
+    if (tid == COLS - 1) sh.first[COLS] = first + total;
+    __syncthreads();
+    const bool staged = sh.first[COLS] <= CAP;      // uniform
+    auto put = [&](int c, int pos, const V& v) {
+        if (staged) {
+            sh.out[pos] = v;
+        } else {
+            const int at = sh.delta[c] + pos;
+            if ((unsigned)at < (unsigned)cap) out_g[at] = v;
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const Interval me = iv[k];
+        int* pos = sh.cnt[wave];
+        if constexpr (STABLE) {
+            uint32_t* lo = sh.lo[wave];
+            uint32_t* hi = sh.hi[wave];
+            uint32_t* own = lane < 32 ? lo : hi;
+            const uint32_t bit = 1u << (lane & 31);
+            const uint32_t mlo = lane < 32 ? bit - 1u : ~0u, mhi = lane < 32 ? 0u : bit - 1u;
+            for (int i = 0; i < me.len; ++i) atomicOr(&own[me.lo + i], bit);
+            wave_lds_sync();
+            for (int i = 0; i < me.len; ++i) {
+                const int c = me.lo + i;
+                put(c, pos[c] + __popc(lo[c] & mlo) + __popc(hi[c] & mhi), val[k]);
+            }
+            if (k + 1 == PER) break;
+            wave_lds_sync();
+            for (int c = lane; c < ncols; c += kWave) {
+                pos[c] += __popc(lo[c]) + __popc(hi[c]);
+                lo[c] = 0u;
+                hi[c] = 0u;
+            }
+            wave_lds_sync();
+        } else {
+            for (int i = 0; i < me.len; ++i) {
+                const int c = me.lo + i;
+                put(c, atomicAdd(&pos[c], 1), val[k]);
+            }
+        }
+    }
+    __syncthreads();
+    if (staged) {
+        // 16 lanes per column: a column's values are one contiguous run
+        for (int c = tid >> 4; c < ncols; c += kRbThreads / 16) {
+            const int end = sh.first[c + 1], to = sh.delta[c];
+            for (int i = sh.first[c] + (tid & 15); i < end; i += 16)
+                if ((unsigned)(to + i) < (unsigned)cap) out_g[to + i] = sh.out[i];
+        }
+    }
+    __syncthreads();
+    return total;
+}
+
+// A partition's intervals in rounds of PER per lane: the stage of a stable
+// placement (whose masks take LDS too) holds half a partition.
+template <int PER, typename V, int COLS, int CAP, bool STABLE>
+__device__ __forceinline__ void place_all(PlaceShared<V, COLS, CAP, STABLE>& sh,
+                                          const Interval* iv, const V* val, int ncols,
+                                          int column_base, V* out_g, int cap) {
+    static_assert(kRbPer % PER == 0, "whole rounds");
+#pragma unroll
+    for (int r = 0; r < kRbPer; r += PER) {
+        if (r > 0) {
+            clear_place(sh);
+            __syncthreads();
+        }
+        column_base = min(column_base + place<PER>(sh, iv + r, val + r, ncols, column_base,
+                                                   out_g, cap),
+                          cap);
+    }
+}
+// Interval k (of kRbPer) of a lane, in rounds of PER: its index within the
+// partition.
+template <int PER>
+__device__ __forceinline__ int interval_index(int k) {
+    const int wave = threadIdx.x >> 6, lane = lane_id();
+    return (k / PER) * (PER * kRbThreads) + wave * (PER * kWave) + (k % PER) * kWave + lane;
+}
+constexpr int round_per(bool stable) { return stable ? 2 : kRbPer; }
+
+// A Gaussian's rectangle clipped to the grid (a rectangle outside it, never
+// the projection's, sets bit 4 of err).
+__device__ __forceinline__ uint2 grid_rect(uint2 rc, int tiles_x, int tiles_y, bool& bad) {
+    int x0, x1, y0, y1;
+    unpack_rect(rc, x0, x1, y0, y1);
+    bad = rect_count(rc) > 0 && (x1 > tiles_x || y1 > tiles_y);
+    if (!bad) return rc;
+    x0 = min(x0, tiles_x);
+    x1 = min(x1, tiles_x);
+    y0 = min(y0, tiles_y);
+    y1 = min(y1, tiles_y);
+    return pack_rect(x0, x1, y0, y1);
+}
+
+// Step 1, counting: partition b holds the Gaussians perm[1024 b ..) (the ids
+// themselves where perm is null).  counts[row * parts + b] = its runs per row,
+// part_tot[b] = its pairs; with perm, in_order[i] = the rectangle of perm[i],
+// so that the random gather is paid once.  Also clears the tile bins and the
+// error word.
+__global__ __launch_bounds__(kRbThreads) void row_count_kernel(
+    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
+    int tiles_y, int parts, uint32_t* __restrict__ counts, uint32_t* __restrict__ part_tot,
+    uint2* __restrict__ in_order, int num_tiles, int2* __restrict__ bins,
+    uint32_t* __restrict__ err) {
+    __shared__ int s_d[kRbThreads];
+    __shared__ uint32_t s_tmp[kRbWaves];
+    const int tid = threadIdx.x, part = blockIdx.x;
+    if (part == 0 && tid == 0) *err = 0u;
+    for (int t = part * kRbThreads + tid; t < num_tiles; t += gridDim.x * kRbThreads)
+        bins[t] = make_int2(0, 0);
+    uint2 rc[kRbPer];
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = part * kRbPart + k * kRbThreads + tid;
+        rc[k] = i < n ? rects[perm ? perm[i] : (uint32_t)i] : make_uint2(0u, 0u);
+    }
+    s_d[tid] = 0;
+    __syncthreads();
+    uint32_t pairs = 0;
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = part * kRbPart + k * kRbThreads + tid;
+        if (perm && i < n) in_order[i] = rc[k];
+        bool bad;
+        pairs += rect_count(rc[k]);
+        const uint2 r = grid_rect(rc[k], tiles_x, tiles_y, bad);
+        if (rect_count(r) > 0)
+            add_differences(s_d, kRbThreads, {(int)(r.x >> 16), (int)(r.y >> 16)});
+    }
+    __syncthreads();
+    const uint32_t d = (uint32_t)s_d[tid];
+    const uint32_t c = block_exclusive_scan256(d, s_tmp) + d;      // wraps back to the count
+    if (tid < tiles_y) counts[(size_t)tid * parts + part] = c;
+    const uint32_t t = block_exclusive_scan256(pairs, s_tmp) + pairs;
+    if (tid == kRbThreads - 1) part_tot[part] = t;
+}
+
+// Step 1, placement: the runs of partition b into the row segments, which lie
+// end to end in runs[0 .. sum of row_len).  rects in perm's order; counts: exclusive over the
+// partitions of a row (column_scan), row_len their totals.  Workgroup 0 also
+// writes the exact pair total and bit 8 of err where it exceeds cap.
+template <bool STABLE, int COLS>
+__global__ __launch_bounds__(kRbThreads) void row_place_kernel(
+    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
+    int tiles_y, int parts, const uint32_t* __restrict__ counts,
+    const uint32_t* __restrict__ row_len, const uint32_t* __restrict__ part_tot,
+    uint2* __restrict__ runs, int cap, unsigned long long* __restrict__ total_out,
+    uint32_t* __restrict__ err) {
+    constexpr int PER = round_per(STABLE);
+    __shared__ PlaceShared<uint2, COLS, 3072, STABLE> sh;
+    __shared__ uint64_t s_sum[kRbWaves];
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, part = blockIdx.x;
+    Interval iv[kRbPer];
+    uint2 val[kRbPer];
+    bool bad_any = false;
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = part * kRbPart + interval_index<PER>(k);
+        const uint32_t id = i < n ? (perm ? perm[i] : (uint32_t)i) : 0u;
+        bool bad;
+        const uint2 rc =
+            grid_rect(i < n ? rects[i] : make_uint2(0u, 0u), tiles_x, tiles_y, bad);
+        bad_any = bad_any || bad;
+        iv[k].lo = (int)(rc.x >> 16);
+        iv[k].len = rect_count(rc) > 0 ? (int)(rc.y >> 16) : 0;
+        val[k] = make_uint2(id, (rc.x & 0xFFFFu) | (rc.y << 16));
+    }
+    if (bad_any) atomicOr(err, 4u);
+    clear_place(sh);
+    // (the rows' runs may sum past 32 bits: positions past cap are all alike)
+    const uint64_t row = tid < tiles_y ? row_len[tid] : 0u;
+    const uint64_t at = block_exclusive_scan256(row, s_sum) +
+                        (tid < tiles_y ? counts[(size_t)tid * parts + part] : 0u);
+    const int base = (int)min(at, (uint64_t)cap);
+    place_all<PER>(sh, iv, val, tiles_y, base, runs, cap);
+    if (part != 0) return;
+    uint64_t sum = 0;
+    for (int i = tid; i < parts; i += kRbThreads) sum += part_tot[i];
+    sum = wave_inclusive_sum(sum);
+    if (lane == kWave - 1) s_sum[wave] = sum;
+    __syncthreads();
+    if (tid == 0) {
+        sum = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+        *total_out = (unsigned long long)sum;
+        if (sum > (uint64_t)cap) atomicOr(err, 8u);
+    }
+}
+
+// Step 2's partitions: row r's runs [e0[r], e0[r + 1]) in partitions
+// [p0[r], p0[r + 1]) of up to kRbPart, none at or past cap.
+struct RowTable {
+    int e0[kRowBinAxis + 1], p0[kRowBinAxis + 1];
+};
+
+// Called by the whole workgroup (kRbThreads threads); ends with a barrier.
+__device__ __forceinline__ void row_table(RowTable& rt, const uint32_t* __restrict__ row_len,
+                                          int tiles_y, int cap, uint64_t* s_tmp) {
+    const int tid = threadIdx.x;
+    const uint64_t len = tid < tiles_y ? row_len[tid] : 0u;
+    const uint64_t e = block_exclusive_scan256(len, s_tmp);
+    const uint64_t lim = (uint64_t)cap;
+    const uint64_t b = min(e, lim), n = min(e + len, lim) - b;
+    const uint64_t np = (n + kRbPart - 1) / kRbPart;
+    const uint64_t p = block_exclusive_scan256(np, s_tmp);
+    rt.e0[tid] = (int)b;
+    rt.p0[tid] = (int)p;
+    if (tid == kRbThreads - 1) {
+        rt.e0[kRowBinAxis] = (int)(b + n);
+        rt.p0[kRowBinAxis] = (int)(p + np);
+    }
+    __syncthreads();
+}
+
+// The row of partition p (largest r with p0[r] <= p; an empty row's p0 equals
+// the next one's, so the search lands on the row that holds p).
+__device__ __forceinline__ int row_of(const RowTable& rt, int p) {
+    int lo = 0, hi = kRowBinAxis;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (rt.p0[mid] <= p) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Persistent walk over the partitions: XCD x (workgroups are dealt round
+// robin) takes a contiguous band, so that the partial lines of one row's lists
+// meet in one L2.
+template <typename F>
+__device__ __forceinline__ void for_partitions(int total, F body) {
+    const int per = (total + 7) / 8, x = blockIdx.x & 7;
+    for (int q = blockIdx.x >> 3; q < per; q += gridDim.x >> 3) {
+        const int p = x * per + q;
+        if (p < total) body(p);
+    }
+}
+
+// Step 2, counting: counts[p * 256 + column] = the runs of partition p that
+// cover the column; desc[p] = (row, first run, end, whether it is the row's
+// first partition), desc[-1].x the number of partitions.
+__global__ __launch_bounds__(kRbThreads) void col_count_kernel(
+    const uint2* __restrict__ runs, const uint32_t* __restrict__ row_len, int tiles_x,
+    int tiles_y, int cap, uint32_t* __restrict__ counts, int4* __restrict__ desc) {
+    __shared__ RowTable rt;
+    __shared__ int s_d[kRbThreads];
+    __shared__ uint32_t s_tmp[kRbWaves];
+    __shared__ uint64_t s_tmp64[kRbWaves];
+    const int tid = threadIdx.x;
+    row_table(rt, row_len, tiles_y, cap, s_tmp64);
+    if (blockIdx.x == 0 && tid == 0) desc[-1] = make_int4(rt.p0[kRowBinAxis], 0, 0, 0);
+    for_partitions(rt.p0[kRowBinAxis], [&](int p) {
+        const int r = row_of(rt, p);
+        const int begin = rt.e0[r] + (p - rt.p0[r]) * kRbPart;
+        const int end = min(rt.e0[r + 1], begin + kRbPart);
+        if (tid == 0) desc[p] = make_int4(r, begin, end, p == rt.p0[r] ? 1 : 0);
+        uint32_t w[kRbPer];
+#pragma unroll
+        for (int k = 0; k < kRbPer; ++k) {
+            const int i = begin + k * kRbThreads + tid;
+            w[k] = i < end ? runs[i].y : 0u;
+        }
+        s_d[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kRbPer; ++k)
+            add_differences(s_d, kRbThreads, {(int)(w[k] & 0xFFFFu), (int)(w[k] >> 16)});
+        __syncthreads();
+        const uint32_t d = (uint32_t)s_d[tid];
+        const uint32_t c = block_exclusive_scan256(d, s_tmp) + d;
+        if (tid < tiles_x) counts[(size_t)p * kRowBinAxis + tid] = c;
+    });
+}
+
+// Step 2, offsets, one workgroup per row: counts become each partition's first
+// position in the column's list, relative to the row's first pair;
+// tile_first[row * 257 + column] the tile's first position, [.. + 256] the
+// row's pairs (all at most cap).  Four groups of 256 threads share the row's
+// partitions.
+constexpr int kRbGroups = 4;
+__global__ __launch_bounds__(kRbThreads * kRbGroups) void col_scan_kernel(
+    const uint32_t* __restrict__ row_len, int tiles_x, int tiles_y, int cap,
+    uint32_t* __restrict__ counts, uint32_t* __restrict__ tile_first) {
+    __shared__ uint32_t s_sum[kRbGroups][kRowBinAxis];
+    __shared__ uint64_t s_w[kRbWaves], s_e[kRbWaves], s_p[kRbWaves];
+    __shared__ int s_range[2];
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    const int c = tid & (kRowBinAxis - 1), g = tid / kRowBinAxis, row = blockIdx.x;
+    // this row's partitions (row_table's numbers, by the first 256 threads)
+    const uint64_t lim = (uint64_t)cap;
+    uint64_t len = 0, e = 0, np = 0, p = 0;
+    if (g == 0) {
+        len = c < tiles_y ? row_len[c] : 0u;
+        e = wave_inclusive_sum(len);
+        if (lane == kWave - 1) s_e[wave] = e;
+    }
+    __syncthreads();
+    if (g == 0) {
+        for (int w = 0; w < wave; ++w) e += s_e[w];
+        const uint64_t b = min(e - len, lim);
+        np = (min(e, lim) - b + kRbPart - 1) / kRbPart;
+        p = wave_inclusive_sum(np);
+        if (lane == kWave - 1) s_p[wave] = p;
+    }
+    __syncthreads();
+    if (g == 0) {
+        for (int w = 0; w < wave; ++w) p += s_p[w];
+        if (c == row) {
+            s_range[0] = (int)(p - np);
+            s_range[1] = (int)p;
+        }
+    }
+    __syncthreads();
+    const int p0 = s_range[0], parts = s_range[1] - p0;
+    const int q0 = p0 + parts * g / kRbGroups, q1 = p0 + parts * (g + 1) / kRbGroups;
+    const bool on = c < tiles_x;
+    uint32_t sum = 0;
+    if (on) {
+#pragma unroll 8
+        for (int q = q0; q < q1; ++q) sum += counts[(size_t)q * kRowBinAxis + c];
+    }
+    s_sum[g][c] = sum;
+    __syncthreads();
+    uint64_t total = 0, before = 0;
+#pragma unroll
+    for (int k = 0; k < kRbGroups; ++k) {
+        const uint32_t v = s_sum[k][c];
+        before += k < g ? v : 0u;
+        total += v;
+    }
+    // exclusive over the columns (every group computes the same)
+    const uint64_t incl = wave_inclusive_sum(total);
+    if (g == 0 && lane == kWave - 1) s_w[wave] = incl;
+    __syncthreads();
+    uint64_t first = incl - total;
+    for (int w = 0; w < (c >> 6); ++w) first += s_w[w];
+    if (g == 0) {
+        uint32_t* tf = tile_first + (size_t)row * (kRowBinAxis + 1);
+        tf[c] = (uint32_t)min(first, lim);
+        if (c == kRowBinAxis - 1) tf[kRowBinAxis] = (uint32_t)min(first + total, lim);
+    }
+    uint64_t run = first + before;
+    if (on) {
+#pragma unroll 8
+        for (int q = q0; q < q1; ++q) {
+            const size_t at = (size_t)q * kRowBinAxis + c;
+            const uint32_t v = counts[at];
+            counts[at] = (uint32_t)min(run, lim);
+            run += v;
+        }
+    }
+}
+
+// Step 2, placement: the ids of every partition's runs into the tiles' lists
+// (rows end to end), and the bins of the rows that have runs.
+template <bool STABLE, int COLS>
+__global__ __launch_bounds__(kRbThreads) void col_place_kernel(
+    const uint2* __restrict__ runs, const int4* __restrict__ desc, int tiles_x, int tiles_y,
+    int cap, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_first,
+    uint32_t* __restrict__ ids, int2* __restrict__ bins) {
+    constexpr int PER = round_per(STABLE);
+    __shared__ PlaceShared<uint32_t, COLS, STABLE ? (COLS == 128 ? 4096 : 3072) : 5120, STABLE> sh;
+    __shared__ int s_row0[kRowBinAxis];
+    __shared__ uint64_t s_tmp[kRbWaves];
+    const int tid = threadIdx.x;
+    const uint64_t pairs =
+        tid < tiles_y ? tile_first[(size_t)tid * (kRowBinAxis + 1) + kRowBinAxis] : 0u;
+    s_row0[tid] = (int)min(block_exclusive_scan256(pairs, s_tmp), (uint64_t)cap);
+    const int parts = uniform_i(desc[-1].x);
+    for_partitions(parts, [&](int p) {
+        const int4 d = desc[p];
+        Interval iv[kRbPer];
+        uint32_t id[kRbPer];
+#pragma unroll
+        for (int k = 0; k < kRbPer; ++k) {
+            const int i = d.y + interval_index<PER>(k);
+            const uint2 run = i < d.z ? runs[i] : make_uint2(0u, 0u);
+            id[k] = run.x;
+            iv[k] = {(int)(run.y & 0xFFFFu), (int)(run.y >> 16)};
+        }
+        clear_place(sh);
+        __syncthreads();
+        // (both terms at most cap < 2^30)
+        const int row0 = s_row0[d.x];
+        const int base = tid < tiles_x
+                             ? min(row0 + (int)counts[(size_t)p * kRowBinAxis + tid], cap)
+                             : 0;
+        if (d.w && tid < tiles_x) {
+            const uint32_t* tf = tile_first + (size_t)d.x * (kRowBinAxis + 1) + tid;
+            const int b = min(row0 + (int)tf[0], cap), e = min(row0 + (int)tf[1], cap);
+            if (e > b) bins[d.x * tiles_x + tid] = make_int2(b, e);
+        }
+        place_all<PER>(sh, iv, id, tiles_x, base, ids, cap);
+    });
+}
+
+// Tile id of every list entry (only where the caller asks for it).
+__global__ void tile_ids_kernel(const int2* __restrict__ bins, uint32_t* __restrict__ tiles) {
+    const int2 b = bins[blockIdx.x];
+    for (int i = b.x + (int)threadIdx.x; i < b.y; i += blockDim.x) tiles[i] = blockIdx.x;
+}
+
+constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
+
+}  // namespace
+
+RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap) {
+    RowBinPlan p{};
+    p.n = n;
+    p.tiles_x = tiles_x;
+    p.tiles_y = tiles_y;
+    p.cap = cap > 0 ? cap : 1;
+    p.parts = (n + kRbPart - 1) / kRbPart;
+    p.max_col_parts = p.cap / kRbPart + tiles_y;
+    size_t o = 0;
+    const size_t parts = (size_t)(p.parts > 0 ? p.parts : 1);
+    p.row_len = o; o = align256(o + 4ull * kRowBinAxis);
+    p.row_counts = o; o = align256(o + 4ull * kRowBinAxis * parts);
+    p.part_tot = o; o = align256(o + 4ull * parts);
+    p.tile_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * (size_t)kRowBinAxis);
+    p.desc = o; o = align256(o + 16ull * ((size_t)p.max_col_parts + 1));
+    p.col_counts = o; o = align256(o + 4ull * kRowBinAxis * (size_t)p.max_col_parts);
+    p.scratch_bytes = o;
+    return p;
+}
+
+hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects,
+                   uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
+                   int2* bins, unsigned long long* total, uint32_t* err, void* scratch,
+                   hipStream_t s) {
+    if (p.tiles_x > kRowBinAxis || p.tiles_y > kRowBinAxis || p.n <= 0)
+        return hipErrorInvalidValue;
+    uint8_t* b = static_cast<uint8_t*>(scratch);
+    auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
+    int4* desc = reinterpret_cast<int4*>(b + p.desc) + 1;
+    const int tiles = p.tiles_x * p.tiles_y;
+    hipError_t e;
+    row_count_kernel<<<p.parts, kRbThreads, 0, s>>>(p.n, perm, rects, p.tiles_x, p.tiles_y,
+                                                    p.parts, U(p.row_counts), U(p.part_tot),
+                                                    in_order, tiles, bins, err);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = column_scan(U(p.row_counts), p.parts, U(p.row_len), p.tiles_y, s)) != hipSuccess)
+        return e;
+#define JSA_ROW(ST, COLS)                                                                     \
+    row_place_kernel<ST, COLS><<<p.parts, kRbThreads, 0, s>>>(                                \
+        p.n, perm, perm ? in_order : rects, p.tiles_x, p.tiles_y, p.parts, U(p.row_counts),   \
+        U(p.row_len),                                                                         \
+        U(p.part_tot), runs, p.cap, total, err)
+    if (narrow(p.tiles_y)) {
+        if (perm) JSA_ROW(true, 128); else JSA_ROW(false, 128);
+    } else {
+        if (perm) JSA_ROW(true, 256); else JSA_ROW(false, 256);
+    }
+#undef JSA_ROW
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    stage_mark(kMarkEmitted, s);
+    // persistent: as many workgroups as fit the chip, or one per partition
+    const int most = 8 * ((p.max_col_parts + 7) / 8);
+    const int grid = most < 2048 ? most : 2048;
+    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_x, p.tiles_y, p.cap,
+                                                 U(p.col_counts), desc);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    col_scan_kernel<<<p.tiles_y, kRbThreads * kRbGroups, 0, s>>>(
+        U(p.row_len), p.tiles_x, p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+#define JSA_COL(ST, COLS)                                                                     \
+    col_place_kernel<ST, COLS><<<grid, kRbThreads, 0, s>>>(                                   \
+        runs, desc, p.tiles_x, p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first), ids, bins)
+    if (narrow(p.tiles_x)) {
+        if (perm) JSA_COL(true, 128); else JSA_COL(false, 128);
+    } else {
+        if (perm) JSA_COL(true, 256); else JSA_COL(false, 256);
+    }
+#undef JSA_COL
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    stage_mark(kMarkTileSorted, s);
+    if (tiles_sorted) {
+        tile_ids_kernel<<<tiles, 256, 0, s>>>(bins, tiles_sorted);
+        e = hipGetLastError();
+    }
+    return e;
+}
+
+}  // namespace jsa

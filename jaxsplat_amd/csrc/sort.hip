@@ -256,6 +256,12 @@ SortPlan sort_plan(int n_cap, int begin_bit, int end_bit) {
     return p;
 }
 
+hipError_t column_scan(uint32_t* counts, int parts, uint32_t* totals, int columns,
+                       hipStream_t s) {
+    radix_colscan<<<columns, kSortThreads, 0, s>>>(counts, parts, totals);
+    return hipGetLastError();
+}
+
 size_t sort_zero_bytes(const SortPlan& p) { return 0; }
 
 uint32_t* sort_first_counts(const SortPlan& p, void* scratch) {
