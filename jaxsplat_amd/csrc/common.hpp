@@ -360,16 +360,63 @@ __device__ __forceinline__ float wave_sums_split(float* v, int lane) {
     return val;
 }
 
+// The records of v's set bits (slot kb + bit), in order, added to (a0, a1,
+// a2): four at a time with their loads in flight together (a missing one reads
+// the zero record).
+template <bool ABS>
+__device__ __forceinline__ void add_records(uint64_t v, int kb, const float* __restrict__ rec,
+                                            float4& a0, float4& a1, float4& a2) {
+    while (v) {
+        int k[4];
+        bool ok[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            ok[i] = v != 0u;
+            k[i] = ok[i] ? kb + __ffsll((unsigned long long)v) - 1 : 0;
+            v &= v - 1u;
+        }
+        float4 r[4][3];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            load_record_from<ABS>(ok[i] ? record_at<ABS>(rec, (size_t)k[i]) : kZeroRecord,
+                                  r[i][0], r[i][1], r[i][2]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 q0 = r[i][0], q1 = r[i][1], q2 = r[i][2];
+            a0.x += q0.x; a0.y += q0.y; a0.z += q0.z; a0.w += q0.w;
+            a1.x += q1.x; a1.y += q1.y; a1.z += q1.z; a1.w += q1.w;
+            a2.x += q2.x;
+            if (ABS) {
+                a2.y += q2.y;
+                a2.z += q2.z;
+            }
+        }
+    }
+}
+
+// Flags of the slots [off, end) in the 64-slot window from bitmap word w (one
+// of the words that hold them).
+__device__ __forceinline__ uint64_t slot_window(const uint32_t* __restrict__ bits, int w, int off,
+                                                int end) {
+    const int w1 = (end - 1) >> 5;
+    const uint32_t lo = bits[w], hi = w < w1 ? bits[w + 1] : 0u;
+    uint64_t v = ((uint64_t)hi << 32) | lo;
+    const int first = off - (w << 5), past = end - (w << 5);       // in the window's bits
+    if (first > 0) v &= ~0ull << first;
+    if (past < 64) v &= (1ull << past) - 1ull;
+    return v;
+}
+
 // Sum of the flagged staged records of slots [off, end) (empty: off == end),
-// in slot order, into (a0, a1, a2) of the calling lane.  Ranges of at most 16
-// slots are summed by their own lane: the (at most two) bitmap words covering
-// the range as one mask (bits outside the range masked off), the set bits
-// taken four records at a time with their loads in flight together (a missing
-// one reads the zero record).  Longer ranges are summed one at a time
-// by the whole wave -- lane l takes slots off + l, off + l + 64, ... -- and
+// into (a0, a1, a2) of the calling lane.  Ranges of at most 16 slots are summed
+// by their own lane in slot order.  Longer ranges are summed one at a time by
+// the whole wave -- lane l takes slots off + l, off + l + 64, ... -- and
 // combined in a fixed tree (wave_sums_split), so that one large Gaussian does
 // not hold its wave for tens of rounds; the results stay independent of
-// scheduling.
+// scheduling.  A longer range of which at most two slots are flagged needs no
+// wave either: zeros change no sum, and two values have one order.  That is
+// most of them where tiles are opaque: the flags of the tiles behind stay
+// clear (3M large Gaussians at 1080p, 33 slots each: tail 300 -> 106 us, 610k with 11: 43 -> 31).
 // Called by every lane of the wave.
 template <bool ABS>
 __device__ __forceinline__ void sum_records(int off, int end, const float* __restrict__ rec,
@@ -380,46 +427,22 @@ __device__ __forceinline__ void sum_records(int off, int end, const float* __res
     // longer per-lane runs hold their wave, and each wave-wide range costs one
     // transposed wave reduction
     constexpr int kBig = 16;
-    const bool big = end - off > kBig;
+    // bitmap words that a lane counts by itself (wider ranges go to the wave)
+    constexpr int kWords = 16;
     const int cnt = end - off;
+    const int w0 = off >> 5, w1 = (end - 1) >> 5;
     static_assert(kBig <= 33, "a per-lane range spans at most two bitmap words");
-    if (cnt > 0 && !big) {
-        // the (at most two) bitmap words of the range as one 64-bit mask, so
-        // that four set bits of either word are taken per step
-        const int wfirst = off >> 5, wlast = (end - 1) >> 5;
-        const uint32_t lo_mask = ~0u << (off & 31);
-        const int hb = (end - 1) & 31;
-        const uint32_t hi_mask = hb == 31 ? ~0u : ((2u << hb) - 1u);
-        const uint32_t wa = bits[wfirst];
-        const uint32_t wb = wlast > wfirst ? bits[wlast] : 0u;
-        uint64_t v = wlast > wfirst ? ((uint64_t)(wb & hi_mask) << 32) | (wa & lo_mask)
-                                    : (uint64_t)(wa & lo_mask & hi_mask);
-        const int kb = wfirst << 5;
-        while (v) {
-            int k[4];
-            bool ok[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                ok[i] = v != 0u;
-                k[i] = ok[i] ? kb + __ffsll((unsigned long long)v) - 1 : 0;
-                v &= v - 1u;
-            }
-            float4 r[4][3];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                load_record_from<ABS>(ok[i] ? record_at<ABS>(rec, (size_t)k[i]) : kZeroRecord,
-                                      r[i][0], r[i][1], r[i][2]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 q0 = r[i][0], q1 = r[i][1], q2 = r[i][2];
-                a0.x += q0.x; a0.y += q0.y; a0.z += q0.z; a0.w += q0.w;
-                a1.x += q1.x; a1.y += q1.y; a1.z += q1.z; a1.w += q1.w;
-                a2.x += q2.x;
-                if (ABS) {
-                    a2.y += q2.y;
-                    a2.z += q2.z;
-                }
-            }
+    uint64_t v = 0;
+    bool big = cnt > kBig;
+    if (cnt > 0 && w1 - w0 < kWords) {
+        v = slot_window(bits, w0, off, end);
+        int flagged = __popcll(v);
+        for (int w = w0 + 2; w <= w1; w += 2) flagged += __popcll(slot_window(bits, w, off, end));
+        big = big && flagged > 2;
+        if (!big && flagged > 0) {
+            add_records<ABS>(v, w0 << 5, rec, a0, a1, a2);
+            for (int w = w0 + 2; w <= w1; w += 2)
+                add_records<ABS>(slot_window(bits, w, off, end), w << 5, rec, a0, a1, a2);
         }
     }
     uint64_t bigm = ballot(big);
