@@ -738,14 +738,14 @@ __device__ __forceinline__ void order_tile_run(int t, const int2* __restrict__ b
 }
 
 // One workgroup per tile (see above), mapped as the raster kernels map the
-// tiles (xcd_tile), so that each XCD orders a band of tiles whose ids its
-// raster workgroups then read through the same L2.
+// tiles (xcd_tile), so that each XCD orders the tiles whose ids its raster
+// workgroups then read through the same L2.
 __global__ __launch_bounds__(kSegThreads) void tile_depth_sort_kernel(
     const int2* __restrict__ bins, int num_bins, const uint32_t* __restrict__ dkeys,
     uint32_t* __restrict__ ids, uint32_t* __restrict__ ka, uint32_t* __restrict__ va,
     uint2* __restrict__ kv_tmp) {
     __shared__ SegShared sh;
-    const int t = xcd_tile(blockIdx.x, num_bins);
+    const int t = xcd_tile(blockIdx.x, kXcdChunkView);
     if (t < num_bins) order_tile_run(t, bins, dkeys, ids, ka, va, kv_tmp, sh);
 }
 
@@ -776,7 +776,7 @@ hipError_t tile_depth_order(const int2* bins, int num_bins, bool xcd, const uint
     // xcd_tile's grid, or two runs per workgroup (A/B at 6 waves per SIMD:
     // multi32 +7%, orbit64 -1% against one run per workgroup; 4 or 8 runs
     // cost orbit64's long runs more)
-    const int grid = xcd ? 8 * ((num_bins + 7) / 8) : (num_bins + 1) / 2;
+    const int grid = xcd ? xcd_grid(num_bins, kXcdChunkView) : (num_bins + 1) / 2;
     if (xcd)
         tile_depth_sort_kernel<<<grid, kSegThreads, 0, s>>>(bins, num_bins, dkeys, ids, ka, va,
                                                            kv_tmp);

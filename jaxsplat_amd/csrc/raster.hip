@@ -29,8 +29,8 @@
 //    with LDS float atomics and flushed with one set of global float atomics
 //    per (Gaussian, tile) instead of one per (Gaussian, wave);
 //  * the tile index is remapped so that each of the 8 XCDs (blocks are issued
-//    round-robin over XCDs) renders a contiguous band of tiles, keeping
-//    neighbouring tiles' Gaussians in the same L2.
+//    round-robin over XCDs) renders chunks of consecutive tiles (xcd_tile),
+//    keeping neighbouring tiles' Gaussians in the same L2.
 #include "common.hpp"
 
 namespace jsa {
@@ -50,6 +50,10 @@ inline int bwd_threads(int block_width, int slots) {
 }
 static_assert((kMaxTileThreads + 3) / 4 <= 64 && 128 / 2 <= 64,
               "one wave covers a tile at 4 (more than 128 pixels) or 2 pixels per lane");
+
+__host__ __device__ __forceinline__ int xcd_chunk(const RasterGrid& g) {
+    return g.views ? kXcdChunkBatch : kXcdChunkView;
+}
 
 constexpr float kTEps = 1e-4f;
 // The batches hold the conic scaled to base 2: (a, b, c) * (log2(e)/2,
@@ -466,7 +470,7 @@ __global__ __launch_bounds__(256) void raster_fwd_kernel(
     const float* __restrict__ colors, const float* __restrict__ opac,
     const float* __restrict__ bgs, float* __restrict__ final_Ts, int* __restrict__ final_idx,
     float* __restrict__ out_img) {
-    const int gt = xcd_tile(blockIdx.x, rg.total_tiles);
+    const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
     if (gt >= rg.total_tiles) return;
     raster_fwd_tile<DEPTH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
                            final_idx, out_img);
@@ -945,7 +949,7 @@ __global__ __launch_bounds__(64) void raster_bwd_kernel(
     const float* __restrict__ v_out_alpha, float* __restrict__ v_rgb,
     float* __restrict__ v_opacity, float* __restrict__ v_xy, float* __restrict__ v_xy_abs,
     float* __restrict__ v_conic, StagedOut st) {
-    const int gt = xcd_tile(blockIdx.x, rg.total_tiles);
+    const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
     if (gt >= rg.total_tiles) return;
     raster_bwd_tile<CONSISTENT, ABS, DEPTH, STAGED, NSLOT>(
         rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts, final_idx, v_out_img,
@@ -1080,8 +1084,6 @@ __global__ void raster_empty_kernel(size_t n_pix, int nch, const float* __restri
     }
 }
 
-int tile_grid(int total_tiles) { return 8 * ((total_tiles + 7) / 8); }
-
 // Workgroups of a persistent work-queue grid: the CUs times the workgroups of
 // `kernel` one CU holds at once (at most one per tile).
 template <typename K>
@@ -1192,7 +1194,7 @@ hipError_t raster_fwd_grid(const RasterGrid& g, const int* items_sorted, const i
     // default: the smallest batch depth that holds one entry per thread (a
     // 12- or 13-pixel tile has 192 threads: 256, two staging rounds)
     const int depth = g.fwd_depth > 0 ? g.fwd_depth : (nthr <= 64 ? 64 : nthr <= 128 ? 128 : 256);
-    const int grid = tile_grid(g.total_tiles);
+    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
     const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
     const float2* x2 = reinterpret_cast<const float2*>(xys);
     if (g.order) {
@@ -1263,7 +1265,7 @@ hipError_t raster_bwd_grid(const RasterGrid& g, const int* items_sorted, const i
     if (g.total_tiles <= 0) return hipSuccess;
     const int slots = bwd_slots(g.block_width);
     const int nthr = bwd_threads(g.block_width, slots);
-    const int grid = tile_grid(g.total_tiles);
+    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
     // 64 Gaussians per batch by default: the LDS partial sums (depth x 9..11 x 4
     // floats) otherwise limit the workgroups per CU (measured fastest on the
     // 1080p, 800x800 and mixed-size workloads)
@@ -1335,7 +1337,7 @@ hipError_t raster_bwd_staged(const Camera& c, int nch, const int* gids_sorted,
         g.splats = splats;
         const int slots = bwd_slots(g.block_width);
         const int nthr = bwd_threads(g.block_width, slots);
-        const int grid = tile_grid(g.total_tiles);
+        const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
         const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
         const float2* x2 = reinterpret_cast<const float2*>(xys);
 #define JSA_LAUNCH_S(CONS, ABS, S)                                                           \
@@ -1398,7 +1400,7 @@ hipError_t raster_bwd_batch_staged(const RasterGrid& g, int max_view_n, const in
     if (e != hipSuccess) return e;
     const int slots = bwd_slots(g.block_width);
     const int nthr = bwd_threads(g.block_width, slots);
-    const int grid = tile_grid(g.total_tiles);
+    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
     const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
     const float2* x2 = reinterpret_cast<const float2*>(xys);
     // work queue (g.order): a persistent grid takes the tiles in that order
