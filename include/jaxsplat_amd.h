@@ -372,6 +372,22 @@ int jaxsplat_rasterize_backward_staged_rects(
     float* v_colors, float* v_opacity, float* v_xy, float* v_xy_abs, float* v_conic, int adjoint,
     void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same for any number of channels (the reference's N-channel backward,
+ * lib/kernels/backward.cu:27-151), in passes of up to eight: a record holds a
+ * pass's channels and the six geometry sums.  tile_rects NULL: the slots follow
+ * the reference's rectangles of xys and radii. */
+size_t jaxsplat_rasterize_backward_staged_nd_workspace_size(const jaxsplat_descriptor* d,
+                                                            uint32_t num_intersects,
+                                                            uint32_t channels);
+int jaxsplat_rasterize_backward_staged_nd(
+    const jaxsplat_descriptor* d, const int32_t* gaussian_ids_sorted, const int32_t* tile_bins,
+    uint32_t num_intersects, const float* xys, const float* conics, const float* colors,
+    const float* opacities, const float* background, uint32_t channels, const int32_t* radii,
+    const uint32_t* tile_rects, const int32_t* cum_tiles_hit, const float* final_Ts,
+    const int32_t* final_idx, const float* v_out_img, const float* v_out_img_alpha,
+    float* v_colors, float* v_opacity, float* v_xy, float* v_conic, int adjoint, void* workspace,
+    size_t workspace_bytes, void* stream);
+
 /*
  * The fused render (no counterpart as one call in the reference, whose render,
  * jaxsplat/__init__.py:6-70, is project then rasterize): the projection with

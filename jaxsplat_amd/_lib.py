@@ -37,7 +37,9 @@ EXPORTS = (
     "jaxsplat_rasterize_backward_staged_workspace_size", "jaxsplat_rasterize_backward_staged",
     "jaxsplat_tile_rects_workspace_size", "jaxsplat_tile_rects", "jaxsplat_bin_depth_sort_rects",
     "jaxsplat_project_forward_rects",
-    "jaxsplat_rasterize_backward_staged_rects", "jaxsplat_render_backward",
+    "jaxsplat_rasterize_backward_staged_rects",
+    "jaxsplat_rasterize_backward_staged_nd_workspace_size",
+    "jaxsplat_rasterize_backward_staged_nd", "jaxsplat_render_backward",
     "jaxsplat_project_forward_splats", "jaxsplat_rasterize_forward_splats",
     "jaxsplat_rasterize_forward_binned", "jaxsplat_rasterize_backward_binned",
     "jaxsplat_rasterize_forward_nd", "jaxsplat_rasterize_backward_nd",
@@ -137,6 +139,9 @@ _SIGS = {
     "jaxsplat_rasterize_forward_splats": (I32, [DP, P, P, U32, P, P, U32, P, P, P, P]),
     "jaxsplat_rasterize_backward_staged": (I32, [DP, P, P, U32, P, P, P, P, P, U32, P, P, P, P, P,
                                                   P, P, P, P, P, P, I32, P, SZ, P]),
+    "jaxsplat_rasterize_backward_staged_nd_workspace_size": (SZ, [DP, U32, U32]),
+    "jaxsplat_rasterize_backward_staged_nd": (I32, [DP, P, P, U32, P, P, P, P, P, U32, P, P, P,
+                                                     P, P, P, P, P, P, P, P, I32, P, SZ, P]),
     "jaxsplat_rasterize_forward_binned": (I32, [DP, P, P, U32] + [P] * 8 + [P]),
     "jaxsplat_rasterize_backward_binned": (I32, [DP, P, P, U32] + [P] * 14 + [I32, P]),
     "jaxsplat_rasterize_forward_nd": (I32, [DP, P, P, U32] + [P] * 5 + [U32] + [P] * 3 + [P]),

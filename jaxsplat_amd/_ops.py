@@ -395,11 +395,18 @@ def _bin_rects(d, depths, rects, cum, dev, capacity=None):
 
 
 def staged_backward_applies(nch, isect):
-    """Whether the rasterize backward takes the staged entry point: up to
-    three channels and fewer than 2^30 intersections (its record slots are
-    31-bit); otherwise the atomic N-channel backward, which has neither limit
-    and differs only in the order of the float additions."""
+    """Whether the backward takes the staged entry points of up to three
+    channels: fewer than 2^30 intersections (record slots are 31-bit).  More
+    channels take the staged N-channel one (``_wide_backward_applies``);
+    otherwise the atomic N-channel backward, which has no limit and differs
+    only in the order of the float additions."""
     return STAGED_BACKWARD and 1 <= nch <= 3 and 0 <= isect <= STAGED_MAX_INTERSECTIONS
+
+
+def _wide_backward_applies(nch, isect):
+    """Whether the rasterize backward takes the staged N-channel entry point,
+    whose passes hold up to eight channels."""
+    return STAGED_BACKWARD and 3 < nch <= 4096 and 0 <= isect <= STAGED_MAX_INTERSECTIONS
 
 
 def _rasterize_forward(d, gids, bins, isect, xys, conics, colors, opacities, background,
@@ -423,12 +430,16 @@ def _rasterize_forward(d, gids, bins, isect, xys, conics, colors, opacities, bac
 
 def _staged_workspace(d, isect, nch, dev):
     """Workspace of the staged rasterize backward (records and bitmap), or
-    None where that backward does not apply or its 52 bytes per intersection
-    do not fit (the atomic backward is then used).  Returns (ws, bytes)."""
-    if not staged_backward_applies(nch, isect):
-        return None, 0
+    None where that backward does not apply or its bytes (52 per intersection,
+    60 beyond four channels) do not fit (the atomic backward is then used).
+    Returns (ws, bytes)."""
     L = _lib.lib()
-    wsb = L.jaxsplat_rasterize_backward_staged_workspace_size(ctypes.byref(d), isect)
+    if staged_backward_applies(nch, isect):
+        wsb = L.jaxsplat_rasterize_backward_staged_workspace_size(ctypes.byref(d), isect)
+    elif _wide_backward_applies(nch, isect):
+        wsb = L.jaxsplat_rasterize_backward_staged_nd_workspace_size(ctypes.byref(d), isect, nch)
+    else:
+        return None, 0
     try:
         return torch.empty(max(wsb, 1), dtype=torch.uint8, device=dev), wsb
     except torch.OutOfMemoryError:
@@ -452,7 +463,13 @@ def _rasterize_backward(d, isect, adjoint, colors, opacities, background, xys, c
     nch = colors.shape[1]
     ws, wsb = _staged_workspace(d, isect, nch, dev)
     with torch.cuda.device(dev):
-        if ws is not None and rects is not None:
+        if ws is not None and nch > 3:
+            _lib.check(L.jaxsplat_rasterize_backward_staged_nd(
+                ctypes.byref(d), _p(gids), _p(bins), isect, _p(xys), _p(conics), _p(colors),
+                _p(opacities), _p(background), nch, _p(radii), _p(rects), _p(cum_tiles_hit),
+                _p(final_Ts), _p(final_idx), _p(v_img), None, _p(v_colors), _p(v_opacity),
+                _p(v_xy), _p(v_conic), adjoint, _p(ws), wsb, _stream(dev)))
+        elif ws is not None and rects is not None:
             _lib.check(L.jaxsplat_rasterize_backward_staged_rects(
                 ctypes.byref(d), _p(gids), _p(bins), isect, _p(xys), _p(conics), _p(colors),
                 _p(opacities), _p(background), nch, _p(radii), _p(rects), _p(cum_tiles_hit),

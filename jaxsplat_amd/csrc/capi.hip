@@ -592,10 +592,10 @@ int jaxsplat_rasterize_forward_nd(const jaxsplat_descriptor* d,
         return fail(JAXSPLAT_ERR_INVALID, "rasterize_forward_nd: NULL required pointer");
     jsa::RasterGrid g = jsa::single_grid(c);
     g.ch_stride = (int)channels;
-    // channels in passes of up to three: the blend decisions are the same in every pass
-    for (int off = 0; off < (int)channels; off += 3) {
+    // channels in passes: the blend decisions are the same in every pass
+    for (int off = 0; off < (int)channels; off += g.ch_n) {
         g.ch_off = off;
-        g.ch_n = std::min(3, (int)channels - off);
+        g.ch_n = jsa::pass_channels((int)channels - off);
         JSA_CHECK_HIP(jsa::raster_fwd_grid(g, gaussian_ids_sorted, tile_bins, xys, conics, colors,
                                            opacities, background, final_Ts, final_idx, out_img,
                                            s),
@@ -694,6 +694,56 @@ int jaxsplat_rasterize_backward_staged(
                                          adjoint == JAXSPLAT_ADJOINT_CONSISTENT,
                                          static_cast<hipStream_t>(stream)),
                   "rasterize_backward_staged");
+    return JAXSPLAT_OK;
+}
+
+size_t jaxsplat_rasterize_backward_staged_nd_workspace_size(const jaxsplat_descriptor* d,
+                                                            uint32_t num_intersects,
+                                                            uint32_t channels) {
+    if (!d || validate(d) || channels < 1 || channels > 4096) return 0;
+    return align256(jsa::raster_bwd_staged_bytes((int)num_intersects, (int)channels));
+}
+
+int jaxsplat_rasterize_backward_staged_nd(
+    const jaxsplat_descriptor* d, const int32_t* gaussian_ids_sorted, const int32_t* tile_bins,
+    uint32_t num_intersects, const float* xys, const float* conics, const float* colors,
+    const float* opacities, const float* background, uint32_t channels, const int32_t* radii,
+    const uint32_t* tile_rects, const int32_t* cum_tiles_hit, const float* final_Ts,
+    const int32_t* final_idx, const float* v_out_img, const float* v_out_img_alpha,
+    float* v_colors, float* v_opacity, float* v_xy, float* v_conic, int adjoint, void* workspace,
+    size_t workspace_bytes, void* stream) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    if (channels < 1 || channels > 4096)
+        return fail(JAXSPLAT_ERR_INVALID, "channels must be in [1, 4096], got %u", channels);
+    if (num_intersects >= (1u << 30))
+        return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
+    if (adjoint != JAXSPLAT_ADJOINT_REFERENCE && adjoint != JAXSPLAT_ADJOINT_CONSISTENT)
+        return fail(JAXSPLAT_ERR_INVALID, "unknown adjoint mode %d", adjoint);
+    if (d->num_points == 0) return JAXSPLAT_OK;
+    if (!v_colors || !v_opacity || !v_xy || !v_conic)
+        return fail(JAXSPLAT_ERR_INVALID, "rasterize_backward_staged_nd: NULL gradient pointer");
+    if (!xys || !radii || !cum_tiles_hit ||
+        (num_intersects > 0 && (!gaussian_ids_sorted || !tile_bins || !conics || !colors ||
+                                !opacities || !background || !final_Ts || !final_idx ||
+                                !v_out_img)))
+        return fail(JAXSPLAT_ERR_INVALID, "rasterize_backward_staged_nd: NULL required pointer");
+    const size_t need =
+        align256(jsa::raster_bwd_staged_bytes((int)num_intersects, (int)channels));
+    if (!workspace || workspace_bytes < need)
+        return fail(JAXSPLAT_ERR_WORKSPACE,
+                    "rasterize_backward_staged_nd: workspace too small (%zu < %zu)",
+                    workspace_bytes, need);
+    JSA_CHECK_HIP(jsa::raster_bwd_staged(camera_of(d), (int)channels, gaussian_ids_sorted,
+                                         tile_bins, (int)num_intersects, xys, conics, colors,
+                                         opacities, background, final_Ts, final_idx, v_out_img,
+                                         v_out_img_alpha, radii,
+                                         reinterpret_cast<const uint2*>(tile_rects),
+                                         cum_tiles_hit, workspace, v_colors, v_opacity, v_xy,
+                                         nullptr, v_conic,
+                                         adjoint == JAXSPLAT_ADJOINT_CONSISTENT,
+                                         static_cast<hipStream_t>(stream)),
+                  "rasterize_backward_staged_nd");
     return JAXSPLAT_OK;
 }
 

@@ -257,62 +257,31 @@ __device__ __forceinline__ uint2 opacity_tile_rect(int bw, int tiles_x, int tile
 // Staged rasterize-backward records (raster.hip writes them; the reduction
 // kernels in raster.hip and project.hip sum them)
 // ---------------------------------------------------------------------------
-// A record holds one (Gaussian, tile) pair's sums at the pair's intersection
-// slot k: 9 floats at rec + 9 k, (rgb 3, conic 3, xy 2, opacity), or with the
-// v_xy_abs sums (ABS) 12 floats at rec + 12 k, (rgb 3, conic a), (conic b,
-// c, xy 2), (opacity, xy_abs 2, -).  bits holds one bit per slot, set when
-// the slot's record was written.  The workspace reserves 48 bytes per slot.
-template <bool ABS>
-__device__ __forceinline__ const float* record_at(const float* __restrict__ rec, size_t k) {
-    return rec + (ABS ? 12 : 9) * k;
-}
+// A record holds one (Gaussian, tile) pair's NV sums at the pair's intersection
+// slot k, floats at rec + record_stride(NV) k: the channels (three, or as many as
+// a wide channel pass holds), conic 3, xy 2, opacity, and after the three
+// channels' nine optionally xy_abs 2 (NV = kAbsValues, padded to 12 floats).  bits
+// holds one bit per slot, set when the slot's record was written.
+constexpr int kAbsValues = 11;
+constexpr int record_stride(int nv) { return nv == kAbsValues ? 12 : nv; }
 
-template <bool ABS>
-__device__ __forceinline__ void load_record_from(const float* __restrict__ q, float4& a0,
-                                                 float4& a1, float4& a2) {
-    if (ABS) {
-        const float4* q4 = reinterpret_cast<const float4*>(q);
-        a0 = q4[0];
-        a1 = q4[1];
-        a2 = q4[2];
-    } else {
-        a0 = make_float4(q[0], q[1], q[2], q[3]);
-        a1 = make_float4(q[4], q[5], q[6], q[7]);
-        a2 = make_float4(q[8], 0.f, 0.f, 0.f);
-    }
-}
-
-template <bool ABS>
-__device__ __forceinline__ void load_record(const float* __restrict__ rec, size_t k, float4& a0,
-                                            float4& a1, float4& a2) {
-    load_record_from<ABS>(record_at<ABS>(rec, k), a0, a1, a2);
+template <int NV>
+__device__ __forceinline__ void load_record(const float* __restrict__ q, float* r) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) r[i] = q[i];
 }
 
 // An all-zero record (zero-initialised, never written): the source of the
 // absent records' loads in sum_records, whose +0 terms leave a sum unchanged.
-static __device__ __align__(16) float kZeroRecord[12];
+static __device__ __align__(16) float kZeroRecord[16];
 
-template <bool ABS>
-__device__ __forceinline__ void store_record(float* __restrict__ rec, size_t k, float4 a0,
-                                             float4 a1, float4 a2) {
-    if (ABS) {
-        float4* q = reinterpret_cast<float4*>(rec) + 3 * k;
-        q[0] = a0;
-        q[1] = a1;
-        q[2] = a2;
-    } else {
-        float* q = rec + 9 * k;
-        q[0] = a0.x;
-        q[1] = a0.y;
-        q[2] = a0.z;
-        q[3] = a0.w;
-        q[4] = a1.x;
-        q[5] = a1.y;
-        q[6] = a1.z;
-        q[7] = a1.w;
-        q[8] = a2.x;
-    }
+template <int NV>
+__device__ __forceinline__ void store_record(float* __restrict__ rec, size_t k, const float* r) {
+    float* q = rec + record_stride(NV) * k;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) q[i] = r[i];
 }
+
 // Row (16-lane) sums of v[0..NV) by recursive halving.  At each DPP level
 // (partner lanes l^1, l^2, l+-4, l+-8 within the row: each flips one lane bit
 // and keeps the lower ones) the values are taken in pairs: a lane whose level
@@ -370,12 +339,12 @@ __device__ __forceinline__ float wave_sums_split(float* v, int lane) {
     return val;
 }
 
-// The records of v's set bits (slot kb + bit), in order, added to (a0, a1,
-// a2): four at a time with their loads in flight together (a missing one reads
-// the zero record).
-template <bool ABS>
+// The records of v's set bits (slot kb + bit), in order, added to acc: four at
+// a time with their loads in flight together (a missing one reads the zero
+// record).
+template <int NV>
 __device__ __forceinline__ void add_records(uint64_t v, int kb, const float* __restrict__ rec,
-                                            float4& a0, float4& a1, float4& a2) {
+                                            float* acc) {
     while (v) {
         int k[4];
         bool ok[4];
@@ -385,22 +354,14 @@ __device__ __forceinline__ void add_records(uint64_t v, int kb, const float* __r
             k[i] = ok[i] ? kb + __ffsll((unsigned long long)v) - 1 : 0;
             v &= v - 1u;
         }
-        float4 r[4][3];
+        float r[4][NV];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            load_record_from<ABS>(ok[i] ? record_at<ABS>(rec, (size_t)k[i]) : kZeroRecord,
-                                  r[i][0], r[i][1], r[i][2]);
+            load_record<NV>(ok[i] ? rec + record_stride(NV) * (size_t)k[i] : kZeroRecord, r[i]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 q0 = r[i][0], q1 = r[i][1], q2 = r[i][2];
-            a0.x += q0.x; a0.y += q0.y; a0.z += q0.z; a0.w += q0.w;
-            a1.x += q1.x; a1.y += q1.y; a1.z += q1.z; a1.w += q1.w;
-            a2.x += q2.x;
-            if (ABS) {
-                a2.y += q2.y;
-                a2.z += q2.z;
-            }
-        }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NV; ++j) acc[j] += r[i][j];
     }
 }
 
@@ -418,7 +379,7 @@ __device__ __forceinline__ uint64_t slot_window(const uint32_t* __restrict__ bit
 }
 
 // Sum of the flagged staged records of slots [off, end) (empty: off == end),
-// into (a0, a1, a2) of the calling lane.  Ranges of at most 16 slots are summed
+// into acc (zeros) of the calling lane.  Ranges of at most 16 slots are summed
 // by their own lane in slot order.  Longer ranges are summed one at a time by
 // the whole wave -- lane l takes slots off + l, off + l + 64, ... -- and
 // combined in a fixed tree (wave_sums_split), so that one large Gaussian does
@@ -428,10 +389,10 @@ __device__ __forceinline__ uint64_t slot_window(const uint32_t* __restrict__ bit
 // most of them where tiles are opaque: the flags of the tiles behind stay
 // clear (3M large Gaussians at 1080p, 33 slots each: tail 300 -> 106 us, 610k with 11: 43 -> 31).
 // Called by every lane of the wave.
-template <bool ABS>
+template <int NV>
 __device__ __forceinline__ void sum_records(int off, int end, const float* __restrict__ rec,
                                             const uint32_t* __restrict__ bits, int lane,
-                                            float4& a0, float4& a1, float4& a2) {
+                                            float* acc) {
     // 16: 56 us for the backward tail of 1M Gaussians at 1080p (24 the same,
     // 32: 60 us; 12: 62 us and 8: 92 us measured before the two-word mask):
     // longer per-lane runs hold their wave, and each wave-wide range costs one
@@ -441,7 +402,6 @@ __device__ __forceinline__ void sum_records(int off, int end, const float* __res
     constexpr int kWords = 16;
     const int cnt = end - off;
     const int w0 = off >> 5, w1 = (end - 1) >> 5;
-    static_assert(kBig <= 33, "a per-lane range spans at most two bitmap words");
     uint64_t v = 0;
     bool big = cnt > kBig;
     if (cnt > 0 && w1 - w0 < kWords) {
@@ -450,9 +410,9 @@ __device__ __forceinline__ void sum_records(int off, int end, const float* __res
         for (int w = w0 + 2; w <= w1; w += 2) flagged += __popcll(slot_window(bits, w, off, end));
         big = big && flagged > 2;
         if (!big && flagged > 0) {
-            add_records<ABS>(v, w0 << 5, rec, a0, a1, a2);
+            add_records<NV>(v, w0 << 5, rec, acc);
             for (int w = w0 + 2; w <= w1; w += 2)
-                add_records<ABS>(slot_window(bits, w, off, end), w << 5, rec, a0, a1, a2);
+                add_records<NV>(slot_window(bits, w, off, end), w << 5, rec, acc);
         }
     }
     uint64_t bigm = ballot(big);
@@ -461,31 +421,25 @@ __device__ __forceinline__ void sum_records(int off, int end, const float* __res
         bigm &= bigm - 1;
         const int boff = __builtin_amdgcn_readlane(off, src);
         const int bend = __builtin_amdgcn_readlane(end, src);
-        float4 b0 = make_float4(0.f, 0.f, 0.f, 0.f), b1 = b0, b2 = b0;
+        float b[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) b[i] = 0.f;
         for (int k = boff + lane; k < bend; k += 64) {
             if (!((bits[k >> 5] >> (k & 31)) & 1u)) continue;
-            float4 r0, r1, r2;
-            load_record<ABS>(rec, (size_t)k, r0, r1, r2);
-            b0.x += r0.x; b0.y += r0.y; b0.z += r0.z; b0.w += r0.w;
-            b1.x += r1.x; b1.y += r1.y; b1.z += r1.z; b1.w += r1.w;
-            b2.x += r2.x; b2.y += r2.y; b2.z += r2.z;
-        }
-        float v[11] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w, b2.x, b2.y, b2.z};
-        // lane j < NV ends with the wave sum of value j (xy_abs sums only with ABS)
-        constexpr int NV = ABS ? 11 : 9;
-        const float val = wave_sums_split<NV>(v, lane);
-        float t[11];
+            float r[NV];
+            load_record<NV>(rec + record_stride(NV) * (size_t)k, r);
 #pragma unroll
-        for (int i = 0; i < NV; ++i)
-            t[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), i));
-        if (lane == src) {
-            a0 = make_float4(t[0], t[1], t[2], t[3]);
-            a1 = make_float4(t[4], t[5], t[6], t[7]);
-            a2 = make_float4(t[8], ABS ? t[9] : 0.f, ABS ? t[10] : 0.f, 0.f);
+            for (int i = 0; i < NV; ++i) b[i] += r[i];
+        }
+        // lane j < NV ends with the wave sum of value j
+        const float val = wave_sums_split<NV>(b, lane);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(val), i));
+            if (lane == src) acc[i] = t;
         }
     }
 }
-
 
 // ---------------------------------------------------------------------------
 // Host-side internal interface (implemented in the .hip files)
@@ -533,8 +487,9 @@ struct RasterGrid {
     int n_items;          // sorted entries name items in [0, n_items)
     int fwd_depth;        // Gaussians staged per batch: 64, 128 or 256 (0: workgroup size)
     int bwd_depth;        // likewise for the backward (0: 64)
-    // channel pass: channels [ch_off, ch_off + ch_n) (ch_n <= 3) of colors,
-    // backgrounds, images and v_colors stored with ch_stride channels per row
+    // channel pass: channels [ch_off, ch_off + ch_n) (ch_n <= pass_channels) of
+    // colors, backgrounds, images and v_colors stored with ch_stride channels per
+    // row
     int ch_stride, ch_off, ch_n;
     // work queue (optional): a permutation of the tiles in the order a
     // persistent grid takes them, and two device counters (forward,
@@ -547,6 +502,13 @@ struct RasterGrid {
     // xys, opacities, conics, colours and rectangles separately
     const float4* splats;
 };
+
+// Channels of a rasterizer pass over the next `left` ones: up to eight (one pass
+// of 7 channels instead of three at 540 x 960 with 200k Gaussians: forward 228 ->
+// 85 us; backward 890 us with atomics -> 250 staged, and 16 for the sums).  Eight:
+// the records stay within the 16 lanes of a row sum, 116 VGPRs (four waves per
+// SIMD, three channels: 80 and six).
+inline int pass_channels(int left) { return left < 8 ? left : 8; }
 
 ViewRec single_view(const Camera& c);
 RasterGrid single_grid(const Camera& c);
@@ -780,9 +742,10 @@ hipError_t raster_fwd_grid(const RasterGrid& g, const int* items_sorted, const i
                            const float* opacities, const float* backgrounds, float* final_Ts,
                            int* final_idx, float* out_img, hipStream_t s);
 // Single-view backward with staged gradients instead of float atomics (see
-// StagedOut in raster.hip): nch <= 3 channels, workspace raster_bwd_staged_bytes;
-// radii and cum_tiles_hit are the projection's.  Writes every gradient row.
-size_t raster_bwd_staged_bytes(int num_isect);
+// StagedOut in raster.hip): nch channels in passes of up to eight (v_xy_abs and
+// splats: nch <= 3), workspace raster_bwd_staged_bytes; radii and cum_tiles_hit are the projection's.  Writes every gradient row.
+// Workspace for nch channels: records of the widest channel pass and bitmap.
+size_t raster_bwd_staged_bytes(int num_isect, int nch = 3);
 // rects (optional, packed as pack_rect) replaces the rectangles computed from
 // xys and radii (and must be the ones the binning used).  records_only: stop
 // after the records and their bitmap (in ws); render_bwd_tail sums them.

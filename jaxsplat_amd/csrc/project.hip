@@ -743,7 +743,7 @@ __global__ __launch_bounds__(256) void render_bwd_tail_kernel(
     const float4 q4 = reinterpret_cast<const float4*>(quats)[gi];
     const float cn[3] = {conics[3 * gi + 0], conics[3 * gi + 1], conics[3 * gi + 2]};
     const bool vis = own && rad > 0;
-    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0, a2 = a0;
+    float a[9] = {};        // rgb 3, conic 3, xy 2, opacity
     int off = 0, end = 0;
     if (vis) {
         int x0, x1, y0, y1;
@@ -752,13 +752,13 @@ __global__ __launch_bounds__(256) void render_bwd_tail_kernel(
         off = end - (x1 - x0) * (y1 - y0);
         if (off < 0 || end > num_isect) off = end = 0;     // inconsistent input: zeros
     }
-    sum_records<false>(off, end, rec, bits, lane, a0, a1, a2);
+    sum_records<9>(off, end, rec, bits, lane, a);
     if (!own) return;
     float* vcol = v_colors + (size_t)nch * idx;
-    vcol[0] = a0.x;
-    if (nch > 1) vcol[1] = a0.y;
-    if (nch > 2) vcol[2] = a0.z;
-    v_opacity[idx] = a2.x;
+    vcol[0] = a[0];
+    if (nch > 1) vcol[1] = a[1];
+    if (nch > 2) vcol[2] = a[2];
+    v_opacity[idx] = a[8];
     float vmean[3] = {0.f, 0.f, 0.f}, vsc[3] = {0.f, 0.f, 0.f}, vq[4] = {0.f, 0.f, 0.f, 0.f};
     if (vis) {                                                  // backward.cu:369-371
         M3 W;
@@ -767,8 +767,8 @@ __global__ __launch_bounds__(256) void render_bwd_tail_kernel(
         const float q[4] = {q4.x, q4.y, q4.z, q4.w};
         const CovParts cp = cov3d_parts(sc, q, c.glob_scale);
         float vc2[3], vc3[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        view_vjp(c, W, pt, m, cp.cov, cn[0], cn[1], cn[2], make_float2(a1.z, a1.w), 0.f, a0.w,
-                 a1.x, a1.y, false, 0.f, 0.f, consistent, vmean, vc2, vc3);
+        view_vjp(c, W, pt, m, cp.cov, cn[0], cn[1], cn[2], make_float2(a[6], a[7]), 0.f, a[3],
+                 a[4], a[5], false, 0.f, 0.f, consistent, vmean, vc2, vc3);
         cov3d_vjp(cp, q, c.glob_scale, vc3, vsc, vq);
     }
 #pragma unroll

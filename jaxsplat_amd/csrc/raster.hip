@@ -108,12 +108,24 @@ __device__ __forceinline__ ViewRec resolve_view(const RasterGrid& g, int gt) {
     return g.views[lo];
 }
 
-// Up to three channels (rg.ch_off .. + rg.ch_n) of row g of a (rows, ch_stride)
-// array; absent channels read as 0.  The default pass is all of an (N, 3) array.
+// The first three channels (rg.ch_off .. + rg.ch_n) of row g of a (rows,
+// ch_stride) array; absent channels read as 0.  The default pass is all of an
+// (N, 3) array.
 __device__ __forceinline__ float4 load_color(const RasterGrid& rg, const float* __restrict__ a,
                                              size_t g) {
     const float* p = a + (size_t)rg.ch_stride * g + rg.ch_off;
     return make_float4(p[0], rg.ch_n > 1 ? p[1] : 0.f, rg.ch_n > 2 ? p[2] : 0.f, 0.f);
+}
+
+// A wide channel pass (CH > 3 channels in one pass over the list: the blend and
+// its adjoint are evaluated once instead of once per three channels): channels
+// 3.. CH - 1 of the row.
+template <int CH>
+__device__ __forceinline__ void load_more(const RasterGrid& rg, const float* __restrict__ a,
+                                          size_t g, float* v) {
+    const float* p = a + (size_t)rg.ch_stride * g + rg.ch_off;
+#pragma unroll
+    for (int k = 3; k < CH; ++k) v[k - 3] = k < rg.ch_n ? p[k] : 0.f;
 }
 
 // One staged entry's inputs: from the splat records when the grid has them
@@ -279,7 +291,7 @@ __device__ __forceinline__ bool group_hit(const CullInfo& k, float4 r) {
 // Tile gt (< rg.total_tiles) of the grid's tile numbering, rendered by the
 // whole workgroup; the flat-grid kernel and the work-queue kernel below both
 // run this body.
-template <int DEPTH>
+template <int DEPTH, int CH>
 __device__ __forceinline__ void raster_fwd_tile(
     const RasterGrid& rg, int gt, const int* __restrict__ gids, const int2* __restrict__ bins,
     const float2* __restrict__ xys, const float* __restrict__ conics,
@@ -289,7 +301,8 @@ __device__ __forceinline__ void raster_fwd_tile(
     constexpr int NW = DEPTH / 64;            // 64-entry words per batch
     __shared__ float4 s_a[DEPTH];             // tile-centred x, y, opacity, id
     __shared__ float4 s_b[DEPTH];             // base-2 conic a', b', c', alpha_limit2(opacity)
-    __shared__ float4 s_c[DEPTH];             // colour
+    __shared__ float4 s_c[DEPTH];             // colour (channel 3: wide passes)
+    __shared__ float4 s_d[CH > 4 ? DEPTH : 1];    // channels 4..7
     __shared__ uint64_t s_mask[4][NW];        // [group][64-entry word]
     __shared__ float4 s_rect[4];
     __shared__ int s_rok[4];
@@ -333,6 +346,7 @@ __device__ __forceinline__ void raster_fwd_tile(
     // pixel terminates, then updates every lane unconditionally.
     float T = 1.f;
     float cr = 0.f, cg = 0.f, cb = 0.f;
+    float ce[CH > 3 ? CH - 3 : 1] = {};
     int cur = 0;
     uint64_t dm = ballot(!inside);
 
@@ -357,6 +371,13 @@ __device__ __forceinline__ void raster_fwd_tile(
                 s_b[e] = make_float4(sp.ca * kHalfLog2e, sp.cb * kLog2e, sp.cc * kHalfLog2e,
                                      sp.lim2);
                 s_c[e] = sp.col;
+                if constexpr (CH > 3) {
+                    float more[CH - 3];
+                    load_more<CH>(rg, colors, it + gshift, more);
+                    s_c[e].w = more[0];
+                    if constexpr (CH > 4)
+                        s_d[e] = make_float4(more[1], more[2], more[3], more[4]);
+                }
                 for (int G = 0; G < nwaves; ++G)
                     if (s_rok[G] && group_hit(ci, s_rect[G])) bits |= 1u << G;
             }
@@ -386,7 +407,8 @@ __device__ __forceinline__ void raster_fwd_tile(
             // byte offset 16 t is moved to a vector register once: it is the
             // LDS address of the three reads and the value that marks the
             // pixel's last blended entry (cur_off).
-            auto fetch = [&](int& t, int& toff, float4& a, float4& b, float4& c) -> bool {
+            auto fetch = [&](int& t, int& toff, float4& a, float4& b, float4& c,
+                             float4& d) -> bool {
                 const bool h = m != 0;
                 t = h ? q * 64 + __ffsll((unsigned long long)m) - 1 : t;
                 m &= m - 1;
@@ -394,10 +416,14 @@ __device__ __forceinline__ void raster_fwd_tile(
                 a = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_a) + toff);
                 b = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_b) + toff);
                 c = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_c) + toff);
+                if constexpr (CH > 4)
+                    d = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_d) +
+                                                         toff);
                 return h;
             };
             // one pair; true when every pixel of the wave is done
-            auto eval = [&](int toff, const float4& a, const float4& b, const float4& col) -> bool {
+            auto eval = [&](int toff, const float4& a, const float4& b, const float4& col,
+                            const float4& d) -> bool {
                 const float dx = a.x - px, dy = a.y - py;
                 const float s2 = sigma2(b, dx, dy);
                 const bool ok = pair_accepted(s2, b.w);
@@ -406,8 +432,10 @@ __device__ __forceinline__ void raster_fwd_tile(
                 const float alpha = fminf(0.999f, a.z * __builtin_amdgcn_exp2f(-s2));
                 const float al = lane_in(take) ? alpha : 0.f;
                 const float vis = al * T;
-                // T (1 - alpha) as T - alpha T, in place; exactly T where al = 0
-                T = T - vis;
+                // T (1 - alpha) as T - alpha T, in place; exactly T where al = 0 (the
+                // contractions are explicit: every pass of the channels must take
+                // the same decisions)
+                T = __builtin_fmaf(-T, al, T);
                 // a pixel with al = 0 keeps its T > 1e-4: fin is within take
                 const uint64_t fin = ballot(T <= kTEps);
                 uint64_t add = take;
@@ -421,24 +449,31 @@ __device__ __forceinline__ void raster_fwd_tile(
                     add = take & ~fin;
                     dm |= fin;
                 }
-                cr += col.x * v;
-                cg += col.y * v;
-                cb += col.z * v;
+                cr = __builtin_fmaf(col.x, v, cr);
+                cg = __builtin_fmaf(col.y, v, cg);
+                cb = __builtin_fmaf(col.z, v, cb);
+                if constexpr (CH > 3) ce[0] = __builtin_fmaf(col.w, v, ce[0]);
+                if constexpr (CH > 4) {
+                    ce[1] = __builtin_fmaf(d.x, v, ce[1]);
+                    ce[2] = __builtin_fmaf(d.y, v, ce[2]);
+                    ce[3] = __builtin_fmaf(d.z, v, ce[3]);
+                    ce[4] = __builtin_fmaf(d.w, v, ce[4]);
+                }
                 cur_off = lane_in(add) ? toff : cur_off;
                 return dm == ~0ull;
             };
             int t0 = 0, t1 = 0, o0, o1;
-            float4 a0, b0, c0, a1, b1, c1;
-            bool h0 = fetch(t0, o0, a0, b0, c0);
+            float4 a0, b0, c0, d0, a1, b1, c1, d1;
+            bool h0 = fetch(t0, o0, a0, b0, c0, d0);
             while (h0) {
-                const bool h1 = fetch(t1, o1, a1, b1, c1);
-                if (eval(o0, a0, b0, c0)) {
+                const bool h1 = fetch(t1, o1, a1, b1, c1, d1);
+                if (eval(o0, a0, b0, c0, d0)) {
                     live = false;
                     break;
                 }
                 if (!h1) break;
-                h0 = fetch(t0, o0, a0, b0, c0);
-                if (eval(o1, a1, b1, c1)) {
+                h0 = fetch(t0, o0, a0, b0, c0, d0);
+                if (eval(o1, a1, b1, c1, d1)) {
                     live = false;
                     break;
                 }
@@ -459,11 +494,18 @@ __device__ __forceinline__ void raster_fwd_tile(
         o[0] = cr + T * bg.x;
         if (rg.ch_n > 1) o[1] = cg + T * bg.y;
         if (rg.ch_n > 2) o[2] = cb + T * bg.z;
+        if constexpr (CH > 3) {
+            float more[CH - 3];
+            load_more<CH>(rg, bgs, vr.view, more);
+#pragma unroll
+            for (int k = 3; k < CH; ++k)
+                if (k < rg.ch_n) o[k] = ce[k - 3] + T * more[k - 3];
+        }
     }
 }
 
 // Flat grid: one workgroup per tile, XCD-aware tile order.
-template <int DEPTH>
+template <int DEPTH, int CH = 3>
 __global__ __launch_bounds__(256) void raster_fwd_kernel(
     RasterGrid rg, const int* __restrict__ gids, const int2* __restrict__ bins,
     const float2* __restrict__ xys, const float* __restrict__ conics,
@@ -472,8 +514,8 @@ __global__ __launch_bounds__(256) void raster_fwd_kernel(
     float* __restrict__ out_img) {
     const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
     if (gt >= rg.total_tiles) return;
-    raster_fwd_tile<DEPTH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
-                           final_idx, out_img);
+    raster_fwd_tile<DEPTH, CH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
+                               final_idx, out_img);
 }
 
 // Next item of a work queue, taken by one workgroup: order[i] for the i-th
@@ -503,14 +545,15 @@ __global__ __launch_bounds__(256) void raster_fwd_queue_kernel(
         const int gt = next_queue_item(counter, order, rg.total_tiles);
         if (gt == -1) return;
         if ((unsigned)gt >= (unsigned)rg.total_tiles) continue;   // never for a valid order
-        raster_fwd_tile<DEPTH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
-                               final_idx, out_img);
+        raster_fwd_tile<DEPTH, 3>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
+                                  final_idx, out_img);
     }
 }
 
 // ---------------------------------------------------------------------------
 // Backward: NSLOT pixels per lane (slots); 64-pixel groups = (slot, wave).
 // ---------------------------------------------------------------------------
+template <int CH>
 struct PixState {
     // px, py: pixel centre relative to the tile's centre corner (exact);
     // pxx, pxy, pyy: its products, the weights of the moment sums
@@ -524,12 +567,14 @@ struct PixState {
     float U, w;
     int fin;
     bool inside;
+    float vo_e[CH > 3 ? CH - 3 : 1];    // v_out of a wide pass's channels 3..
 };
 
 // One pixel's contribution to the per-Gaussian partial sums, branch-free
 // (an invalid pair contributes zeros and leaves the pixel state unchanged).
 // Only pixel-dependent sums are accumulated; the per-Gaussian factors are
 // applied once per (Gaussian, tile) by finish_grads:
+// (three channels; the CH of a wide pass shift the other sums along)
 //   g[0..2] = sum fac * v_out                       (v_rgb)
 //   g[3..5] = sum vs dx^2, vs dx dy, vs dy^2         (v_conic, x 0.5 / 1 / 0.5)
 //   g[6..7] = sum vs dx, vs dy                       (v_xy = conic * (sum vs d))
@@ -544,16 +589,17 @@ struct PixState {
 // with all 64 lanes active (the call sites branch on scalar mask bits only):
 // a lane masked off around the call would be missing from the ballots, and
 // its pairs from the per-Gaussian sums.
-template <bool CONSISTENT, int NV>
-__device__ __forceinline__ uint64_t bwd_pixel(PixState& s, float dx, float dy, float s2,
+template <bool CONSISTENT, int NV, int CH>
+__device__ __forceinline__ uint64_t bwd_pixel(PixState<CH>& s, float dx, float dy, float s2,
                                               const float4 a, const float4 b, const float4 col,
-                                              int k, float* g) {
+                                              const float* more, int k, float* g) {
 #define JSA_ACC(i, v) (g[i] += (v))
     constexpr float kClamp = CONSISTENT ? 0.999f : 0.99f;
     const float raw = a.z * __builtin_amdgcn_exp2f(-s2);
     // a pixel outside the image has fin = -1 (k >= 0), so live implies inside
     const bool live = k <= s.fin;
-    const bool acc = pair_accepted(s2, col.w);
+    // (a wide pass, whose colours fill col, keeps the limit beside the position)
+    const bool acc = pair_accepted(s2, CH > 3 ? a.w : col.w);
     const bool valid = live && acc;
     // an invalid pair acts as alpha = 0: U and w unchanged exactly, no weight
     const float rv = valid ? raw : 0.f;
@@ -565,9 +611,18 @@ __device__ __forceinline__ uint64_t bwd_pixel(PixState& s, float dx, float dy, f
     JSA_ACC(0, fac * s.vo_r);
     JSA_ACC(1, fac * s.vo_g);
     JSA_ACC(2, fac * s.vo_b);
+    if constexpr (CH > 3) {
+#pragma unroll
+        for (int c = 3; c < CH; ++c) JSA_ACC(c, fac * s.vo_e[c - 3]);
+    }
+    constexpr int C0 = CH;
     // v_alpha = sum_ch (col T - buf / (1 - alpha)) v_out
     //           + T_final (v_out_alpha - bg . v_out) / (1 - alpha) = T (cv - w)
-    const float cv = col.x * s.vo_r + col.y * s.vo_g + col.z * s.vo_b;
+    float cv = col.x * s.vo_r + col.y * s.vo_g + col.z * s.vo_b;
+    if constexpr (CH > 3) {
+#pragma unroll
+        for (int c = 3; c < CH; ++c) cv = __builtin_fmaf(more[c - 3], s.vo_e[c - 3], cv);
+    }
     const float dcw = cv - s.w;
     const float v_alpha = T * dcw;
     s.w = __builtin_fmaf(al, dcw, s.w);
@@ -586,11 +641,11 @@ __device__ __forceinline__ uint64_t bwd_pixel(PixState& s, float dx, float dy, f
     } else {
         // moments of vs over the pixel positions; finish_grads turns them
         // into the sums over the offsets (dx, dy) = Gaussian - pixel
-        JSA_ACC(3, vs * s.pxx);
-        JSA_ACC(4, vs * s.pxy);
-        JSA_ACC(5, vs * s.pyy);
-        JSA_ACC(6, vs * s.px);
-        JSA_ACC(7, vs * s.py);
+        JSA_ACC(C0 + 0, vs * s.pxx);
+        JSA_ACC(C0 + 1, vs * s.pxy);
+        JSA_ACC(C0 + 2, vs * s.pyy);
+        JSA_ACC(C0 + 3, vs * s.px);
+        JSA_ACC(C0 + 4, vs * s.py);
     }
     JSA_ACC(NV - 1, vs);
 #undef JSA_ACC
@@ -602,31 +657,32 @@ __device__ __forceinline__ uint64_t bwd_pixel(PixState& s, float dx, float dy, f
 // scaled conic and opacity o of the Gaussian): r[] becomes (v_rgb 3, v_conic 3,
 // v_xy 2, [v_xy_abs 2], v_opacity).  o > 0 whenever a pair was valid
 // (alpha >= 1/255).
-template <int NV>
+template <int NV, int CH>
 __device__ __forceinline__ void finish_grads(float* r, float4 conic2, float o, float gx,
                                              float gy) {
     constexpr float kInvLog2e = 1.f / kLog2e;
-    if (NV == 9) {
+    float* c = r + CH;          // conic 3, xy 2
+    if (NV != kAbsValues) {
         // moments -> offset sums, with (gx, gy) the tile-centred Gaussian
         // position: sum vs (gx - px) = gx S - Sx, sum vs (gx - px)^2 =
         // gx (gx S - 2 Sx) + Sxx, sum vs (gx - px)(gy - py) =
         // gx (gy S - Sy) - gy Sx + Sxy
-        const float S = r[NV - 1], Sx = r[6], Sy = r[7];
+        const float S = r[NV - 1], Sx = c[3], Sy = c[4];
         const float ex = fmaf(gx, S, -Sx), ey = fmaf(gy, S, -Sy);
-        r[3] = fmaf(gx, ex - Sx, r[3]);
-        r[4] = fmaf(gx, ey, fmaf(-gy, Sx, r[4]));
-        r[5] = fmaf(gy, ey - Sy, r[5]);
-        r[6] = ex;
-        r[7] = ey;
+        c[0] = fmaf(gx, ex - Sx, c[0]);
+        c[1] = fmaf(gx, ey, fmaf(-gy, Sx, c[1]));
+        c[2] = fmaf(gy, ey - Sy, c[2]);
+        c[3] = ex;
+        c[4] = ey;
     }
     const float ca = conic2.x * (2.f * kInvLog2e), cb = conic2.y * kInvLog2e,
                 cc = conic2.z * (2.f * kInvLog2e);
-    r[3] *= 0.5f;
-    r[5] *= 0.5f;
-    const float sp = r[6], sq = r[7];
-    r[6] = ca * sp + cb * sq;
-    r[7] = cb * sp + cc * sq;
-    if (NV == 11) {
+    c[0] *= 0.5f;
+    c[2] *= 0.5f;
+    const float sp = c[3], sq = c[4];
+    c[3] = ca * sp + cb * sq;
+    c[4] = cb * sp + cc * sq;
+    if (NV == kAbsValues) {
         r[8] *= kInvLog2e;
         r[9] *= kInvLog2e;
     }
@@ -639,7 +695,8 @@ __device__ __forceinline__ void finish_grads(float* r, float4 conic2, float o, f
 // intersection slot in the reference's emission order, cum_tiles_hit[g] -
 // num_tiles_hit[g] + the tile's row-major offset in g's tile rectangle, and
 // sets the slot's bit in a bitmap (one 32-bit atomic OR per flush, where the
-// direct path adds nine floats atomically); raster_bwd_reduce_kernel (or the
+// direct path adds nine floats atomically; a wide channel pass's records hold its
+// CH channels); raster_bwd_reduce_kernel (or the
 // fused render's tail) then sums each Gaussian's flagged records in slot
 // order, so the result does not depend on the order in which tiles finish.
 struct StagedOut {
@@ -654,7 +711,7 @@ struct StagedOut {
 
 // NSLOT pixels per lane (slots), so each (Gaussian, wave) reduction covers
 // 64 * NSLOT pixels; 64-pixel groups = (slot, wave).
-template <bool CONSISTENT, bool ABS, int DEPTH, bool STAGED, int NSLOT>
+template <bool CONSISTENT, bool ABS, int DEPTH, bool STAGED, int NSLOT, int CH>
 __device__ __forceinline__ void raster_bwd_tile(
     const RasterGrid& rg, int gt, const int* __restrict__ gids, const int2* __restrict__ bins,
     const float2* __restrict__ xys, const float* __restrict__ conics,
@@ -664,11 +721,13 @@ __device__ __forceinline__ void raster_bwd_tile(
     const float* __restrict__ v_out_alpha, float* __restrict__ v_rgb,
     float* __restrict__ v_opacity, float* __restrict__ v_xy, float* __restrict__ v_xy_abs,
     float* __restrict__ v_conic, const StagedOut& st) {
-    constexpr int NV = ABS ? 11 : 9;     // rgb3, conic3, xy2, [xy_abs2], opacity
+    static_assert(CH == 3 || (STAGED && !ABS), "wide channel passes: staged, without v_xy_abs");
+    constexpr int NV = ABS ? kAbsValues : CH + 6;   // channels, conic3, xy2, [xy_abs2], opacity
     constexpr int NW = DEPTH / 64;       // 64-entry words per batch
-    __shared__ float4 s_a[DEPTH];        // tile-centred x, y, opacity, id
+    __shared__ float4 s_a[DEPTH];        // tile-centred x, y, opacity, id (wide: limit)
     __shared__ float4 s_b[DEPTH];        // base-2 conic a', b', c', staged slot
-    __shared__ float4 s_c[DEPTH];        // colour, alpha_limit2(opacity)
+    __shared__ float4 s_c[DEPTH];        // colour, alpha_limit2(opacity) (wide: channel 3)
+    __shared__ float4 s_d[CH > 4 ? DEPTH : 1];      // channels 4..7
     // one wave per workgroup (bwd_threads: NSLOT pixels per lane cover the
     // tile in 64 lanes); its per-entry sums, kept until the batch's flush
     __shared__ float s_g[DEPTH][NV];
@@ -700,7 +759,10 @@ __device__ __forceinline__ void raster_bwd_tile(
     const float4 bg4 = load_color(rg, bgs, vr.view);
     const float bgr = bg4.x, bgg = bg4.y, bgb = bg4.z;
 
-    PixState ps[NSLOT];
+    float bg_more[CH > 3 ? CH - 3 : 1];
+    if constexpr (CH > 3) load_more<CH>(rg, bgs, vr.view, bg_more);
+
+    PixState<CH> ps[NSLOT];
     int slot_fin[NSLOT];                 // per slot: largest final index over the wave
 #pragma unroll
     for (int sl = 0; sl < NSLOT; ++sl) {
@@ -718,7 +780,7 @@ __device__ __forceinline__ void raster_bwd_tile(
         }
         const int i = y_org + r;
         const int j = x_org + c;
-        PixState& s = ps[sl];
+        PixState<CH>& s = ps[sl];
         s.inside = pixel && i < vr.img_h && j < vr.img_w;
         s.px = (float)(j - cx0) + 0.5f;
         s.py = (float)(i - cy0) + 0.5f;
@@ -738,6 +800,14 @@ __device__ __forceinline__ void raster_bwd_tile(
         const float vo_a = (s.inside && v_out_alpha) ? v_out_alpha[pix] : 0.f;
         // w = B / T_final with B's background term only
         s.w = (bgr * s.vo_r + bgg * s.vo_g + bgb * s.vo_b) - vo_a;
+        if constexpr (CH > 3) {
+            load_more<CH>(rg, v_out_img, pix, s.vo_e);
+#pragma unroll
+            for (int k = 0; k < CH - 3; ++k) {
+                if (!s.inside) s.vo_e[k] = 0.f;
+                s.w = __builtin_fmaf(bg_more[k], s.vo_e[k], s.w);
+            }
+        }
         slot_fin[sl] = uniform_i(wave_max_i(s.fin));
     }
     if (tid < ngroups) {
@@ -799,6 +869,14 @@ __device__ __forceinline__ void raster_bwd_tile(
                 const CullInfo ci = cull_info(sp.x, sp.y, sp.ca, sp.cb, sp.cc, sp.lim2);
                 float4 col = sp.col;
                 col.w = ci.lim2;                 // colour, acceptance limit
+                if constexpr (CH > 3) {
+                    float more[CH - 3];
+                    load_more<CH>(rg, colors, it + gshift, more);
+                    col.w = more[0];
+                    s_a[e].w = ci.lim2;
+                    if constexpr (CH > 4)
+                        s_d[e] = make_float4(more[1], more[2], more[3], more[4]);
+                }
                 s_c[e] = col;
                 for (int G = 0; G < ngroups; ++G)
                     if (s_rok[G] && group_hit(ci, s_rect[G])) bits |= 1u << G;
@@ -836,6 +914,15 @@ __device__ __forceinline__ void raster_bwd_tile(
                 const float4 a = s_a[t];
                 const float4 bb = s_b[t];
                 const float4 col = s_c[t];
+                float more[CH > 3 ? CH - 3 : 1];
+                if constexpr (CH > 3) more[0] = col.w;
+                if constexpr (CH > 4) {
+                    const float4 d = s_d[t];
+                    more[1] = d.x;
+                    more[2] = d.y;
+                    more[3] = d.z;
+                    more[4] = d.w;
+                }
                 float g[NV];
 #pragma unroll
                 // -0 + x is x exactly, so the first slot's sums need no add
@@ -858,13 +945,13 @@ __device__ __forceinline__ void raster_bwd_tile(
                             const float dy = a.y - ps[s0].py;
                             const float bdy = bb.y * dy, cdy = bb.z * dy;
                             if (h0)
-                                any |= bwd_pixel<CONSISTENT, NV>(
+                                any |= bwd_pixel<CONSISTENT, NV, CH>(
                                     ps[s0], dxa, dy, sigma2_terms(bb.x, dxa, bdy, cdy, dy), a,
-                                    bb, col, k, g);
+                                    bb, col, more, k, g);
                             if (h1)
-                                any |= bwd_pixel<CONSISTENT, NV>(
+                                any |= bwd_pixel<CONSISTENT, NV, CH>(
                                     ps[s0 + 1], dxb, dy, sigma2_terms(bb.x, dxb, bdy, cdy, dy),
-                                    a, bb, col, k, g);
+                                    a, bb, col, more, k, g);
                         }
                     }
                 }
@@ -873,8 +960,8 @@ __device__ __forceinline__ void raster_bwd_tile(
                     for (int sl = 0; sl < NSLOT; ++sl)
                         if ((ms[sl] >> b) & 1ull) {
                             const float dx = a.x - ps[sl].px, dy = a.y - ps[sl].py;
-                            any |= bwd_pixel<CONSISTENT, NV>(ps[sl], dx, dy, sigma2(bb, dx, dy),
-                                                             a, bb, col, k, g);
+                            any |= bwd_pixel<CONSISTENT, NV, CH>(
+                                ps[sl], dx, dy, sigma2(bb, dx, dy), a, bb, col, more, k, g);
                         }
                 }
                 if (any == 0) continue;
@@ -907,14 +994,17 @@ __device__ __forceinline__ void raster_bwd_tile(
                 s_g[e][v] = 0.f;
             }
             s_flag[e] = 0;
-            finish_grads<NV>(r, s_b[e], s_a[e].z, s_a[e].x, s_a[e].y);
+            finish_grads<NV, CH>(r, s_b[e], s_a[e].z, s_a[e].x, s_a[e].y);
             if (STAGED) {
                 const int slot = __float_as_int(s_b[e].w);
                 if (slot < 0) continue;
-                store_record<ABS>(st.rec, (size_t)slot, make_float4(r[0], r[1], r[2], r[3]),
-                                  make_float4(r[4], r[5], r[6], r[7]),
-                                  make_float4(r[NV - 1], ABS ? r[8] : 0.f, ABS ? r[9] : 0.f,
-                                              0.f));
+                if (ABS) {              // opacity before xy_abs
+                    const float op = r[NV - 1];
+                    r[10] = r[9];
+                    r[9] = r[8];
+                    r[8] = op;
+                }
+                store_record<NV>(st.rec, (size_t)slot, r);
                 atomicOr(&st.bits[slot >> 5], 1u << (slot & 31));
                 continue;
             }
@@ -939,7 +1029,7 @@ __device__ __forceinline__ void raster_bwd_tile(
     }
 }
 
-template <bool CONSISTENT, bool ABS, int DEPTH, bool STAGED, int NSLOT>
+template <bool CONSISTENT, bool ABS, int DEPTH, bool STAGED, int NSLOT, int CH = 3>
 __global__ __launch_bounds__(64) void raster_bwd_kernel(
     RasterGrid rg, const int* __restrict__ gids, const int2* __restrict__ bins,
     const float2* __restrict__ xys, const float* __restrict__ conics,
@@ -951,7 +1041,7 @@ __global__ __launch_bounds__(64) void raster_bwd_kernel(
     float* __restrict__ v_conic, StagedOut st) {
     const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
     if (gt >= rg.total_tiles) return;
-    raster_bwd_tile<CONSISTENT, ABS, DEPTH, STAGED, NSLOT>(
+    raster_bwd_tile<CONSISTENT, ABS, DEPTH, STAGED, NSLOT, CH>(
         rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts, final_idx, v_out_img,
         v_out_alpha, v_rgb, v_opacity, v_xy, v_xy_abs, v_conic, st);
 }
@@ -969,7 +1059,7 @@ __global__ __launch_bounds__(64) void raster_bwd_queue_kernel(
         const int gt = next_queue_item(counter, order, rg.total_tiles);
         if (gt == -1) return;
         if ((unsigned)gt >= (unsigned)rg.total_tiles) continue;   // never for a valid order
-        raster_bwd_tile<CONSISTENT, false, DEPTH, true, NSLOT>(
+        raster_bwd_tile<CONSISTENT, false, DEPTH, true, NSLOT, 3>(
             rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts, final_idx, v_out_img,
             nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, st);
     }
@@ -978,19 +1068,22 @@ __global__ __launch_bounds__(64) void raster_bwd_queue_kernel(
 // Per Gaussian: the sum of its flagged staged records, in slot order, as the
 // final gradients (every output row is written; a Gaussian with no flagged
 // record gets zeros).  num_isect bounds the slots (a radius or cum_tiles_hit
-// inconsistent with it yields zeros rather than an out-of-range read).
-template <bool ABS>
+// inconsistent with it yields zeros rather than an out-of-range read).  Channels
+// [ch_off, ch_off + ch_n) of nch; a later channel pass (ch_off > 0) adds to the
+// geometry's gradients, which are linear in the channels.
+template <bool ABS, int CH>
 __global__ __launch_bounds__(256) void raster_bwd_reduce_kernel(
     Camera c, int num_isect, const float2* __restrict__ xys, const int* __restrict__ radii,
     const uint2* __restrict__ rects, const int* __restrict__ cum, const float* __restrict__ rec,
-    const uint32_t* __restrict__ bits, int nch, float* __restrict__ v_rgb,
+    const uint32_t* __restrict__ bits, int nch, int ch_off, int ch_n, float* __restrict__ v_rgb,
     float* __restrict__ v_opacity, float* __restrict__ v_xy, float* __restrict__ v_xy_abs,
     float* __restrict__ v_conic) {
+    constexpr int NV = ABS ? kAbsValues : CH + 6;
     // no early exit: the wave-wide pass of sum_records needs every lane
     const int g = blockIdx.x * 256 + threadIdx.x;
     const int lane = lane_id();
     const bool own = g < c.num_points;
-    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0, a2 = a0;
+    float a[NV] = {};
     int off = 0, end = 0;
     if (own && radii[g] > 0) {
         int x0, x1, y0, y1;
@@ -1002,21 +1095,33 @@ __global__ __launch_bounds__(256) void raster_bwd_reduce_kernel(
         off = end - (x1 - x0) * (y1 - y0);
         if (off < 0 || end > num_isect) off = end = 0;     // inconsistent input: zeros
     }
-    sum_records<ABS>(off, end, rec, bits, lane, a0, a1, a2);
+    sum_records<NV>(off, end, rec, bits, lane, a);
     if (!own) return;
-    float* vc = v_rgb + (size_t)nch * g;
-    vc[0] = a0.x;
-    if (nch > 1) vc[1] = a0.y;
-    if (nch > 2) vc[2] = a0.z;
-    v_conic[3 * (size_t)g + 0] = a0.w;
-    v_conic[3 * (size_t)g + 1] = a1.x;
-    v_conic[3 * (size_t)g + 2] = a1.y;
-    v_xy[2 * (size_t)g + 0] = a1.z;
-    v_xy[2 * (size_t)g + 1] = a1.w;
-    v_opacity[g] = a2.x;
+    float* vc = v_rgb + (size_t)nch * g + ch_off;
+#pragma unroll
+    for (int k = 0; k < CH; ++k)
+        if (k < ch_n) vc[k] = a[k];
+    const float* q = a + CH;
+    float* vcn = v_conic + 3 * (size_t)g;
+    float* vxy = v_xy + 2 * (size_t)g;
+    if (ch_off > 0) {
+        vcn[0] += q[0];
+        vcn[1] += q[1];
+        vcn[2] += q[2];
+        vxy[0] += q[3];
+        vxy[1] += q[4];
+        v_opacity[g] += q[5];
+        return;
+    }
+    vcn[0] = q[0];
+    vcn[1] = q[1];
+    vcn[2] = q[2];
+    vxy[0] = q[3];
+    vxy[1] = q[4];
+    v_opacity[g] = q[5];
     if (ABS) {
-        v_xy_abs[2 * (size_t)g + 0] = a2.y;
-        v_xy_abs[2 * (size_t)g + 1] = a2.z;
+        v_xy_abs[2 * (size_t)g + 0] = a[9];
+        v_xy_abs[2 * (size_t)g + 1] = a[10];
     }
 }
 
@@ -1036,7 +1141,7 @@ __global__ __launch_bounds__(256) void raster_bwd_batch_reduce_kernel(
     const int lane = lane_id();
     const bool own = k < vr.n;
     const size_t it = (size_t)vr.item_off + (own ? k : 0);
-    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0, a2 = a0;
+    float a[9] = {};
     int off = 0, end = 0;
     if (own && radii[it] > 0) {
         const int cnt = (int)rect_count(item_rects[it]);
@@ -1048,14 +1153,14 @@ __global__ __launch_bounds__(256) void raster_bwd_batch_reduce_kernel(
             }
         }
     }
-    sum_records<false>(off, end, rec, bits, lane, a0, a1, a2);
+    sum_records<9>(off, end, rec, bits, lane, a);
     if (!own) return;
-    v_conic[3 * it + 0] = a0.w;
-    v_conic[3 * it + 1] = a1.x;
-    v_conic[3 * it + 2] = a1.y;
-    v_xy[2 * it + 0] = a1.z;
-    v_xy[2 * it + 1] = a1.w;
-    v_rgbo[it] = make_float4(a0.x, a0.y, a0.z, a2.x);
+    v_conic[3 * it + 0] = a[3];
+    v_conic[3 * it + 1] = a[4];
+    v_conic[3 * it + 2] = a[5];
+    v_xy[2 * it + 0] = a[6];
+    v_xy[2 * it + 1] = a[7];
+    v_rgbo[it] = make_float4(a[0], a[1], a[2], a[8]);
 }
 
 struct ZeroList {
@@ -1220,10 +1325,23 @@ hipError_t raster_fwd_grid(const RasterGrid& g, const int* items_sorted, const i
 #undef JSA_QUEUE
         return hipGetLastError();
     }
-#define JSA_LAUNCH(D)                                                                        \
-    raster_fwd_kernel<D><<<grid, nthr, 0, s>>>(g, items_sorted, b2, x2, conics, colors,     \
-                                               opacities, backgrounds, final_Ts, final_idx,  \
-                                               out_img)
+#define JSA_LAUNCH(...)                                                                      \
+    raster_fwd_kernel<__VA_ARGS__><<<grid, nthr, 0, s>>>(                                    \
+        g, items_sorted, b2, x2, conics, colors, opacities, backgrounds, final_Ts, final_idx, \
+        out_img)
+    if (g.ch_n > 3) {           // a wide pass (single view): one depth per tile size
+        if (g.splats || g.ch_n > 8) return hipErrorInvalidValue;
+        if (g.ch_n > 4) {
+            if (nthr <= 64) JSA_LAUNCH(64, 8);
+            else if (nthr <= 128) JSA_LAUNCH(128, 8);
+            else JSA_LAUNCH(256, 8);
+        } else {
+            if (nthr <= 64) JSA_LAUNCH(64, 4);
+            else if (nthr <= 128) JSA_LAUNCH(128, 4);
+            else JSA_LAUNCH(256, 4);
+        }
+        return hipGetLastError();
+    }
     switch (depth) {
         case 64: JSA_LAUNCH(64); break;
         case 128: JSA_LAUNCH(128); break;
@@ -1300,9 +1418,15 @@ hipError_t raster_bwd_grid(const RasterGrid& g, const int* items_sorted, const i
     return hipGetLastError();
 }
 
-size_t raster_bwd_staged_bytes(int num_isect) {
+// Floats of a staged record of nch channels (of the widest pass).
+static int record_floats(int nch) {
+    return nch <= 3 ? 12 : nch == 4 ? 10 : 14;      // (three channels: room for v_xy_abs)
+}
+
+size_t raster_bwd_staged_bytes(int num_isect, int nch) {
     const size_t n = (size_t)(num_isect > 0 ? num_isect : 1);
-    return ((48 * n + 255) & ~size_t(255)) + ((4 * ((n + 31) / 32) + 255) & ~size_t(255));
+    return ((4 * record_floats(nch) * n + 255) & ~size_t(255)) +
+           ((4 * ((n + 31) / 32) + 255) & ~size_t(255));
 }
 
 hipError_t raster_bwd_staged(const Camera& c, int nch, const int* gids_sorted,
@@ -1316,61 +1440,73 @@ hipError_t raster_bwd_staged(const Camera& c, int nch, const int* gids_sorted,
                              float* v_conic, int consistent, hipStream_t s, bool records_only,
                              const float4* splats) {
     if (c.num_points <= 0) return hipSuccess;
-    if (nch < 1 || nch > 3) return hipErrorInvalidValue;
+    if (nch < 1 || (nch > 3 && (v_xy_abs || records_only || splats)))
+        return hipErrorInvalidValue;
     uint8_t* w = static_cast<uint8_t*>(ws);
     const size_t n = (size_t)(num_isect > 0 ? num_isect : 1);
     StagedOut st;
     st.rec = reinterpret_cast<float*>(w);
-    st.bits = reinterpret_cast<uint32_t*>(w + ((48 * n + 255) & ~size_t(255)));
+    st.bits = reinterpret_cast<uint32_t*>(w + ((4 * record_floats(nch) * n + 255) & ~size_t(255)));
     st.cum = cum_tiles_hit;
     st.first = nullptr;
     st.rects = rects;
     st.radii = radii;
     st.n_slots = num_isect;
+    RasterGrid g = single_grid(c);
+    g.ch_stride = nch;
+    g.splats = splats;
+    const int slots = bwd_slots(g.block_width);
+    const int nthr = bwd_threads(g.block_width, slots);
+    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
+    const int blocks = (c.num_points + 255) / 256;
+    const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
+    const float2* x2 = reinterpret_cast<const float2*>(xys);
     hipError_t e = hipSuccess;
-    if (num_isect > 0) {
-        const size_t words = ((size_t)num_isect + 31) / 32;
-        if ((e = fill_zero(st.bits, 4 * words, s)) != hipSuccess) return e;
-        RasterGrid g = single_grid(c);
-        g.ch_stride = nch;
-        g.ch_n = nch;
-        g.splats = splats;
-        const int slots = bwd_slots(g.block_width);
-        const int nthr = bwd_threads(g.block_width, slots);
-        const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
-        const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
-        const float2* x2 = reinterpret_cast<const float2*>(xys);
-#define JSA_LAUNCH_S(CONS, ABS, S)                                                           \
-    raster_bwd_kernel<CONS, ABS, 64, true, S><<<grid, nthr, 0, s>>>(                        \
-        g, gids_sorted, b2, x2, conics, colors, opacities, background, final_Ts, final_idx,  \
-        v_out, v_out_alpha, nullptr, nullptr, nullptr, nullptr, nullptr, st)
-#define JSA_LAUNCH(CONS, ABS)                                                                \
+    // channel passes of up to eight (the alpha cotangent enters once)
+    for (int off = 0; off < nch; off += pass_channels(nch - off)) {
+        g.ch_off = off;
+        g.ch_n = pass_channels(nch - off);
+        if (num_isect > 0) {
+            const size_t words = ((size_t)num_isect + 31) / 32;
+            if ((e = fill_zero(st.bits, 4 * words, s)) != hipSuccess) return e;
+            const float* va = off == 0 ? v_out_alpha : nullptr;
+#define JSA_LAUNCH_C(CONS, ABS, CH)                                                          \
     do {                                                                                     \
-        if (slots == 4) JSA_LAUNCH_S(CONS, ABS, 4);                                          \
-        else JSA_LAUNCH_S(CONS, ABS, 2);                                                     \
+        if (slots == 4)                                                                      \
+            raster_bwd_kernel<CONS, ABS, 64, true, 4, CH><<<grid, nthr, 0, s>>>(             \
+                g, gids_sorted, b2, x2, conics, colors, opacities, background, final_Ts,     \
+                final_idx, v_out, va, nullptr, nullptr, nullptr, nullptr, nullptr, st);      \
+        else                                                                                 \
+            raster_bwd_kernel<CONS, ABS, 64, true, 2, CH><<<grid, nthr, 0, s>>>(             \
+                g, gids_sorted, b2, x2, conics, colors, opacities, background, final_Ts,     \
+                final_idx, v_out, va, nullptr, nullptr, nullptr, nullptr, nullptr, st);      \
     } while (0)
-        if (consistent) {
-            if (v_xy_abs) JSA_LAUNCH(true, true); else JSA_LAUNCH(true, false);
-        } else {
-            if (v_xy_abs) JSA_LAUNCH(false, true); else JSA_LAUNCH(false, false);
-        }
+#define JSA_LAUNCH(CONS)                                                                     \
+    do {                                                                                     \
+        if (g.ch_n > 4) JSA_LAUNCH_C(CONS, false, 8);                                        \
+        else if (g.ch_n > 3) JSA_LAUNCH_C(CONS, false, 4);                                   \
+        else if (v_xy_abs) JSA_LAUNCH_C(CONS, true, 3);                                      \
+        else JSA_LAUNCH_C(CONS, false, 3);                                                   \
+    } while (0)
+            if (consistent) JSA_LAUNCH(true); else JSA_LAUNCH(false);
 #undef JSA_LAUNCH
-#undef JSA_LAUNCH_S
+#undef JSA_LAUNCH_C
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        stage_mark(kMarkRecords, s);
+        if (records_only) return hipSuccess;
+#define JSA_REDUCE(ABS, CH)                                                                  \
+    raster_bwd_reduce_kernel<ABS, CH><<<blocks, 256, 0, s>>>(                                \
+        c, num_isect, x2, radii, rects, cum_tiles_hit, st.rec, st.bits, nch, off, g.ch_n,    \
+        v_colors, v_opacity, v_xy, v_xy_abs, v_conic)
+        if (g.ch_n > 4) JSA_REDUCE(false, 8);
+        else if (g.ch_n > 3) JSA_REDUCE(false, 4);
+        else if (v_xy_abs) JSA_REDUCE(true, 3);
+        else JSA_REDUCE(false, 3);
+#undef JSA_REDUCE
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    stage_mark(kMarkRecords, s);
-    if (records_only) return hipSuccess;
-    const int blocks = (c.num_points + 255) / 256;
-    const float2* x2 = reinterpret_cast<const float2*>(xys);
-    if (v_xy_abs)
-        raster_bwd_reduce_kernel<true><<<blocks, 256, 0, s>>>(
-            c, num_isect, x2, radii, rects, cum_tiles_hit, st.rec, st.bits, nch, v_colors,
-            v_opacity, v_xy, v_xy_abs, v_conic);
-    else
-        raster_bwd_reduce_kernel<false><<<blocks, 256, 0, s>>>(
-            c, num_isect, x2, radii, rects, cum_tiles_hit, st.rec, st.bits, nch, v_colors,
-            v_opacity, v_xy, nullptr, v_conic);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t raster_bwd_batch_staged(const RasterGrid& g, int max_view_n, const int* items_sorted,
