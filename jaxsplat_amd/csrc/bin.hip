@@ -485,15 +485,16 @@ __global__ __launch_bounds__(256) void tile_bins_kernel(const uint32_t* __restri
 // buckets instead; the order is exact whatever the distribution, only the
 // counting reads grow with the bucket sizes.
 //
-// One 256-thread workgroup per tile: runs of up to kSegCap entries are held
+// One 256-thread workgroup per tile: runs of up to seg_cap(256) entries are held
 // in registers and placed in LDS; longer ones go through global scratch at
-// the run's own offsets (L2-resident), with the bucket counts in LDS.
+// the run's own offsets (L2-resident), with the bucket counts in LDS.  Where the
+// lists are long on average these are left to a second launch of larger
+// workgroups, whose registers and LDS hold them (see tile_depth_order).
 constexpr int kSegThreads = 256;
-constexpr int kSegWaves = kSegThreads / kWave;
+constexpr int kSegThreadsLong = 512;                   // (1024: 2.2 times as long)
 constexpr int kSegItems = 6;                           // entries per lane
-constexpr int kSegCap = kSegThreads * kSegItems;       // 1536
-constexpr int kSegBucketBits = 11;
-constexpr int kSegBuckets = 1 << kSegBucketBits;
+constexpr int kSegBucketsPer = 8;                      // and buckets
+constexpr int seg_cap(int threads) { return threads * kSegItems; }      // 256: 1536
 
 // Unsigned min / max over the 64 lanes (full EXEC): DPP inside the rows,
 // then the four rows by readlane.
@@ -509,21 +510,24 @@ __device__ __forceinline__ uint32_t wave_extreme_u32(uint32_t v) {
               op((uint32_t)__builtin_amdgcn_readlane(a, 32), (uint32_t)__builtin_amdgcn_readlane(a, 48)));
 }
 
-// 20 KB, so that eight workgroups fit a CU.  red and tmp are used before the
-// entries are placed, so they share kv's space.
+// 20 KB per 256 threads, so that a CU is full of waves.  red and tmp are used
+// before the entries are placed, so they share kv's space.
+template <int THREADS>
 struct SegShared {
+    static constexpr int kWaves = THREADS / kWave;
+    static constexpr int kCap = seg_cap(THREADS);
+    static constexpr int kBuckets = kSegBucketsPer * THREADS;
     union {
-        uint2 kv[kSegCap];                          // placed (key, id)
+        uint2 kv[kCap];                             // placed (key, id)
         struct {
-            uint32_t red[4 * kSegWaves];
-            uint32_t tmp[kSegWaves];
+            uint32_t red[4 * kWaves];
+            uint32_t tmp[kWaves];
         };
     };
-    uint32_t cnt[kSegBuckets];                      // bucket counts / starts; then the ids
+    uint32_t cnt[kBuckets];                         // bucket counts / starts; then the ids
 };
-static_assert(kSegBuckets >= kSegCap, "the ids are staged in cnt");
-static_assert(sizeof(SegShared) <= 20480, "eight workgroups per CU");
-static_assert(kSegBuckets % kSegThreads == 0, "bucket scan: whole runs per thread");
+static_assert(kSegBucketsPer >= kSegItems, "the ids are staged in cnt");
+static_assert(sizeof(SegShared<256>) <= 20480, "eight workgroups per CU");
 
 // The run's composite bucketing: v = (key - kmin) << ib | (id - imin),
 // bucket = v >> shift.
@@ -538,8 +542,11 @@ struct Buckets {
 
 // Block min / max of the keys and ids (ids of a run of two or more entries
 // differ, so the composite range is never empty).  Ends with a barrier.
+template <int THREADS>
 __device__ __forceinline__ Buckets block_buckets(uint32_t kmin, uint32_t kmax, uint32_t imin,
-                                                 uint32_t imax, SegShared& sh) {
+                                                 uint32_t imax, SegShared<THREADS>& sh) {
+    constexpr int kSegWaves = SegShared<THREADS>::kWaves;
+    constexpr int kSegBucketBits = __builtin_ctz(SegShared<THREADS>::kBuckets);
     const int wave = threadIdx.x >> 6;
     kmin = wave_extreme_u32<false>(kmin);
     kmax = wave_extreme_u32<true>(kmax);
@@ -585,8 +592,9 @@ __device__ __forceinline__ uint32_t bucket_word(uint32_t b) {
 // Counts in sh.cnt[bucket_word(0..kSegBuckets)) -> exclusive starts (the last
 // bucket ends at the run's length).  Each thread scans a run of consecutive
 // buckets.  Ends with a barrier.
-__device__ __forceinline__ void bucket_scan(SegShared& sh) {
-    constexpr int per = kSegBuckets / kSegThreads;
+template <int THREADS>
+__device__ __forceinline__ void bucket_scan(SegShared<THREADS>& sh) {
+    constexpr int per = kSegBucketsPer;
     const int tid = threadIdx.x;
     const int b0 = tid * per;
     uint32_t c[per];
@@ -596,7 +604,7 @@ __device__ __forceinline__ void bucket_scan(SegShared& sh) {
         c[k] = sh.cnt[bucket_word(b0 + k)];
         sum += c[k];
     }
-    uint32_t run = block_exclusive_scan256(sum, sh.tmp);
+    uint32_t run = block_exclusive_scan<SegShared<THREADS>::kWaves>(sum, sh.tmp);
 #pragma unroll
     for (int k = 0; k < per; ++k) {
         sh.cnt[bucket_word(b0 + k)] = run;
@@ -606,8 +614,9 @@ __device__ __forceinline__ void bucket_scan(SegShared& sh) {
 }
 
 // End of bucket bk: the next bucket's start, or n for the last one.
-__device__ __forceinline__ uint32_t bucket_end(const SegShared& sh, uint32_t bk, int n) {
-    return bk + 1 < (uint32_t)kSegBuckets ? sh.cnt[bucket_word(bk + 1)] : (uint32_t)n;
+template <int THREADS>
+__device__ __forceinline__ uint32_t bucket_end(const SegShared<THREADS>& sh, uint32_t bk, int n) {
+    return bk + 1 < (uint32_t)SegShared<THREADS>::kBuckets ? sh.cnt[bucket_word(bk + 1)] : (uint32_t)n;
 }
 
 // (key, id) order of two entries.
@@ -624,13 +633,15 @@ __device__ __forceinline__ uint32_t bucket_rank(KV kv, uint32_t s, uint32_t c, u
     return rank;
 }
 
-// Runs of more than kSegCap entries: the same order through global scratch
+// Runs of more than seg_cap(THREADS) entries: the same order through global scratch
 // at the run's offsets: ka the keys, va the slots in the buckets, kv the
 // placed (key, id).  Every lane of the block calls it (barriers inside).
+template <int THREADS>
 __device__ void long_run_order(int base, int n, const uint32_t* __restrict__ dkeys,
                                uint32_t* __restrict__ ids, uint32_t* __restrict__ ka,
                                uint32_t* __restrict__ va, uint2* __restrict__ kv,
-                               SegShared& sh) {
+                               SegShared<THREADS>& sh) {
+    constexpr int kSegThreads = THREADS, kSegBuckets = SegShared<THREADS>::kBuckets;
     const int tid = threadIdx.x;
     uint32_t kmin = ~0u, kmax = 0u, imin = ~0u, imax = 0u;
     for (int e = tid; e < n; e += kSegThreads) {
@@ -664,18 +675,20 @@ __device__ void long_run_order(int base, int n, const uint32_t* __restrict__ dke
     }
 }
 
-// Orders run t (all lanes of the block; barriers inside).
-__device__ __forceinline__ void order_tile_run(int t, const int2* __restrict__ bins,
+// Orders run b of the ids (all lanes of the block; barriers inside).
+template <int THREADS>
+__device__ __forceinline__ void order_run(int2 b,
                                                const uint32_t* __restrict__ dkeys,
                                                uint32_t* __restrict__ ids,
                                                uint32_t* __restrict__ ka,
                                                uint32_t* __restrict__ va,
-                                               uint2* __restrict__ kv_tmp, SegShared& sh) {
-    const int2 b = bins[t];
+                                               uint2* __restrict__ kv_tmp,
+                                               SegShared<THREADS>& sh) {
+    constexpr int kSegThreads = THREADS, kSegBuckets = SegShared<THREADS>::kBuckets;
     const int n = b.y - b.x;
     if (n <= 1) return;                                 // uniform
-    if (n > kSegCap) {
-        long_run_order(b.x, n, dkeys, ids, ka, va, kv_tmp, sh);
+    if (n > seg_cap(THREADS)) {
+        long_run_order<THREADS>(b.x, n, dkeys, ids, ka, va, kv_tmp, sh);
         return;
     }
     const int tid = threadIdx.x;
@@ -739,50 +752,72 @@ __device__ __forceinline__ void order_tile_run(int t, const int2* __restrict__ b
 
 // One workgroup per tile (see above), mapped as the raster kernels map the
 // tiles (xcd_tile), so that each XCD orders the tiles whose ids its raster
-// workgroups then read through the same L2.
+// workgroups then read through the same L2.  Runs of more than `most` entries
+// are left for tile_depth_sort_long_kernel.
 __global__ __launch_bounds__(kSegThreads) void tile_depth_sort_kernel(
-    const int2* __restrict__ bins, int num_bins, const uint32_t* __restrict__ dkeys,
+    const int2* __restrict__ bins, int num_bins, int most, const uint32_t* __restrict__ dkeys,
     uint32_t* __restrict__ ids, uint32_t* __restrict__ ka, uint32_t* __restrict__ va,
     uint2* __restrict__ kv_tmp) {
-    __shared__ SegShared sh;
+    __shared__ SegShared<kSegThreads> sh;
     const int t = xcd_tile(blockIdx.x, kXcdChunkView);
-    if (t < num_bins) order_tile_run(t, bins, dkeys, ids, ka, va, kv_tmp, sh);
+    if (t >= num_bins) return;
+    const int2 b = bins[t];
+    if (b.y - b.x <= most) order_run(b, dkeys, ids, ka, va, kv_tmp, sh);
 }
 
-// A batch's bins (view << tile_bits | tile: many empty, many short): each
+// The runs of least .. most entries of a batch's bins (view << tile_bits | tile:
+// many empty, many short), or those that are long for 256 threads: each
 // workgroup takes the runs blockIdx.x, + gridDim.x, ..., so an empty one costs
 // a load rather than a workgroup.  At least 6 waves per SIMD (78 VGPRs; the
 // loop took 87 unbounded).
-__global__ __launch_bounds__(kSegThreads, 6) void tile_depth_sort_loop_kernel(
-    const int2* __restrict__ bins, int num_bins, const uint32_t* __restrict__ dkeys,
-    uint32_t* __restrict__ ids, uint32_t* __restrict__ ka, uint32_t* __restrict__ va,
-    uint2* __restrict__ kv_tmp) {
-    __shared__ SegShared sh;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS, 6) void tile_depth_sort_loop_kernel(
+    const int2* __restrict__ bins, int num_bins, int least, int most,
+    const uint32_t* __restrict__ dkeys, uint32_t* __restrict__ ids, uint32_t* __restrict__ ka,
+    uint32_t* __restrict__ va, uint2* __restrict__ kv_tmp) {
+    __shared__ SegShared<THREADS> sh;
     for (int t = blockIdx.x; t < num_bins; t += gridDim.x) {
-        order_tile_run(t, bins, dkeys, ids, ka, va, kv_tmp, sh);
+        const int2 b = bins[t];
+        if (b.y - b.x < least || b.y - b.x > most) continue;    // uniform
+        order_run(b, dkeys, ids, ka, va, kv_tmp, sh);
         __syncthreads();                                // LDS is reused by the next run
     }
 }
 
-// The per-tile depth order of every run of bins[0..num_bins).  ka, va: free
-// buffers of the intersection capacity; kv_tmp: a free one of twice that.
-// xcd: the bins are one view's tiles in the raster kernels' numbering (the
-// batch's bins, view << tile_bits | tile, are not: a band per XCD would also
-// be uneven there).
-hipError_t tile_depth_order(const int2* bins, int num_bins, bool xcd, const uint32_t* dkeys,
-                            uint32_t* ids, uint32_t* ka, uint32_t* va, uint2* kv_tmp,
-                            hipStream_t s) {
+// The per-tile depth order of every run of bins[0..num_bins), cap entries at
+// most.  ka, va: free buffers of the intersection capacity; kv_tmp: a free one
+// of twice that.  batch: the bins are view << tile_bits | tile, else one view's
+// tiles in the raster kernels' numbering.
+//
+// Runs of up to 1536 entries are bound by the gather of the keys and by LDS
+// latency, with eight workgroups per CU; a longer one in a 256-thread workgroup
+// goes through global scratch and holds its CU's other waves back.  12 views of
+// 500k Gaussians at 800 x 800 (26M pairs, 85% of them in runs of 1537 to 4467):
+// 422 us in one launch of 256 threads, 64 + 197 in two.  A view takes the second
+// launch where its average run (of the capacity) is long: it costs 7 us where
+// none is (1M Gaussians spread over 1080p, 808 pairs per tile: 46 us alone);
+// 500k Gaussians in half of an 800 x 800 image, 848 per tile: 53 us in one, 43
+// in two; 1M, 1700: 136 and 92; 1.5M, 2540: 239 and 166.
+hipError_t tile_depth_order(const int2* bins, int num_bins, int cap, bool batch,
+                            const uint32_t* dkeys, uint32_t* ids, uint32_t* ka, uint32_t* va,
+                            uint2* kv_tmp, hipStream_t s) {
     if (num_bins <= 0) return hipSuccess;
-    // xcd_tile's grid, or two runs per workgroup (A/B at 6 waves per SIMD:
-    // multi32 +7%, orbit64 -1% against one run per workgroup; 4 or 8 runs
-    // cost orbit64's long runs more)
-    const int grid = xcd ? xcd_grid(num_bins, kXcdChunkView) : (num_bins + 1) / 2;
-    if (xcd)
-        tile_depth_sort_kernel<<<grid, kSegThreads, 0, s>>>(bins, num_bins, dkeys, ids, ka, va,
-                                                           kv_tmp);
+    // two bins per workgroup (A/B at 6 waves per SIMD: multi32 +7%, orbit64 -1%
+    // against one; 4 or 8 cost orbit64's long runs more)
+    const int pairs = (num_bins + 1) / 2;
+    const int whole = seg_cap(kSegThreads);
+    const bool two = cap > whole && (batch || cap > whole * (long long)num_bins);
+    const int most = two ? whole : INT32_MAX;
+    if (batch)
+        tile_depth_sort_loop_kernel<kSegThreads><<<pairs, kSegThreads, 0, s>>>(
+            bins, num_bins, 0, most, dkeys, ids, ka, va, kv_tmp);
     else
-        tile_depth_sort_loop_kernel<<<grid, kSegThreads, 0, s>>>(bins, num_bins, dkeys, ids, ka,
-                                                                va, kv_tmp);
+        tile_depth_sort_kernel<<<xcd_grid(num_bins, kXcdChunkView), kSegThreads, 0, s>>>(
+            bins, num_bins, most, dkeys, ids, ka, va, kv_tmp);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !two) return e;
+    tile_depth_sort_loop_kernel<kSegThreadsLong><<<pairs, kSegThreadsLong, 0, s>>>(
+        bins, num_bins, whole + 1, INT32_MAX, dkeys, ids, ka, va, kv_tmp);
     return hipGetLastError();
 }
 
@@ -986,8 +1021,8 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
     stage_mark(kMarkBinned, s);
     if (p.by_depth) return hipSuccess;
     const size_t i4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
-    return tile_depth_order(bins, p.num_tiles, true, dkeys, ids, U(L.runs), U(L.runs + i4),
-                            reinterpret_cast<uint2*>(b + L.kv), s);
+    return tile_depth_order(bins, p.num_tiles, p.isect_cap, false, dkeys, ids, U(L.runs),
+                            U(L.runs + i4), reinterpret_cast<uint2*>(b + L.kv), s);
 }
 
 }  // namespace
@@ -995,7 +1030,7 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 // Pairs of the capacity per Gaussian from which the lists are ordered by one
 // depth sort of the Gaussians and stable placements, instead of tile by tile:
 // the depth sort costs 40 us + 36 us per 1M Gaussians, the order of the tiles
-// 7.6 us per 1M pairs in runs of up to kSegCap and several times that beyond.
+// 7.6 us per 1M pairs in runs of up to 1536 and several times that beyond.
 // Forward of 50k Gaussians with 100 pairs each at 900 x 1600: 232 us by depth,
 // 392 tile by tile; 610k Gaussians with 11 pairs each at 1080p: 664 against
 // 607 us (forward and backward).
@@ -1088,9 +1123,9 @@ hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
     stage_mark(kMarkBinned, s);
     // per-tile depth order; the emission's pair buffers and the sort's
     // ping-pong buffers (adjacent) are free again and serve the longer runs
-    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, true, dkeys,
-                            ids, U(L.tiles), U(L.gids), reinterpret_cast<uint2*>(b + L.ttmp_k),
-                            s);
+    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.isect_cap,
+                            false, dkeys, ids, U(L.tiles), U(L.gids),
+                            reinterpret_cast<uint2*>(b + L.ttmp_k), s);
 }
 
 // Binning of given tile rectangles with their inclusive counts (the render
@@ -1148,8 +1183,8 @@ hipError_t bin_rects(const BinPlan& p, const Camera& c, const float* depths,
                                                    reinterpret_cast<int2*>(tile_bins), err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     stage_mark(kMarkBinned, s);
-    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, true,
-                            reinterpret_cast<const uint32_t*>(depths), ids, U(L.tiles),
+    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.isect_cap,
+                            false, reinterpret_cast<const uint32_t*>(depths), ids, U(L.tiles),
                             U(L.gids), reinterpret_cast<uint2*>(b + L.ttmp_k), s);
 }
 
@@ -1269,7 +1304,7 @@ hipError_t batch_bin(const BatchBinPlan& p, const ViewRec* views, const uint2* i
     tile_bins_kernel<<<nb > 0 ? nb : 1, 256, 0, s>>>(U(L.keys_sorted), 0, count, p.num_bins,
                                                    reinterpret_cast<int2*>(tile_bins), err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_bins, false,
+    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_bins, p.isect_cap, true,
                             depth_keys, ids, U(L.keys), U(L.vals),
                             reinterpret_cast<uint2*>(b + L.ttmp_k), s);
 }

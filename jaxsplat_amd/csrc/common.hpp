@@ -158,10 +158,10 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, int bits, uint64_t v
     return peers;
 }
 
-// Exclusive scan of one value per thread over a 256-thread block (s_tmp: 4
-// words of LDS; two barriers).
-template <typename T>
-__device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
+// Exclusive scan of one value per thread over a block of WAVES waves (s_tmp: a
+// word of LDS per wave; two barriers).
+template <int WAVES, typename T>
+__device__ __forceinline__ T block_exclusive_scan(T v, T* s_tmp) {
     const int tid = threadIdx.x;
     const int lane = lane_id();
     const int wave = tid >> 6;
@@ -170,9 +170,13 @@ __device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
     __syncthreads();
     T off = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) off += (w < wave) ? s_tmp[w] : T(0);
+    for (int w = 0; w < WAVES; ++w) off += (w < wave) ? s_tmp[w] : T(0);
     __syncthreads();
     return off + incl - v;
+}
+template <typename T>
+__device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
+    return block_exclusive_scan<4>(v, s_tmp);
 }
 
 // Tile rectangle [x0, x1) x [y0, y1) of a Gaussian from its centre and integer
