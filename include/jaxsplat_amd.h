@@ -438,6 +438,60 @@ int jaxsplat_render_backward(
     const float* v_out_img, float* v_colors, float* v_opacity, float* v_mean3d, float* v_scale,
     float* v_quat, int adjoint, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * Host reads of a count (an inclusive count's last entry) without a copy or an
+ * event: jaxsplat_count_begin queues a kernel that writes *count with a ticket to
+ * a pinned word of the calling thread, and jaxsplat_count_wait (same thread)
+ * returns it as soon as it has arrived, whatever else the stream still holds.  A
+ * capturing stream is refused.
+ */
+int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream);
+int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, void* stream);
+
+/*
+ * The error word and the exact total of a binning's workspace (its first 16
+ * bytes) accumulated into *err (or) and *total (maximum), on the stream.
+ */
+int jaxsplat_bin_record(const void* workspace, int32_t* err, int64_t* total, void* stream);
+
+/*
+ * The fused render as two calls over two opaque buffers (16-byte aligned):
+ * render_begin is jaxsplat_project_forward_splats into `state`
+ * (jaxsplat_render_state_size bytes), and, with a ticket, jaxsplat_count_begin of
+ * the intersection count (jaxsplat_render_count waits for it); render_finish is
+ * jaxsplat_bin_rects_sort and jaxsplat_rasterize_forward_splats into `lists`
+ * (jaxsplat_render_lists_size bytes) and out_img, with bin_ws a workspace of
+ * jaxsplat_bin_emit_workspace_size bytes, and, with err, jaxsplat_bin_record.
+ * render_finish_backward is jaxsplat_render_backward over them.  render_layout
+ * gives the byte offsets of splats, conics, depths, radii, cum_tiles_hit and
+ * tile_rects in `state` and of gaussian_ids_sorted, tile_bins, final_Ts and
+ * final_idx in `lists`.
+ */
+size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d);
+size_t jaxsplat_render_lists_size(const jaxsplat_descriptor* d, uint32_t num_intersects);
+int jaxsplat_render_layout(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                           size_t* offsets);
+int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
+                          const float* scales, const float* quats, const float* viewmat,
+                          const float* opacities, const float* colors, uint32_t channels,
+                          void* state, size_t state_bytes, uint64_t* ticket, void* stream);
+int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint64_t ticket,
+                          int32_t* num_intersects, void* stream);
+int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                           const void* state, size_t state_bytes, const float* background,
+                           uint32_t channels, void* lists, size_t lists_bytes, void* bin_ws,
+                           size_t bin_ws_bytes, float* out_img, int32_t* err, int64_t* total,
+                           void* stream);
+int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                    const float* means3d, const float* scales,
+                                    const float* quats, const float* viewmat,
+                                    const void* state, size_t state_bytes, const void* lists,
+                                    size_t lists_bytes, const float* background,
+                                    uint32_t channels, const float* v_out_img,
+                                    float* v_colors, float* v_opacity, float* v_mean3d,
+                                    float* v_scale, float* v_quat, int adjoint,
+                                    void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Batched rendering: many views of one or more scenes in one pass.
  *

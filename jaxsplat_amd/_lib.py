@@ -40,6 +40,10 @@ EXPORTS = (
     "jaxsplat_rasterize_backward_staged_rects",
     "jaxsplat_rasterize_backward_staged_nd_workspace_size",
     "jaxsplat_rasterize_backward_staged_nd", "jaxsplat_render_backward",
+    "jaxsplat_count_begin", "jaxsplat_count_wait", "jaxsplat_bin_record",
+    "jaxsplat_render_state_size", "jaxsplat_render_lists_size", "jaxsplat_render_layout",
+    "jaxsplat_render_begin", "jaxsplat_render_count", "jaxsplat_render_finish",
+    "jaxsplat_render_finish_backward",
     "jaxsplat_project_forward_splats", "jaxsplat_rasterize_forward_splats",
     "jaxsplat_rasterize_forward_binned", "jaxsplat_rasterize_backward_binned",
     "jaxsplat_rasterize_forward_nd", "jaxsplat_rasterize_backward_nd",
@@ -99,6 +103,7 @@ _lib = None
 
 P = ctypes.c_void_p
 U32 = ctypes.c_uint32
+U64 = ctypes.c_uint64
 I32 = ctypes.c_int
 F32 = ctypes.c_float
 SZ = ctypes.c_size_t
@@ -135,6 +140,17 @@ _SIGS = {
                                                         P]),
     "jaxsplat_render_backward": (I32, [DP, P, P, U32] + [P] * 7 + [U32] + [P] * 11
                                  + [I32, P, SZ, P]),
+    "jaxsplat_count_begin": (I32, [P, ctypes.POINTER(U64), P]),
+    "jaxsplat_count_wait": (I32, [P, U64, ctypes.POINTER(ctypes.c_int32), P]),
+    "jaxsplat_bin_record": (I32, [P, P, P, P]),
+    "jaxsplat_render_state_size": (SZ, [DP]),
+    "jaxsplat_render_lists_size": (SZ, [DP, U32]),
+    "jaxsplat_render_layout": (I32, [DP, U32, ctypes.POINTER(SZ)]),
+    "jaxsplat_render_begin": (I32, [DP] + [P] * 6 + [U32, P, SZ, ctypes.POINTER(U64), P]),
+    "jaxsplat_render_count": (I32, [DP, P, U64, ctypes.POINTER(ctypes.c_int32), P]),
+    "jaxsplat_render_finish": (I32, [DP, U32, P, SZ, P, U32, P, SZ, P, SZ, P, P, P, P]),
+    "jaxsplat_render_finish_backward": (I32, [DP, U32, P, P, P, P, P, SZ, P, SZ, P, U32]
+                                        + [P] * 6 + [I32, P, SZ, P]),
     "jaxsplat_project_forward_splats": (I32, [DP] + [P] * 6 + [U32] + [P] * 9 + [P, SZ, P]),
     "jaxsplat_rasterize_forward_splats": (I32, [DP, P, P, U32, P, P, U32, P, P, P, P]),
     "jaxsplat_rasterize_backward_staged": (I32, [DP, P, P, U32, P, P, P, P, P, U32, P, P, P, P, P,

@@ -54,19 +54,40 @@ class ShapeDtypeError(AssertionError, TypeError):
 def _expect(name, t, shape, dtype):
     if not isinstance(t, torch.Tensor):
         raise ShapeDtypeError(f"{name}: expected a torch.Tensor, got {type(t).__name__}")
-    if tuple(t.shape) != tuple(shape) or t.dtype != dtype:
+    if t.shape != shape or t.dtype != dtype:
         raise ShapeDtypeError(
             f"{name}: expected shape {tuple(shape)} {dtype}, got {tuple(t.shape)} {t.dtype}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ShapeDtypeError(f"{name}: expected a GPU tensor, got device {t.device}")
 
 
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # (no Stream object: a fifth of the time, several times per call)
+    if device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+class _Here:
+    """A context that changes nothing."""
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on(dev):
+    """The device of a call's tensors made current, if it is not already."""
+    return _HERE if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
 
 
 def _adjoint(mode):
@@ -94,7 +115,7 @@ def _project_forward(d, means3d, scales, quats, viewmat, opacities=None):
     rects = torch.empty((N if opacities is not None else 0, 2), dtype=torch.int32, device=dev)
     ws_bytes = L.jaxsplat_project_workspace_size(ctypes.byref(d))
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         if opacities is not None:
             _lib.check(L.jaxsplat_project_forward_rects(
                 ctypes.byref(d), _p(means3d), _p(scales), _p(quats), _p(viewmat),
@@ -124,7 +145,7 @@ def _project_backward(d, adjoint, means3d, scales, quats, viewmat, radii, conics
     v_scale = torch.empty_like(scales)
     v_quat = torch.empty_like(quats)
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.jaxsplat_project_backward(
             ctypes.byref(d), _p(means3d), _p(scales), _p(quats), _p(viewmat),
             _p(radii), _p(conics), _p(comp), _p(v_xys), _p(v_depths), _p(v_conics),
@@ -227,7 +248,7 @@ def _bin(d, xys, depths, radii, isect, dev, return_tiles=False):
     bins = torch.empty((ntiles, 2), dtype=torch.int32, device=dev)
     ws_bytes = L.jaxsplat_bin_workspace_size(ctypes.byref(d), isect)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.jaxsplat_bin_and_sort(
             ctypes.byref(d), _p(xys), _p(depths), _p(radii), isect, _p(gids), _p(tiles),
             _p(bins), _p(ws), ws_bytes, _stream(dev)))
@@ -269,10 +290,17 @@ class IsectCapacity:
         self._total = torch.zeros(1, dtype=torch.int64, device=self.device)
         self.last_total = 0
 
+    def _words(self, dev):
+        """The accumulators' addresses, for a binning on dev."""
+        if self._err.device != dev:
+            raise RuntimeError(f"the capacity is on {self._err.device}, the render on {dev}")
+        return self._err.data_ptr(), self._total.data_ptr()
+
     def _record(self, ws):
         # emission workspace header: error word at byte 0, exact total (uint64) at byte 8
-        torch.bitwise_or(self._err, ws[0:4].view(torch.int32), out=self._err)
-        torch.maximum(self._total, ws[8:16].view(torch.int64), out=self._total)
+        with _on(ws.device):
+            _lib.check(_lib.lib().jaxsplat_bin_record(_p(ws), *self._words(ws.device),
+                                                      _stream(ws.device)))
 
     def check(self):
         """Largest intersection total since the last check (host sync);
@@ -310,38 +338,43 @@ def _emit(d, dws, isect, dev, capacity):
     return gids[:isect], bins, isect
 
 
-def _read_count(cum, dev):
-    """Queue a copy of the last inclusive count to pinned memory; returns
-    (host tensor, event) -- the caller waits on the event after queueing the
-    depth stage, so that the read overlaps it."""
-    count = torch.empty(1, dtype=torch.int32, pin_memory=True)
-    count.copy_(cum.reshape(-1)[-1:], non_blocking=True)
-    ready = torch.cuda.Event()
-    ready.record()
-    return count, ready
+def _begin_count(cum, dev):
+    """Queue the host read of the last inclusive count; returns what
+    ``_end_count`` waits for, so that what the caller queues in between overlaps
+    the read."""
+    ticket = ctypes.c_uint64()
+    last = cum.data_ptr() + 4 * (cum.numel() - 1)
+    _lib.check(_lib.lib().jaxsplat_count_begin(last, ctypes.byref(ticket), _stream(dev)))
+    return last, ticket
+
+
+def _end_count(read, dev):
+    last, ticket = read
+    count = ctypes.c_int32()
+    _lib.check(_lib.lib().jaxsplat_count_wait(last, ticket, ctypes.byref(count), _stream(dev)))
+    return count.value
 
 
 def _bin_overlapped(d, xys, depths, radii, cum_tiles_hit, dev, capacity=None):
     """Binning into the reference's tile rectangles.  By default the host read
     of num_intersects = cum_tiles_hit[N-1] (which sizes the outputs, as in the
-    reference) overlaps the depth stage: the count is copied to pinned memory
-    and the depth sort queued behind it before the host waits.  With a
+    reference) overlaps the depth stage, which is queued behind it before the
+    host waits.  With a
     capacity (IsectCapacity) nothing is read back.  Returns
     (gaussian_ids_sorted, tile_bins, isect)."""
     N = xys.shape[0]
     if N == 0:
         return _bin(d, xys, depths, radii, 0, dev)
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         if capacity is None:
-            count, ready = _read_count(cum_tiles_hit, dev)
+            read = _begin_count(cum_tiles_hit, dev)
         dws_bytes = L.jaxsplat_bin_depth_workspace_size(ctypes.byref(d))
         dws = torch.empty(max(dws_bytes, 1), dtype=torch.uint8, device=dev)
         _lib.check(L.jaxsplat_bin_depth_sort(ctypes.byref(d), _p(xys), _p(depths), _p(radii),
                                              _p(dws), dws_bytes, _stream(dev)))
         if capacity is None:
-            ready.synchronize()
-            isect = int(count[0])
+            isect = _end_count(read, dev)
         else:
             isect = capacity.capacity
         return _emit(d, dws, isect, dev, capacity)
@@ -358,7 +391,7 @@ def _bin_tight(d, xys, depths, radii, conics, opacities, dev, capacity=None):
     if N == 0:
         gids, bins, isect = _bin(d, xys, depths, radii, 0, dev)
         return gids, bins, isect, rects, cum
-    with torch.cuda.device(dev):
+    with _on(dev):
         rws_bytes = L.jaxsplat_tile_rects_workspace_size(ctypes.byref(d))
         rws = torch.empty(max(rws_bytes, 1), dtype=torch.uint8, device=dev)
         _lib.check(L.jaxsplat_tile_rects(ctypes.byref(d), _p(xys), _p(radii), _p(conics),
@@ -375,11 +408,9 @@ def _bin_rects(d, depths, rects, cum, dev, capacity=None):
     capacity) no read.  Returns (gaussian_ids_sorted, tile_bins, isect)."""
     L = _lib.lib()
     ntiles = d.grid_dim_2d.x * d.grid_dim_2d.y
-    with torch.cuda.device(dev):
+    with _on(dev):
         if capacity is None:
-            count, ready = _read_count(cum, dev)
-            ready.synchronize()
-            isect = int(count[0])
+            isect = _end_count(_begin_count(cum, dev), dev)
         else:
             isect = capacity.capacity
         gids = torch.empty(max(isect, 1), dtype=torch.int32, device=dev)
@@ -420,7 +451,7 @@ def _rasterize_forward(d, gids, bins, isect, xys, conics, colors, opacities, bac
     final_idx = torch.empty((H, W, 1), dtype=torch.int32, device=dev)
     img = torch.empty((H, W, nch), dtype=torch.float32, device=dev)
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.check(L.jaxsplat_rasterize_forward_nd(
             ctypes.byref(d), _p(gids), _p(bins), isect, _p(xys), _p(conics), _p(colors),
             _p(opacities), _p(background), nch, _p(final_Ts), _p(final_idx), _p(img),
@@ -462,7 +493,7 @@ def _rasterize_backward(d, isect, adjoint, colors, opacities, background, xys, c
     L = _lib.lib()
     nch = colors.shape[1]
     ws, wsb = _staged_workspace(d, isect, nch, dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         if ws is not None and nch > 3:
             _lib.check(L.jaxsplat_rasterize_backward_staged_nd(
                 ctypes.byref(d), _p(gids), _p(bins), isect, _p(xys), _p(conics), _p(colors),
@@ -554,55 +585,57 @@ class _Render(torch.autograd.Function):
         H, W = img_shape
         d = _lib.make_descriptor(N, img_shape, f, c, glob_scale, clip_thresh, block_width)
         L = _lib.lib()
-        # no xys or per-Gaussian counts: the splat records hold the positions
-        # and cum the counts
-        depths = torch.empty((N, 1), dtype=torch.float32, device=dev)
-        radii = torch.empty((N, 1), dtype=torch.int32, device=dev)
-        conics = torch.empty((N, 3), dtype=torch.float32, device=dev)
-        cum = torch.empty((N, 1), dtype=torch.int32, device=dev)
-        rects = torch.empty((N, 2), dtype=torch.int32, device=dev)
-        splats = torch.empty((N, 12), dtype=torch.float32, device=dev)
-        ws_bytes = L.jaxsplat_project_workspace_size(ctypes.byref(d))
-        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
-            _lib.check(L.jaxsplat_project_forward_splats(
-                ctypes.byref(d), _p(means3d), _p(scales), _p(quats), _p(viewmat),
-                _p(opacities), _p(colors), nch, None, _p(depths), _p(radii), _p(conics),
-                None, None, _p(cum), _p(rects), _p(splats), _p(ws), ws_bytes,
-                _stream(dev)))
-        if N == 0:
-            gids, bins, isect = _bin(d, splats[:, :2].contiguous(), depths, radii, 0, dev)
-        else:
-            gids, bins, isect = _bin_rects(d, depths, rects, cum, dev, capacity)
-        final_Ts = torch.empty((H, W, 1), dtype=torch.float32, device=dev)
-        final_idx = torch.empty((H, W, 1), dtype=torch.int32, device=dev)
-        img = torch.empty((H, W, nch), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
-            _lib.check(L.jaxsplat_rasterize_forward_splats(
-                ctypes.byref(d), _p(gids), _p(bins), isect, _p(splats), _p(background), nch,
-                _p(final_Ts), _p(final_idx), _p(img), _stream(dev)))
+        # two buffers that the C entries lay out, kept for the backward: the
+        # per-Gaussian state and the tiles' lists with the pixels' residuals
+        db = ctypes.byref(d)
+        state_bytes = L.jaxsplat_render_state_size(db)
+        state = torch.empty(state_bytes // 4, dtype=torch.int32, device=dev)
+        s = _stream(dev)
+        ticket = ctypes.c_uint64() if capacity is None else None
+        words = capacity._words(dev) if capacity is not None else (None, None)
+        with _on(dev):
+            _lib.check(L.jaxsplat_render_begin(
+                db, _p(means3d), _p(scales), _p(quats), _p(viewmat), _p(opacities), _p(colors),
+                nch, _p(state), state_bytes, ticket, s))
+            img = torch.empty((H, W, nch), dtype=torch.float32, device=dev)
+            if capacity is None:
+                count = ctypes.c_int32()
+                _lib.check(L.jaxsplat_render_count(db, _p(state), ticket, ctypes.byref(count), s))
+                isect = count.value
+            else:
+                isect = capacity.capacity if N else 0
+            lists_bytes = L.jaxsplat_render_lists_size(db, isect)
+            ws_bytes = L.jaxsplat_bin_emit_workspace_size(db, isect)
+            lists = torch.empty(lists_bytes // 4, dtype=torch.int32, device=dev)
+            ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
+            _lib.check(L.jaxsplat_render_finish(
+                db, isect, _p(state), state_bytes, _p(background), nch, _p(lists), lists_bytes,
+                _p(ws), ws_bytes, _p(img), *words, s))
         ctx.d = d
         ctx.isect = isect
         ctx.adjoint = adjoint
         ctx.save_for_backward(means3d, scales, quats, viewmat, colors, opacities, background,
-                              conics, radii, cum, rects, splats, gids, bins, final_Ts,
-                              final_idx)
+                              state, lists)
         return img
 
     @staticmethod
     def backward(ctx, v_img):
-        means3d, scales, quats, viewmat, colors, opacities, background, conics, radii, \
-            cum, rects, splats, gids, bins, final_Ts, final_idx = ctx.saved_tensors
+        means3d, scales, quats, viewmat, colors, opacities, background, state, lists = \
+            ctx.saved_tensors
+        d, isect = ctx.d, ctx.isect
         dev = means3d.device
         nch = colors.shape[1]
-        ws, wsb = _staged_workspace(ctx.d, ctx.isect, nch, dev)
+        state, lists = _aligned(state), _aligned(lists)
+        ws, wsb = _staged_workspace(d, isect, nch, dev)
         if ws is None:
-            xys = splats[:, :2].contiguous()
+            N = means3d.shape[0]
+            xys, conics, radii, cum, rects, gids, bins, final_Ts, final_idx = _render_views(
+                d, isect, N, state, lists)
             v_colors, v_opacity, v_xy, v_conic = _rasterize_backward(
-                ctx.d, ctx.isect, ctx.adjoint, colors, opacities, background, xys, conics, gids,
+                d, isect, ctx.adjoint, colors, opacities, background, xys, conics, gids,
                 bins, final_Ts, final_idx, radii, cum, rects, v_img)
             v_mean3d, v_scale, v_quat = _project_backward(
-                ctx.d, ctx.adjoint, means3d, scales, quats, viewmat, radii, conics, None, v_xy,
+                d, ctx.adjoint, means3d, scales, quats, viewmat, radii, conics, None, v_xy,
                 None, v_conic, None)
             return None, v_mean3d, v_scale, v_quat, v_colors, v_opacity, None, None, None
         v_img = v_img.contiguous()
@@ -611,15 +644,39 @@ class _Render(torch.autograd.Function):
         v_mean3d = torch.empty_like(means3d)
         v_scale = torch.empty_like(scales)
         v_quat = torch.empty_like(quats)
-        L = _lib.lib()
-        with torch.cuda.device(dev):
-            _lib.check(L.jaxsplat_render_backward(
-                ctypes.byref(ctx.d), _p(gids), _p(bins), ctx.isect, _p(means3d), _p(scales),
-                _p(quats), _p(viewmat), _p(splats), _p(conics), _p(background), nch, _p(radii),
-                _p(rects), _p(cum), _p(final_Ts), _p(final_idx), _p(v_img), _p(v_colors),
-                _p(v_opacity), _p(v_mean3d), _p(v_scale), _p(v_quat), ctx.adjoint, _p(ws), wsb,
-                _stream(dev)))
+        with _on(dev):
+            _lib.check(_lib.lib().jaxsplat_render_finish_backward(
+                ctypes.byref(d), isect, _p(means3d), _p(scales), _p(quats), _p(viewmat),
+                _p(state), 4 * state.numel(), _p(lists), 4 * lists.numel(), _p(background), nch,
+                _p(v_img), _p(v_colors), _p(v_opacity), _p(v_mean3d), _p(v_scale), _p(v_quat),
+                ctx.adjoint, _p(ws), wsb, _stream(dev)))
         return None, v_mean3d, v_scale, v_quat, v_colors, v_opacity, None, None, None
+
+
+def _aligned(buf):
+    """A buffer of the fused render as its C entries take it (a saved-tensor
+    hook may hand back a view of something larger)."""
+    return buf if buf.is_contiguous() and buf.data_ptr() % 16 == 0 else \
+        buf.clone(memory_format=torch.contiguous_format)
+
+
+def _render_views(d, isect, N, state, lists):
+    """The arrays in the fused render's buffers: (xys, conics, radii, cum,
+    rects, gids, bins, final_Ts, final_idx)."""
+    off = (ctypes.c_size_t * 10)()
+    _lib.check(_lib.lib().jaxsplat_render_layout(ctypes.byref(d), isect, off))
+
+    def part(buf, i, rows, cols, dtype=torch.int32):
+        a = off[i] // 4
+        return buf[a:a + rows * cols].view(dtype).view(rows, cols)
+
+    f32 = torch.float32
+    T = d.grid_dim_2d.x * d.grid_dim_2d.y
+    pixels = d.img_shape.x * d.img_shape.y
+    xys = part(state, 0, N, 12, f32)[:, :2].contiguous()
+    return (xys, part(state, 1, N, 3, f32), part(state, 3, N, 1), part(state, 4, N, 1),
+            part(state, 5, N, 2), part(lists, 6, isect, 1), part(lists, 7, T, 2),
+            part(lists, 8, pixels, 1, f32), part(lists, 9, pixels, 1))
 
 
 def render_fused(means3d, scales, quats, colors, opacities, *, viewmat, background, img_shape, f,

@@ -2,7 +2,10 @@
 // include/jaxsplat_amd.h): argument validation, descriptor -> camera
 // conversion, workspace carving, and the four reference-compatible XLA
 // custom-call targets.
+#include <unistd.h>
+
 #include <algorithm>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -823,6 +826,283 @@ int jaxsplat_rasterize_forward_splats(const jaxsplat_descriptor* d,
                                          final_Ts, final_idx, out_img, s),
                   "rasterize_forward_splats");
     return JAXSPLAT_OK;
+}
+
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// Counts read by the host
+// ---------------------------------------------------------------------------
+namespace {
+
+// A pinned, coherent word of a thread: (ticket << 32 | count).  The GPU idles
+// from the count until the launches that need it arrive, so what counts is the
+// time from the store to the next launch.  This read and the two-call render
+// below, in place of a copy to pinned memory with an event, and nine allocations
+// and a call less: 105 -> 59 us per view of 2k Gaussians at 256 x 256 (bound by
+// the host), 658 -> 637 us per step of 1M at 1080p (bound by the kernels).  The
+// ticket tells a late store of an abandoned read from the awaited one; the word
+// is given back with its thread.
+struct CountWord {
+    uint64_t* host = nullptr;
+    uint64_t* dev = nullptr;
+    uint32_t ticket = 0;
+    pid_t pid = 0;
+    ~CountWord() {
+        if (host && pid == getpid()) (void)hipHostFree(host);
+    }
+};
+thread_local CountWord t_count;
+
+__global__ void count_kernel(const int32_t* __restrict__ count, uint64_t* __restrict__ out,
+                             uint32_t ticket) {
+    __hip_atomic_store(out, (uint64_t)ticket << 32 | (uint32_t)*count, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void bin_record_kernel(const uint32_t* __restrict__ header, int32_t* __restrict__ err,
+                                  long long* __restrict__ total) {
+    *err |= (int32_t)header[0];
+    const long long t = (long long)((uint64_t)header[2] | (uint64_t)header[3] << 32);
+    *total = *total > t ? *total : t;
+}
+
+}  // namespace
+
+extern "C" {
+
+int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream) {
+    g_err.clear();
+    if (!count || !ticket) return fail(JAXSPLAT_ERR_INVALID, "count_begin: NULL required pointer");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    JSA_CHECK_HIP(hipStreamIsCapturing(s, &capturing), "count_begin");
+    if (capturing != hipStreamCaptureStatusNone)
+        return fail(JAXSPLAT_ERR_INVALID,
+                    "a count cannot be read while its stream is capturing (give a capacity)");
+    CountWord& w = t_count;
+    if (!w.host) {
+        void *h = nullptr, *p = nullptr;
+        JSA_CHECK_HIP(hipHostMalloc(&h, 64, hipHostMallocCoherent | hipHostMallocMapped |
+                                                hipHostMallocPortable),
+                      "count_begin");
+        if (hipHostGetDevicePointer(&p, h, 0) != hipSuccess) {
+            (void)hipHostFree(h);
+            return fail(JAXSPLAT_ERR_HIP, "count_begin: no device pointer of pinned memory");
+        }
+        w.host = static_cast<uint64_t*>(h);
+        w.dev = static_cast<uint64_t*>(p);
+        w.pid = getpid();
+        *w.host = 0;
+    }
+    if (++w.ticket == 0) w.ticket = 1;
+    count_kernel<<<1, 1, 0, s>>>(count, w.dev, w.ticket);
+    JSA_CHECK_HIP(hipGetLastError(), "count_begin");
+    *ticket = w.ticket;
+    return JAXSPLAT_OK;
+}
+
+int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, void* stream) {
+    g_err.clear();
+    if (!count || !value) return fail(JAXSPLAT_ERR_INVALID, "count_wait: NULL required pointer");
+    const CountWord& w = t_count;
+    if (!w.host || ticket != w.ticket)
+        return fail(JAXSPLAT_ERR_INVALID, "count_wait: not this thread's last ticket");
+    auto arrived = [&]() {
+        const uint64_t v = __atomic_load_n(w.host, __ATOMIC_ACQUIRE);
+        if ((uint32_t)(v >> 32) != (uint32_t)ticket) return false;
+        *value = (int32_t)(uint32_t)v;
+        return true;
+    };
+    // polled for 2 ms; a stream with more than that before the count is waited for
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    for (unsigned i = 0; (i & 63u) != 63u || std::chrono::steady_clock::now() < until; ++i) {
+        if (arrived()) return JAXSPLAT_OK;
+        __builtin_ia32_pause();
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    JSA_CHECK_HIP(hipStreamSynchronize(s), "count_wait");
+    if (arrived()) return JAXSPLAT_OK;
+    JSA_CHECK_HIP(hipMemcpyAsync(value, count, 4, hipMemcpyDeviceToHost, s), "count_wait");
+    JSA_CHECK_HIP(hipStreamSynchronize(s), "count_wait");
+    return JAXSPLAT_OK;
+}
+
+int jaxsplat_bin_record(const void* workspace, int32_t* err, int64_t* total, void* stream) {
+    g_err.clear();
+    if (!workspace || !err || !total)
+        return fail(JAXSPLAT_ERR_INVALID, "bin_record: NULL required pointer");
+    bin_record_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const uint32_t*>(workspace), err, reinterpret_cast<long long*>(total));
+    JSA_CHECK_HIP(hipGetLastError(), "bin_record");
+    return JAXSPLAT_OK;
+}
+
+}  // extern "C"
+
+// ---------------------------------------------------------------------------
+// The fused render over two buffers
+// ---------------------------------------------------------------------------
+namespace {
+
+struct RenderState {
+    size_t splats, conics, depths, radii, cum, rects, ws, ws_bytes, end;
+};
+RenderState render_state(const jaxsplat_descriptor* d) {
+    const size_t n = d->num_points ? d->num_points : 1;
+    RenderState r;
+    size_t o = 0;
+    r.splats = o; o = align256(o + 48 * n);
+    r.conics = o; o = align256(o + 12 * n);
+    r.depths = o; o = align256(o + 4 * n);
+    r.radii = o; o = align256(o + 4 * n);
+    r.cum = o; o = align256(o + 4 * n);
+    r.rects = o; o = align256(o + 8 * n);
+    r.ws = o;
+    r.ws_bytes = jaxsplat_project_workspace_size(d);
+    r.end = align256(o + r.ws_bytes);
+    return r;
+}
+
+struct RenderLists {
+    size_t gids, bins, final_ts, final_idx, end;
+};
+RenderLists render_lists(const jaxsplat_descriptor* d, uint32_t isect) {
+    const size_t tiles = (size_t)d->grid_dim_2d.x * d->grid_dim_2d.y;
+    const size_t pixels = (size_t)d->img_shape.x * d->img_shape.y;
+    RenderLists r;
+    size_t o = 0;
+    r.bins = o; o = align256(o + 8 * tiles);
+    r.final_ts = o; o = align256(o + 4 * pixels);
+    r.final_idx = o; o = align256(o + 4 * pixels);
+    r.gids = o; o = align256(o + 4 * (size_t)(isect ? isect : 1));
+    r.end = o;
+    return r;
+}
+
+template <typename T>
+T* at(void* base, size_t offset) {
+    return reinterpret_cast<T*>(static_cast<uint8_t*>(base) + offset);
+}
+template <typename T>
+const T* at(const void* base, size_t offset) {
+    return reinterpret_cast<const T*>(static_cast<const uint8_t*>(base) + offset);
+}
+bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) != 0; }
+
+}  // namespace
+
+extern "C" {
+
+size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d) {
+    return d && !validate(d) ? render_state(d).end : 0;
+}
+
+size_t jaxsplat_render_lists_size(const jaxsplat_descriptor* d, uint32_t num_intersects) {
+    return d && !validate(d) ? render_lists(d, num_intersects).end : 0;
+}
+
+int jaxsplat_render_layout(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                           size_t* offsets) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    if (!offsets) return fail(JAXSPLAT_ERR_INVALID, "render_layout: offsets is NULL");
+    const RenderState r = render_state(d);
+    const RenderLists l = render_lists(d, num_intersects);
+    const size_t all[10] = {r.splats, r.conics, r.depths, r.radii, r.cum,
+                            r.rects, l.gids, l.bins, l.final_ts, l.final_idx};
+    std::copy(all, all + 10, offsets);
+    return JAXSPLAT_OK;
+}
+
+int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
+                          const float* scales, const float* quats, const float* viewmat,
+                          const float* opacities, const float* colors, uint32_t channels,
+                          void* state, size_t state_bytes, uint64_t* ticket, void* stream) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    const RenderState r = render_state(d);
+    if (!state || misaligned(state) || state_bytes < r.end)
+        return fail(JAXSPLAT_ERR_WORKSPACE, "render_begin: state too small or misaligned");
+    if (int st = jaxsplat_project_forward_splats(
+            d, means3d, scales, quats, viewmat, opacities, colors, channels, nullptr,
+            at<float>(state, r.depths), at<int32_t>(state, r.radii), at<float>(state, r.conics),
+            nullptr, nullptr, at<int32_t>(state, r.cum), at<uint32_t>(state, r.rects),
+            at<float>(state, r.splats), at<void>(state, r.ws), r.ws_bytes, stream))
+        return st;
+    if (!ticket || d->num_points == 0) return JAXSPLAT_OK;
+    return jaxsplat_count_begin(at<int32_t>(state, r.cum) + (d->num_points - 1), ticket, stream);
+}
+
+int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint64_t ticket,
+                          int32_t* num_intersects, void* stream) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    if (!state || !num_intersects)
+        return fail(JAXSPLAT_ERR_INVALID, "render_count: NULL required pointer");
+    if (d->num_points == 0) {
+        *num_intersects = 0;
+        return JAXSPLAT_OK;
+    }
+    return jaxsplat_count_wait(at<int32_t>(state, render_state(d).cum) + (d->num_points - 1),
+                               ticket, num_intersects, stream);
+}
+
+int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                           const void* state, size_t state_bytes, const float* background,
+                           uint32_t channels, void* lists, size_t lists_bytes, void* bin_ws,
+                           size_t bin_ws_bytes, float* out_img, int32_t* err, int64_t* total,
+                           void* stream) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    if (num_intersects >= (1u << 30))
+        return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
+    const RenderState r = render_state(d);
+    const RenderLists l = render_lists(d, num_intersects);
+    if (!state || misaligned(state) || state_bytes < r.end || !lists || misaligned(lists) ||
+        lists_bytes < l.end)
+        return fail(JAXSPLAT_ERR_WORKSPACE, "render_finish: buffer too small or misaligned");
+    int32_t* gids = at<int32_t>(lists, l.gids);
+    int32_t* bins = at<int32_t>(lists, l.bins);
+    if (int st = jaxsplat_bin_rects_sort(d, at<float>(state, r.depths),
+                                         at<uint32_t>(state, r.rects), at<int32_t>(state, r.cum),
+                                         num_intersects, gids, nullptr, bins, bin_ws,
+                                         bin_ws_bytes, stream))
+        return st;
+    if (int st = jaxsplat_rasterize_forward_splats(
+            d, gids, bins, num_intersects, at<float>(state, r.splats), background, channels,
+            at<float>(lists, l.final_ts), at<int32_t>(lists, l.final_idx), out_img, stream))
+        return st;
+    if (!err || num_intersects == 0 || d->num_points == 0) return JAXSPLAT_OK;
+    return jaxsplat_bin_record(bin_ws, err, total, stream);
+}
+
+int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                    const float* means3d, const float* scales,
+                                    const float* quats, const float* viewmat,
+                                    const void* state, size_t state_bytes, const void* lists,
+                                    size_t lists_bytes, const float* background,
+                                    uint32_t channels, const float* v_out_img,
+                                    float* v_colors, float* v_opacity, float* v_mean3d,
+                                    float* v_scale, float* v_quat, int adjoint,
+                                    void* workspace, size_t workspace_bytes, void* stream) {
+    g_err.clear();
+    if (int st = validate(d)) return st;
+    if (num_intersects >= (1u << 30))
+        return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
+    const RenderState r = render_state(d);
+    const RenderLists l = render_lists(d, num_intersects);
+    if (!state || misaligned(state) || state_bytes < r.end || !lists || misaligned(lists) ||
+        lists_bytes < l.end)
+        return fail(JAXSPLAT_ERR_WORKSPACE,
+                    "render_finish_backward: buffer too small or misaligned");
+    return jaxsplat_render_backward(
+        d, at<int32_t>(lists, l.gids), at<int32_t>(lists, l.bins), num_intersects, means3d,
+        scales, quats, viewmat, at<float>(state, r.splats), at<float>(state, r.conics),
+        background, channels, at<int32_t>(state, r.radii), at<uint32_t>(state, r.rects),
+        at<int32_t>(state, r.cum), at<float>(lists, l.final_ts), at<int32_t>(lists, l.final_idx),
+        v_out_img, v_colors, v_opacity, v_mean3d, v_scale, v_quat, adjoint, workspace,
+        workspace_bytes, stream);
 }
 
 int jaxsplat_rasterize_backward_staged_rects(
