@@ -797,7 +797,10 @@ __global__ __launch_bounds__(THREADS, 6) void tile_depth_sort_loop_kernel(
 // launch where its average run (of the capacity) is long: it costs 7 us where
 // none is (1M Gaussians spread over 1080p, 808 pairs per tile: 46 us alone);
 // 500k Gaussians in half of an 800 x 800 image, 848 per tile: 53 us in one, 43
-// in two; 1M, 1700: 136 and 92; 1.5M, 2540: 239 and 166.
+// in two; 1M, 1700: 136 and 92; 1.5M, 2540: 239 and 166.  A batch, many of whose
+// bins are empty, takes it from a sixth of that (535 pairs per bin above; 5 views
+// of 15k at 492 x 383, 37 per bin: 214 us per step in one, 223 in two).
+constexpr int kLongBatchPairs = 256;
 hipError_t tile_depth_order(const int2* bins, int num_bins, int cap, bool batch,
                             const uint32_t* dkeys, uint32_t* ids, uint32_t* ka, uint32_t* va,
                             uint2* kv_tmp, hipStream_t s) {
@@ -806,7 +809,8 @@ hipError_t tile_depth_order(const int2* bins, int num_bins, int cap, bool batch,
     // against one; 4 or 8 cost orbit64's long runs more)
     const int pairs = (num_bins + 1) / 2;
     const int whole = seg_cap(kSegThreads);
-    const bool two = cap > whole && (batch || cap > whole * (long long)num_bins);
+    const bool two =
+        cap > whole && cap > (batch ? kLongBatchPairs : whole) * (long long)num_bins;
     const int most = two ? whole : INT32_MAX;
     if (batch)
         tile_depth_sort_loop_kernel<kSegThreads><<<pairs, kSegThreads, 0, s>>>(
@@ -1027,14 +1031,18 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 
 }  // namespace
 
-// Pairs of the capacity per Gaussian from which the lists are ordered by one
-// depth sort of the Gaussians and stable placements, instead of tile by tile:
-// the depth sort costs 40 us + 36 us per 1M Gaussians, the order of the tiles
-// 7.6 us per 1M pairs in runs of up to 1536 and several times that beyond.
-// Forward of 50k Gaussians with 100 pairs each at 900 x 1600: 232 us by depth,
-// 392 tile by tile; 610k Gaussians with 11 pairs each at 1080p: 664 against
-// 607 us (forward and backward).
+// Pairs of the capacity per Gaussian and per tile from which the lists are
+// ordered by one depth sort of the Gaussians and stable placements, instead of
+// tile by tile: the depth sort costs 45 us + 36 us per 1M Gaussians, the order of
+// the tiles 7.6 us per 1M pairs in runs of up to 1536 and two to three times that
+// beyond.  Many pairs per Gaussian mean large Gaussians, whose overlap makes some
+// runs several times the average.  By depth against tile by tile, forward, us:
+//   per Gaussian, per tile    50k: 95, 804: 219, 263      50k: 29, 939: 167, 176
+//                             1M: 18, 2513: 355, 470     25k: 29, 467: 157, 127
+//                             30k: 20, 427: 165, 111     25k: 95, 400: 196, 180
+//                             300k: 10, 1061: 203, 159     2k: 93, 32: 160, 116
 constexpr int kByDepthPairs = 16;
+constexpr int kByDepthTilePairs = 640;
 // Grids of up to this many tiles are one radix pass of the emitted pairs,
 // whose three launches fewer are worth more than the traffic of few pairs
 // (2k Gaussians at 256 x 256: 50 against 61 us of kernels).
@@ -1048,7 +1056,8 @@ BinPlan bin_plan(const Camera& c, int isect_cap) {
     p.tile_bits = bitlen((uint32_t)(p.num_tiles > 1 ? p.num_tiles - 1 : 1));
     p.by_rows = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
                 p.num_tiles > kOnePassTiles;
-    p.by_depth = p.by_rows && (long long)isect_cap > kByDepthPairs * (long long)p.n;
+    p.by_depth = p.by_rows && (long long)isect_cap > kByDepthPairs * (long long)p.n &&
+                 (long long)isect_cap > kByDepthTilePairs * (long long)p.num_tiles;
     p.rows = row_bin_plan(p.n, c.tiles_x, c.tiles_y, isect_cap);
     p.depth_sort = sort_plan(p.n, 0, 32);
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);

@@ -53,3 +53,25 @@ def test_row_binning_bitexact(tiles, n, radius, path):
         keys = (tids.astype(np.int64) << 32) | depths.view(np.int32)[gids].astype(np.int64)
         assert np.array_equal(keys, ks)
     assert np.array_equal(bins, bs)
+
+
+@pytest.mark.parametrize("path", [{}, {"rects": True}], ids=["one", "rects"])
+@pytest.mark.parametrize("tiles", [(17, 17), (128, 3), (129, 3), (3, 128), (3, 129), (2, 256),
+                                   (256, 2)], ids=str)
+def test_depth_order_bitexact(tiles, path):
+    """Many pairs per Gaussian and per tile: most rectangles cover the grid."""
+    n = 1700
+    xys, depths, radii, _, img = _scene(n, tiles, 90, seed=sum(tiles))
+    radii[: 6 * n // 10] = max(img) + 20
+    perm = np.random.default_rng(5).permutation(n)
+    xys, radii = xys[perm], radii[perm]
+    x0, x1, y0, y1 = oracle.project.tile_rect(xys[:, 0], xys[:, 1], radii.astype(np.float32),
+                                              tiles[1], tiles[0], BW)
+    cum = np.cumsum(np.where(radii > 0, (x1 - x0) * (y1 - y0), 0)).astype(np.int32)
+    assert cum[-1] > 16 * n and cum[-1] > 640 * tiles[0] * tiles[1]
+    gids, tids, bins, isect = H.gpu_bin(xys, depths, radii, cum, img_shape=img, block_width=BW,
+                                        **path)
+    ks, gs, bs = oracle.binning.bin_and_sort(xys, depths, radii, cum, img_shape=img,
+                                             block_width=BW)
+    assert isect == ks.size and np.array_equal(gids, gs) and np.array_equal(bins, bs)
+    assert np.array_equal(tids, ks >> 32)
