@@ -140,7 +140,7 @@ int jaxsplat_project_forward(const jaxsplat_descriptor* d, const float* means3d,
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  Same arguments and results as jaxsplat_project_forward
  * without the workspace; the scan's scratch is a library-held device array
- * of 512 KiB per GPU, so num_points is at most 2^26 (JAXSPLAT_ERR_CAPACITY
+ * of 1 MiB per GPU, so num_points is at most 2^26 (JAXSPLAT_ERR_CAPACITY
  * above).  All calls on one GPU share that array: calls that overlap on one
  * GPU (other streams, other threads) race and must be serialised by the
  * caller.

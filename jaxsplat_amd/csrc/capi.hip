@@ -166,6 +166,38 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // namespace
 
+namespace {
+
+// jaxsplat_project_forward_splats; count_out (optional): see project_fwd.
+int project_splats(const jaxsplat_descriptor* d, const float* means3d, const float* scales,
+                   const float* quats, const float* viewmat, const float* opacities,
+                   const float* colors, uint32_t channels, float* xys, float* depths,
+                   int32_t* radii, float* conics, float* compensation, int32_t* num_tiles_hit,
+                   int32_t* cum_tiles_hit, uint32_t* tile_rects, float* splats, void* workspace,
+                   size_t workspace_bytes, uint64_t* count_out, uint32_t ticket, void* stream) {
+    if (int st = validate(d)) return st;
+    if (channels < 1 || channels > 3)
+        return fail(JAXSPLAT_ERR_INVALID,
+                    "project_forward_splats: channels must be in [1, 3], got %u", channels);
+    if (d->num_points == 0) return JAXSPLAT_OK;
+    if (!means3d || !scales || !quats || !viewmat || !opacities || !colors || !depths ||
+        !radii || !conics || !cum_tiles_hit || !tile_rects || !splats)
+        return fail(JAXSPLAT_ERR_INVALID, "project_forward_splats: NULL required pointer");
+    if (!workspace ||
+        workspace_bytes < align256(jsa::project_fwd_scratch_bytes((int)d->num_points)))
+        return fail(JAXSPLAT_ERR_WORKSPACE, "project_forward_splats: workspace too small");
+    JSA_CHECK_HIP(jsa::project_fwd(camera_of(d), means3d, scales, quats, viewmat, nullptr, xys,
+                                   depths, radii, conics, compensation, num_tiles_hit,
+                                   cum_tiles_hit, opacities,
+                                   reinterpret_cast<uint2*>(tile_rects), workspace,
+                                   static_cast<hipStream_t>(stream), colors, (int)channels,
+                                   reinterpret_cast<float4*>(splats), count_out, ticket),
+                  "project_forward_splats");
+    return JAXSPLAT_OK;
+}
+
+}  // namespace
+
 extern "C" {
 
 const char* jaxsplat_version(void) { return "jaxsplat_amd 0.1.0 (gfx950)"; }
@@ -308,24 +340,9 @@ int jaxsplat_project_forward_splats(const jaxsplat_descriptor* d, const float* m
                                     int32_t* cum_tiles_hit, uint32_t* tile_rects, float* splats,
                                     void* workspace, size_t workspace_bytes, void* stream) {
     g_err.clear();
-    if (int st = validate(d)) return st;
-    if (channels < 1 || channels > 3)
-        return fail(JAXSPLAT_ERR_INVALID,
-                    "project_forward_splats: channels must be in [1, 3], got %u", channels);
-    if (d->num_points == 0) return JAXSPLAT_OK;
-    if (!means3d || !scales || !quats || !viewmat || !opacities || !colors || !depths ||
-        !radii || !conics || !cum_tiles_hit || !tile_rects || !splats)
-        return fail(JAXSPLAT_ERR_INVALID, "project_forward_splats: NULL required pointer");
-    if (!workspace || workspace_bytes < jaxsplat_project_workspace_size(d))
-        return fail(JAXSPLAT_ERR_WORKSPACE, "project_forward_splats: workspace too small");
-    JSA_CHECK_HIP(jsa::project_fwd(camera_of(d), means3d, scales, quats, viewmat, nullptr, xys,
-                                   depths, radii, conics, compensation, num_tiles_hit,
-                                   cum_tiles_hit, opacities,
-                                   reinterpret_cast<uint2*>(tile_rects), workspace,
-                                   static_cast<hipStream_t>(stream), colors, (int)channels,
-                                   reinterpret_cast<float4*>(splats)),
-                  "project_forward_splats");
-    return JAXSPLAT_OK;
+    return project_splats(d, means3d, scales, quats, viewmat, opacities, colors, channels, xys,
+                          depths, radii, conics, compensation, num_tiles_hit, cum_tiles_hit,
+                          tile_rects, splats, workspace, workspace_bytes, nullptr, 0u, stream);
 }
 
 int jaxsplat_project_backward(const jaxsplat_descriptor* d, const float* means3d,
@@ -856,25 +873,11 @@ thread_local CountWord t_count;
 
 __global__ void count_kernel(const int32_t* __restrict__ count, uint64_t* __restrict__ out,
                              uint32_t ticket) {
-    __hip_atomic_store(out, (uint64_t)ticket << 32 | (uint32_t)*count, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
+    jsa::store_count(out, *count, ticket);
 }
 
-__global__ void bin_record_kernel(const uint32_t* __restrict__ header, int32_t* __restrict__ err,
-                                  long long* __restrict__ total) {
-    *err |= (int32_t)header[0];
-    const long long t = (long long)((uint64_t)header[2] | (uint64_t)header[3] << 32);
-    *total = *total > t ? *total : t;
-}
-
-}  // namespace
-
-extern "C" {
-
-int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream) {
-    g_err.clear();
-    if (!count || !ticket) return fail(JAXSPLAT_ERR_INVALID, "count_begin: NULL required pointer");
-    hipStream_t s = static_cast<hipStream_t>(stream);
+// A new ticket of this thread's word (t_count) for a count on stream s.
+int next_ticket(hipStream_t s) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     JSA_CHECK_HIP(hipStreamIsCapturing(s, &capturing), "count_begin");
     if (capturing != hipStreamCaptureStatusNone)
@@ -896,7 +899,26 @@ int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream) {
         *w.host = 0;
     }
     if (++w.ticket == 0) w.ticket = 1;
-    count_kernel<<<1, 1, 0, s>>>(count, w.dev, w.ticket);
+    return JAXSPLAT_OK;
+}
+
+__global__ void bin_record_kernel(const uint32_t* __restrict__ header, int32_t* __restrict__ err,
+                                  long long* __restrict__ total) {
+    *err |= (int32_t)header[0];
+    const long long t = (long long)((uint64_t)header[2] | (uint64_t)header[3] << 32);
+    *total = *total > t ? *total : t;
+}
+
+}  // namespace
+
+extern "C" {
+
+int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream) {
+    g_err.clear();
+    if (!count || !ticket) return fail(JAXSPLAT_ERR_INVALID, "count_begin: NULL required pointer");
+    if (int st = next_ticket(static_cast<hipStream_t>(stream))) return st;
+    const CountWord& w = t_count;
+    count_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(count, w.dev, w.ticket);
     JSA_CHECK_HIP(hipGetLastError(), "count_begin");
     *ticket = w.ticket;
     return JAXSPLAT_OK;
@@ -1024,14 +1046,20 @@ int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
     const RenderState r = render_state(d);
     if (!state || misaligned(state) || state_bytes < r.end)
         return fail(JAXSPLAT_ERR_WORKSPACE, "render_begin: state too small or misaligned");
-    if (int st = jaxsplat_project_forward_splats(
-            d, means3d, scales, quats, viewmat, opacities, colors, channels, nullptr,
-            at<float>(state, r.depths), at<int32_t>(state, r.radii), at<float>(state, r.conics),
-            nullptr, nullptr, at<int32_t>(state, r.cum), at<uint32_t>(state, r.rects),
-            at<float>(state, r.splats), at<void>(state, r.ws), r.ws_bytes, stream))
-        return st;
-    if (!ticket || d->num_points == 0) return JAXSPLAT_OK;
-    return jaxsplat_count_begin(at<int32_t>(state, r.cum) + (d->num_points - 1), ticket, stream);
+    if (ticket) {
+        *ticket = 0;
+        if (d->num_points > 0) {
+            if (int st = next_ticket(static_cast<hipStream_t>(stream))) return st;
+            *ticket = t_count.ticket;
+        }
+    }
+    const bool count = ticket && d->num_points > 0;
+    return project_splats(d, means3d, scales, quats, viewmat, opacities, colors, channels,
+                          nullptr, at<float>(state, r.depths), at<int32_t>(state, r.radii),
+                          at<float>(state, r.conics), nullptr, nullptr,
+                          at<int32_t>(state, r.cum), at<uint32_t>(state, r.rects),
+                          at<float>(state, r.splats), at<void>(state, r.ws), r.ws_bytes,
+                          count ? t_count.dev : nullptr, count ? t_count.ticket : 0u, stream);
 }
 
 int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint64_t ticket,

@@ -179,6 +179,12 @@ __device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
     return block_exclusive_scan<4>(v, s_tmp);
 }
 
+// A count with its ticket into a pinned, coherent word of the host's.
+__device__ __forceinline__ void store_count(uint64_t* out, int count, uint32_t ticket) {
+    __hip_atomic_store(out, (uint64_t)ticket << 32 | (uint32_t)count, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Tile rectangle [x0, x1) x [y0, y1) of a Gaussian from its centre and integer
 // radius: forward.cu:152-161 / helpers.h:9-32 (the binning and the staged
 // backward must agree bit for bit, so both use this one function).
@@ -552,7 +558,8 @@ hipError_t project_fwd(const Camera& c, const float* means3d, const float* scale
                        float* xys, float* depths, int* radii, float* conics,
                        float* compensation, int* num_tiles_hit, int* cum_tiles_hit,
                        const float* opacities, uint2* rects, void* scratch, hipStream_t s,
-                       const float* colors = nullptr, int nch = 0, float4* splats = nullptr);
+                       const float* colors = nullptr, int nch = 0, float4* splats = nullptr,
+                       uint64_t* count_out = nullptr, uint32_t ticket = 0);
 // Opacity-limited tile rectangles (opacity_tile_rect) of projected Gaussians,
 // their counts (num_tiles_hit optional) and inclusive sums; scratch
 // project_fwd_scratch_bytes(c.num_points).

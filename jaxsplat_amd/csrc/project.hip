@@ -133,8 +133,11 @@ __device__ __forceinline__ M3 ewa_jacobian(float fx, float fy, float tx, float t
     return J;
 }
 
-constexpr int kProjPer = 4;                   // Gaussians per lane
-constexpr int kProjPart = 256 * kProjPer;    // Gaussians per scan partition
+constexpr int kProjPart = 256;      // Gaussians per workgroup and scan partition
+// Partitions per workgroup of the scan's second kernel: few, so that it has
+// workgroups enough, but what each sums grows with their number.
+constexpr int kScanPer = 4, kScanPerMany = 16, kScanMany = 1 << 20;
+constexpr int kBatchPer = 4;        // Gaussians per lane of the batched projection
 
 // Projected attributes of one Gaussian (culled ones keep the zeros).
 struct Proj {
@@ -298,7 +301,7 @@ __device__ __forceinline__ Camera view_camera(const ViewRec& v, float glob_scale
     return c;
 }
 
-// Batched forward: blockIdx.y = view, kProjPer Gaussians per lane of the
+// Batched forward: blockIdx.y = view, kBatchPer Gaussians per lane of the
 // view's scene.  Writes the item rows the binning and rasterizer read, and the
 // depth sort key; no scan (the emission scans in depth order itself).
 __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
@@ -308,7 +311,7 @@ __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
     const float* __restrict__ opacities, float* __restrict__ xys, float* __restrict__ conics,
     int* __restrict__ radii, uint32_t* __restrict__ dkeys, uint2* __restrict__ rects) {
     const ViewRec vr = views[blockIdx.y];
-    const int first = blockIdx.x * kProjPart;
+    const int first = blockIdx.x * (256 * kBatchPer);
     if (first >= vr.n) return;
     const Camera c = view_camera(vr, glob_scale, clip_thresh, block_width);
     M3 W;
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
     const float* sc = scales + 3 * (size_t)vr.g0;
     const float* qt = quats + 4 * (size_t)vr.g0;
 #pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
+    for (int k = 0; k < kBatchPer; ++k) {
         const int local = first + k * 256 + (int)threadIdx.x;
         if (local >= vr.n) break;
         const Proj r = project_core(c, local, W, pt, m3, sc, qt);
@@ -341,6 +344,17 @@ __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
     }
 }
 
+// The workgroup's inclusive sums of the tile counts (project_scan_add_kernel adds
+// the partition's offset) and their total.
+__device__ __forceinline__ void count_scan(uint32_t cnt, int idx, int n,
+                                           int* __restrict__ cum_tiles_hit,
+                                           uint32_t* __restrict__ part_tot, uint32_t* s_tmp) {
+    const uint32_t incl = block_exclusive_scan256(cnt, s_tmp) + cnt;
+    if (idx < n) cum_tiles_hit[idx] = (int)incl;
+    if (threadIdx.x == 255) part_tot[blockIdx.x] = incl;
+}
+
+
 __global__ __launch_bounds__(256) void project_fwd_kernel(
     Camera c, const float* __restrict__ means3d, const float* __restrict__ scales,
     const float* __restrict__ quats, const float* __restrict__ viewmat,
@@ -350,47 +364,18 @@ __global__ __launch_bounds__(256) void project_fwd_kernel(
     const float* __restrict__ opacities, uint2* __restrict__ rects,
     uint32_t* __restrict__ part_tot, const float* __restrict__ colors, int nch,
     float4* __restrict__ splats) {
-    __shared__ uint32_t s_wave_tot[kProjPer][4];
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = tid >> 6;
-    const int part = blockIdx.x;
+    __shared__ uint32_t s_tmp[4];
+    const int idx = blockIdx.x * kProjPart + (int)threadIdx.x;
     M3 W;
     float pt[3];
     load_view(viewmat, W, pt);
-
-    // element k*256 + tid of the partition, k = 0..kProjPer-1 (coalesced slabs)
-    int incl[kProjPer];
-    int cnt[kProjPer];
-#pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
-        const int idx = part * kProjPart + k * 256 + tid;
-        cnt[k] = idx < c.num_points
-                     ? project_one(c, idx, W, pt, means3d, scales, quats, cov3d_out, xys,
-                                   depths, radii, conics, comp_out, num_tiles_hit, opacities,
-                                   rects, colors, nch, splats)
-                     : 0;
-        incl[k] = wave_inclusive_sum(cnt[k]);
-        if (lane == 63) s_wave_tot[k][wave] = (uint32_t)incl[k];
-    }
-    __syncthreads();
-    // partition-local inclusive sums; project_scan_add_kernel adds the
-    // partition's offset
-    uint32_t total = 0;
-#pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
-        uint32_t w_off = 0, slab = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t v = s_wave_tot[k][w];
-            w_off += (w < wave) ? v : 0u;
-            slab += v;
-        }
-        const int idx = part * kProjPart + k * 256 + tid;
-        if (idx < c.num_points) cum_tiles_hit[idx] = (int)(total + w_off + (uint32_t)incl[k]);
-        total += slab;
-    }
-    if (tid == 0) part_tot[part] = total;
+    const uint32_t cnt =
+        idx < c.num_points
+            ? (uint32_t)project_one(c, idx, W, pt, means3d, scales, quats, cov3d_out, xys,
+                                    depths, radii, conics, comp_out, num_tiles_hit, opacities,
+                                    rects, colors, nch, splats)
+            : 0u;
+    count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
 }
 
 // Opacity-limited tile rectangles (opacity_tile_rect) of the projected
@@ -402,68 +387,52 @@ __global__ __launch_bounds__(256) void tile_rects_kernel(
     const float* __restrict__ conics, const float* __restrict__ opacities,
     uint2* __restrict__ rects, int* __restrict__ num_tiles_hit, int* __restrict__ cum_tiles_hit,
     uint32_t* __restrict__ part_tot) {
-    __shared__ uint32_t s_wave_tot[kProjPer][4];
-    const int tid = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = tid >> 6;
-    const int part = blockIdx.x;
-    int incl[kProjPer];
-    int cnt[kProjPer];
-#pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
-        const int idx = part * kProjPart + k * 256 + tid;
-        cnt[k] = 0;
-        if (idx < c.num_points) {
-            const int rad = radii[idx];
-            uint2 rc = make_uint2(0u, 0u);
-            if (rad > 0)
-                rc = opacity_tile_rect(c.block_width, c.tiles_x, c.tiles_y, xys[idx], rad,
-                                       conics[3 * idx + 0], conics[3 * idx + 1],
-                                       conics[3 * idx + 2], opacities[idx]);
-            rects[idx] = rc;
-            cnt[k] = (int)rect_count(rc);
-            if (num_tiles_hit) num_tiles_hit[idx] = cnt[k];
-        }
-        incl[k] = wave_inclusive_sum(cnt[k]);
-        if (lane == 63) s_wave_tot[k][wave] = (uint32_t)incl[k];
+    __shared__ uint32_t s_tmp[4];
+    const int idx = blockIdx.x * kProjPart + (int)threadIdx.x;
+    uint32_t cnt = 0;
+    if (idx < c.num_points) {
+        const int rad = radii[idx];
+        uint2 rc = make_uint2(0u, 0u);
+        if (rad > 0)
+            rc = opacity_tile_rect(c.block_width, c.tiles_x, c.tiles_y, xys[idx], rad,
+                                   conics[3 * idx + 0], conics[3 * idx + 1],
+                                   conics[3 * idx + 2], opacities[idx]);
+        rects[idx] = rc;
+        cnt = rect_count(rc);
+        if (num_tiles_hit) num_tiles_hit[idx] = (int)cnt;
     }
-    __syncthreads();
-    uint32_t total = 0;
-#pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
-        uint32_t w_off = 0, slab = 0;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint32_t v = s_wave_tot[k][w];
-            w_off += (w < wave) ? v : 0u;
-            slab += v;
-        }
-        const int idx = part * kProjPart + k * 256 + tid;
-        if (idx < c.num_points) cum_tiles_hit[idx] = (int)(total + w_off + (uint32_t)incl[k]);
-        total += slab;
-    }
-    if (tid == 0) part_tot[part] = total;
+    count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
 }
 
-// cum_tiles_hit += its partition's offset, one workgroup per partition
-// p >= 1: the workgroup sums the totals of partitions 0..p-1 itself (at most a
-// few KB from L2 at 1M Gaussians), so no separate scan kernel runs between
-// the projection and this one.
+// cum_tiles_hit += its partition's offset, `per` partitions per workgroup: the
+// workgroup sums the totals of all earlier partitions itself (a few KB from L2
+// at 1M Gaussians), so no separate scan kernel runs between the projection and
+// this one.  Partitions are one workgroup of the projection, a Gaussian per lane:
+// four per lane left CUs without work up to 260k Gaussians and took 11 us at any
+// size below that (now 5; 3M: 101 + 10 us, now 89 + 11).  count_out (optional):
+// where the last count goes for the host, with its ticket.
 __global__ __launch_bounds__(256) void project_scan_add_kernel(
-    int n, const uint32_t* __restrict__ part_tot, int* __restrict__ cum_tiles_hit) {
+    int n, int parts, int per, const uint32_t* __restrict__ part_tot,
+    int* __restrict__ cum_tiles_hit, uint64_t* __restrict__ count_out, uint32_t ticket) {
     __shared__ uint32_t s_w[4];
     const int tid = threadIdx.x;
-    const int p = blockIdx.x + 1;
+    const int p = blockIdx.x * per;
     uint32_t sum = 0;
     for (int q = tid; q < p; q += 256) sum += part_tot[q];
     sum = wave_inclusive_sum(sum);
     if (lane_id() == 63) s_w[tid >> 6] = sum;
     __syncthreads();
-    const int off = (int)((s_w[0] + s_w[1]) + (s_w[2] + s_w[3]));
-#pragma unroll
-    for (int k = 0; k < kProjPer; ++k) {
-        const int idx = p * kProjPart + k * 256 + tid;
-        if (idx < n) cum_tiles_hit[idx] += off;
+    uint32_t off = (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
+    const int end = min(p + per, parts);
+#pragma unroll 4
+    for (int q = p; q < end; ++q) {
+        const int idx = q * kProjPart + tid;
+        if (idx < n) {
+            const int cum = cum_tiles_hit[idx] + (int)off;
+            cum_tiles_hit[idx] = cum;
+            if (count_out && idx == n - 1) store_count(count_out, cum, ticket);
+        }
+        off += part_tot[q];
     }
 }
 
@@ -896,22 +865,22 @@ hipError_t fill_value_f32x3(float* dst, size_t n_pixels, const float* rgb, hipSt
     return hipGetLastError();
 }
 
-// scratch layout: [counter u32 | err u32 | pad to 16 | status u64 x parts]
+// One total per partition.
 size_t project_fwd_scratch_bytes(int n) {
     const size_t parts = ((size_t)n + kProjPart - 1) / kProjPart;
-    return 16 + 8 * (parts > 0 ? parts : 1);
+    return 4 * (parts > 0 ? parts : 1);
 }
 
 // Projection scratch held by the library, for callers that cannot allocate
-// (jaxsplat_project_forward_noalloc): the fused scan's partition totals and
-// offsets for up to kStaticProjectPoints Gaussians, 512 KiB + 256 B.  Each
+// (jaxsplat_project_forward_noalloc): the scan's partition totals for up to
+// kStaticProjectPoints Gaussians, 1 MiB.  Each
 // device holds its own copy until the process ends.  In host code the array's
 // name is not a device address: kernels get the address that
 // hipGetSymbolAddress returns for the current device.  Nothing in it needs
 // to start at zero (the forward kernel writes every partition total before
 // the scan reads it); calls that overlap on one device race on it.
 constexpr size_t kStaticProjectScratch =
-    (16 + 8 * (size_t)(kStaticProjectPoints / kProjPart) + 255) & ~(size_t)255;
+    (4 * (size_t)(kStaticProjectPoints / kProjPart) + 255) & ~(size_t)255;
 static_assert(kStaticProjectPoints % kProjPart == 0, "whole partitions");
 static __device__ __align__(256) uint8_t scratch[kStaticProjectScratch];
 
@@ -937,12 +906,23 @@ hipError_t project_static_scratch(void** out) {
     return hipSuccess;
 }
 
+// The counts' scan over the partitions (a single one's sums are final) and the
+// host's copy of the last.
+static hipError_t scan_add(int n, int parts, const uint32_t* part_tot, int* cum_tiles_hit,
+                           uint64_t* count_out, uint32_t ticket, hipStream_t s) {
+    if (parts == 1 && !count_out) return hipSuccess;
+    const int per = n <= kScanMany ? kScanPer : kScanPerMany;
+    project_scan_add_kernel<<<(parts + per - 1) / per, 256, 0, s>>>(
+        n, parts, per, part_tot, cum_tiles_hit, count_out, ticket);
+    return hipGetLastError();
+}
+
 hipError_t project_fwd(const Camera& c, const float* means3d, const float* scales,
                        const float* quats, const float* viewmat, float* cov3d, float* xys,
                        float* depths, int* radii, float* conics, float* compensation,
                        int* num_tiles_hit, int* cum_tiles_hit, const float* opacities,
                        uint2* rects, void* scratch, hipStream_t s, const float* colors, int nch,
-                       float4* splats) {
+                       float4* splats, uint64_t* count_out, uint32_t ticket) {
     if (c.num_points <= 0) return hipSuccess;
     if (splats && (!opacities || !rects || !colors || nch < 1 || nch > 3))
         return hipErrorInvalidValue;
@@ -952,10 +932,10 @@ hipError_t project_fwd(const Camera& c, const float* means3d, const float* scale
                                              depths, radii, conics, compensation, num_tiles_hit,
                                              cum_tiles_hit, opacities, rects, part_tot, colors,
                                              nch, splats);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || parts == 1) return e;
-    project_scan_add_kernel<<<parts - 1, 256, 0, s>>>(c.num_points, part_tot, cum_tiles_hit);
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess
+               ? e
+               : scan_add(c.num_points, parts, part_tot, cum_tiles_hit, count_out, ticket, s);
 }
 
 hipError_t tile_rects(const Camera& c, const float* xys, const int* radii, const float* conics,
@@ -967,10 +947,10 @@ hipError_t tile_rects(const Camera& c, const float* xys, const int* radii, const
     tile_rects_kernel<<<parts, 256, 0, s>>>(c, reinterpret_cast<const float2*>(xys), radii,
                                             conics, opacities, rects, num_tiles_hit,
                                             cum_tiles_hit, part_tot);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || parts == 1) return e;
-    project_scan_add_kernel<<<parts - 1, 256, 0, s>>>(c.num_points, part_tot, cum_tiles_hit);
-    return hipGetLastError();
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess
+               ? e
+               : scan_add(c.num_points, parts, part_tot, cum_tiles_hit, nullptr, 0u, s);
 }
 
 hipError_t project_bwd(const Camera& c, const float* means3d, const float* scales,
@@ -1016,7 +996,7 @@ hipError_t project_batch_fwd(const ViewRec* views, int num_views, int max_view_n
                              float* conics, int* radii, uint32_t* depth_keys, uint2* item_rects,
                              hipStream_t s) {
     if (num_views <= 0 || max_view_n <= 0) return hipSuccess;
-    const dim3 grid((max_view_n + kProjPart - 1) / kProjPart, num_views);
+    const dim3 grid((max_view_n + 256 * kBatchPer - 1) / (256 * kBatchPer), num_views);
     project_batch_fwd_kernel<<<grid, 256, 0, s>>>(views, glob_scale, clip_thresh, block_width,
                                                   means3d, scales, quats, viewmats, opacities,
                                                   xys, conics, radii, depth_keys, item_rects);
