@@ -232,6 +232,7 @@ struct EmitEntries {
 struct FirstCounts {
     uint32_t* counts;
     int tile, parts, shift, bits;
+    size_t digit_stride, part_stride;
 };
 
 FirstCounts first_counts(const SortPlan& sp, uint8_t* sort_scratch) {
@@ -241,6 +242,8 @@ FirstCounts first_counts(const SortPlan& sp, uint8_t* sort_scratch) {
     fc.parts = sp.parts;
     fc.shift = sp.first_shift;
     fc.bits = sp.first_bits;
+    fc.digit_stride = sp.digit_stride;
+    fc.part_stride = sp.part_stride;
     return fc;
 }
 
@@ -417,7 +420,7 @@ __global__ __launch_bounds__(256) void emit_expand_kernel(
     if (fc.counts) {
         __syncthreads();
         const int d = threadIdx.x;
-        fc.counts[(size_t)d * fc.parts + blockIdx.x] =
+        fc.counts[d * fc.digit_stride + blockIdx.x * fc.part_stride] =
             (s_hist[0][d] + s_hist[1][d]) + (s_hist[2][d] + s_hist[3][d]);
     }
 }

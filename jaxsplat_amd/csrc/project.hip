@@ -137,7 +137,7 @@ constexpr int kProjPart = 256;      // Gaussians per workgroup and scan partitio
 // Partitions per workgroup of the scan's second kernel: few, so that it has
 // workgroups enough, but what each sums grows with their number.
 constexpr int kScanPer = 4, kScanPerMany = 16, kScanMany = 1 << 20;
-constexpr int kBatchPer = 4;        // Gaussians per lane of the batched projection
+constexpr int kBatchPer = 1;        // Gaussians per lane of the batched projection
 
 // Projected attributes of one Gaussian (culled ones keep the zeros).
 struct Proj {

@@ -235,14 +235,15 @@ __device__ __forceinline__ uint2 grid_rect(uint2 rc, int tiles_x, int tiles_y, b
 }
 
 // Step 1, counting: partition b holds the Gaussians perm[1024 b ..) (the ids
-// themselves where perm is null).  counts[row * parts + b] = its runs per row,
+// themselves where perm is null).  counts[row * row_stride + b * part_stride] =
+// its runs per row,
 // part_tot[b] = its pairs; with perm, in_order[i] = the rectangle of perm[i],
 // so that the random gather is paid once.  Also clears the tile bins and the
 // error word.
 __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
     int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
-    int tiles_y, int parts, uint32_t* __restrict__ counts, uint32_t* __restrict__ part_tot,
-    uint2* __restrict__ in_order, int num_tiles, int2* __restrict__ bins,
+    int tiles_y, int row_stride, int part_stride, uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ part_tot, uint2* __restrict__ in_order, int num_tiles, int2* __restrict__ bins,
     uint32_t* __restrict__ err) {
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
@@ -272,20 +273,20 @@ __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
     __syncthreads();
     const uint32_t d = (uint32_t)s_d[tid];
     const uint32_t c = block_exclusive_scan256(d, s_tmp) + d;      // wraps back to the count
-    if (tid < tiles_y) counts[(size_t)tid * parts + part] = c;
+    if (tid < tiles_y) counts[(size_t)tid * row_stride + (size_t)part * part_stride] = c;
     const uint32_t t = block_exclusive_scan256(pairs, s_tmp) + pairs;
     if (tid == kRbThreads - 1) part_tot[part] = t;
 }
 
 // Step 1, placement: the runs of partition b into the row segments, which lie
 // end to end in runs[0 .. sum of row_len).  rects in perm's order; counts: exclusive over the
-// partitions of a row (column_scan), row_len their totals.  Workgroup 0 also
-// writes the exact pair total and bit 8 of err where it exceeds cap.
+// partitions of a row (column_scan), row_len their totals, or with fold the
+// counts themselves, and workgroup 0 writes row_len.  Workgroup 0 also writes the exact pair total and bit 8 of err where it exceeds cap.
 template <bool STABLE, int COLS>
 __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
-    int tiles_y, int parts, const uint32_t* __restrict__ counts,
-    const uint32_t* __restrict__ row_len, const uint32_t* __restrict__ part_tot,
+    int tiles_y, int parts, bool fold, const uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ row_len, const uint32_t* __restrict__ part_tot,
     uint2* __restrict__ runs, int cap, unsigned long long* __restrict__ total_out,
     uint32_t* __restrict__ err) {
     constexpr int PER = round_per(STABLE);
@@ -310,9 +311,12 @@ __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     if (bad_any) atomicOr(err, 4u);
     clear_place(sh);
     // (the rows' runs may sum past 32 bits: positions past cap are all alike)
-    const uint64_t row = tid < tiles_y ? row_len[tid] : 0u;
-    const uint64_t at = block_exclusive_scan256(row, s_sum) +
-                        (tid < tiles_y ? counts[(size_t)tid * parts + part] : 0u);
+    uint2 own = make_uint2(0u, 0u);         // before this partition, of the row
+    if (tid < tiles_y)
+        own = fold ? fold_counts(counts, parts, part, tid)
+                   : make_uint2(counts[(size_t)tid * parts + part], row_len[tid]);
+    if (fold && part == 0 && tid < tiles_y) row_len[tid] = own.y;
+    const uint64_t at = block_exclusive_scan256((uint64_t)own.y, s_sum) + own.x;
     const int base = (int)min(at, (uint64_t)cap);
     place_all<PER>(sh, iv, val, tiles_y, base, runs, cap);
     if (part != 0) return;
@@ -552,6 +556,7 @@ RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap) {
     p.tiles_y = tiles_y;
     p.cap = cap > 0 ? cap : 1;
     p.parts = (n + kRbPart - 1) / kRbPart;
+    p.fold = p.parts <= kFoldParts;
     p.max_col_parts = p.cap / kRbPart + tiles_y;
     size_t o = 0;
     const size_t parts = (size_t)(p.parts > 0 ? p.parts : 1);
@@ -577,14 +582,18 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     const int tiles = p.tiles_x * p.tiles_y;
     hipError_t e;
     row_count_kernel<<<p.parts, kRbThreads, 0, s>>>(p.n, perm, rects, p.tiles_x, p.tiles_y,
-                                                    p.parts, U(p.row_counts), U(p.part_tot),
+                                                    p.fold ? 1 : p.parts,
+                                                    p.fold ? kRowBinAxis : 1, U(p.row_counts),
+                                                    U(p.part_tot),
                                                     in_order, tiles, bins, err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = column_scan(U(p.row_counts), p.parts, U(p.row_len), p.tiles_y, s)) != hipSuccess)
+    if (!p.fold && (e = column_scan(U(p.row_counts), p.parts, U(p.row_len), p.tiles_y, s)) !=
+                       hipSuccess)
         return e;
 #define JSA_ROW(ST, COLS)                                                                     \
     row_place_kernel<ST, COLS><<<p.parts, kRbThreads, 0, s>>>(                                \
-        p.n, perm, perm ? in_order : rects, p.tiles_x, p.tiles_y, p.parts, U(p.row_counts),   \
+        p.n, perm, perm ? in_order : rects, p.tiles_x, p.tiles_y, p.parts, p.fold,            \
+        U(p.row_counts),                                                                      \
         U(p.row_len),                                                                         \
         U(p.part_tot), runs, p.cap, total, err)
     if (narrow(p.tiles_y)) {

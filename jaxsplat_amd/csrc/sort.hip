@@ -8,7 +8,8 @@
 //    (1024 or 4096 keys) into per-wave LDS histograms and writes the 256
 //    counts digit-major, counts[d * parts + part];
 //  * radix_colscan: one workgroup per digit turns its column into exclusive
-//    prefixes over the partitions and records the digit total;
+//    prefixes over the partitions and records the digit total (not for few
+//    partitions, whose counts the downsweep sums itself);
 //  * radix_downsweep: each workgroup ranks its keys stably -- each wave ranks
 //    64 keys per round with 64-lane ballots (one ballot per digit bit gives
 //    the mask of lanes holding the same digit; the highest lane of a peer
@@ -39,7 +40,7 @@ __device__ __forceinline__ int read_n(int n_host, const int* n_dev) {
 template <int ITEMS>
 __global__ __launch_bounds__(kSortThreads) void radix_upsweep(
     const uint32_t* __restrict__ keys, int n_host, const int* __restrict__ n_dev, int shift,
-    int bits, int parts, uint32_t* __restrict__ counts) {
+    int bits, size_t digit_stride, size_t part_stride, uint32_t* __restrict__ counts) {
     constexpr int TILE = kSortThreads * ITEMS;
     __shared__ uint32_t s_hist[kSortWaves][kBins];
     const int tid = threadIdx.x;
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_upsweep(
     uint32_t v = 0;
 #pragma unroll
     for (int w = 0; w < kSortWaves; ++w) v += s_hist[w][tid];
-    counts[(size_t)tid * parts + part] = v;
+    counts[tid * digit_stride + part * part_stride] = v;
 }
 
 // In-place exclusive scan of one digit's column counts[d * parts + 0..parts)
@@ -134,9 +135,9 @@ template <int ITEMS, bool STABLE>
 __global__ __launch_bounds__(kSortThreads) void radix_downsweep(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int n_host,
-    const int* __restrict__ n_dev, int shift, int bits, int parts,
-    const uint32_t* __restrict__ counts /* scanned, digit-major */,
-    const uint32_t* __restrict__ totals /* per digit */) {
+    const int* __restrict__ n_dev, int shift, int bits, int parts, bool fold,
+    const uint32_t* __restrict__ counts /* fold: as counted; else scanned, digit-major */,
+    const uint32_t* __restrict__ totals /* per digit (not fold) */) {
     constexpr int TILE = kSortThreads * ITEMS;
     __shared__ uint32_t s_keys[TILE];
     __shared__ uint32_t s_vals[TILE];
@@ -172,6 +173,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_downsweep(
         val[r] = in ? (vals_in ? vals_in[p] : (uint32_t)p) : 0u;
         keep[r] = in;
     }
+    // this digit's keys before the partition and in all (the loads overlap the
+    // keys' and the ranking)
+    const uint2 own = fold ? fold_counts(counts, parts, part, tid)
+                           : make_uint2(counts[(size_t)tid * parts + part], totals[tid]);
     // ---- wave-local ranking: stable with 64-lane ballots, else atomics ----
 #pragma unroll
     for (int r = 0; r < ITEMS; ++r) {
@@ -200,10 +205,10 @@ __global__ __launch_bounds__(kSortThreads) void radix_downsweep(
         s_whist[w][d] = total;
         total += c;
     }
-    const uint32_t dstart = block_exclusive_scan256(totals[d], s_tmp);
+    const uint32_t dstart = block_exclusive_scan256(own.y, s_tmp);
     const uint32_t lstart = block_exclusive_scan256(total, s_tmp);
     s_lstart[d] = lstart;
-    s_gbase[d] = dstart + counts[(size_t)d * parts + part];
+    s_gbase[d] = dstart + own.x;
     if (d == kBins - 1) s_valid = lstart + total;      // keys kept in this partition
     __syncthreads();
 
@@ -250,6 +255,9 @@ SortPlan sort_plan(int n_cap, int begin_bit, int end_bit) {
     const int per = p.passes > 0 ? (p.end_bit - p.begin_bit + p.passes - 1) / p.passes : 0;
     p.first_shift = p.begin_bit;
     p.first_bits = min(per, p.end_bit - p.begin_bit);
+    p.fold = p.parts <= kFoldParts;
+    p.digit_stride = p.fold ? 1 : (size_t)p.parts;
+    p.part_stride = p.fold ? kBins : 1;
     // [totals 256][counts 256 * parts]
     p.scratch_bytes = 4ull * kBins + 4ull * kBins * (size_t)p.parts;
     p.scratch_bytes = (p.scratch_bytes + 255) & ~size_t(255);
@@ -300,17 +308,20 @@ hipError_t sort_pairs(const SortPlan& p, const uint32_t* keys_in, const uint32_t
     do {                                                                                     \
         if (count_here) {                                                                    \
             radix_upsweep<IT><<<p.parts, kSortThreads, 0, s>>>(ki, n_host, n_dev, shift,     \
-                                                                bits, p.parts, counts);      \
+                                                                bits, p.digit_stride,        \
+                                                                p.part_stride, counts);      \
             if ((e = hipGetLastError()) != hipSuccess) return e;                             \
         }                                                                                    \
-        radix_colscan<<<kBins, kSortThreads, 0, s>>>(counts, p.parts, totals);               \
-        if ((e = hipGetLastError()) != hipSuccess) return e;                                 \
+        if (!p.fold) {                                                                       \
+            radix_colscan<<<kBins, kSortThreads, 0, s>>>(counts, p.parts, totals);           \
+            if ((e = hipGetLastError()) != hipSuccess) return e;                             \
+        }                                                                                    \
         if (stable)                                                                          \
             radix_downsweep<IT, true><<<p.parts, kSortThreads, 0, s>>>(                      \
-                ki, vi, ko, vo, n_host, n_dev, shift, bits, p.parts, counts, totals);        \
+                ki, vi, ko, vo, n_host, n_dev, shift, bits, p.parts, p.fold, counts, totals);        \
         else                                                                                 \
             radix_downsweep<IT, false><<<p.parts, kSortThreads, 0, s>>>(                     \
-                ki, vi, ko, vo, n_host, n_dev, shift, bits, p.parts, counts, totals);        \
+                ki, vi, ko, vo, n_host, n_dev, shift, bits, p.parts, p.fold, counts, totals);        \
         if ((e = hipGetLastError()) != hipSuccess) return e;                                 \
     } while (0)
         if (items == 16) JSA_PASS(16);
