@@ -464,17 +464,21 @@ int jaxsplat_bin_record(const void* workspace, int32_t* err, int64_t* total, voi
  * jaxsplat_bin_emit_workspace_size bytes, and, with err, jaxsplat_bin_record.
  * render_finish_backward is jaxsplat_render_backward over them.  render_layout
  * gives the byte offsets of splats, conics, depths, radii, cum_tiles_hit and
- * tile_rects in `state` and of gaussian_ids_sorted, tile_bins, final_Ts and
- * final_idx in `lists`.
+ * tile_rects in `state`, of gaussian_ids_sorted, tile_bins, final_Ts and
+ * final_idx in `lists`, and of the compensation in `state`.  antialiased (0 or 1,
+ * the same in every call): the blend takes opacity times the projection's
+ * compensation (its opacities are given to the backward again), with gradients
+ * through both.
  */
-size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d);
+size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d, int antialiased);
 size_t jaxsplat_render_lists_size(const jaxsplat_descriptor* d, uint32_t num_intersects);
 int jaxsplat_render_layout(const jaxsplat_descriptor* d, uint32_t num_intersects,
                            size_t* offsets);
 int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
                           const float* scales, const float* quats, const float* viewmat,
                           const float* opacities, const float* colors, uint32_t channels,
-                          void* state, size_t state_bytes, uint64_t* ticket, void* stream);
+                          int antialiased, void* state, size_t state_bytes, uint64_t* ticket,
+                          void* stream);
 int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint64_t ticket,
                           int32_t* num_intersects, void* stream);
 int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects,
@@ -487,7 +491,8 @@ int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_i
                                     const float* quats, const float* viewmat,
                                     const void* state, size_t state_bytes, const void* lists,
                                     size_t lists_bytes, const float* background,
-                                    uint32_t channels, const float* v_out_img,
+                                    uint32_t channels, const float* opacities,
+                                    int antialiased, const float* v_out_img,
                                     float* v_colors, float* v_opacity, float* v_mean3d,
                                     float* v_scale, float* v_quat, int adjoint,
                                     void* workspace, size_t workspace_bytes, void* stream);

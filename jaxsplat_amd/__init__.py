@@ -54,7 +54,7 @@ def render(means3d, scales, quats, colors, opacities, *, viewmat, background, im
     """
     fusable = (isinstance(colors, _ops.torch.Tensor) and colors.dim() == 2 and
                1 <= colors.shape[1] <= 3)
-    if _ops.TIGHT_TILES and _ops.FUSED_RENDER and not antialiased and fusable:
+    if _ops.TIGHT_TILES and _ops.FUSED_RENDER and fusable:
         # one autograd node (up to 3 channels): projection with the
         # opacity-limited rectangles and splat records, binning,
         # rasterization; its backward sums the rasterize records and runs the
@@ -63,7 +63,7 @@ def render(means3d, scales, quats, colors, opacities, *, viewmat, background, im
                                  background=background, img_shape=img_shape, f=f, c=c,
                                  glob_scale=glob_scale, clip_thresh=clip_thresh,
                                  block_width=block_size, adjoint=adjoint,
-                                 isect_capacity=isect_capacity)
+                                 isect_capacity=isect_capacity, antialiased=antialiased)
     if _ops.TIGHT_TILES:
         # one projection pass also yields the opacity-limited tile rectangles
         # (of the raw opacities: compensation <= 1 only shrinks the region)

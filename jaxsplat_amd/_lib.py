@@ -143,14 +143,14 @@ _SIGS = {
     "jaxsplat_count_begin": (I32, [P, ctypes.POINTER(U64), P]),
     "jaxsplat_count_wait": (I32, [P, U64, ctypes.POINTER(ctypes.c_int32), P]),
     "jaxsplat_bin_record": (I32, [P, P, P, P]),
-    "jaxsplat_render_state_size": (SZ, [DP]),
+    "jaxsplat_render_state_size": (SZ, [DP, I32]),
     "jaxsplat_render_lists_size": (SZ, [DP, U32]),
     "jaxsplat_render_layout": (I32, [DP, U32, ctypes.POINTER(SZ)]),
-    "jaxsplat_render_begin": (I32, [DP] + [P] * 6 + [U32, P, SZ, ctypes.POINTER(U64), P]),
+    "jaxsplat_render_begin": (I32, [DP] + [P] * 6 + [U32, I32, P, SZ, ctypes.POINTER(U64), P]),
     "jaxsplat_render_count": (I32, [DP, P, U64, ctypes.POINTER(ctypes.c_int32), P]),
     "jaxsplat_render_finish": (I32, [DP, U32, P, SZ, P, U32, P, SZ, P, SZ, P, P, P, P]),
-    "jaxsplat_render_finish_backward": (I32, [DP, U32, P, P, P, P, P, SZ, P, SZ, P, U32]
-                                        + [P] * 6 + [I32, P, SZ, P]),
+    "jaxsplat_render_finish_backward": (I32, [DP, U32, P, P, P, P, P, SZ, P, SZ, P, U32,
+                                                P, I32] + [P] * 6 + [I32, P, SZ, P]),
     "jaxsplat_project_forward_splats": (I32, [DP] + [P] * 6 + [U32] + [P] * 9 + [P, SZ, P]),
     "jaxsplat_rasterize_forward_splats": (I32, [DP, P, P, U32, P, P, U32, P, P, P, P]),
     "jaxsplat_rasterize_backward_staged": (I32, [DP, P, P, U32, P, P, P, P, P, U32, P, P, P, P, P,

@@ -579,7 +579,7 @@ class _Render(torch.autograd.Function):
     @staticmethod
     def forward(ctx, cfg, means3d, scales, quats, colors, opacities, viewmat, background,
                 capacity):
-        img_shape, f, c, glob_scale, clip_thresh, block_width, adjoint = cfg
+        img_shape, f, c, glob_scale, clip_thresh, block_width, adjoint, aa = cfg
         N, nch = colors.shape
         dev = means3d.device
         H, W = img_shape
@@ -588,7 +588,7 @@ class _Render(torch.autograd.Function):
         # two buffers that the C entries lay out, kept for the backward: the
         # per-Gaussian state and the tiles' lists with the pixels' residuals
         db = ctypes.byref(d)
-        state_bytes = L.jaxsplat_render_state_size(db)
+        state_bytes = L.jaxsplat_render_state_size(db, aa)
         state = torch.empty(state_bytes // 4, dtype=torch.int32, device=dev)
         s = _stream(dev)
         ticket = ctypes.c_uint64() if capacity is None else None
@@ -596,7 +596,7 @@ class _Render(torch.autograd.Function):
         with _on(dev):
             _lib.check(L.jaxsplat_render_begin(
                 db, _p(means3d), _p(scales), _p(quats), _p(viewmat), _p(opacities), _p(colors),
-                nch, _p(state), state_bytes, ticket, s))
+                nch, aa, _p(state), state_bytes, ticket, s))
             img = torch.empty((H, W, nch), dtype=torch.float32, device=dev)
             if capacity is None:
                 count = ctypes.c_int32()
@@ -614,6 +614,7 @@ class _Render(torch.autograd.Function):
         ctx.d = d
         ctx.isect = isect
         ctx.adjoint = adjoint
+        ctx.aa = aa
         ctx.save_for_backward(means3d, scales, quats, viewmat, colors, opacities, background,
                               state, lists)
         return img
@@ -629,14 +630,17 @@ class _Render(torch.autograd.Function):
         ws, wsb = _staged_workspace(d, isect, nch, dev)
         if ws is None:
             N = means3d.shape[0]
-            xys, conics, radii, cum, rects, gids, bins, final_Ts, final_idx = _render_views(
-                d, isect, N, state, lists)
+            xys, conics, radii, cum, rects, gids, bins, final_Ts, final_idx, comp = \
+                _render_views(d, isect, N, state, lists, ctx.aa)
             v_colors, v_opacity, v_xy, v_conic = _rasterize_backward(
-                d, isect, ctx.adjoint, colors, opacities, background, xys, conics, gids,
-                bins, final_Ts, final_idx, radii, cum, rects, v_img)
+                d, isect, ctx.adjoint, colors, opacities * comp if ctx.aa else opacities,
+                background, xys, conics, gids, bins, final_Ts, final_idx, radii, cum, rects,
+                v_img)
+            v_comp = v_opacity * opacities if ctx.aa else None
+            v_opacity = v_opacity * comp if ctx.aa else v_opacity
             v_mean3d, v_scale, v_quat = _project_backward(
-                d, ctx.adjoint, means3d, scales, quats, viewmat, radii, conics, None, v_xy,
-                None, v_conic, None)
+                d, ctx.adjoint, means3d, scales, quats, viewmat, radii, conics, comp, v_xy,
+                None, v_conic, v_comp)
             return None, v_mean3d, v_scale, v_quat, v_colors, v_opacity, None, None, None
         v_img = v_img.contiguous()
         v_colors = torch.empty_like(colors)
@@ -648,7 +652,7 @@ class _Render(torch.autograd.Function):
             _lib.check(_lib.lib().jaxsplat_render_finish_backward(
                 ctypes.byref(d), isect, _p(means3d), _p(scales), _p(quats), _p(viewmat),
                 _p(state), 4 * state.numel(), _p(lists), 4 * lists.numel(), _p(background), nch,
-                _p(v_img), _p(v_colors), _p(v_opacity), _p(v_mean3d), _p(v_scale), _p(v_quat),
+                _p(opacities), ctx.aa, _p(v_img), _p(v_colors), _p(v_opacity), _p(v_mean3d), _p(v_scale), _p(v_quat),
                 ctx.adjoint, _p(ws), wsb, _stream(dev)))
         return None, v_mean3d, v_scale, v_quat, v_colors, v_opacity, None, None, None
 
@@ -660,10 +664,10 @@ def _aligned(buf):
         buf.clone(memory_format=torch.contiguous_format)
 
 
-def _render_views(d, isect, N, state, lists):
+def _render_views(d, isect, N, state, lists, aa):
     """The arrays in the fused render's buffers: (xys, conics, radii, cum,
-    rects, gids, bins, final_Ts, final_idx)."""
-    off = (ctypes.c_size_t * 10)()
+    rects, gids, bins, final_Ts, final_idx, compensation or None)."""
+    off = (ctypes.c_size_t * 11)()
     _lib.check(_lib.lib().jaxsplat_render_layout(ctypes.byref(d), isect, off))
 
     def part(buf, i, rows, cols, dtype=torch.int32):
@@ -676,15 +680,16 @@ def _render_views(d, isect, N, state, lists):
     xys = part(state, 0, N, 12, f32)[:, :2].contiguous()
     return (xys, part(state, 1, N, 3, f32), part(state, 3, N, 1), part(state, 4, N, 1),
             part(state, 5, N, 2), part(lists, 6, isect, 1), part(lists, 7, T, 2),
-            part(lists, 8, pixels, 1, f32), part(lists, 9, pixels, 1))
+            part(lists, 8, pixels, 1, f32), part(lists, 9, pixels, 1),
+            part(state, 10, N, 1, f32) if aa else None)
 
 
 def render_fused(means3d, scales, quats, colors, opacities, *, viewmat, background, img_shape, f,
                  c, glob_scale, clip_thresh, block_width, adjoint="reference",
-                 isect_capacity=None):
+                 isect_capacity=None, antialiased=False):
     """``render`` as one autograd node (``_Render``): the opacity-limited
     binning and the fused backward tail.  Same arguments and result as
-    ``render`` without the antialiased mode."""
+    ``render``, up to three channels."""
     adj = _adjoint(adjoint)
     N = means3d.shape[0] if isinstance(means3d, torch.Tensor) else -1
     nch = colors.shape[1] if isinstance(colors, torch.Tensor) and colors.dim() == 2 else 3
@@ -700,7 +705,7 @@ def render_fused(means3d, scales, quats, colors, opacities, *, viewmat, backgrou
     if isect_capacity is not None and not isinstance(isect_capacity, IsectCapacity):
         raise TypeError("isect_capacity must be an IsectCapacity")
     cfg = (tuple(img_shape), tuple(f), tuple(c), float(glob_scale), float(clip_thresh),
-           int(block_width), adj)
+           int(block_width), adj, 1 if antialiased else 0)
     return _Render.apply(cfg, means3d.contiguous(), scales.contiguous(), quats.contiguous(),
                          colors.contiguous(), opacities.contiguous(), viewmat.contiguous(),
                          background.contiguous(), isect_capacity)

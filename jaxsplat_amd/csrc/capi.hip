@@ -174,7 +174,8 @@ int project_splats(const jaxsplat_descriptor* d, const float* means3d, const flo
                    const float* colors, uint32_t channels, float* xys, float* depths,
                    int32_t* radii, float* conics, float* compensation, int32_t* num_tiles_hit,
                    int32_t* cum_tiles_hit, uint32_t* tile_rects, float* splats, void* workspace,
-                   size_t workspace_bytes, uint64_t* count_out, uint32_t ticket, void* stream) {
+                   size_t workspace_bytes, uint64_t* count_out, uint32_t ticket,
+                   bool antialiased, void* stream) {
     if (int st = validate(d)) return st;
     if (channels < 1 || channels > 3)
         return fail(JAXSPLAT_ERR_INVALID,
@@ -191,7 +192,8 @@ int project_splats(const jaxsplat_descriptor* d, const float* means3d, const flo
                                    cum_tiles_hit, opacities,
                                    reinterpret_cast<uint2*>(tile_rects), workspace,
                                    static_cast<hipStream_t>(stream), colors, (int)channels,
-                                   reinterpret_cast<float4*>(splats), count_out, ticket),
+                                   reinterpret_cast<float4*>(splats), count_out, ticket,
+                                   antialiased),
                   "project_forward_splats");
     return JAXSPLAT_OK;
 }
@@ -342,7 +344,8 @@ int jaxsplat_project_forward_splats(const jaxsplat_descriptor* d, const float* m
     g_err.clear();
     return project_splats(d, means3d, scales, quats, viewmat, opacities, colors, channels, xys,
                           depths, radii, conics, compensation, num_tiles_hit, cum_tiles_hit,
-                          tile_rects, splats, workspace, workspace_bytes, nullptr, 0u, stream);
+                          tile_rects, splats, workspace, workspace_bytes, nullptr, 0u, false,
+                          stream);
 }
 
 int jaxsplat_project_backward(const jaxsplat_descriptor* d, const float* means3d,
@@ -767,15 +770,21 @@ int jaxsplat_rasterize_backward_staged_nd(
     return JAXSPLAT_OK;
 }
 
-int jaxsplat_render_backward(
+}  // extern "C"
+
+namespace {
+
+// jaxsplat_render_backward; opacities and compensation (optional, both): of an
+// antialiased render.
+int render_backward(
     const jaxsplat_descriptor* d, const int32_t* gaussian_ids_sorted, const int32_t* tile_bins,
     uint32_t num_intersects, const float* means3d, const float* scales, const float* quats,
     const float* viewmat, const float* splats, const float* conics, const float* background,
     uint32_t channels, const int32_t* radii, const uint32_t* tile_rects,
     const int32_t* cum_tiles_hit, const float* final_Ts, const int32_t* final_idx,
     const float* v_out_img, float* v_colors, float* v_opacity, float* v_mean3d, float* v_scale,
-    float* v_quat, int adjoint, void* workspace, size_t workspace_bytes, void* stream) {
-    g_err.clear();
+    float* v_quat, int adjoint, void* workspace, size_t workspace_bytes, void* stream,
+    const float* opacities, const float* compensation) {
     if (int st = validate(d)) return st;
     if (channels < 1 || channels > 3)
         return fail(JAXSPLAT_ERR_INVALID, "render_backward: channels must be in [1, 3], got %u",
@@ -810,9 +819,29 @@ int jaxsplat_render_backward(
     JSA_CHECK_HIP(jsa::render_bwd_tail(c, (int)channels, (int)num_intersects, means3d, scales,
                                        quats, viewmat, radii, rects, cum_tiles_hit, conics,
                                        workspace, v_colors, v_opacity, v_mean3d, v_scale, v_quat,
-                                       consistent, s),
+                                       consistent, s, opacities, compensation),
                   "render_backward (tail)");
     return JAXSPLAT_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int jaxsplat_render_backward(
+    const jaxsplat_descriptor* d, const int32_t* gaussian_ids_sorted, const int32_t* tile_bins,
+    uint32_t num_intersects, const float* means3d, const float* scales, const float* quats,
+    const float* viewmat, const float* splats, const float* conics, const float* background,
+    uint32_t channels, const int32_t* radii, const uint32_t* tile_rects,
+    const int32_t* cum_tiles_hit, const float* final_Ts, const int32_t* final_idx,
+    const float* v_out_img, float* v_colors, float* v_opacity, float* v_mean3d, float* v_scale,
+    float* v_quat, int adjoint, void* workspace, size_t workspace_bytes, void* stream) {
+    g_err.clear();
+    return render_backward(d, gaussian_ids_sorted, tile_bins, num_intersects, means3d, scales,
+                           quats, viewmat, splats, conics, background, channels, radii,
+                           tile_rects, cum_tiles_hit, final_Ts, final_idx, v_out_img, v_colors,
+                           v_opacity, v_mean3d, v_scale, v_quat, adjoint, workspace,
+                           workspace_bytes, stream, nullptr, nullptr);
 }
 
 int jaxsplat_rasterize_forward_splats(const jaxsplat_descriptor* d,
@@ -968,9 +997,9 @@ int jaxsplat_bin_record(const void* workspace, int32_t* err, int64_t* total, voi
 namespace {
 
 struct RenderState {
-    size_t splats, conics, depths, radii, cum, rects, ws, ws_bytes, end;
+    size_t splats, conics, depths, radii, cum, rects, comp, ws, ws_bytes, end;
 };
-RenderState render_state(const jaxsplat_descriptor* d) {
+RenderState render_state(const jaxsplat_descriptor* d, int antialiased) {
     const size_t n = d->num_points ? d->num_points : 1;
     RenderState r;
     size_t o = 0;
@@ -980,6 +1009,7 @@ RenderState render_state(const jaxsplat_descriptor* d) {
     r.radii = o; o = align256(o + 4 * n);
     r.cum = o; o = align256(o + 4 * n);
     r.rects = o; o = align256(o + 8 * n);
+    r.comp = o; o = align256(o + (antialiased ? 4 * n : 0));
     r.ws = o;
     r.ws_bytes = jaxsplat_project_workspace_size(d);
     r.end = align256(o + r.ws_bytes);
@@ -1016,8 +1046,8 @@ bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) !
 
 extern "C" {
 
-size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d) {
-    return d && !validate(d) ? render_state(d).end : 0;
+size_t jaxsplat_render_state_size(const jaxsplat_descriptor* d, int antialiased) {
+    return d && !validate(d) ? render_state(d, antialiased).end : 0;
 }
 
 size_t jaxsplat_render_lists_size(const jaxsplat_descriptor* d, uint32_t num_intersects) {
@@ -1029,21 +1059,22 @@ int jaxsplat_render_layout(const jaxsplat_descriptor* d, uint32_t num_intersects
     g_err.clear();
     if (int st = validate(d)) return st;
     if (!offsets) return fail(JAXSPLAT_ERR_INVALID, "render_layout: offsets is NULL");
-    const RenderState r = render_state(d);
+    const RenderState r = render_state(d, 1);
     const RenderLists l = render_lists(d, num_intersects);
-    const size_t all[10] = {r.splats, r.conics, r.depths, r.radii, r.cum,
-                            r.rects, l.gids, l.bins, l.final_ts, l.final_idx};
-    std::copy(all, all + 10, offsets);
+    const size_t all[11] = {r.splats, r.conics, r.depths, r.radii, r.cum, r.rects,
+                            l.gids, l.bins, l.final_ts, l.final_idx, r.comp};
+    std::copy(all, all + 11, offsets);
     return JAXSPLAT_OK;
 }
 
 int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
                           const float* scales, const float* quats, const float* viewmat,
                           const float* opacities, const float* colors, uint32_t channels,
-                          void* state, size_t state_bytes, uint64_t* ticket, void* stream) {
+                          int antialiased, void* state, size_t state_bytes, uint64_t* ticket,
+                          void* stream) {
     g_err.clear();
     if (int st = validate(d)) return st;
-    const RenderState r = render_state(d);
+    const RenderState r = render_state(d, antialiased);
     if (!state || misaligned(state) || state_bytes < r.end)
         return fail(JAXSPLAT_ERR_WORKSPACE, "render_begin: state too small or misaligned");
     if (ticket) {
@@ -1056,10 +1087,12 @@ int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
     const bool count = ticket && d->num_points > 0;
     return project_splats(d, means3d, scales, quats, viewmat, opacities, colors, channels,
                           nullptr, at<float>(state, r.depths), at<int32_t>(state, r.radii),
-                          at<float>(state, r.conics), nullptr, nullptr,
+                          at<float>(state, r.conics),
+                          antialiased ? at<float>(state, r.comp) : nullptr, nullptr,
                           at<int32_t>(state, r.cum), at<uint32_t>(state, r.rects),
                           at<float>(state, r.splats), at<void>(state, r.ws), r.ws_bytes,
-                          count ? t_count.dev : nullptr, count ? t_count.ticket : 0u, stream);
+                          count ? t_count.dev : nullptr, count ? t_count.ticket : 0u,
+                          antialiased != 0, stream);
 }
 
 int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint64_t ticket,
@@ -1072,7 +1105,7 @@ int jaxsplat_render_count(const jaxsplat_descriptor* d, const void* state, uint6
         *num_intersects = 0;
         return JAXSPLAT_OK;
     }
-    return jaxsplat_count_wait(at<int32_t>(state, render_state(d).cum) + (d->num_points - 1),
+    return jaxsplat_count_wait(at<int32_t>(state, render_state(d, 0).cum) + (d->num_points - 1),
                                ticket, num_intersects, stream);
 }
 
@@ -1085,7 +1118,7 @@ int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects
     if (int st = validate(d)) return st;
     if (num_intersects >= (1u << 30))
         return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
-    const RenderState r = render_state(d);
+    const RenderState r = render_state(d, 0);
     const RenderLists l = render_lists(d, num_intersects);
     if (!state || misaligned(state) || state_bytes < r.end || !lists || misaligned(lists) ||
         lists_bytes < l.end)
@@ -1110,7 +1143,8 @@ int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_i
                                     const float* quats, const float* viewmat,
                                     const void* state, size_t state_bytes, const void* lists,
                                     size_t lists_bytes, const float* background,
-                                    uint32_t channels, const float* v_out_img,
+                                    uint32_t channels, const float* opacities,
+                                    int antialiased, const float* v_out_img,
                                     float* v_colors, float* v_opacity, float* v_mean3d,
                                     float* v_scale, float* v_quat, int adjoint,
                                     void* workspace, size_t workspace_bytes, void* stream) {
@@ -1118,19 +1152,22 @@ int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_i
     if (int st = validate(d)) return st;
     if (num_intersects >= (1u << 30))
         return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
-    const RenderState r = render_state(d);
+    const RenderState r = render_state(d, antialiased);
     const RenderLists l = render_lists(d, num_intersects);
     if (!state || misaligned(state) || state_bytes < r.end || !lists || misaligned(lists) ||
         lists_bytes < l.end)
         return fail(JAXSPLAT_ERR_WORKSPACE,
                     "render_finish_backward: buffer too small or misaligned");
-    return jaxsplat_render_backward(
+    if (antialiased && d->num_points > 0 && !opacities)
+        return fail(JAXSPLAT_ERR_INVALID, "render_finish_backward: NULL required pointer");
+    return render_backward(
         d, at<int32_t>(lists, l.gids), at<int32_t>(lists, l.bins), num_intersects, means3d,
         scales, quats, viewmat, at<float>(state, r.splats), at<float>(state, r.conics),
         background, channels, at<int32_t>(state, r.radii), at<uint32_t>(state, r.rects),
         at<int32_t>(state, r.cum), at<float>(lists, l.final_ts), at<int32_t>(lists, l.final_idx),
         v_out_img, v_colors, v_opacity, v_mean3d, v_scale, v_quat, adjoint, workspace,
-        workspace_bytes, stream);
+        workspace_bytes, stream, antialiased ? opacities : nullptr,
+        antialiased ? at<float>(state, r.comp) : nullptr);
 }
 
 int jaxsplat_rasterize_backward_staged_rects(

@@ -559,7 +559,8 @@ hipError_t project_fwd(const Camera& c, const float* means3d, const float* scale
                        float* compensation, int* num_tiles_hit, int* cum_tiles_hit,
                        const float* opacities, uint2* rects, void* scratch, hipStream_t s,
                        const float* colors = nullptr, int nch = 0, float4* splats = nullptr,
-                       uint64_t* count_out = nullptr, uint32_t ticket = 0);
+                       uint64_t* count_out = nullptr, uint32_t ticket = 0,
+                       bool antialiased = false);
 // Opacity-limited tile rectangles (opacity_tile_rect) of projected Gaussians,
 // their counts (num_tiles_hit optional) and inclusive sums; scratch
 // project_fwd_scratch_bytes(c.num_points).
@@ -585,7 +586,9 @@ hipError_t render_bwd_tail(const Camera& c, int nch, int num_isect, const float*
                            const int* radii, const uint2* rects, const int* cum,
                            const float* conics, const void* ws, float* v_colors,
                            float* v_opacity, float* v_mean3d, float* v_scale, float* v_quat,
-                           int consistent, hipStream_t s);
+                           int consistent, hipStream_t s,
+                           const float* opacities = nullptr,
+                           const float* compensation = nullptr);
 
 // ---- LSD radix sort (uint32 keys, uint32 values) ----
 // Partitions up to which a scatter sums the counts of all partitions itself

@@ -119,3 +119,33 @@ def test_capturing_stream_refuses_the_read():
     t.cuda.synchronize()
     assert _same(_step(p, size, cap), want) and _same(_step(p, size), want)
     assert cap.check() > 0
+
+
+@pytest.mark.parametrize("adjoint", ["reference", "consistent"])
+@pytest.mark.parametrize("nch", [1, 3])
+@pytest.mark.parametrize("size", SIZES, ids=str)
+def test_antialiased_fused_equals_composition(size, nch, adjoint, monkeypatch):
+    """The antialiased render as one node: images and gradients bit for bit those
+    of the projection, the product and the rasterization as separate nodes."""
+    t = H.torch()
+    h, w = size
+    params = _scene(5)
+    params[1] = params[1] * 0.2         # footprints below a pixel: compensation well below 1
+    params[3] = params[3][:, :nch].contiguous()
+    v = t.linspace(-1, 1, h * w * nch, device="cuda").view(h, w, nch)
+
+    def step(staged=True):
+        monkeypatch.setattr(_ops, "STAGED_BACKWARD", staged)
+        p = [x.detach().requires_grad_(True) for x in params]
+        img = render(*p, viewmat=H.dev(scenes.IDENTITY), background=v[0, 0].abs().contiguous(),
+                     img_shape=size, f=(float(w), float(w)), c=(w / 2, h / 2), glob_scale=1.0,
+                     clip_thresh=0.01, adjoint=adjoint, antialiased=True)
+        return [img.detach()] + list(t.autograd.grad(img, p, v))
+
+    fused, atomic = step(), step(staged=False)
+    monkeypatch.setattr(_ops, "FUSED_RENDER", False)
+    separate = step()
+    assert _same(fused, separate)
+    for g, s in zip(atomic, separate):
+        ref = H.host(s).astype(np.float64)
+        assert np.all(np.abs(H.host(g) - ref) <= 1e-5 * np.abs(ref) + 1e-6 * np.abs(ref).max())
