@@ -206,7 +206,7 @@ def main():
 # ---------------------------------------------------------------------------
 # Committed counter summaries (rocprofv3) and their validity
 # ---------------------------------------------------------------------------
-RENDER_BWD = "raster_bwd_kernel<*, *, *, true, *> + render_bwd_tail_kernel"
+RENDER_BWD = "raster_bwd_kernel<*, *, *, true, *, 3> + render_bwd_tail_kernel<false>"
 
 
 def source_hash():
@@ -460,21 +460,32 @@ def stage_breakdown(torch, sc, cam, params, target, iters):
     # colour) and writes 80 (depth, radius, conic, inclusive sum, rectangle,
     # 48-byte splat record) + 8 of scan; a staged list entry costs
     # its id and its splat record (52 B), in the backward also its inclusive
-    # sum; a flushed record is 36 B.
+    # sum; a flushed record is 36 B.  Binning by tile rows: "emission" reads the
+    # rectangles twice and writes a run of 8 B per tile row of a rectangle,
+    # "tile_sort" reads the runs twice and writes an id per pair; with many pairs
+    # per Gaussian and per tile (csrc/bin.hip), "emission" is led by a depth sort
+    # of the Gaussians (four passes of 20 B) and the lists are then in order.
+    # Small grids and more than 256 tiles per axis emit and sort the pairs.
+    by_rows = T > 256 and max(d.grid_dim_2d.x, d.grid_dim_2d.y) <= 256
+    by_depth = by_rows and isect > 16 * N and isect > 640 * T
+    runs = int((rects[:, 1] >> 16).sum().item())
     stage_bytes = {
         "project_fwd": 144 * N,
-        "emission": 24 * N + 8 * isect,
-        "tile_sort": 40 * isect,
-        "bin_edges": 4 * isect + 8 * T,
-        "tile_depth_sort": 12 * isect + 8 * T,
+        "emission": (16 + 84 * by_depth) * N + 8 * runs if by_rows else 24 * N + 8 * isect,
+        "tile_sort": 16 * runs + 4 * isect + 8 * T if by_rows else 40 * isect,
+        "bin_edges": 0 if by_rows else 4 * isect + 8 * T,
+        "tile_depth_sort": 0 if by_depth else 12 * isect + 8 * T,
         "raster_fwd": 52 * L_ft + 8 * T + 20 * Px,
         "loss_grad": 36 * Px,
         "raster_bwd_records": 56 * L_bt + 8 * T + 20 * Px + 36 * R + (isect + 7) // 8,
         "bwd_tail": 36 * R + (isect + 7) // 8 + 16 * N + 56 * V + 4 * (N - V) + 40 * N,
     }
     # the raster kernels are bound by VALU issue, the per-tile depth sort by
-    # the latency of its LDS ranking rounds and barriers, the rest by HBM
+    # the latency of its LDS ranking rounds and barriers, the binning by tile
+    # rows by its LDS accesses, the rest by HBM
     bound_by = {"raster_fwd": "valu", "raster_bwd_records": "valu", "tile_depth_sort": "lds"}
+    if by_rows:
+        bound_by.update(emission="lds", tile_sort="lds")
     stages = {}
     for k in names:
         ms_k = acc[k]
@@ -501,9 +512,9 @@ def stage_breakdown(torch, sc, cam, params, target, iters):
             "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5),
             "traffic": None, "avg_ms": round(ms_bwd, 4), "bytes_per_launch": int(bytes_bwd)}
     if counters is not None:
-        kr = _kernel_entry(counters, "jsa::raster_bwd_kernel<false, false, 64, true, 4>")
-        kd = _kernel_entry(counters, "jsa::render_bwd_tail_kernel")
-        kf = _kernel_entry(counters, "jsa::raster_fwd_kernel<256>")
+        kr = _kernel_entry(counters, "jsa::raster_bwd_kernel<false, false, 64, true, 4, 3>")
+        kd = _kernel_entry(counters, "jsa::render_bwd_tail_kernel<false>")
+        kf = _kernel_entry(counters, "jsa::raster_fwd_kernel<256, 3>")
         if kr and kd and kr.get("hbm_bytes") and kd.get("hbm_bytes"):
             roof["traffic"] = int(kr["hbm_bytes"] + kd["hbm_bytes"])
             roof["traffic_over_alg"] = round(roof["traffic"] / bytes_bwd, 3)
