@@ -1217,7 +1217,8 @@ hipError_t bin_and_sort(const BinPlan& p, const Camera& c, const float* xys, con
 // Batched binning (items of many views; see ViewRec)
 // ---------------------------------------------------------------------------
 // Items are numbered view by view (ViewRec::item_off), so the item order is
-// the (view, item) order:
+// the (view, item) order.  Up to 256 tiles per axis: by tile rows (batch_row_bin),
+// then step 5 below.  Larger grids:
 //  1. view_keys: every item's view;
 //  2. emission (BATCH) in item order: keys view << tile_bits | tile, values =
 //     item ids, with the total and the clamped count published on the device;
@@ -1231,16 +1232,25 @@ struct BatchLayout {
     size_t err, count, total, zero_end;
     size_t tile_sort, vkeys, keys, vals, ttmp_k, ttmp_v, keys_sorted, end;
     EmitLayout emit;
+    size_t rows, runs, kv;      // by_rows (as for one view)
 };
 
 BatchLayout batch_layout(const BatchBinPlan& p) {
-    BatchLayout L;
+    BatchLayout L{};
     size_t o = 0;
     L.err = o; o += 16;
     L.count = o; o += 16;
     L.total = o; o += 16;
     L.zero_end = o;
     o = align256(o);
+    if (p.by_rows) {
+        const size_t c4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
+        L.rows = o; o = align256(o + p.rows.scratch_bytes);
+        L.runs = o; o += 2 * c4;
+        L.kv = o; o += 2 * c4;
+        L.end = o;
+        return L;
+    }
     L.tile_sort = o; o = align256(o + p.tile_sort.scratch_bytes);
     o = emit_layout(o, p.n_items, p.isect_cap, true, L.emit);
     const size_t n4 = align256(4ull * (p.n_items > 0 ? p.n_items : 1));
@@ -1257,8 +1267,9 @@ BatchLayout batch_layout(const BatchBinPlan& p) {
 
 }  // namespace
 
-BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int isect_cap) {
-    BatchBinPlan p;
+BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int max_x,
+                            int max_y, int isect_cap) {
+    BatchBinPlan p{};
     p.n_items = n_items;
     p.num_views = num_views;
     p.isect_cap = isect_cap;
@@ -1266,6 +1277,8 @@ BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int 
     p.view_bits = bitlen((uint32_t)(num_views > 1 ? num_views - 1 : 0));
     p.num_bins = num_views << p.tile_bits;
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
+    p.by_rows = max_x <= kRowBinAxis && max_y <= kRowBinAxis && num_views <= kMaxBatchViews;
+    if (p.by_rows) p.rows = batch_row_plan(num_views, parts, max_x, max_y, isect_cap);
     p.scratch_bytes = batch_layout(p).end;
     return p;
 }
@@ -1290,15 +1303,27 @@ hipError_t batch_bin(const BatchBinPlan& p, const ViewRec* views, const uint2* i
                      uint32_t* item_first, void* scratch, hipStream_t s) {
     const BatchLayout L = batch_layout(p);
     uint8_t* b = static_cast<uint8_t*>(scratch);
-    hipError_t e = fill_zero(b, L.zero_end, s);
-    if (e != hipSuccess) return e;
+    uint32_t* err = reinterpret_cast<uint32_t*>(b + L.err);
+    int* count = reinterpret_cast<int*>(b + L.count);
+    auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
+    hipError_t e;
+    if (p.by_rows && p.n_items > 0) {
+        uint32_t* ids = reinterpret_cast<uint32_t*>(items_sorted);
+        int2* bins = reinterpret_cast<int2*>(tile_bins);
+        e = batch_row_bin(p.rows, views, item_rects, reinterpret_cast<uint2*>(b + L.runs), ids,
+                          p.num_bins, bins, item_first, count,
+                          reinterpret_cast<unsigned long long*>(b + L.total), err, b + L.rows,
+                          s);
+        if (e != hipSuccess) return e;
+        const size_t c4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
+        return tile_depth_order(bins, p.num_bins, p.isect_cap, true, depth_keys, ids, U(L.runs),
+                                U(L.runs + c4), reinterpret_cast<uint2*>(b + L.kv), s);
+    }
+    if ((e = fill_zero(b, L.zero_end, s)) != hipSuccess) return e;
     e = fill_zero(tile_bins, 8ull * p.num_bins, s);
     if (e != hipSuccess) return e;
     if (p.n_items <= 0) return hipSuccess;
     if (p.num_views > kMaxBatchViews) return hipErrorInvalidValue;
-    uint32_t* err = reinterpret_cast<uint32_t*>(b + L.err);
-    int* count = reinterpret_cast<int*>(b + L.count);
-    auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
 
     view_keys_kernel<<<(p.n_items + 255) / 256, 256, 0, s>>>(nullptr, p.n_items, nullptr, views,
                                                               p.num_views, U(L.vkeys));

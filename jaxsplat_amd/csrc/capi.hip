@@ -1477,7 +1477,8 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
         return fail(JAXSPLAT_ERR_INVALID, "too many Gaussians (%lld)", g);
     }
     b->n_gauss = (int)g;
-    long long items = 0, tiles = 0, pix = 0;
+    long long items = 0, tiles = 0, pix = 0, parts = 0;
+    int max_x = 1, max_y = 1;
     int prev_scene = 0;
     for (int s = 0; s < num_scenes; ++s) b->scenes[s].v_begin = b->scenes[s].v_end = 0;
     for (int v = 0; v < num_views; ++v) {
@@ -1511,6 +1512,10 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
         r.tile_off = (int)tiles;
         r.view = v;
         r.pix_off = pix;
+        r.part_off = (int)parts;
+        parts += (r.n + jsa::kRowBinPart - 1) / jsa::kRowBinPart;
+        max_x = std::max(max_x, r.tiles_x);
+        max_y = std::max(max_y, r.tiles_y);
         items += r.n;
         tiles += (long long)r.tiles_x * r.tiles_y;
         pix += (long long)w.img_w * w.img_h;
@@ -1526,7 +1531,8 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
     b->n_items = (int)items;
     b->total_tiles = (int)tiles;
     b->num_pixels = pix;
-    b->bin = jsa::batch_bin_plan(b->n_items, num_views, b->max_view_tiles, (int)isect_capacity);
+    b->bin = jsa::batch_bin_plan(b->n_items, num_views, b->max_view_tiles, (int)parts,
+                                 max_x, max_y, (int)isect_capacity);
     if (b->bin.tile_bits + b->bin.view_bits > 31) {
         delete b;
         return fail(JAXSPLAT_ERR_INVALID, "views x tiles exceed 2^31 bins");

@@ -477,7 +477,8 @@ struct alignas(16) ViewRec {
     int bin_off;          // first tile bin (view << tile_bits)
     int view;             // row of viewmats and backgrounds
     long long pix_off;    // first pixel in the image-sized buffers
-    long long reserved;
+    int part_off;         // first binning partition (kRowBinPart items)
+    int reserved;
 };
 static_assert(sizeof(ViewRec) == 80, "ViewRec layout");
 
@@ -646,7 +647,8 @@ hipError_t sort_pairs(const SortPlan& p, const uint32_t* keys_in, const uint32_t
 hipError_t column_scan(uint32_t* counts, int parts, uint32_t* totals, int columns, hipStream_t s);
 
 // ---- binning by tile rows (rowbin.hip) ----
-constexpr int kRowBinAxis = 256;    // tiles per axis, at most
+constexpr int kRowBinAxis = 256;
+constexpr int kRowBinPart = 1024;       // Gaussians or runs per partition    // tiles per axis, at most
 struct RowBinPlan {
     int n, tiles_x, tiles_y, cap;
     int parts;              // partitions of the Gaussians
@@ -668,6 +670,22 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
                    uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
                    int2* bins, unsigned long long* total, uint32_t* err, void* scratch,
                    hipStream_t s);
+
+// The same over the items of a batch's views (tile counts up to kRowBinAxis per
+// axis, ViewRec::part_off set, parts in all): bins[view's bin_off + tile] (all
+// num_bins cleared first), ids in arbitrary order inside a list, *count = min(
+// *total, cap), and every item's first pair in item order (item_first, optional;
+// at most cap).
+struct BatchRowPlan {
+    int num_views, parts, max_x, max_y, rows, cap, max_col_parts;
+    size_t counts, part_tot, part_pair, row_first, row_off, row_part, row_pair, tile_first, desc,
+        col_counts, scratch_bytes;
+};
+BatchRowPlan batch_row_plan(int num_views, int parts, int max_x, int max_y, int cap);
+hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint2* rects,
+                         uint2* runs, uint32_t* ids, int num_bins, int2* bins,
+                         uint32_t* item_first, int* count, unsigned long long* total,
+                         uint32_t* err, void* scratch, hipStream_t s);
 
 // ---- binning ----
 struct BinPlan {
@@ -744,9 +762,14 @@ struct BatchBinPlan {
     int tile_bits, view_bits;
     int num_bins;       // num_views << tile_bits
     SortPlan tile_sort;
+    bool by_rows;       // batch_row_bin
+    BatchRowPlan rows;
     size_t scratch_bytes;
 };
-BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int isect_cap);
+// parts: binning partitions of all views (ViewRec::part_off); max_x, max_y: the
+// largest tile counts per axis.
+BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int max_x,
+                            int max_y, int isect_cap);
 // Sorted item ids of every (view, tile) and bins[view << tile_bits | tile].
 // The scratch keeps the intersection count clamped to the capacity (the
 // length the sorts and bins use), the exact total (64 bits) and an error word:

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256) void tile_rects_kernel(
 // at 1M Gaussians), so no separate scan kernel runs between the projection and
 // this one.  Partitions are one workgroup of the projection, a Gaussian per lane:
 // four per lane left CUs without work up to 260k Gaussians and took 11 us at any
-// size below that (now 5; 3M: 101 + 10 us, now 89 + 11).  count_out (optional):
+// size below that (now 5; 3M: 101 + 10 us with this kernel, now 89 + 14).  count_out (optional):
 // where the last count goes for the host, with its ticket.
 __global__ __launch_bounds__(256) void project_scan_add_kernel(
     int n, int parts, int per, const uint32_t* __restrict__ part_tot,
@@ -419,6 +419,7 @@ __global__ __launch_bounds__(256) void project_scan_add_kernel(
     const int tid = threadIdx.x;
     const int p = blockIdx.x * per;
     uint32_t sum = 0;
+#pragma unroll 8
     for (int q = tid; q < p; q += 256) sum += part_tot[q];
     sum = wave_inclusive_sum(sum);
     if (lane_id() == 63) s_w[tid >> 6] = sum;

@@ -42,7 +42,7 @@ namespace {
 
 constexpr int kRbThreads = 256;
 constexpr int kRbWaves = kRbThreads / kWave;
-constexpr int kRbPart = 1024;                       // intervals per partition
+constexpr int kRbPart = kRowBinPart;                // intervals per partition
 constexpr int kRbPer = kRbPart / kRbThreads;        // and per lane
 static_assert(kRowBinAxis == kRbThreads, "one thread per column");
 
@@ -446,12 +446,35 @@ __device__ __forceinline__ void for_partitions(int total, F body) {
     }
 }
 
+// counts[column] = the runs [begin, end) that cover the column, all 256 of them.
+// Called by the whole workgroup.
+__device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, int begin, int end,
+                                              int* s_d, uint32_t* s_tmp,
+                                              uint32_t* __restrict__ counts) {
+    const int tid = threadIdx.x;
+    uint32_t w[kRbPer];
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = begin + k * kRbThreads + tid;
+        w[k] = i < end ? runs[i].y : 0u;
+    }
+    s_d[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k)
+        add_differences(s_d, kRbThreads, {(int)(w[k] & 0xFFFFu), (int)(w[k] >> 16)});
+    __syncthreads();
+    const uint32_t d = (uint32_t)s_d[tid];
+    const uint32_t c = block_exclusive_scan256(d, s_tmp) + d;
+    counts[tid] = c;
+}
+
 // Step 2, counting: counts[p * 256 + column] = the runs of partition p that
 // cover the column; desc[p] = (row, first run, end, whether it is the row's
 // first partition), desc[-1].x the number of partitions.
 __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
-    const uint2* __restrict__ runs, const uint32_t* __restrict__ row_len, int tiles_x,
-    int tiles_y, int cap, uint32_t* __restrict__ counts, int4* __restrict__ desc) {
+    const uint2* __restrict__ runs, const uint32_t* __restrict__ row_len, int tiles_y, int cap,
+    uint32_t* __restrict__ counts, int4* __restrict__ desc) {
     __shared__ RowTable rt;
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
@@ -464,35 +487,81 @@ __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
         const int begin = rt.e0[r] + (p - rt.p0[r]) * kRbPart;
         const int end = min(rt.e0[r + 1], begin + kRbPart);
         if (tid == 0) desc[p] = make_int4(r, begin, end, p == rt.p0[r] ? 1 : 0);
-        uint32_t w[kRbPer];
-#pragma unroll
-        for (int k = 0; k < kRbPer; ++k) {
-            const int i = begin + k * kRbThreads + tid;
-            w[k] = i < end ? runs[i].y : 0u;
-        }
-        s_d[tid] = 0;
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < kRbPer; ++k)
-            add_differences(s_d, kRbThreads, {(int)(w[k] & 0xFFFFu), (int)(w[k] >> 16)});
-        __syncthreads();
-        const uint32_t d = (uint32_t)s_d[tid];
-        const uint32_t c = block_exclusive_scan256(d, s_tmp) + d;
-        if (tid < tiles_x) counts[(size_t)p * kRowBinAxis + tid] = c;
+        count_columns(runs, begin, end, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
     });
 }
+
+constexpr int kScanThreads = 1024;
+struct ScanShared {
+    uint32_t sum[kScanThreads];
+    uint64_t w[kRbWaves];
+};
+// The counts of partitions [p0, p0 + parts), 256 columns each of which the first
+// COLS may be set, become each partition's first position in its column's list,
+// relative to the columns' first; first_out[c] the column's first position, [256]
+// the total (all at most cap).  1024 / COLS groups of threads share the
+// partitions, whose loads are what it waits for (489 partitions of 50 rows: 26 us
+// with four groups of 256 columns, 11 with sixteen of 64).
+template <int COLS>
+__device__ __forceinline__ void scan_columns(ScanShared& sh, int p0, int parts, int cap,
+                                             uint32_t* __restrict__ counts,
+                                             uint32_t* __restrict__ first_out) {
+    constexpr int kGroups = kScanThreads / COLS;
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+    const int c = tid & (COLS - 1), g = tid / COLS;
+    const uint64_t lim = (uint64_t)cap;
+    const int q0 = p0 + (int)((long long)parts * g / kGroups);
+    const int q1 = p0 + (int)((long long)parts * (g + 1) / kGroups);
+    uint32_t sum = 0;
+#pragma unroll 8
+    for (int q = q0; q < q1; ++q) sum += counts[(size_t)q * kRowBinAxis + c];
+    sh.sum[tid] = sum;
+    __syncthreads();
+    uint64_t total = 0, before = 0;
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) {
+        const uint32_t v = sh.sum[k * COLS + c];
+        before += k < g ? v : 0u;
+        total += v;
+    }
+    // exclusive over the columns (every group computes the same)
+    const uint64_t incl = wave_inclusive_sum(total);
+    if (g == 0 && lane == kWave - 1) sh.w[wave] = incl;
+    __syncthreads();
+    uint64_t first = incl - total, all = 0;
+#pragma unroll
+    for (int w = 0; w < COLS / kWave; ++w) {
+        first += w < (c >> 6) ? sh.w[w] : 0u;
+        all += sh.w[w];
+    }
+    if (tid <= kRowBinAxis) first_out[tid] = (uint32_t)min(tid < COLS ? first : all, lim);
+    uint64_t run = first + before;
+#pragma unroll 8
+    for (int q = q0; q < q1; ++q) {
+        const size_t at = (size_t)q * kRowBinAxis + c;
+        const uint32_t v = counts[at];
+        counts[at] = (uint32_t)min(run, lim);
+        run += v;
+    }
+}
+// The instantiation for columns [0, n).
+#define JSA_SCAN(n, LAUNCH)                                                                   \
+    do {                                                                                      \
+        if ((n) <= 64) LAUNCH(64);                                                            \
+        else if ((n) <= 128) LAUNCH(128);                                                     \
+        else LAUNCH(256);                                                                     \
+    } while (0)
 
 // Step 2, offsets, one workgroup per row: counts become each partition's first
 // position in the column's list, relative to the row's first pair;
 // tile_first[row * 257 + column] the tile's first position, [.. + 256] the
-// row's pairs (all at most cap).  Four groups of 256 threads share the row's
-// partitions.
-constexpr int kRbGroups = 4;
-__global__ __launch_bounds__(kRbThreads * kRbGroups) void col_scan_kernel(
-    const uint32_t* __restrict__ row_len, int tiles_x, int tiles_y, int cap,
+// row's pairs (all at most cap).
+template <int COLS>
+__global__ __launch_bounds__(kScanThreads) void col_scan_kernel(
+    const uint32_t* __restrict__ row_len, int tiles_y, int cap,
     uint32_t* __restrict__ counts, uint32_t* __restrict__ tile_first) {
-    __shared__ uint32_t s_sum[kRbGroups][kRowBinAxis];
-    __shared__ uint64_t s_w[kRbWaves], s_e[kRbWaves], s_p[kRbWaves];
+    __shared__ ScanShared sh;
+    __shared__ uint64_t s_e[kRbWaves], s_p[kRbWaves];
     __shared__ int s_range[2];
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const int c = tid & (kRowBinAxis - 1), g = tid / kRowBinAxis, row = blockIdx.x;
@@ -521,44 +590,8 @@ __global__ __launch_bounds__(kRbThreads * kRbGroups) void col_scan_kernel(
         }
     }
     __syncthreads();
-    const int p0 = s_range[0], parts = s_range[1] - p0;
-    const int q0 = p0 + parts * g / kRbGroups, q1 = p0 + parts * (g + 1) / kRbGroups;
-    const bool on = c < tiles_x;
-    uint32_t sum = 0;
-    if (on) {
-#pragma unroll 8
-        for (int q = q0; q < q1; ++q) sum += counts[(size_t)q * kRowBinAxis + c];
-    }
-    s_sum[g][c] = sum;
-    __syncthreads();
-    uint64_t total = 0, before = 0;
-#pragma unroll
-    for (int k = 0; k < kRbGroups; ++k) {
-        const uint32_t v = s_sum[k][c];
-        before += k < g ? v : 0u;
-        total += v;
-    }
-    // exclusive over the columns (every group computes the same)
-    const uint64_t incl = wave_inclusive_sum(total);
-    if (g == 0 && lane == kWave - 1) s_w[wave] = incl;
-    __syncthreads();
-    uint64_t first = incl - total;
-    for (int w = 0; w < (c >> 6); ++w) first += s_w[w];
-    if (g == 0) {
-        uint32_t* tf = tile_first + (size_t)row * (kRowBinAxis + 1);
-        tf[c] = (uint32_t)min(first, lim);
-        if (c == kRowBinAxis - 1) tf[kRowBinAxis] = (uint32_t)min(first + total, lim);
-    }
-    uint64_t run = first + before;
-    if (on) {
-#pragma unroll 8
-        for (int q = q0; q < q1; ++q) {
-            const size_t at = (size_t)q * kRowBinAxis + c;
-            const uint32_t v = counts[at];
-            counts[at] = (uint32_t)min(run, lim);
-            run += v;
-        }
-    }
+    scan_columns<COLS>(sh, s_range[0], s_range[1] - s_range[0], cap, counts,
+                       tile_first + (size_t)row * (kRowBinAxis + 1));
 }
 
 // Step 2, placement: the ids of every partition's runs into the tiles' lists
@@ -599,6 +632,266 @@ __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
             const uint32_t* tf = tile_first + (size_t)d.x * (kRowBinAxis + 1) + tid;
             const int b = min(row0 + (int)tf[0], cap), e = min(row0 + (int)tf[1], cap);
             if (e > b) bins[d.x * tiles_x + tid] = make_int2(b, e);
+        }
+        place_all<PER>(sh, iv, id, tiles_x, base, ids, cap);
+    });
+}
+
+// ---- batches ----
+// The same two steps over the items of many views: a partition of items lies in
+// one view, a "row" is a tile row of a view, r = view * max_y + y, and the
+// offsets that one view's workgroups find by themselves come from tables.  12
+// views of 500k Gaussians at 800 x 800 (26M pairs of 6M items): 192 us in eight
+// launches, where emitting the pairs and sorting them by tile took 442 in
+// thirteen; step 2552 -> 2280 us.
+
+// The view that owns partition p.
+__device__ __forceinline__ int view_of_part(const ViewRec* __restrict__ views, int num_views,
+                                            int p) {
+    int lo = 0, hi = num_views;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (views[mid].part_off <= p) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Step 1, counting (row_count_kernel): counts[p * 256 + y], part_tot[p].
+__global__ __launch_bounds__(kRbThreads) void batch_row_count_kernel(
+    const ViewRec* __restrict__ views, int num_views, const uint2* __restrict__ rects,
+    uint32_t* __restrict__ counts, uint32_t* __restrict__ part_tot, int num_bins,
+    int2* __restrict__ bins, uint32_t* __restrict__ err) {
+    __shared__ int s_d[kRbThreads];
+    __shared__ uint32_t s_tmp[kRbWaves];
+    const int tid = threadIdx.x, part = blockIdx.x;
+    if (part == 0 && tid == 0) *err = 0u;
+    for (int t = part * kRbThreads + tid; t < num_bins; t += gridDim.x * kRbThreads)
+        bins[t] = make_int2(0, 0);
+    const ViewRec vr = views[view_of_part(views, num_views, part)];
+    const int local = (part - vr.part_off) * kRbPart;
+    s_d[tid] = 0;
+    __syncthreads();
+    uint32_t pairs = 0;
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = local + k * kRbThreads + tid;
+        const uint2 rc = i < vr.n ? rects[vr.item_off + i] : make_uint2(0u, 0u);
+        bool bad;
+        pairs += rect_count(rc);
+        const uint2 r = grid_rect(rc, vr.tiles_x, vr.tiles_y, bad);
+        if (rect_count(r) > 0)
+            add_differences(s_d, kRbThreads, {(int)(r.x >> 16), (int)(r.y >> 16)});
+    }
+    __syncthreads();
+    const uint32_t d = (uint32_t)s_d[tid];
+    counts[(size_t)part * kRowBinAxis + tid] = block_exclusive_scan256(d, s_tmp) + d;
+    const uint32_t t = block_exclusive_scan256(pairs, s_tmp) + pairs;
+    if (tid == kRbThreads - 1) part_tot[part] = t;
+}
+
+// Step 1, offsets: a view's rows are the columns of its partitions' counts;
+// row_first[view * 257 + y] the row's first run, relative to the view's.
+template <int COLS>
+__global__ __launch_bounds__(kScanThreads) void batch_row_scan_kernel(
+    const ViewRec* __restrict__ views, int cap, uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ row_first) {
+    __shared__ ScanShared sh;
+    const ViewRec vr = views[blockIdx.x];
+    scan_columns<COLS>(sh, vr.part_off, (vr.n + kRbPart - 1) / kRbPart, cap, counts,
+                       row_first + (size_t)blockIdx.x * (kRowBinAxis + 1));
+}
+
+// Exclusive scan of get(0..n) by one workgroup of 1024 threads, in rounds;
+// put(i, exclusive sum, value).  Returns the total.
+template <typename G, typename P>
+__device__ __forceinline__ uint64_t scan_rounds(int n, uint64_t* s_tmp, G get, P put) {
+    uint64_t carry = 0;
+    for (int b = 0; b < n; b += 1024) {
+        const int i = b + (int)threadIdx.x;
+        const uint64_t v = i < n ? get(i) : 0u;
+        const uint64_t e = block_exclusive_scan<16>(v, s_tmp);
+        if (i < n) put(i, carry + e, v);
+        if (threadIdx.x == 1023) s_tmp[16] = e + v;
+        __syncthreads();
+        carry += s_tmp[16];
+        __syncthreads();
+    }
+    return carry;
+}
+
+// Workgroup 0: every row's first run (row_off) and partition (row_part, R + 1
+// entries) of step 2, and those partitions' descriptors (col_count_kernel's).
+// Workgroup 1: every partition's first pair in item order (part_pair), and the
+// totals: *total, *count = min(total, cap), bit 8 of err.
+__global__ __launch_bounds__(1024) void batch_table_kernel(
+    int max_y, int rows, const uint32_t* __restrict__ row_first, int cap,
+    int* __restrict__ row_off, int* __restrict__ row_part, int4* __restrict__ desc, int parts,
+    const uint32_t* __restrict__ part_tot, uint32_t* __restrict__ part_pair,
+    int* __restrict__ count, unsigned long long* __restrict__ total,
+    uint32_t* __restrict__ err) {
+    __shared__ uint64_t s_tmp[17];
+    const uint64_t lim = (uint64_t)cap;
+    if (blockIdx.x == 1) {
+        const uint64_t sum = scan_rounds(
+            parts, s_tmp, [&](int i) { return (uint64_t)part_tot[i]; },
+            [&](int i, uint64_t e, uint64_t) { part_pair[i] = (uint32_t)min(e, lim); });
+        if (threadIdx.x == 0) {
+            *total = (unsigned long long)sum;
+            *count = (int)min(sum, lim);
+            if (sum > lim) atomicOr(err, 8u);
+        }
+        return;
+    }
+    auto len = [&](int r) {
+        const uint32_t* f = row_first + (size_t)(r / max_y) * (kRowBinAxis + 1) + r % max_y;
+        return (uint64_t)(f[1] - f[0]);
+    };
+    auto np = [](int b, int e) { return (e - b + kRbPart - 1) / kRbPart; };
+    scan_rounds(rows, s_tmp, len, [&](int r, uint64_t e, uint64_t v) {
+        row_off[r] = (int)min(e, lim);
+        row_part[r] = np((int)min(e, lim), (int)min(e + v, lim));       // for now
+    });
+    const uint64_t all = scan_rounds(
+        rows, s_tmp, [&](int r) { return (uint64_t)row_part[r]; },
+        [&](int r, uint64_t e, uint64_t v) {
+            row_part[r] = (int)e;
+            const int begin = row_off[r];
+            const int end = (int)min((uint64_t)begin + len(r), lim);
+            for (int q = 0; q < (int)v; ++q)
+                desc[(int)e + q] = make_int4(r, begin + q * kRbPart,
+                                             min(end, begin + (q + 1) * kRbPart), q == 0);
+        });
+    if (threadIdx.x == 0) {
+        row_part[rows] = (int)all;
+        desc[-1] = make_int4((int)all, 0, 0, 0);
+    }
+}
+
+// Step 1, placement (row_place_kernel), and every item's first pair.
+template <int COLS>
+__global__ __launch_bounds__(kRbThreads) void batch_row_place_kernel(
+    const ViewRec* __restrict__ views, int num_views, int max_y,
+    const uint2* __restrict__ rects, const uint32_t* __restrict__ counts,
+    const int* __restrict__ row_off, const uint32_t* __restrict__ part_pair,
+    uint2* __restrict__ runs, uint32_t* __restrict__ item_first, int cap,
+    uint32_t* __restrict__ err) {
+    constexpr int PER = round_per(false);
+    __shared__ PlaceShared<uint2, COLS, 3072, false> sh;
+    __shared__ uint32_t s_pairs[kRbWaves];
+    const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, part = blockIdx.x;
+    const int v = view_of_part(views, num_views, part);
+    const ViewRec vr = views[v];
+    const int local = (part - vr.part_off) * kRbPart;
+    static_assert(PER == kRbPer, "a wave's items are consecutive");
+    Interval iv[kRbPer];
+    uint2 val[kRbPer];
+    uint32_t before[kRbPer], pairs = 0;
+    bool bad_any = false;
+#pragma unroll
+    for (int k = 0; k < kRbPer; ++k) {
+        const int i = local + interval_index<PER>(k);
+        const uint2 own = i < vr.n ? rects[vr.item_off + i] : make_uint2(0u, 0u);
+        const uint32_t n = rect_count(own), incl = wave_inclusive_sum(n);
+        before[k] = pairs + incl - n;
+        pairs += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        bool bad;
+        const uint2 rc = grid_rect(own, vr.tiles_x, vr.tiles_y, bad);
+        bad_any = bad_any || bad;
+        iv[k].lo = (int)(rc.x >> 16);
+        iv[k].len = rect_count(rc) > 0 ? (int)(rc.y >> 16) : 0;
+        val[k] = make_uint2((uint32_t)(vr.item_off + i), (rc.x & 0xFFFFu) | (rc.y << 16));
+    }
+    if (bad_any) atomicOr(err, 4u);
+    if (lane == 0) s_pairs[wave] = pairs;
+    clear_place(sh);
+    __syncthreads();
+    if (item_first) {
+        uint32_t at = part_pair[part];
+        for (int w = 0; w < wave; ++w) at += s_pairs[w];
+#pragma unroll
+        for (int k = 0; k < kRbPer; ++k) {
+            const int i = local + interval_index<PER>(k);
+            if (i < vr.n) item_first[vr.item_off + i] = min(at + before[k], (uint32_t)cap);
+        }
+    }
+    const int base =
+        tid < vr.tiles_y
+            ? (int)min((uint64_t)row_off[v * max_y] + counts[(size_t)part * kRowBinAxis + tid],
+                       (uint64_t)cap)
+            : 0;
+    place_all<PER>(sh, iv, val, vr.tiles_y, base, runs, cap);
+}
+
+// Step 2, counting, over the descriptors.
+__global__ __launch_bounds__(kRbThreads) void batch_col_count_kernel(
+    const uint2* __restrict__ runs, const int4* __restrict__ desc,
+    uint32_t* __restrict__ counts) {
+    __shared__ int s_d[kRbThreads];
+    __shared__ uint32_t s_tmp[kRbWaves];
+    const int tid = threadIdx.x;
+    for_partitions(uniform_i(desc[-1].x), [&](int p) {
+        const int4 d = desc[p];
+        count_columns(runs, d.y, d.z, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
+    });
+}
+
+// Step 2, offsets, one workgroup per row.
+template <int COLS>
+__global__ __launch_bounds__(kScanThreads) void batch_col_scan_kernel(
+    const int* __restrict__ row_part, int cap, uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ tile_first) {
+    __shared__ ScanShared sh;
+    const int row = blockIdx.x, p0 = row_part[row];
+    scan_columns<COLS>(sh, p0, row_part[row + 1] - p0, cap, counts,
+                       tile_first + (size_t)row * (kRowBinAxis + 1));
+}
+
+// Every row's first pair.
+__global__ __launch_bounds__(1024) void batch_pair_scan_kernel(
+    int rows, const uint32_t* __restrict__ tile_first, int cap, int* __restrict__ row_pair) {
+    __shared__ uint64_t s_tmp[17];
+    scan_rounds(
+        rows, s_tmp,
+        [&](int r) {
+            return (uint64_t)tile_first[(size_t)r * (kRowBinAxis + 1) + kRowBinAxis];
+        },
+        [&](int r, uint64_t e, uint64_t) { row_pair[r] = (int)min(e, (uint64_t)cap); });
+}
+
+// Step 2, placement (col_place_kernel).
+template <int COLS>
+__global__ __launch_bounds__(kRbThreads) void batch_col_place_kernel(
+    const ViewRec* __restrict__ views, int max_y, const uint2* __restrict__ runs,
+    const int4* __restrict__ desc, int cap, const uint32_t* __restrict__ counts,
+    const uint32_t* __restrict__ tile_first, const int* __restrict__ row_pair,
+    uint32_t* __restrict__ ids, int2* __restrict__ bins) {
+    constexpr int PER = round_per(false);
+    __shared__ PlaceShared<uint32_t, COLS, 5120, false> sh;
+    const int tid = threadIdx.x;
+    for_partitions(uniform_i(desc[-1].x), [&](int p) {
+        const int4 d = desc[p];
+        const int v = d.x / max_y, ty = d.x - v * max_y;
+        const int tiles_x = views[v].tiles_x;
+        Interval iv[kRbPer];
+        uint32_t id[kRbPer];
+#pragma unroll
+        for (int k = 0; k < kRbPer; ++k) {
+            const int i = d.y + interval_index<PER>(k);
+            const uint2 run = i < d.z ? runs[i] : make_uint2(0u, 0u);
+            id[k] = run.x;
+            iv[k] = {(int)(run.y & 0xFFFFu), (int)(run.y >> 16)};
+        }
+        clear_place(sh);
+        __syncthreads();
+        const int row0 = row_pair[d.x];
+        const int base = tid < tiles_x
+                             ? min(row0 + (int)counts[(size_t)p * kRowBinAxis + tid], cap)
+                             : 0;
+        if (d.w && tid < tiles_x) {
+            const uint32_t* tf = tile_first + (size_t)d.x * (kRowBinAxis + 1) + tid;
+            const int b = min(row0 + (int)tf[0], cap), e = min(row0 + (int)tf[1], cap);
+            if (e > b) bins[views[v].bin_off + ty * tiles_x + tid] = make_int2(b, e);
         }
         place_all<PER>(sh, iv, id, tiles_x, base, ids, cap);
     });
@@ -672,11 +965,14 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     // persistent: as many workgroups as fit the chip, or one per partition
     const int most = 8 * ((p.max_col_parts + 7) / 8);
     const int grid = most < 2048 ? most : 2048;
-    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_x, p.tiles_y, p.cap,
+    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_y, p.cap,
                                                  U(p.col_counts), desc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    col_scan_kernel<<<p.tiles_y, kRbThreads * kRbGroups, 0, s>>>(
-        U(p.row_len), p.tiles_x, p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first));
+#define JSA_LAUNCH(COLS)                                                                      \
+    col_scan_kernel<COLS><<<p.tiles_y, kScanThreads, 0, s>>>(                                 \
+        U(p.row_len), p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first))
+    JSA_SCAN(p.tiles_x, JSA_LAUNCH);
+#undef JSA_LAUNCH
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_COL(ST, COLS)                                                                     \
     col_place_kernel<ST, COLS><<<grid, kRbThreads, 0, s>>>(                                   \
@@ -694,6 +990,83 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
         e = hipGetLastError();
     }
     return e;
+}
+
+BatchRowPlan batch_row_plan(int num_views, int parts, int max_x, int max_y, int cap) {
+    BatchRowPlan p{};
+    p.num_views = num_views;
+    p.parts = parts;
+    p.max_x = max_x;
+    p.max_y = max_y;
+    p.rows = num_views * max_y;
+    p.cap = cap > 0 ? cap : 1;
+    p.max_col_parts = p.cap / kRbPart + p.rows;
+    const size_t np = (size_t)(parts > 0 ? parts : 1), rows = (size_t)(p.rows > 0 ? p.rows : 1);
+    size_t o = 0;
+    p.counts = o; o = align256(o + 4ull * kRowBinAxis * np);
+    p.part_tot = o; o = align256(o + 4ull * np);
+    p.part_pair = o; o = align256(o + 4ull * np);
+    p.row_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * (size_t)num_views);
+    p.row_off = o; o = align256(o + 4ull * rows);
+    p.row_part = o; o = align256(o + 4ull * (rows + 1));
+    p.row_pair = o; o = align256(o + 4ull * rows);
+    p.tile_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * rows);
+    p.desc = o; o = align256(o + 16ull * ((size_t)p.max_col_parts + 1));
+    p.col_counts = o; o = align256(o + 4ull * kRowBinAxis * (size_t)p.max_col_parts);
+    p.scratch_bytes = o;
+    return p;
+}
+
+hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint2* rects,
+                         uint2* runs, uint32_t* ids, int num_bins, int2* bins,
+                         uint32_t* item_first, int* count, unsigned long long* total,
+                         uint32_t* err, void* scratch, hipStream_t s) {
+    uint8_t* b = static_cast<uint8_t*>(scratch);
+    auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
+    auto I = [&](size_t off) { return reinterpret_cast<int*>(b + off); };
+    int4* desc = reinterpret_cast<int4*>(b + p.desc) + 1;
+    hipError_t e;
+    batch_row_count_kernel<<<p.parts, kRbThreads, 0, s>>>(
+        views, p.num_views, rects, U(p.counts), U(p.part_tot), num_bins, bins, err);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+#define JSA_LAUNCH(COLS)                                                                      \
+    batch_row_scan_kernel<COLS><<<p.num_views, kScanThreads, 0, s>>>(                         \
+        views, p.cap, U(p.counts), U(p.row_first))
+    JSA_SCAN(p.max_y, JSA_LAUNCH);
+#undef JSA_LAUNCH
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    batch_table_kernel<<<2, 1024, 0, s>>>(p.max_y, p.rows, U(p.row_first), p.cap,
+                                          I(p.row_off), I(p.row_part), desc, p.parts,
+                                          U(p.part_tot), U(p.part_pair), count, total, err);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+#define JSA_ROW(COLS)                                                                         \
+    batch_row_place_kernel<COLS><<<p.parts, kRbThreads, 0, s>>>(                              \
+        views, p.num_views, p.max_y, rects, U(p.counts), I(p.row_off), U(p.part_pair), runs,  \
+        item_first, p.cap, err)
+    if (narrow(p.max_y)) JSA_ROW(128);
+    else JSA_ROW(256);
+#undef JSA_ROW
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const int most = 8 * ((p.max_col_parts + 7) / 8);
+    const int grid = most < 2048 ? most : 2048;
+    batch_col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, desc, U(p.col_counts));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+#define JSA_LAUNCH(COLS)                                                                      \
+    batch_col_scan_kernel<COLS><<<p.rows, kScanThreads, 0, s>>>(                              \
+        I(p.row_part), p.cap, U(p.col_counts), U(p.tile_first))
+    JSA_SCAN(p.max_x, JSA_LAUNCH);
+#undef JSA_LAUNCH
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    batch_pair_scan_kernel<<<1, 1024, 0, s>>>(p.rows, U(p.tile_first), p.cap, I(p.row_pair));
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+#define JSA_COL(COLS)                                                                         \
+    batch_col_place_kernel<COLS><<<grid, kRbThreads, 0, s>>>(                                 \
+        views, p.max_y, runs, desc, p.cap, U(p.col_counts), U(p.tile_first), I(p.row_pair),   \
+        ids, bins)
+    if (narrow(p.max_x)) JSA_COL(128);
+    else JSA_COL(256);
+#undef JSA_COL
+    return hipGetLastError();
 }
 
 }  // namespace jsa
