@@ -482,6 +482,16 @@ struct alignas(16) ViewRec {
 };
 static_assert(sizeof(ViewRec) == 80, "ViewRec layout");
 
+// A batch's staged records as the projection backward sums them (rec null: it
+// takes the items' sums instead).
+struct BatchRecords {
+    const float* rec = nullptr;
+    const uint32_t* bits = nullptr;
+    const uint2* rects = nullptr;       // per item
+    const uint32_t* first = nullptr;    // per item: first slot
+    int n_slots = 0;
+};
+
 // Scenes of a batch: Gaussians [g0, g0 + n) seen by views [v_begin, v_end).
 struct SceneRec {
     int g0, n, v_begin, v_end;
@@ -743,14 +753,15 @@ hipError_t project_batch_fwd(const ViewRec* views, int num_views, int max_view_n
                              float* conics, int* radii, uint32_t* depth_keys, uint2* item_rects,
                              hipStream_t s);
 // Backward: one lane per Gaussian, summing the contributions of its scene's
-// views; writes v_mean3d, v_scale, v_quat for every Gaussian of every scene,
-// and with v_rgbo (per item: rgb, opacity; optional) also v_colors and
-// v_opacity as the sums of the Gaussian's items over the views.
+// views; writes all gradients of every Gaussian of every scene.  The items' sums
+// are taken from br's records, or with br.rec null from v_xy, v_conic and v_rgbo
+// (per item: rgb, opacity).
 hipError_t project_batch_bwd(const SceneRec* scenes, int num_scenes, int max_scene_n,
                              const ViewRec* views, float glob_scale, float clip_thresh,
                              const float* means3d, const float* scales, const float* quats,
                              const float* viewmats, const int* radii, const float* conics,
                              const float* v_xy, const float* v_conic, const float* v_rgbo,
+                             const BatchRecords& br,
                              float* v_mean3d, float* v_scale, float* v_quat, float* v_colors,
                              float* v_opacity, int consistent, hipStream_t s);
 
@@ -830,7 +841,7 @@ hipError_t raster_fwd_splats(const Camera& c, int nch, const int* gids_sorted,
 // item_first[item] + the tile's row-major offset in the item's rectangle
 // (item_rects, the ones the binning used; workspace raster_bwd_staged_bytes(cap)),
 // summed per item into v_xy, v_conic and v_rgbo (4 floats per item: rgb,
-// opacity); every item row is written.  g.views is the device view table;
+// opacity), every item row (not with v_xy null).  g.views is the device view table;
 // max_view_n the largest view's item count.
 hipError_t raster_bwd_batch_staged(const RasterGrid& g, int max_view_n, const int* items_sorted,
                                    const int* tile_bins, int cap, const float* xys,

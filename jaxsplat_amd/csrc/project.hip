@@ -760,20 +760,26 @@ __global__ __launch_bounds__(256) void render_bwd_tail_kernel(
 // Batched backward: blockIdx.y = scene, one lane per Gaussian; the views of
 // the scene are walked in order and their v_mean3d / v_cov3d contributions
 // summed in registers (the scale/rotation VJP is linear in v_cov3d, so it
-// runs once on the sum), and likewise the items' colour and opacity gradients
-// when v_rgbo is given.  No atomics; every Gaussian of the scene is written.
+// runs once on the sum), and likewise the items' colour and opacity gradients.
+// No atomics; every Gaussian of the scene is written.
+// SUM: the items' record sums are taken here, view after view, instead of by
+// raster_bwd_batch_reduce_kernel, whose 36 bytes per item are then neither written
+// nor read.
+template <bool SUM>
 __global__ __launch_bounds__(256) void project_batch_bwd_kernel(
     const SceneRec* __restrict__ scenes, const ViewRec* __restrict__ views, float glob_scale,
     float clip_thresh, const float* __restrict__ means3d, const float* __restrict__ scales,
     const float* __restrict__ quats, const float* __restrict__ viewmats,
     const int* __restrict__ radii, const float* __restrict__ conics,
     const float* __restrict__ v_xy, const float* __restrict__ v_conic,
-    const float4* __restrict__ v_rgbo, float* __restrict__ v_mean3d,
+    const float4* __restrict__ v_rgbo, const BatchRecords br, float* __restrict__ v_mean3d,
     float* __restrict__ v_scale, float* __restrict__ v_quat, float* __restrict__ v_colors,
     float* __restrict__ v_opacity, int consistent) {
     const SceneRec sc = scenes[blockIdx.y];
-    const int k = blockIdx.x * 256 + (int)threadIdx.x;
-    if (k >= sc.n) return;
+    if ((int)blockIdx.x * 256 >= sc.n) return;          // uniform over the block
+    const bool own = blockIdx.x * 256 + (int)threadIdx.x < sc.n;
+    const int k = own ? blockIdx.x * 256 + (int)threadIdx.x : 0;
+    const int lane = lane_id();
     const size_t g = (size_t)sc.g0 + k;
     const float m[3] = {means3d[3 * g + 0], means3d[3 * g + 1], means3d[3 * g + 2]};
     const float s[3] = {scales[3 * g + 0], scales[3 * g + 1], scales[3 * g + 2]};
@@ -786,14 +792,38 @@ __global__ __launch_bounds__(256) void project_batch_bwd_kernel(
     for (int v = sc.v_begin; v < sc.v_end; ++v) {
         const ViewRec vr = views[v];
         const size_t it = (size_t)vr.item_off + k;
-        if (radii[it] <= 0) continue;
-        if (v_rgbo) {
+        const int rad = own ? radii[it] : 0;
+        float a[9] = {};            // rgb 3, conic 3, xy 2, opacity
+        if constexpr (SUM) {
+            int off = 0, end = 0;
+            if (rad > 0) {
+                const int cnt = (int)rect_count(br.rects[it]);
+                const long long f = br.first[it];
+                if (cnt > 0 && f + cnt <= (long long)br.n_slots) {
+                    off = (int)f;
+                    end = off + cnt;
+                }
+            }
+            sum_records<9>(off, end, br.rec, br.bits, lane, a);
+            if (rad <= 0) continue;
+        } else {
+            if (rad <= 0) continue;
             const float4 c = v_rgbo[it];
-            rgbo.x += c.x;
-            rgbo.y += c.y;
-            rgbo.z += c.z;
-            rgbo.w += c.w;
+            const float2 xy = reinterpret_cast<const float2*>(v_xy)[it];
+            a[0] = c.x;
+            a[1] = c.y;
+            a[2] = c.z;
+            a[3] = v_conic[3 * it + 0];
+            a[4] = v_conic[3 * it + 1];
+            a[5] = v_conic[3 * it + 2];
+            a[6] = xy.x;
+            a[7] = xy.y;
+            a[8] = c.w;
         }
+        rgbo.x += a[0];
+        rgbo.y += a[1];
+        rgbo.z += a[2];
+        rgbo.w += a[8];
         if (!any) {
             cp = cov3d_parts(s, q, glob_scale);
             any = true;
@@ -804,14 +834,14 @@ __global__ __launch_bounds__(256) void project_batch_bwd_kernel(
         load_view(viewmats + 16 * vr.view, W, pt);
         float vm[3], v2[3], v3[6];
         view_vjp(c, W, pt, m, cp.cov, conics[3 * it + 0], conics[3 * it + 1], conics[3 * it + 2],
-                 reinterpret_cast<const float2*>(v_xy)[it], 0.f, v_conic[3 * it + 0],
-                 v_conic[3 * it + 1], v_conic[3 * it + 2], false, 0.f, 0.f, consistent, vm, v2,
-                 v3);
+                 make_float2(a[6], a[7]), 0.f, a[3], a[4], a[5], false, 0.f, 0.f, consistent, vm,
+                 v2, v3);
 #pragma unroll
         for (int j = 0; j < 3; ++j) vmean[j] += vm[j];
 #pragma unroll
         for (int j = 0; j < 6; ++j) vc3[j] += v3[j];
     }
+    if (!own) return;
     float vsc[3] = {0.f, 0.f, 0.f}, vq[4] = {0.f, 0.f, 0.f, 0.f};
     if (any) cov3d_vjp(cp, q, glob_scale, vc3, vsc, vq);
 #pragma unroll
@@ -820,12 +850,10 @@ __global__ __launch_bounds__(256) void project_batch_bwd_kernel(
         v_scale[3 * g + j] = vsc[j];
     }
     reinterpret_cast<float4*>(v_quat)[g] = make_float4(vq[0], vq[1], vq[2], vq[3]);
-    if (v_rgbo) {
-        v_colors[3 * g + 0] = rgbo.x;
-        v_colors[3 * g + 1] = rgbo.y;
-        v_colors[3 * g + 2] = rgbo.z;
-        v_opacity[g] = rgbo.w;
-    }
+    v_colors[3 * g + 0] = rgbo.x;
+    v_colors[3 * g + 1] = rgbo.y;
+    v_colors[3 * g + 2] = rgbo.z;
+    v_opacity[g] = rgbo.w;
 }
 
 // n words set to v, then tail (0..3) zero bytes after them.
@@ -1022,14 +1050,19 @@ hipError_t project_batch_bwd(const SceneRec* scenes, int num_scenes, int max_sce
                              const float* means3d, const float* scales, const float* quats,
                              const float* viewmats, const int* radii, const float* conics,
                              const float* v_xy, const float* v_conic, const float* v_rgbo,
+                             const BatchRecords& br,
                              float* v_mean3d, float* v_scale, float* v_quat, float* v_colors,
                              float* v_opacity, int consistent, hipStream_t s) {
     if (num_scenes <= 0 || max_scene_n <= 0) return hipSuccess;
     const dim3 grid((max_scene_n + 255) / 256, num_scenes);
-    project_batch_bwd_kernel<<<grid, 256, 0, s>>>(
-        scenes, views, glob_scale, clip_thresh, means3d, scales, quats, viewmats, radii, conics,
-        v_xy, v_conic, reinterpret_cast<const float4*>(v_rgbo), v_mean3d, v_scale, v_quat,
-        v_colors, v_opacity, consistent);
+#define JSA_LAUNCH(SUM)                                                                      \
+    project_batch_bwd_kernel<SUM><<<grid, 256, 0, s>>>(                                      \
+        scenes, views, glob_scale, clip_thresh, means3d, scales, quats, viewmats, radii,     \
+        conics, v_xy, v_conic, reinterpret_cast<const float4*>(v_rgbo), br, v_mean3d,        \
+        v_scale, v_quat, v_colors, v_opacity, consistent)
+    if (br.rec) JSA_LAUNCH(true);
+    else JSA_LAUNCH(false);
+#undef JSA_LAUNCH
     return hipGetLastError();
 }
 

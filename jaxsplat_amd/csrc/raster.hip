@@ -1572,7 +1572,7 @@ hipError_t raster_bwd_batch_staged(const RasterGrid& g, int max_view_n, const in
 #undef JSA_LAUNCH
 #undef JSA_LAUNCH_D
 #undef JSA_LAUNCH_S
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = hipGetLastError()) != hipSuccess || !v_xy) return e;
     const dim3 rgrid((max_view_n + 255) / 256, g.num_views);
     raster_bwd_batch_reduce_kernel<<<rgrid, 256, 0, s>>>(
         g.views, cap, radii, item_rects, item_first, st.rec, st.bits, v_xy, v_conic,

@@ -78,3 +78,39 @@ def test_batch_rows(bw):
         again = render_batch(*params, vm, bg, plan=exact)
     assert exact.check() == total
     assert np.array_equal(H.host(again).view(np.uint32), H.host(runs[0][0]).view(np.uint32))
+
+
+@pytest.mark.parametrize("adjoint", ["reference", "consistent"])
+def test_batch_of_many_gaussians(adjoint):
+    """With 131072 Gaussians or more the projection backward sums the records."""
+    t = H.torch()
+    rng = np.random.default_rng(9)
+    sizes = (131072, 700)
+    params = [H.dev(a) for a in scenes.gaussians(rng, sum(sizes), (-1.5, -1.2, 2),
+                                                 (1.5, 1.2, 6), np.log(0.02))]
+    hw, f, c = (120, 150), (120.0, 120.0), (75.0, 60.0)
+    views = [ViewSpec(s, hw, f, c) for s in (0, 0, 1)]
+    vms = [H.dev(scenes.look_at((x, 0.2, -1.0), target=(0, 0, 4)).astype(np.float32))
+           for x in (0.5, -0.5, 0.0)]
+    bg = H.dev(np.zeros((3, 3), np.float32))
+    plan = BatchPlan(list(sizes), views, glob_scale=1.0, clip_thresh=0.01,
+                     isect_capacity=1 << 20)
+    runs = []
+    for _ in range(2):
+        p = [x.detach().clone().requires_grad_(True) for x in params]
+        flat = render_batch(*p, t.stack(vms), bg, plan=plan, adjoint=adjoint)
+        v = t.linspace(-1, 1, flat.numel(), device="cuda").view(flat.shape)
+        runs.append(t.autograd.grad(flat, p, v))
+    assert plan.check() > 0
+    for a, b in zip(*runs):
+        assert np.array_equal(H.host(a).view(np.uint32), H.host(b).view(np.uint32))
+    sums = [np.zeros(tuple(x.shape)) for x in params]
+    for k, vk in enumerate(plan.split(v)):
+        rows = slice(0, sizes[0]) if k < 2 else slice(sizes[0], sum(sizes))
+        p = [x[rows].detach().contiguous().requires_grad_(True) for x in params]
+        one = render(*p, viewmat=vms[k], background=bg[k].contiguous(), img_shape=hw, f=f, c=c,
+                     glob_scale=1.0, clip_thresh=0.01, adjoint=adjoint)
+        for s, g in zip(sums, t.autograd.grad(one, p, vk.contiguous())):
+            s[rows] += H.host(g)
+    for g, s in zip(runs[0], sums):
+        assert np.all(np.abs(H.host(g) - s) <= 1e-3 * np.abs(s) + 1e-4 * np.abs(s).max())
