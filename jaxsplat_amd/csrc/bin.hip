@@ -9,10 +9,10 @@
 // the reference's final order is the lexicographic order
 // (tile, depth bits, gaussian id).
 //
-// Single view: grids of up to 256 tiles per axis are binned by tile rows
-// (rowbin.hip), of the Gaussians in depth order where they have many pairs
-// each, else in id order with step 5 below after it.  Smaller (one radix pass)
-// and larger grids, and batches:
+// Grids of up to 256 tiles per axis are binned by tile rows (rowbin.hip): of a
+// view's Gaussians in depth order where they have many pairs each and the lists
+// are long, else, and in batches, in id order with step 5 below after it.  Views
+// of up to 256 tiles in all (one radix pass) and larger grids:
 //  1. depth_keys_kernel: per Gaussian its depth bits and packed tile
 //     rectangle;
 //  2. emission in Gaussian id order: a reduce-then-scan of the Gaussians'
