@@ -602,6 +602,10 @@ class _Render(torch.autograd.Function):
                 count = ctypes.c_int32()
                 _lib.check(L.jaxsplat_render_count(db, _p(state), ticket, ctypes.byref(count), s))
                 isect = count.value
+                if not 0 <= isect <= STAGED_MAX_INTERSECTIONS:
+                    raise _lib.JaxsplatError(
+                        _lib.ERR_CAPACITY,
+                        f"num_intersects {isect & 0xFFFFFFFF} exceeds 2^30")
             else:
                 isect = capacity.capacity if N else 0
             lists_bytes = L.jaxsplat_render_lists_size(db, isect)
