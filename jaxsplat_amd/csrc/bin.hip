@@ -38,14 +38,17 @@
 namespace jsa {
 namespace {
 
-// Per Gaussian (id order): the depth sort key and the packed tile rectangle.
-__global__ void depth_keys_kernel(Camera c, const float* __restrict__ depths,
-                                  const int* __restrict__ radii, const float2* __restrict__ xys,
-                                  const uint2* __restrict__ rects_in, uint32_t* __restrict__ keys,
-                                  uint2* __restrict__ rects) {
+// Per Gaussian (id order): the depth sort key and the packed tile rectangle, and
+// (cum, optional) the workgroup's inclusive sums of the tile counts.
+__global__ __launch_bounds__(kCountPart) void depth_keys_kernel(
+    Camera c, const float* __restrict__ depths, const int* __restrict__ radii,
+    const float2* __restrict__ xys, const uint2* __restrict__ rects_in,
+    uint32_t* __restrict__ keys, uint2* __restrict__ rects, int* __restrict__ cum,
+    uint32_t* __restrict__ part_tot) {
+    __shared__ uint32_t s_tmp[4];
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= c.num_points) return;
-    const int rad = radii[g];
+    const bool own = g < c.num_points;
+    const int rad = own ? radii[g] : 0;
     uint2 rc = make_uint2(0u, 0u);
     if (rad > 0) {
         if (rects_in) {
@@ -56,9 +59,12 @@ __global__ void depth_keys_kernel(Camera c, const float* __restrict__ depths,
             rc = pack_rect(x0, x1, y0, y1);
         }
     }
-    // Gaussians that emit nothing get the key the depth sort drops
-    keys[g] = rect_count(rc) > 0 ? __float_as_uint(depths[g]) : 0xFFFFFFFFu;
-    rects[g] = rc;
+    if (own) {
+        // Gaussians that emit nothing get the key the depth sort drops
+        keys[g] = rect_count(rc) > 0 ? __float_as_uint(depths[g]) : 0xFFFFFFFFu;
+        rects[g] = rc;
+    }
+    if (cum) block_count_scan(rect_count(rc), g, c.num_points, cum, part_tot, s_tmp);
 }
 
 // View of each item of the emission order (largest v with item_off[v] <=
@@ -935,11 +941,11 @@ hipError_t emit(int n, const int* n_dev, int tiles_x_plain, const ViewRec* views
     return hipGetLastError();
 }
 
-// Depth stage: per-Gaussian depth keys and rectangles.  It needs no
-// intersection count, so a caller can run it while it reads the count back;
-// its workspace depends on the Gaussian count only.
+// Depth stage: per-Gaussian depth keys and rectangles and (by_rows) the inclusive
+// counts of the tiles.  It needs no intersection count, so a caller can run it while
+// it reads the count back; its workspace depends on the Gaussian count only.
 struct DepthLayout {
-    size_t dkeys, rect_by_id, end;
+    size_t dkeys, rect_by_id, cum, part_tot, end;
 };
 
 DepthLayout depth_layout(const BinPlan& p) {
@@ -948,6 +954,8 @@ DepthLayout depth_layout(const BinPlan& p) {
     const size_t n4 = align256(4ull * (p.n > 0 ? p.n : 1));
     L.dkeys = o; o += n4;
     L.rect_by_id = o; o += 2 * n4;
+    L.cum = o; o += n4;
+    L.part_tot = o; o = align256(o + 4ull * ((size_t)p.n / kCountPart + 1));
     L.end = o;
     return L;
 }
@@ -1007,7 +1015,7 @@ int bitlen(uint32_t v) { return v ? 32 - __builtin_clz(v) : 0; }
 // tiles' lists are then ordered as they are placed, or in id order and every
 // tile's run ordered where it lies.  dkeys: the depth bits.
 hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rects,
-                       int* gids_sorted, int* tiles_sorted, int* tile_bins, void* scratch,
+                       const int* cum, int* gids_sorted, int* tiles_sorted, int* tile_bins, void* scratch,
                        hipStream_t s) {
     const BinLayout L = layout(p);
     uint8_t* b = static_cast<uint8_t*>(scratch);
@@ -1020,7 +1028,7 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
                         U(L.dtmp_v), p.n, nullptr, b + L.depth_sort, nullptr, s)) != hipSuccess)
         return e;
     // (the depth sort's ping-pong buffers, adjacent, are free again)
-    e = row_bin(p.rows, p.by_depth ? U(L.perm) : nullptr, rects,
+    e = row_bin(p.rows, p.by_depth ? U(L.perm) : nullptr, rects, cum,
                 reinterpret_cast<uint2*>(b + L.dtmp_k), reinterpret_cast<uint2*>(b + L.runs), ids,
                 reinterpret_cast<uint32_t*>(tiles_sorted), bins,
                 reinterpret_cast<unsigned long long*>(b + L.total), U(L.err), b + L.rows, s);
@@ -1079,10 +1087,14 @@ hipError_t bin_depth(const BinPlan& p, const Camera& c, const float* xys, const 
     if (p.n <= 0) return hipSuccess;
     const DepthLayout D = depth_layout(p);
     uint8_t* b = static_cast<uint8_t*>(depth_ws);
-    depth_keys_kernel<<<(p.n + 255) / 256, 256, 0, s>>>(
+    int* cum = p.by_rows ? reinterpret_cast<int*>(b + D.cum) : nullptr;
+    uint32_t* part_tot = reinterpret_cast<uint32_t*>(b + D.part_tot);
+    depth_keys_kernel<<<(p.n + kCountPart - 1) / kCountPart, kCountPart, 0, s>>>(
         c, depths, radii, reinterpret_cast<const float2*>(xys), rects,
-        reinterpret_cast<uint32_t*>(b + D.dkeys), reinterpret_cast<uint2*>(b + D.rect_by_id));
-    return hipGetLastError();
+        reinterpret_cast<uint32_t*>(b + D.dkeys), reinterpret_cast<uint2*>(b + D.rect_by_id),
+        cum, part_tot);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess || !cum ? e : count_scan_add(p.n, part_tot, cum, s);
 }
 
 hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
@@ -1095,8 +1107,8 @@ hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
     const uint32_t* dkeys = reinterpret_cast<const uint32_t*>(d + D.dkeys);
     const uint2* rect_by_id = reinterpret_cast<const uint2*>(d + D.rect_by_id);
     if (p.by_rows && p.n > 0)
-        return bin_by_rows(p, dkeys, rect_by_id, gids_sorted, tiles_sorted, tile_bins, scratch,
-                           s);
+        return bin_by_rows(p, dkeys, rect_by_id, reinterpret_cast<const int*>(d + D.cum),
+                           gids_sorted, tiles_sorted, tile_bins, scratch, s);
     hipError_t e = fill_zero(b, L.zero_end, s);
     if (e != hipSuccess) return e;
     e = fill_zero(tile_bins, 8ull * p.num_tiles, s);
@@ -1156,7 +1168,7 @@ hipError_t bin_rects(const BinPlan& p, const Camera& c, const float* depths,
         return fill_zero(tile_bins, 8ull * p.num_tiles, s);
     }
     if (p.by_rows)
-        return bin_by_rows(p, reinterpret_cast<const uint32_t*>(depths), rects, gids_sorted,
+        return bin_by_rows(p, reinterpret_cast<const uint32_t*>(depths), rects, cum, gids_sorted,
                            tiles_sorted, tile_bins, scratch, s);
     uint32_t* err = reinterpret_cast<uint32_t*>(b + L.err);
     auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };

@@ -193,6 +193,18 @@ __device__ __forceinline__ T block_exclusive_scan256(T v, T* s_tmp) {
     return block_exclusive_scan<4>(v, s_tmp);
 }
 
+// A workgroup's inclusive sums of its kCountPart counts and their total (s_tmp: 4
+// words of LDS); count_scan_add adds the offsets of the partitions.
+constexpr int kCountPart = 256;
+__device__ __forceinline__ void block_count_scan(uint32_t cnt, int idx, int n,
+                                                 int* __restrict__ cum,
+                                                 uint32_t* __restrict__ part_tot,
+                                                 uint32_t* s_tmp) {
+    const uint32_t incl = block_exclusive_scan256(cnt, s_tmp) + cnt;
+    if (idx < n) cum[idx] = (int)incl;
+    if (threadIdx.x == kCountPart - 1) part_tot[blockIdx.x] = incl;
+}
+
 // A count with its ticket into a pinned, coherent word of the host's.
 __device__ __forceinline__ void store_count(uint64_t* out, int count, uint32_t ticket) {
     __hip_atomic_store(out, (uint64_t)ticket << 32 | (uint32_t)count, __ATOMIC_RELAXED,
@@ -586,6 +598,9 @@ hipError_t project_fwd(const Camera& c, const float* means3d, const float* scale
                        const float* colors = nullptr, int nch = 0, float4* splats = nullptr,
                        uint64_t* count_out = nullptr, uint32_t ticket = 0,
                        bool antialiased = false);
+// Adds the offsets of the partitions (kCountPart counts each, totals part_tot) to
+// the partitions' inclusive sums cum (block_count_scan's).
+hipError_t count_scan_add(int n, const uint32_t* part_tot, int* cum, hipStream_t s);
 // Opacity-limited tile rectangles (opacity_tile_rect) of projected Gaussians,
 // their counts (num_tiles_hit optional) and inclusive sums; scratch
 // project_fwd_scratch_bytes(c.num_points).
@@ -678,20 +693,21 @@ struct RowBinPlan {
     int parts;              // partitions of the Gaussians
     int max_col_parts;      // partitions of the runs, at most
     bool fold;              // kFoldParts
-    size_t row_len, row_counts, part_tot, tile_first, desc, col_counts;  // offsets in the scratch
+    size_t cut, row_len, row_counts, part_tot, tile_first, desc, col_counts;    // in the scratch
     size_t scratch_bytes;
 };
 RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap);
 // The tiles' lists of the packed rectangles rects (tile counts up to
 // kRowBinAxis per axis): bins (cleared first; empty tiles stay (0, 0)) and
-// ids, at most p.cap of them (the pairs past it are dropped and bit 8 of *err
-// set; *err is cleared first), *total the exact pair total.  With perm (n
-// Gaussian ids, each once) every tile's list is in perm's order; without, its
-// order is arbitrary.  in_order (with perm): n rectangles of scratch; runs: 8
+// ids, at most p.cap of them (of more pairs the first p.cap in emission order, by
+// id and then row by row; bit 8 of *err is set then; *err is cleared first), *total
+// the exact pair total.  cum: the rectangles' inclusive tile counts by id.  With
+// perm (n Gaussian ids, each once) every tile's list is in perm's order; without,
+// its order is arbitrary.  in_order (with perm): n rectangles of scratch; runs: 8
 // bytes per pair of the capacity.  tiles_sorted (optional): every entry's tile
 // id.
 hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects,
-                   uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
+                   const int* cum, uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
                    int2* bins, unsigned long long* total, uint32_t* err, void* scratch,
                    hipStream_t s);
 

@@ -133,7 +133,7 @@ __device__ __forceinline__ M3 ewa_jacobian(float fx, float fy, float tx, float t
     return J;
 }
 
-constexpr int kProjPart = 256;      // Gaussians per workgroup and scan partition
+constexpr int kProjPart = kCountPart;   // Gaussians per workgroup and scan partition
 // Partitions per workgroup of the scan's second kernel: few, so that it has
 // workgroups enough, but what each sums grows with their number.
 constexpr int kScanPer = 4, kScanPerMany = 16, kScanMany = 1 << 20;
@@ -345,17 +345,6 @@ __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
     }
 }
 
-// The workgroup's inclusive sums of the tile counts (project_scan_add_kernel adds
-// the partition's offset) and their total.
-__device__ __forceinline__ void count_scan(uint32_t cnt, int idx, int n,
-                                           int* __restrict__ cum_tiles_hit,
-                                           uint32_t* __restrict__ part_tot, uint32_t* s_tmp) {
-    const uint32_t incl = block_exclusive_scan256(cnt, s_tmp) + cnt;
-    if (idx < n) cum_tiles_hit[idx] = (int)incl;
-    if (threadIdx.x == 255) part_tot[blockIdx.x] = incl;
-}
-
-
 __global__ __launch_bounds__(256) void project_fwd_kernel(
     Camera c, const float* __restrict__ means3d, const float* __restrict__ scales,
     const float* __restrict__ quats, const float* __restrict__ viewmat,
@@ -376,7 +365,7 @@ __global__ __launch_bounds__(256) void project_fwd_kernel(
                                     depths, radii, conics, comp_out, num_tiles_hit, opacities,
                                     rects, colors, nch, splats, antialiased)
             : 0u;
-    count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
+    block_count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
 }
 
 // Opacity-limited tile rectangles (opacity_tile_rect) of the projected
@@ -402,7 +391,7 @@ __global__ __launch_bounds__(256) void tile_rects_kernel(
         cnt = rect_count(rc);
         if (num_tiles_hit) num_tiles_hit[idx] = (int)cnt;
     }
-    count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
+    block_count_scan(cnt, idx, c.num_points, cum_tiles_hit, part_tot, s_tmp);
 }
 
 // cum_tiles_hit += its partition's offset, `per` partitions per workgroup: the
@@ -952,6 +941,10 @@ static hipError_t scan_add(int n, int parts, const uint32_t* part_tot, int* cum_
     project_scan_add_kernel<<<(parts + per - 1) / per, 256, 0, s>>>(
         n, parts, per, part_tot, cum_tiles_hit, count_out, ticket);
     return hipGetLastError();
+}
+
+hipError_t count_scan_add(int n, const uint32_t* part_tot, int* cum, hipStream_t s) {
+    return scan_add(n, (n + kCountPart - 1) / kCountPart, part_tot, cum, nullptr, 0u, s);
 }
 
 hipError_t project_fwd(const Camera& c, const float* means3d, const float* scales,

@@ -299,28 +299,72 @@ __device__ __forceinline__ uint2 grid_rect(uint2 rc, int tiles_x, int tiles_y, b
     return pack_rect(x0, x1, y0, y1);
 }
 
+// Where the pairs exceed the capacity, the first cap of them in emission order
+// (Gaussian by Gaussian, a rectangle row by row) are binned: the Gaussians before
+// `id` whole, of `id` the first `rows` rows, of the last of them (tile row `row`)
+// the first `width` tiles, the others not at all.  id = n, row = -1: all pairs.
+struct Cut {
+    int id, rows, row, width;
+};
+// cum: the inclusive tile counts in id order (one load where nothing is cut).
+__device__ __forceinline__ Cut emission_cut(const int* __restrict__ cum,
+                                            const uint2* __restrict__ rects, int n, int cap) {
+    if ((uint32_t)cum[n - 1] <= (uint32_t)cap) return {n, 0, -1, 0};
+    int id = 0, hi = n - 1;         // the first id whose count exceeds cap
+    while (id < hi) {
+        const int mid = (id + hi) >> 1;
+        if ((uint32_t)cum[mid] > (uint32_t)cap) hi = mid;
+        else id = mid + 1;
+    }
+    const uint2 rc = rects[id];
+    const uint32_t w = rc.y & 0xFFFFu;
+    const uint32_t left =
+        min((uint32_t)cap - (id > 0 ? (uint32_t)cum[id - 1] : 0u), rect_count(rc));
+    const int rows = w > 0 ? (int)((left + w - 1) / w) : 0;
+    if (rows == 0) return {id, 0, -1, 0};
+    return {id, rows, (int)(rc.x >> 16) + rows - 1, (int)(left - (uint32_t)(rows - 1) * w)};
+}
+// Gaussian id's rectangle up to the cut (its last row whole: run_span).
+__device__ __forceinline__ uint2 cut_rect(uint2 rc, uint32_t id, const Cut& cut) {
+    if (id < (uint32_t)cut.id) return rc;
+    const uint32_t rows = id == (uint32_t)cut.id ? (uint32_t)cut.rows : 0u;
+    return make_uint2(rc.x, (rc.y & 0xFFFFu) | min(rc.y >> 16, rows) << 16);
+}
+// A run's columns (x0 | w << 16); here: it lies in the cut's last row.
+__device__ __forceinline__ uint32_t run_span(uint2 run, const Cut& cut, bool here) {
+    if (!here || run.x != (uint32_t)cut.id) return run.y;
+    return (run.y & 0xFFFFu) | min(run.y >> 16, (uint32_t)cut.width) << 16;
+}
+
 // Step 1, counting: partition b holds the Gaussians perm[1024 b ..) (the ids
 // themselves where perm is null).  counts[row * row_stride + b * part_stride] =
 // its runs per row,
 // part_tot[b] = its pairs; with perm, in_order[i] = the rectangle of perm[i],
-// so that the random gather is paid once.  Also clears the tile bins and the
-// error word.
+// so that the random gather is paid once (and up to the cut).  Also clears the tile
+// bins and the error word and keeps the cut for the steps after it.
 __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
-    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
-    int tiles_y, int row_stride, int part_stride, uint32_t* __restrict__ counts,
-    uint32_t* __restrict__ part_tot, uint2* __restrict__ in_order, int num_tiles, int2* __restrict__ bins,
-    uint32_t* __restrict__ err) {
+    int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects,
+    const int* __restrict__ cum, int cap, int tiles_x, int tiles_y, int row_stride,
+    int part_stride, uint32_t* __restrict__ counts, uint32_t* __restrict__ part_tot,
+    uint2* __restrict__ in_order, int num_tiles, int2* __restrict__ bins,
+    Cut* __restrict__ cut_out, uint32_t* __restrict__ err) {
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
     const int tid = threadIdx.x, part = blockIdx.x;
-    if (part == 0 && tid == 0) *err = 0u;
+    const Cut cut = emission_cut(cum, rects, n, cap);
+    if (part == 0 && tid == 0) {
+        *err = 0u;
+        *cut_out = cut;
+    }
     for (int t = part * kRbThreads + tid; t < num_tiles; t += gridDim.x * kRbThreads)
         bins[t] = make_int2(0, 0);
     uint2 rc[kRbPer];
+    uint32_t id[kRbPer];
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
         const int i = part * kRbPart + k * kRbThreads + tid;
-        rc[k] = i < n ? rects[perm ? perm[i] : (uint32_t)i] : make_uint2(0u, 0u);
+        id[k] = i < n ? (perm ? perm[i] : (uint32_t)i) : 0u;
+        rc[k] = i < n ? rects[id[k]] : make_uint2(0u, 0u);
     }
     s_d[tid] = 0;
     __syncthreads();
@@ -328,10 +372,11 @@ __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
         const int i = part * kRbPart + k * kRbThreads + tid;
-        if (perm && i < n) in_order[i] = rc[k];
         bool bad;
         pairs += rect_count(rc[k]);
-        const uint2 r = grid_rect(rc[k], tiles_x, tiles_y, bad);
+        const uint2 kept = cut_rect(rc[k], id[k], cut);
+        if (perm && i < n) in_order[i] = kept;
+        const uint2 r = grid_rect(kept, tiles_x, tiles_y, bad);
         if (rect_count(r) > 0)
             add_differences(s_d, kRbThreads, {(int)(r.x >> 16), (int)(r.y >> 16)});
     }
@@ -352,8 +397,8 @@ __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
     int tiles_y, int parts, bool fold, const uint32_t* __restrict__ counts,
     uint32_t* __restrict__ row_len, const uint32_t* __restrict__ part_tot,
-    uint2* __restrict__ runs, int cap, unsigned long long* __restrict__ total_out,
-    uint32_t* __restrict__ err) {
+    uint2* __restrict__ runs, int cap, const Cut* __restrict__ cut_in,
+    unsigned long long* __restrict__ total_out, uint32_t* __restrict__ err) {
     constexpr int PER = round_per(STABLE);
     __shared__ PlaceShared<uint2, COLS, 3072, STABLE> sh;
     __shared__ uint64_t s_sum[kRbWaves];
@@ -361,13 +406,14 @@ __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     Interval iv[kRbPer];
     uint2 val[kRbPer];
     bool bad_any = false;
+    const Cut cut = *cut_in;
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
         const int i = part * kRbPart + interval_index<PER>(k);
         const uint32_t id = i < n ? (perm ? perm[i] : (uint32_t)i) : 0u;
         bool bad;
-        const uint2 rc =
-            grid_rect(i < n ? rects[i] : make_uint2(0u, 0u), tiles_x, tiles_y, bad);
+        const uint2 rc = grid_rect(cut_rect(i < n ? rects[i] : make_uint2(0u, 0u), id, cut),
+                                   tiles_x, tiles_y, bad);
         bad_any = bad_any || bad;
         iv[k].lo = (int)(rc.x >> 16);
         iv[k].len = rect_count(rc) > 0 ? (int)(rc.y >> 16) : 0;
@@ -447,16 +493,16 @@ __device__ __forceinline__ void for_partitions(int total, F body) {
 }
 
 // counts[column] = the runs [begin, end) that cover the column, all 256 of them.
-// Called by the whole workgroup.
+// here: see run_span.  Called by the whole workgroup.
 __device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, int begin, int end,
-                                              int* s_d, uint32_t* s_tmp,
-                                              uint32_t* __restrict__ counts) {
+                                              const Cut& cut, bool here, int* s_d,
+                                              uint32_t* s_tmp, uint32_t* __restrict__ counts) {
     const int tid = threadIdx.x;
     uint32_t w[kRbPer];
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
         const int i = begin + k * kRbThreads + tid;
-        w[k] = i < end ? runs[i].y : 0u;
+        w[k] = i < end ? run_span(runs[i], cut, here) : 0u;
     }
     s_d[tid] = 0;
     __syncthreads();
@@ -474,12 +520,13 @@ __device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, in
 // first partition), desc[-1].x the number of partitions.
 __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
     const uint2* __restrict__ runs, const uint32_t* __restrict__ row_len, int tiles_y, int cap,
-    uint32_t* __restrict__ counts, int4* __restrict__ desc) {
+    const Cut* __restrict__ cut_in, uint32_t* __restrict__ counts, int4* __restrict__ desc) {
     __shared__ RowTable rt;
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
     __shared__ uint64_t s_tmp64[kRbWaves];
     const int tid = threadIdx.x;
+    const Cut cut = *cut_in;
     row_table(rt, row_len, tiles_y, cap, s_tmp64);
     if (blockIdx.x == 0 && tid == 0) desc[-1] = make_int4(rt.p0[kRowBinAxis], 0, 0, 0);
     for_partitions(rt.p0[kRowBinAxis], [&](int p) {
@@ -487,7 +534,8 @@ __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
         const int begin = rt.e0[r] + (p - rt.p0[r]) * kRbPart;
         const int end = min(rt.e0[r + 1], begin + kRbPart);
         if (tid == 0) desc[p] = make_int4(r, begin, end, p == rt.p0[r] ? 1 : 0);
-        count_columns(runs, begin, end, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
+        count_columns(runs, begin, end, cut, r == cut.row, s_d, s_tmp,
+                      counts + (size_t)p * kRowBinAxis);
     });
 }
 
@@ -599,8 +647,9 @@ __global__ __launch_bounds__(kScanThreads) void col_scan_kernel(
 template <bool STABLE, int COLS>
 __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
     const uint2* __restrict__ runs, const int4* __restrict__ desc, int tiles_x, int tiles_y,
-    int cap, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_first,
-    uint32_t* __restrict__ ids, int2* __restrict__ bins) {
+    int cap, const Cut* __restrict__ cut_in, const uint32_t* __restrict__ counts,
+    const uint32_t* __restrict__ tile_first, uint32_t* __restrict__ ids,
+    int2* __restrict__ bins) {
     constexpr int PER = round_per(STABLE);
     __shared__ PlaceShared<uint32_t, COLS, STABLE ? (COLS == 128 ? 4096 : 3072) : 5120, STABLE> sh;
     __shared__ int s_row0[kRowBinAxis];
@@ -610,16 +659,19 @@ __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
         tid < tiles_y ? tile_first[(size_t)tid * (kRowBinAxis + 1) + kRowBinAxis] : 0u;
     s_row0[tid] = (int)min(block_exclusive_scan256(pairs, s_tmp), (uint64_t)cap);
     const int parts = uniform_i(desc[-1].x);
+    const Cut cut = *cut_in;
     for_partitions(parts, [&](int p) {
         const int4 d = desc[p];
+        const bool here = d.x == cut.row;
         Interval iv[kRbPer];
         uint32_t id[kRbPer];
 #pragma unroll
         for (int k = 0; k < kRbPer; ++k) {
             const int i = d.y + interval_index<PER>(k);
             const uint2 run = i < d.z ? runs[i] : make_uint2(0u, 0u);
+            const uint32_t span = run_span(run, cut, here);
             id[k] = run.x;
-            iv[k] = {(int)(run.y & 0xFFFFu), (int)(run.y >> 16)};
+            iv[k] = {(int)(span & 0xFFFFu), (int)(span >> 16)};
         }
         clear_place(sh);
         __syncthreads();
@@ -832,7 +884,8 @@ __global__ __launch_bounds__(kRbThreads) void batch_col_count_kernel(
     const int tid = threadIdx.x;
     for_partitions(uniform_i(desc[-1].x), [&](int p) {
         const int4 d = desc[p];
-        count_columns(runs, d.y, d.z, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
+        count_columns(runs, d.y, d.z, Cut{}, false, s_d, s_tmp,
+                      counts + (size_t)p * kRowBinAxis);
     });
 }
 
@@ -918,6 +971,7 @@ RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap) {
     p.max_col_parts = p.cap / kRbPart + tiles_y;
     size_t o = 0;
     const size_t parts = (size_t)(p.parts > 0 ? p.parts : 1);
+    p.cut = o; o = align256(o + sizeof(Cut));
     p.row_len = o; o = align256(o + 4ull * kRowBinAxis);
     p.row_counts = o; o = align256(o + 4ull * kRowBinAxis * parts);
     p.part_tot = o; o = align256(o + 4ull * parts);
@@ -929,7 +983,7 @@ RowBinPlan row_bin_plan(int n, int tiles_x, int tiles_y, int cap) {
 }
 
 hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects,
-                   uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
+                   const int* cum, uint2* in_order, uint2* runs, uint32_t* ids, uint32_t* tiles_sorted,
                    int2* bins, unsigned long long* total, uint32_t* err, void* scratch,
                    hipStream_t s) {
     if (p.tiles_x > kRowBinAxis || p.tiles_y > kRowBinAxis || p.n <= 0)
@@ -937,13 +991,12 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     uint8_t* b = static_cast<uint8_t*>(scratch);
     auto U = [&](size_t off) { return reinterpret_cast<uint32_t*>(b + off); };
     int4* desc = reinterpret_cast<int4*>(b + p.desc) + 1;
+    Cut* cut = reinterpret_cast<Cut*>(b + p.cut);
     const int tiles = p.tiles_x * p.tiles_y;
     hipError_t e;
-    row_count_kernel<<<p.parts, kRbThreads, 0, s>>>(p.n, perm, rects, p.tiles_x, p.tiles_y,
-                                                    p.fold ? 1 : p.parts,
-                                                    p.fold ? kRowBinAxis : 1, U(p.row_counts),
-                                                    U(p.part_tot),
-                                                    in_order, tiles, bins, err);
+    row_count_kernel<<<p.parts, kRbThreads, 0, s>>>(
+        p.n, perm, rects, cum, p.cap, p.tiles_x, p.tiles_y, p.fold ? 1 : p.parts,
+        p.fold ? kRowBinAxis : 1, U(p.row_counts), U(p.part_tot), in_order, tiles, bins, cut, err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!p.fold && (e = column_scan(U(p.row_counts), p.parts, U(p.row_len), p.tiles_y, s)) !=
                        hipSuccess)
@@ -951,9 +1004,7 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
 #define JSA_ROW(ST, COLS)                                                                     \
     row_place_kernel<ST, COLS><<<p.parts, kRbThreads, 0, s>>>(                                \
         p.n, perm, perm ? in_order : rects, p.tiles_x, p.tiles_y, p.parts, p.fold,            \
-        U(p.row_counts),                                                                      \
-        U(p.row_len),                                                                         \
-        U(p.part_tot), runs, p.cap, total, err)
+        U(p.row_counts), U(p.row_len), U(p.part_tot), runs, p.cap, cut, total, err)
     if (narrow(p.tiles_y)) {
         if (perm) JSA_ROW(true, 128); else JSA_ROW(false, 128);
     } else {
@@ -965,7 +1016,7 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     // persistent: as many workgroups as fit the chip, or one per partition
     const int most = 8 * ((p.max_col_parts + 7) / 8);
     const int grid = most < 2048 ? most : 2048;
-    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_y, p.cap,
+    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_y, p.cap, cut,
                                                  U(p.col_counts), desc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_LAUNCH(COLS)                                                                      \
@@ -976,7 +1027,8 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_COL(ST, COLS)                                                                     \
     col_place_kernel<ST, COLS><<<grid, kRbThreads, 0, s>>>(                                   \
-        runs, desc, p.tiles_x, p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first), ids, bins)
+        runs, desc, p.tiles_x, p.tiles_y, p.cap, cut, U(p.col_counts), U(p.tile_first), ids,  \
+        bins)
     if (narrow(p.tiles_x)) {
         if (perm) JSA_COL(true, 128); else JSA_COL(false, 128);
     } else {
