@@ -36,6 +36,7 @@
 // stored contiguously; with more values than the stage holds (long intervals,
 // whose columns then hold many values anyway) they are stored directly.
 #include "common.hpp"
+#include "positions.hpp"
 
 namespace jsa {
 namespace {
@@ -207,8 +208,8 @@ __device__ __forceinline__ int place(PlaceShared<V, COLS, CAP, STABLE>& sh, cons
         if (staged) {
             sh.out[pos] = v;
         } else {
-            const int at = sh.delta[c] + pos;
-            if ((unsigned)at < (unsigned)cap) out_g[at] = v;
+            const uint32_t at = (uint32_t)sh.delta[c] + (uint32_t)pos;
+            if (at < (uint32_t)cap) out_g[at] = v;
         }
     };
     int* pos = sh.cnt[wave];
@@ -249,9 +250,10 @@ __device__ __forceinline__ int place(PlaceShared<V, COLS, CAP, STABLE>& sh, cons
     if (staged) {
         // 16 lanes per column: a column's values are one contiguous run
         for (int c = tid >> 4; c < ncols; c += kRbThreads / 16) {
-            const int end = sh.first[c + 1], to = sh.delta[c];
+            const int end = sh.first[c + 1];
+            const uint32_t to = (uint32_t)sh.delta[c];
             for (int i = sh.first[c] + (tid & 15); i < end; i += 16)
-                if ((unsigned)(to + i) < (unsigned)cap) out_g[to + i] = sh.out[i];
+                if (to + (uint32_t)i < (uint32_t)cap) out_g[to + (uint32_t)i] = sh.out[i];
         }
     }
     __syncthreads();
@@ -271,9 +273,9 @@ __device__ __forceinline__ void place_all(PlaceShared<V, COLS, CAP, STABLE>& sh,
             clear_place(sh);
             __syncthreads();
         }
-        column_base = min(column_base + place<PER>(sh, iv + r, val + r, ncols, column_base,
-                                                   out_g, cap),
-                          cap);
+        column_base = clamped_sum(
+            column_base,
+            (uint32_t)place<PER>(sh, iv + r, val + r, ncols, column_base, out_g, cap), cap);
     }
 }
 // Interval k (of kRbPer) of a lane, in rounds of PER: its index within the
@@ -501,8 +503,8 @@ __device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, in
     uint32_t w[kRbPer];
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
-        const int i = begin + k * kRbThreads + tid;
-        w[k] = i < end ? run_span(runs[i], cut, here) : 0u;
+        const int i = k * kRbThreads + tid;
+        w[k] = i < end - begin ? run_span(runs[begin + i], cut, here) : 0u;
     }
     s_d[tid] = 0;
     __syncthreads();
@@ -532,7 +534,7 @@ __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
     for_partitions(rt.p0[kRowBinAxis], [&](int p) {
         const int r = row_of(rt, p);
         const int begin = rt.e0[r] + (p - rt.p0[r]) * kRbPart;
-        const int end = min(rt.e0[r + 1], begin + kRbPart);
+        const int end = part_end(begin, rt.e0[r + 1], kRbPart);
         if (tid == 0) desc[p] = make_int4(r, begin, end, p == rt.p0[r] ? 1 : 0);
         count_columns(runs, begin, end, cut, r == cut.row, s_d, s_tmp,
                       counts + (size_t)p * kRowBinAxis);
@@ -667,22 +669,20 @@ __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
         uint32_t id[kRbPer];
 #pragma unroll
         for (int k = 0; k < kRbPer; ++k) {
-            const int i = d.y + interval_index<PER>(k);
-            const uint2 run = i < d.z ? runs[i] : make_uint2(0u, 0u);
+            const int i = interval_index<PER>(k);
+            const uint2 run = i < d.z - d.y ? runs[d.y + i] : make_uint2(0u, 0u);
             const uint32_t span = run_span(run, cut, here);
             id[k] = run.x;
             iv[k] = {(int)(span & 0xFFFFu), (int)(span >> 16)};
         }
         clear_place(sh);
         __syncthreads();
-        // (both terms at most cap < 2^30)
         const int row0 = s_row0[d.x];
-        const int base = tid < tiles_x
-                             ? min(row0 + (int)counts[(size_t)p * kRowBinAxis + tid], cap)
-                             : 0;
+        const int base =
+            tid < tiles_x ? clamped_sum(row0, counts[(size_t)p * kRowBinAxis + tid], cap) : 0;
         if (d.w && tid < tiles_x) {
             const uint32_t* tf = tile_first + (size_t)d.x * (kRowBinAxis + 1) + tid;
-            const int b = min(row0 + (int)tf[0], cap), e = min(row0 + (int)tf[1], cap);
+            const int b = clamped_sum(row0, tf[0], cap), e = clamped_sum(row0, tf[1], cap);
             if (e > b) bins[d.x * tiles_x + tid] = make_int2(b, e);
         }
         place_all<PER>(sh, iv, id, tiles_x, base, ids, cap);
@@ -799,10 +799,9 @@ __global__ __launch_bounds__(1024) void batch_table_kernel(
         const uint32_t* f = row_first + (size_t)(r / max_y) * (kRowBinAxis + 1) + r % max_y;
         return (uint64_t)(f[1] - f[0]);
     };
-    auto np = [](int b, int e) { return (e - b + kRbPart - 1) / kRbPart; };
     scan_rounds(rows, s_tmp, len, [&](int r, uint64_t e, uint64_t v) {
         row_off[r] = (int)min(e, lim);
-        row_part[r] = np((int)min(e, lim), (int)min(e + v, lim));       // for now
+        row_part[r] = part_count((int)min(e, lim), (int)min(e + v, lim), kRbPart);  // for now
     });
     const uint64_t all = scan_rounds(
         rows, s_tmp, [&](int r) { return (uint64_t)row_part[r]; },
@@ -810,9 +809,10 @@ __global__ __launch_bounds__(1024) void batch_table_kernel(
             row_part[r] = (int)e;
             const int begin = row_off[r];
             const int end = (int)min((uint64_t)begin + len(r), lim);
-            for (int q = 0; q < (int)v; ++q)
-                desc[(int)e + q] = make_int4(r, begin + q * kRbPart,
-                                             min(end, begin + (q + 1) * kRbPart), q == 0);
+            for (int q = 0; q < (int)v; ++q) {
+                const int at = begin + q * kRbPart;
+                desc[(int)e + q] = make_int4(r, at, part_end(at, end, kRbPart), q == 0);
+            }
         });
     if (threadIdx.x == 0) {
         row_part[rows] = (int)all;
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(kRbThreads) void batch_row_place_kernel(
         bad_any = bad_any || bad;
         iv[k].lo = (int)(rc.x >> 16);
         iv[k].len = rect_count(rc) > 0 ? (int)(rc.y >> 16) : 0;
-        val[k] = make_uint2((uint32_t)(vr.item_off + i), (rc.x & 0xFFFFu) | (rc.y << 16));
+        val[k] = make_uint2((uint32_t)vr.item_off + (uint32_t)i, (rc.x & 0xFFFFu) | (rc.y << 16));
     }
     if (bad_any) atomicOr(err, 4u);
     if (lane == 0) s_pairs[wave] = pairs;
@@ -930,20 +930,19 @@ __global__ __launch_bounds__(kRbThreads) void batch_col_place_kernel(
         uint32_t id[kRbPer];
 #pragma unroll
         for (int k = 0; k < kRbPer; ++k) {
-            const int i = d.y + interval_index<PER>(k);
-            const uint2 run = i < d.z ? runs[i] : make_uint2(0u, 0u);
+            const int i = interval_index<PER>(k);
+            const uint2 run = i < d.z - d.y ? runs[d.y + i] : make_uint2(0u, 0u);
             id[k] = run.x;
             iv[k] = {(int)(run.y & 0xFFFFu), (int)(run.y >> 16)};
         }
         clear_place(sh);
         __syncthreads();
         const int row0 = row_pair[d.x];
-        const int base = tid < tiles_x
-                             ? min(row0 + (int)counts[(size_t)p * kRowBinAxis + tid], cap)
-                             : 0;
+        const int base =
+            tid < tiles_x ? clamped_sum(row0, counts[(size_t)p * kRowBinAxis + tid], cap) : 0;
         if (d.w && tid < tiles_x) {
             const uint32_t* tf = tile_first + (size_t)d.x * (kRowBinAxis + 1) + tid;
-            const int b = min(row0 + (int)tf[0], cap), e = min(row0 + (int)tf[1], cap);
+            const int b = clamped_sum(row0, tf[0], cap), e = clamped_sum(row0, tf[1], cap);
             if (e > b) bins[views[v].bin_off + ty * tiles_x + tid] = make_int2(b, e);
         }
         place_all<PER>(sh, iv, id, tiles_x, base, ids, cap);
