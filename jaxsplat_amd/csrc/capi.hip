@@ -2,15 +2,15 @@
 // include/jaxsplat_amd.h): argument validation, descriptor -> camera
 // conversion, workspace carving, and the four reference-compatible XLA
 // custom-call targets.
-#include <unistd.h>
-
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -887,18 +887,56 @@ namespace {
 // below, in place of a copy to pinned memory with an event, and nine allocations
 // and a call less: 105 -> 59 us per view of 2k Gaussians at 256 x 256 (bound by
 // the host), 658 -> 637 us per step of 1M at 1080p (bound by the kernels).  The
-// ticket tells a late store of an abandoned read from the awaited one; the word
-// is given back with its thread.
+// ticket tells a late store of an abandoned read from the awaited one.
+//
+// A thread that ends gives its word to the next one and never frees it: a kernel
+// of a read that it abandoned may still be queued and store to it.  So there are as
+// many words (64 bytes) as threads have read counts at once, and the tickets are
+// the process's, not the word's.
 struct CountWord {
-    uint64_t* host = nullptr;
-    uint64_t* dev = nullptr;
+    uint64_t* host;
+    uint64_t* dev;
+    CountWord* next;
+};
+std::mutex g_count_lock;
+CountWord* g_count_free = nullptr;
+std::atomic<uint32_t> g_ticket{0};
+
+struct OwnCount {
+    CountWord* word = nullptr;
     uint32_t ticket = 0;
-    pid_t pid = 0;
-    ~CountWord() {
-        if (host && pid == getpid()) (void)hipHostFree(host);
+    ~OwnCount() {
+        if (!word) return;
+        std::lock_guard<std::mutex> lock(g_count_lock);
+        word->next = g_count_free;
+        g_count_free = word;
     }
 };
-thread_local CountWord t_count;
+thread_local OwnCount t_count;
+
+// A word that no thread has, or null.
+CountWord* take_count_word() {
+    {
+        std::lock_guard<std::mutex> lock(g_count_lock);
+        if (CountWord* w = g_count_free) {
+            g_count_free = w->next;
+            return w;
+        }
+    }
+    void *h = nullptr, *p = nullptr;
+    if (hipHostMalloc(&h, 64, hipHostMallocCoherent | hipHostMallocMapped |
+                                  hipHostMallocPortable) != hipSuccess)
+        return nullptr;
+    CountWord* w = hipHostGetDevicePointer(&p, h, 0) == hipSuccess ? new (std::nothrow) CountWord
+                                                                 : nullptr;
+    if (!w) {
+        (void)hipHostFree(h);       // (no kernel has seen it)
+        return nullptr;
+    }
+    *w = {static_cast<uint64_t*>(h), static_cast<uint64_t*>(p), nullptr};
+    *w->host = 0;
+    return w;
+}
 
 __global__ void count_kernel(const int32_t* __restrict__ count, uint64_t* __restrict__ out,
                              uint32_t ticket) {
@@ -912,22 +950,10 @@ int next_ticket(hipStream_t s) {
     if (capturing != hipStreamCaptureStatusNone)
         return fail(JAXSPLAT_ERR_INVALID,
                     "a count cannot be read while its stream is capturing (give a capacity)");
-    CountWord& w = t_count;
-    if (!w.host) {
-        void *h = nullptr, *p = nullptr;
-        JSA_CHECK_HIP(hipHostMalloc(&h, 64, hipHostMallocCoherent | hipHostMallocMapped |
-                                                hipHostMallocPortable),
-                      "count_begin");
-        if (hipHostGetDevicePointer(&p, h, 0) != hipSuccess) {
-            (void)hipHostFree(h);
-            return fail(JAXSPLAT_ERR_HIP, "count_begin: no device pointer of pinned memory");
-        }
-        w.host = static_cast<uint64_t*>(h);
-        w.dev = static_cast<uint64_t*>(p);
-        w.pid = getpid();
-        *w.host = 0;
-    }
-    if (++w.ticket == 0) w.ticket = 1;
+    if (!t_count.word && !(t_count.word = take_count_word()))
+        return fail(JAXSPLAT_ERR_HIP, "count_begin: no pinned memory");
+    do t_count.ticket = ++g_ticket;
+    while (t_count.ticket == 0);        // (0 is a new word's)
     return JAXSPLAT_OK;
 }
 
@@ -946,21 +972,21 @@ int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream) {
     g_err.clear();
     if (!count || !ticket) return fail(JAXSPLAT_ERR_INVALID, "count_begin: NULL required pointer");
     if (int st = next_ticket(static_cast<hipStream_t>(stream))) return st;
-    const CountWord& w = t_count;
-    count_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(count, w.dev, w.ticket);
+    count_kernel<<<1, 1, 0, static_cast<hipStream_t>(stream)>>>(count, t_count.word->dev,
+                                                                t_count.ticket);
     JSA_CHECK_HIP(hipGetLastError(), "count_begin");
-    *ticket = w.ticket;
+    *ticket = t_count.ticket;
     return JAXSPLAT_OK;
 }
 
 int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, void* stream) {
     g_err.clear();
     if (!count || !value) return fail(JAXSPLAT_ERR_INVALID, "count_wait: NULL required pointer");
-    const CountWord& w = t_count;
-    if (!w.host || ticket != w.ticket)
+    const CountWord* w = t_count.word;
+    if (!w || ticket != t_count.ticket)
         return fail(JAXSPLAT_ERR_INVALID, "count_wait: not this thread's last ticket");
     auto arrived = [&]() {
-        const uint64_t v = __atomic_load_n(w.host, __ATOMIC_ACQUIRE);
+        const uint64_t v = __atomic_load_n(w->host, __ATOMIC_ACQUIRE);
         if ((uint32_t)(v >> 32) != (uint32_t)ticket) return false;
         *value = (int32_t)(uint32_t)v;
         return true;
@@ -1091,7 +1117,7 @@ int jaxsplat_render_begin(const jaxsplat_descriptor* d, const float* means3d,
                           antialiased ? at<float>(state, r.comp) : nullptr, nullptr,
                           at<int32_t>(state, r.cum), at<uint32_t>(state, r.rects),
                           at<float>(state, r.splats), at<void>(state, r.ws), r.ws_bytes,
-                          count ? t_count.dev : nullptr, count ? t_count.ticket : 0u,
+                          count ? t_count.word->dev : nullptr, count ? t_count.ticket : 0u,
                           antialiased != 0, stream);
 }
 
