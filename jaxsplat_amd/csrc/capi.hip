@@ -12,6 +12,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -991,14 +992,31 @@ int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, v
         *value = (int32_t)(uint32_t)v;
         return true;
     };
-    // polled for 2 ms; a stream with more than that before the count is waited for
-    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
-    for (unsigned i = 0; (i & 63u) != 63u || std::chrono::steady_clock::now() < until; ++i) {
-        if (arrived()) return JAXSPLAT_OK;
-        __builtin_ia32_pause();
-    }
+    // Polled until it arrives, whatever is queued behind it: for 2 ms at once, then
+    // giving up the processor in between, and after 20 ms asleep for the most part.
+    // The stream itself is asked at 2, 4, 8, ... ms: one that failed ends the wait, and
+    // where it has ended without the count (another read's late store took the
+    // word) the count is copied.
+    using namespace std::chrono;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    JSA_CHECK_HIP(hipStreamSynchronize(s), "count_wait");
+    const auto begin = steady_clock::now();
+    for (auto ask = milliseconds(2);;) {
+        for (int i = 0; i < 64; ++i) {
+            if (arrived()) return JAXSPLAT_OK;
+            __builtin_ia32_pause();
+        }
+        const auto waited = steady_clock::now() - begin;
+        if (waited < milliseconds(2)) continue;
+        if (waited >= ask) {
+            ask *= 2;
+            const hipError_t q = hipStreamQuery(s);
+            if (q == hipSuccess) break;
+            if (q != hipErrorNotReady) JSA_CHECK_HIP(q, "count_wait");
+            (void)hipGetLastError();            // not ready is no error
+        }
+        if (waited < milliseconds(20)) std::this_thread::yield();
+        else std::this_thread::sleep_for(microseconds(50));
+    }
     if (arrived()) return JAXSPLAT_OK;
     JSA_CHECK_HIP(hipMemcpyAsync(value, count, 4, hipMemcpyDeviceToHost, s), "count_wait");
     JSA_CHECK_HIP(hipStreamSynchronize(s), "count_wait");

@@ -89,3 +89,19 @@ def test_thread_ends_before_its_count_is_stored():
     run(read)
     assert got == [8] * 12
     assert _wait(mine, _begin(mine, idle), idle) == 7
+
+
+@pytest.mark.parametrize("ms", [0, 4, 30])
+def test_wait_does_not_wait_for_what_is_behind(ms):
+    """A count behind `ms` of work and before 300 ms more arrives while that runs."""
+    t = H.torch()
+    before, behind = _work(ms), _work(300)
+    (count,) = _counts(12345)
+    s = t.cuda.Stream()
+    with t.cuda.stream(s):
+        before()
+        ticket = _begin(count, s)
+        behind()
+    assert _wait(count, ticket, s) == 12345
+    assert not s.query(), "the work behind the count has ended"
+    s.synchronize()
