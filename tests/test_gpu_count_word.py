@@ -105,3 +105,29 @@ def test_wait_does_not_wait_for_what_is_behind(ms):
     assert _wait(count, ticket, s) == 12345
     assert not s.query(), "the work behind the count has ended"
     s.synchronize()
+
+
+def test_late_store_of_an_abandoned_read():
+    """A read abandoned behind 20 ms of work stores over the count of the next one,
+    which is then copied; the abandoned ticket is refused, before and after."""
+    t, L = H.torch(), _lib.lib()
+    queue = _work(20)
+    first, second = _counts(111, 222)
+    slow, idle = t.cuda.Stream(), t.cuda.Stream()
+    value = ctypes.c_int32(-1)
+
+    def refused():
+        return L.jaxsplat_count_wait(H.P(first), abandoned, ctypes.byref(value),
+                                     _stream(slow)) == _lib.ERR_INVALID and value.value == -1
+
+    with t.cuda.stream(slow):
+        queue()
+        abandoned = _begin(first, slow)
+    ticket = _begin(second, idle)
+    assert refused()
+    idle.synchronize()
+    assert not slow.query(), "the late store came too early for this test"
+    slow.synchronize()                  # now the word holds the abandoned read's count
+    assert _wait(second, ticket, idle) == 222
+    assert refused()
+    assert _wait(first, _begin(first, idle), idle) == 111
