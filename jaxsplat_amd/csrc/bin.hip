@@ -1279,8 +1279,8 @@ BatchLayout batch_layout(const BatchBinPlan& p) {
 
 }  // namespace
 
-BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int max_x,
-                            int max_y, int isect_cap) {
+BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int rows,
+                            int max_x, int max_y, int isect_cap) {
     BatchBinPlan p{};
     p.n_items = n_items;
     p.num_views = num_views;
@@ -1290,7 +1290,7 @@ BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int 
     p.num_bins = num_views << p.tile_bits;
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
     p.by_rows = max_x <= kRowBinAxis && max_y <= kRowBinAxis && num_views <= kMaxBatchViews;
-    if (p.by_rows) p.rows = batch_row_plan(num_views, parts, max_x, max_y, isect_cap);
+    if (p.by_rows) p.rows = batch_row_plan(num_views, parts, rows, max_x, max_y, isect_cap);
     p.scratch_bytes = batch_layout(p).end;
     return p;
 }

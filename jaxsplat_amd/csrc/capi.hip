@@ -1521,7 +1521,7 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
         return fail(JAXSPLAT_ERR_INVALID, "too many Gaussians (%lld)", g);
     }
     b->n_gauss = (int)g;
-    long long items = 0, tiles = 0, pix = 0, parts = 0;
+    long long items = 0, tiles = 0, pix = 0, parts = 0, rows = 0;
     int max_x = 1, max_y = 1;
     int prev_scene = 0;
     for (int s = 0; s < num_scenes; ++s) b->scenes[s].v_begin = b->scenes[s].v_end = 0;
@@ -1558,6 +1558,8 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
         r.pix_off = pix;
         r.part_off = (int)parts;
         parts += (r.n + jsa::kRowBinPart - 1) / jsa::kRowBinPart;
+        r.row_off = (int)rows;
+        rows += r.tiles_y;
         max_x = std::max(max_x, r.tiles_x);
         max_y = std::max(max_y, r.tiles_y);
         items += r.n;
@@ -1576,7 +1578,7 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
     b->total_tiles = (int)tiles;
     b->num_pixels = pix;
     b->bin = jsa::batch_bin_plan(b->n_items, num_views, b->max_view_tiles, (int)parts,
-                                 max_x, max_y, (int)isect_capacity);
+                                 (int)rows, max_x, max_y, (int)isect_capacity);
     if (b->bin.tile_bits + b->bin.view_bits > 31) {
         delete b;
         return fail(JAXSPLAT_ERR_INVALID, "views x tiles exceed 2^31 bins");

@@ -504,7 +504,7 @@ struct alignas(16) ViewRec {
     int view;             // row of viewmats and backgrounds
     long long pix_off;    // first pixel in the image-sized buffers
     int part_off;         // first binning partition (kRowBinPart items)
-    int reserved;
+    int row_off;          // first tile row over all views
 };
 static_assert(sizeof(ViewRec) == 80, "ViewRec layout");
 
@@ -712,16 +712,16 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
                    hipStream_t s);
 
 // The same over the items of a batch's views (tile counts up to kRowBinAxis per
-// axis, ViewRec::part_off set, parts in all): bins[view's bin_off + tile] (all
+// axis, ViewRec::part_off and row_off set, parts and rows in all): bins[view's bin_off + tile] (all
 // num_bins cleared first), ids in arbitrary order inside a list, *count = min(
 // *total, cap), and every item's first pair in item order (item_first, optional;
 // at most cap).
 struct BatchRowPlan {
     int num_views, parts, max_x, max_y, rows, cap, max_col_parts;
-    size_t counts, part_tot, part_pair, row_first, row_off, row_part, row_pair, tile_first, desc,
-        col_counts, scratch_bytes;
+    size_t counts, part_tot, part_pair, row_first, row_view, row_len, row_off, row_part, row_pair,
+        tile_first, desc, col_counts, scratch_bytes;
 };
-BatchRowPlan batch_row_plan(int num_views, int parts, int max_x, int max_y, int cap);
+BatchRowPlan batch_row_plan(int num_views, int parts, int rows, int max_x, int max_y, int cap);
 hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint2* rects,
                          uint2* runs, uint32_t* ids, int num_bins, int2* bins,
                          uint32_t* item_first, int* count, unsigned long long* total,
@@ -807,10 +807,10 @@ struct BatchBinPlan {
     BatchRowPlan rows;
     size_t scratch_bytes;
 };
-// parts: binning partitions of all views (ViewRec::part_off); max_x, max_y: the
-// largest tile counts per axis.
-BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int max_x,
-                            int max_y, int isect_cap);
+// parts, rows: binning partitions and tile rows of all views (ViewRec::part_off,
+// row_off); max_x, max_y: the largest tile counts per axis.
+BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int rows,
+                            int max_x, int max_y, int isect_cap);
 // Sorted item ids of every (view, tile) and bins[view << tile_bits | tile].
 // The scratch keeps the intersection count clamped to the capacity (the
 // length the sorts and bins use), the exact total (64 bits) and an error word:

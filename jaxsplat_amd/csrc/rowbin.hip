@@ -691,8 +691,10 @@ __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
 
 // ---- batches ----
 // The same two steps over the items of many views: a partition of items lies in
-// one view, a "row" is a tile row of a view, r = view * max_y + y, and the
-// offsets that one view's workgroups find by themselves come from tables.  12
+// one view, a "row" is a tile row of a view, r = the view's row_off + y, and the
+// offsets that one view's workgroups find by themselves come from tables.  (Rows
+// of the tallest view for every view: 2000 views of 32 x 32 and one of 4096 rows of
+// pixels took 6370 us instead of 1270, and 1.1 GB more.)  12
 // views of 500k Gaussians at 800 x 800 (26M pairs of 6M items): 192 us in eight
 // launches, where emitting the pairs and sorting them by tile took 442 in
 // thirteen; step 2552 -> 2280 us.
@@ -743,15 +745,22 @@ __global__ __launch_bounds__(kRbThreads) void batch_row_count_kernel(
 }
 
 // Step 1, offsets: a view's rows are the columns of its partitions' counts;
-// row_first[view * 257 + y] the row's first run, relative to the view's.
+// row_first[view * 257 + y] the row's first run, relative to the view's; row_len and
+// row_view the runs and the view of every row.
 template <int COLS>
 __global__ __launch_bounds__(kScanThreads) void batch_row_scan_kernel(
     const ViewRec* __restrict__ views, int cap, uint32_t* __restrict__ counts,
-    uint32_t* __restrict__ row_first) {
+    uint32_t* row_first, uint32_t* __restrict__ row_len, int* __restrict__ row_view) {
     __shared__ ScanShared sh;
     const ViewRec vr = views[blockIdx.x];
-    scan_columns<COLS>(sh, vr.part_off, (vr.n + kRbPart - 1) / kRbPart, cap, counts,
-                       row_first + (size_t)blockIdx.x * (kRowBinAxis + 1));
+    uint32_t* first = row_first + (size_t)blockIdx.x * (kRowBinAxis + 1);
+    scan_columns<COLS>(sh, vr.part_off, (vr.n + kRbPart - 1) / kRbPart, cap, counts, first);
+    __syncthreads();            // first is written by several waves
+    const int y = threadIdx.x;
+    if (y < vr.tiles_y) {
+        row_len[vr.row_off + y] = first[y + 1] - first[y];
+        row_view[vr.row_off + y] = blockIdx.x;
+    }
 }
 
 // Exclusive scan of get(0..n) by one workgroup of 1024 threads, in rounds;
@@ -777,8 +786,8 @@ __device__ __forceinline__ uint64_t scan_rounds(int n, uint64_t* s_tmp, G get, P
 // Workgroup 1: every partition's first pair in item order (part_pair), and the
 // totals: *total, *count = min(total, cap), bit 8 of err.
 __global__ __launch_bounds__(1024) void batch_table_kernel(
-    int max_y, int rows, const uint32_t* __restrict__ row_first, int cap,
-    int* __restrict__ row_off, int* __restrict__ row_part, int4* __restrict__ desc, int parts,
+    int rows, const uint32_t* __restrict__ row_len, int cap, int* __restrict__ row_off,
+    int* __restrict__ row_part, int4* __restrict__ desc, int parts,
     const uint32_t* __restrict__ part_tot, uint32_t* __restrict__ part_pair,
     int* __restrict__ count, unsigned long long* __restrict__ total,
     uint32_t* __restrict__ err) {
@@ -795,10 +804,7 @@ __global__ __launch_bounds__(1024) void batch_table_kernel(
         }
         return;
     }
-    auto len = [&](int r) {
-        const uint32_t* f = row_first + (size_t)(r / max_y) * (kRowBinAxis + 1) + r % max_y;
-        return (uint64_t)(f[1] - f[0]);
-    };
+    auto len = [&](int r) { return (uint64_t)row_len[r]; };
     scan_rounds(rows, s_tmp, len, [&](int r, uint64_t e, uint64_t v) {
         row_off[r] = (int)min(e, lim);
         row_part[r] = part_count((int)min(e, lim), (int)min(e + v, lim), kRbPart);  // for now
@@ -823,9 +829,8 @@ __global__ __launch_bounds__(1024) void batch_table_kernel(
 // Step 1, placement (row_place_kernel), and every item's first pair.
 template <int COLS>
 __global__ __launch_bounds__(kRbThreads) void batch_row_place_kernel(
-    const ViewRec* __restrict__ views, int num_views, int max_y,
-    const uint2* __restrict__ rects, const uint32_t* __restrict__ counts,
-    const int* __restrict__ row_off, const uint32_t* __restrict__ part_pair,
+    const ViewRec* __restrict__ views, int num_views, const uint2* __restrict__ rects,
+    const uint32_t* __restrict__ counts, const int* __restrict__ row_off, const uint32_t* __restrict__ part_pair,
     uint2* __restrict__ runs, uint32_t* __restrict__ item_first, int cap,
     uint32_t* __restrict__ err) {
     constexpr int PER = round_per(false);
@@ -869,8 +874,7 @@ __global__ __launch_bounds__(kRbThreads) void batch_row_place_kernel(
     }
     const int base =
         tid < vr.tiles_y
-            ? (int)min((uint64_t)row_off[v * max_y] + counts[(size_t)part * kRowBinAxis + tid],
-                       (uint64_t)cap)
+            ? clamped_sum(row_off[vr.row_off], counts[(size_t)part * kRowBinAxis + tid], cap)
             : 0;
     place_all<PER>(sh, iv, val, vr.tiles_y, base, runs, cap);
 }
@@ -915,8 +919,8 @@ __global__ __launch_bounds__(1024) void batch_pair_scan_kernel(
 // Step 2, placement (col_place_kernel).
 template <int COLS>
 __global__ __launch_bounds__(kRbThreads) void batch_col_place_kernel(
-    const ViewRec* __restrict__ views, int max_y, const uint2* __restrict__ runs,
-    const int4* __restrict__ desc, int cap, const uint32_t* __restrict__ counts,
+    const ViewRec* __restrict__ views, const int* __restrict__ row_view,
+    const uint2* __restrict__ runs, const int4* __restrict__ desc, int cap, const uint32_t* __restrict__ counts,
     const uint32_t* __restrict__ tile_first, const int* __restrict__ row_pair,
     uint32_t* __restrict__ ids, int2* __restrict__ bins) {
     constexpr int PER = round_per(false);
@@ -924,7 +928,7 @@ __global__ __launch_bounds__(kRbThreads) void batch_col_place_kernel(
     const int tid = threadIdx.x;
     for_partitions(uniform_i(desc[-1].x), [&](int p) {
         const int4 d = desc[p];
-        const int v = d.x / max_y, ty = d.x - v * max_y;
+        const int v = row_view[d.x], ty = d.x - views[v].row_off;
         const int tiles_x = views[v].tiles_x;
         Interval iv[kRbPer];
         uint32_t id[kRbPer];
@@ -1043,25 +1047,27 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     return e;
 }
 
-BatchRowPlan batch_row_plan(int num_views, int parts, int max_x, int max_y, int cap) {
+BatchRowPlan batch_row_plan(int num_views, int parts, int rows, int max_x, int max_y, int cap) {
     BatchRowPlan p{};
     p.num_views = num_views;
     p.parts = parts;
     p.max_x = max_x;
     p.max_y = max_y;
-    p.rows = num_views * max_y;
+    p.rows = rows;
     p.cap = cap > 0 ? cap : 1;
     p.max_col_parts = p.cap / kRbPart + p.rows;
-    const size_t np = (size_t)(parts > 0 ? parts : 1), rows = (size_t)(p.rows > 0 ? p.rows : 1);
+    const size_t np = (size_t)(parts > 0 ? parts : 1), nr = (size_t)(rows > 0 ? rows : 1);
     size_t o = 0;
     p.counts = o; o = align256(o + 4ull * kRowBinAxis * np);
     p.part_tot = o; o = align256(o + 4ull * np);
     p.part_pair = o; o = align256(o + 4ull * np);
     p.row_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * (size_t)num_views);
-    p.row_off = o; o = align256(o + 4ull * rows);
-    p.row_part = o; o = align256(o + 4ull * (rows + 1));
-    p.row_pair = o; o = align256(o + 4ull * rows);
-    p.tile_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * rows);
+    p.row_view = o; o = align256(o + 4ull * nr);
+    p.row_len = o; o = align256(o + 4ull * nr);
+    p.row_off = o; o = align256(o + 4ull * nr);
+    p.row_part = o; o = align256(o + 4ull * (nr + 1));
+    p.row_pair = o; o = align256(o + 4ull * nr);
+    p.tile_first = o; o = align256(o + 4ull * (kRowBinAxis + 1) * nr);
     p.desc = o; o = align256(o + 16ull * ((size_t)p.max_col_parts + 1));
     p.col_counts = o; o = align256(o + 4ull * kRowBinAxis * (size_t)p.max_col_parts);
     p.scratch_bytes = o;
@@ -1082,17 +1088,17 @@ hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_LAUNCH(COLS)                                                                      \
     batch_row_scan_kernel<COLS><<<p.num_views, kScanThreads, 0, s>>>(                         \
-        views, p.cap, U(p.counts), U(p.row_first))
+        views, p.cap, U(p.counts), U(p.row_first), U(p.row_len), I(p.row_view))
     JSA_SCAN(p.max_y, JSA_LAUNCH);
 #undef JSA_LAUNCH
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    batch_table_kernel<<<2, 1024, 0, s>>>(p.max_y, p.rows, U(p.row_first), p.cap,
-                                          I(p.row_off), I(p.row_part), desc, p.parts,
-                                          U(p.part_tot), U(p.part_pair), count, total, err);
+    batch_table_kernel<<<2, 1024, 0, s>>>(p.rows, U(p.row_len), p.cap, I(p.row_off),
+                                          I(p.row_part), desc, p.parts, U(p.part_tot),
+                                          U(p.part_pair), count, total, err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_ROW(COLS)                                                                         \
     batch_row_place_kernel<COLS><<<p.parts, kRbThreads, 0, s>>>(                              \
-        views, p.num_views, p.max_y, rects, U(p.counts), I(p.row_off), U(p.part_pair), runs,  \
+        views, p.num_views, rects, U(p.counts), I(p.row_off), U(p.part_pair), runs,           \
         item_first, p.cap, err)
     if (narrow(p.max_y)) JSA_ROW(128);
     else JSA_ROW(256);
@@ -1112,8 +1118,8 @@ hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_COL(COLS)                                                                         \
     batch_col_place_kernel<COLS><<<grid, kRbThreads, 0, s>>>(                                 \
-        views, p.max_y, runs, desc, p.cap, U(p.col_counts), U(p.tile_first), I(p.row_pair),   \
-        ids, bins)
+        views, I(p.row_view), runs, desc, p.cap, U(p.col_counts), U(p.tile_first),            \
+        I(p.row_pair), ids, bins)
     if (narrow(p.max_x)) JSA_COL(128);
     else JSA_COL(256);
 #undef JSA_COL
