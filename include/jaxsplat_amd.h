@@ -218,6 +218,20 @@ int jaxsplat_bin_emit_sort(const jaxsplat_descriptor* d, uint32_t num_intersects
                            size_t workspace_bytes, void* stream);
 
 /*
+ * How the binning calls order the lists depends on how many intersections they
+ * expect (the results do not): jaxsplat_bin_and_sort, jaxsplat_bin_emit_sort and
+ * jaxsplat_bin_rects_sort expect num_intersects.  The _expecting forms take the
+ * number separately, for a num_intersects that is a capacity with headroom: the
+ * count of an earlier, similar binning, or 0 where none is known (from 2^19
+ * Gaussians the capacity then stands for it).  Same workspace.
+ */
+int jaxsplat_bin_emit_sort_expecting(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                     uint32_t expected, const void* depth_workspace,
+                                     int32_t* gaussian_ids_sorted, int32_t* tile_ids_sorted,
+                                     int32_t* tile_bins, void* workspace,
+                                     size_t workspace_bytes, void* stream);
+
+/*
  * Opacity-limited tile rectangles.  No counterpart in the reference; for a
  * fused projection + rasterization (the reference's render,
  * jaxsplat/__init__.py:6-70) whose intermediate tile lists the caller never
@@ -275,6 +289,14 @@ int jaxsplat_bin_rects_sort(const jaxsplat_descriptor* d, const float* depths,
                             uint32_t num_intersects, int32_t* gaussian_ids_sorted,
                             int32_t* tile_ids_sorted, int32_t* tile_bins, void* workspace,
                             size_t workspace_bytes, void* stream);
+
+/* See jaxsplat_bin_emit_sort_expecting. */
+int jaxsplat_bin_rects_sort_expecting(const jaxsplat_descriptor* d, const float* depths,
+                                      const uint32_t* tile_rects, const int32_t* cum_tiles_hit,
+                                      uint32_t num_intersects, uint32_t expected,
+                                      int32_t* gaussian_ids_sorted, int32_t* tile_ids_sorted,
+                                      int32_t* tile_bins, void* workspace,
+                                      size_t workspace_bytes, void* stream);
 
 /*
  * Synchronise `stream` and report an error recorded in the workspace of the
@@ -486,6 +508,15 @@ int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects
                            uint32_t channels, void* lists, size_t lists_bytes, void* bin_ws,
                            size_t bin_ws_bytes, float* out_img, int32_t* err, int64_t* total,
                            void* stream);
+/* With the intersections that are expected given separately
+ * (jaxsplat_bin_emit_sort_expecting; jaxsplat_render_finish expects num_intersects,
+ * or with err, where that is a capacity, does not know). */
+int jaxsplat_render_finish_expecting(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                     uint32_t expected, const void* state, size_t state_bytes,
+                                     const float* background, uint32_t channels, void* lists,
+                                     size_t lists_bytes, void* bin_ws, size_t bin_ws_bytes,
+                                     float* out_img, int32_t* err, int64_t* total,
+                                     void* stream);
 int jaxsplat_render_finish_backward(const jaxsplat_descriptor* d, uint32_t num_intersects,
                                     const float* means3d, const float* scales,
                                     const float* quats, const float* viewmat,

@@ -43,7 +43,8 @@ EXPORTS = (
     "jaxsplat_count_begin", "jaxsplat_count_wait", "jaxsplat_bin_record",
     "jaxsplat_render_state_size", "jaxsplat_render_lists_size", "jaxsplat_render_layout",
     "jaxsplat_render_begin", "jaxsplat_render_count", "jaxsplat_render_finish",
-    "jaxsplat_render_finish_backward",
+    "jaxsplat_render_finish_backward", "jaxsplat_render_finish_expecting",
+    "jaxsplat_bin_emit_sort_expecting", "jaxsplat_bin_rects_sort_expecting",
     "jaxsplat_project_forward_splats", "jaxsplat_rasterize_forward_splats",
     "jaxsplat_rasterize_forward_binned", "jaxsplat_rasterize_backward_binned",
     "jaxsplat_rasterize_forward_nd", "jaxsplat_rasterize_backward_nd",
@@ -130,6 +131,8 @@ _SIGS = {
     "jaxsplat_bin_emit_workspace_size": (SZ, [DP, U32]),
     "jaxsplat_bin_emit_sort": (I32, [DP, U32, P, P, P, P, P, SZ, P]),
     "jaxsplat_bin_rects_sort": (I32, [DP, P, P, P, U32, P, P, P, P, SZ, P]),
+    "jaxsplat_bin_emit_sort_expecting": (I32, [DP, U32, U32, P, P, P, P, P, SZ, P]),
+    "jaxsplat_bin_rects_sort_expecting": (I32, [DP, P, P, P, U32, U32, P, P, P, P, SZ, P]),
     "jaxsplat_rasterize_backward_staged_workspace_size": (SZ, [DP, U32]),
     "jaxsplat_tile_rects_workspace_size": (SZ, [DP]),
     "jaxsplat_tile_rects": (I32, [DP] + [P] * 7 + [P, SZ, P]),
@@ -149,6 +152,8 @@ _SIGS = {
     "jaxsplat_render_begin": (I32, [DP] + [P] * 6 + [U32, I32, P, SZ, ctypes.POINTER(U64), P]),
     "jaxsplat_render_count": (I32, [DP, P, U64, ctypes.POINTER(ctypes.c_int32), P]),
     "jaxsplat_render_finish": (I32, [DP, U32, P, SZ, P, U32, P, SZ, P, SZ, P, P, P, P]),
+    "jaxsplat_render_finish_expecting": (I32, [DP, U32, U32, P, SZ, P, U32, P, SZ, P, SZ, P, P, P,
+                                               P]),
     "jaxsplat_render_finish_backward": (I32, [DP, U32, P, P, P, P, P, SZ, P, SZ, P, U32,
                                                 P, I32] + [P] * 6 + [I32, P, SZ, P]),
     "jaxsplat_project_forward_splats": (I32, [DP] + [P] * 6 + [U32] + [P] * 9 + [P, SZ, P]),

@@ -272,7 +272,10 @@ class IsectCapacity:
     host synchronisation) and raises ``JaxsplatError`` (``ERR_CAPACITY``)
     after an overflow -- whose images and gradients miss the intersections
     beyond the capacity -- having grown ``capacity`` to ``headroom`` times the
-    largest total seen (re-run, and re-capture a graph, after that).
+    largest total seen (re-run, and re-capture a graph, after that).  The total
+    that ``check()`` reads also tells later renders which order of the lists is
+    the faster one (a graph keeps the one that it was captured with); call it
+    once before a loop over dense scenes.
 
     Results equal the default path bit for bit, except that a render with no
     intersections at all keeps final_Ts = 1 internally (the reference writes 0
@@ -289,6 +292,11 @@ class IsectCapacity:
         self._err = torch.zeros(1, dtype=torch.int32, device=self.device)
         self._total = torch.zeros(1, dtype=torch.int64, device=self.device)
         self.last_total = 0
+        # the largest total that the last check() with a render before it read (0:
+        # none yet): with headroom the capacity says little about how many
+        # intersections there are, and how the lists are ordered depends on that
+        # (the results do not)
+        self._expected = 0
 
     def _words(self, dev):
         """The accumulators' addresses, for a binning on dev."""
@@ -309,6 +317,8 @@ class IsectCapacity:
         self._err.zero_()
         self._total.zero_()
         self.last_total = total
+        if total > 0:
+            self._expected = total
         if err & 8:
             old = self.capacity
             self.capacity = min(max(int(total * self.headroom), total + 1),
@@ -321,6 +331,11 @@ class IsectCapacity:
         return total
 
 
+def _expected(isect, capacity):
+    """The number of intersections as far as it is known (0: unknown)."""
+    return isect if capacity is None else capacity._expected
+
+
 def _emit(d, dws, isect, dev, capacity):
     """Emission, tile sort and bin edges over a depth-stage workspace, for
     isect intersections (the exact count, or capacity.capacity).  Returns
@@ -331,8 +346,9 @@ def _emit(d, dws, isect, dev, capacity):
     bins = torch.empty((ntiles, 2), dtype=torch.int32, device=dev)
     ws_bytes = L.jaxsplat_bin_emit_workspace_size(ctypes.byref(d), isect)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
-    _lib.check(L.jaxsplat_bin_emit_sort(ctypes.byref(d), isect, _p(dws), _p(gids), None,
-                                        _p(bins), _p(ws), ws_bytes, _stream(dev)))
+    _lib.check(L.jaxsplat_bin_emit_sort_expecting(
+        ctypes.byref(d), isect, _expected(isect, capacity), _p(dws), _p(gids), None, _p(bins),
+        _p(ws), ws_bytes, _stream(dev)))
     if capacity is not None:
         capacity._record(ws)
     return gids[:isect], bins, isect
@@ -417,9 +433,9 @@ def _bin_rects(d, depths, rects, cum, dev, capacity=None):
         bins = torch.empty((ntiles, 2), dtype=torch.int32, device=dev)
         ws_bytes = L.jaxsplat_bin_emit_workspace_size(ctypes.byref(d), isect)
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
-        _lib.check(L.jaxsplat_bin_rects_sort(ctypes.byref(d), _p(depths), _p(rects), _p(cum),
-                                             isect, _p(gids), None, _p(bins), _p(ws), ws_bytes,
-                                             _stream(dev)))
+        _lib.check(L.jaxsplat_bin_rects_sort_expecting(
+            ctypes.byref(d), _p(depths), _p(rects), _p(cum), isect, _expected(isect, capacity),
+            _p(gids), None, _p(bins), _p(ws), ws_bytes, _stream(dev)))
     if capacity is not None:
         capacity._record(ws)
     return gids[:isect], bins, isect
@@ -612,9 +628,9 @@ class _Render(torch.autograd.Function):
             ws_bytes = L.jaxsplat_bin_emit_workspace_size(db, isect)
             lists = torch.empty(lists_bytes // 4, dtype=torch.int32, device=dev)
             ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
-            _lib.check(L.jaxsplat_render_finish(
-                db, isect, _p(state), state_bytes, _p(background), nch, _p(lists), lists_bytes,
-                _p(ws), ws_bytes, _p(img), *words, s))
+            _lib.check(L.jaxsplat_render_finish_expecting(
+                db, isect, _expected(isect, capacity), _p(state), state_bytes, _p(background), nch,
+                _p(lists), lists_bytes, _p(ws), ws_bytes, _p(img), *words, s))
         ctx.d = d
         ctx.isect = isect
         ctx.adjoint = adjoint

@@ -793,8 +793,8 @@ __global__ __launch_bounds__(THREADS, 6) void tile_depth_sort_loop_kernel(
     }
 }
 
-// The per-tile depth order of every run of bins[0..num_bins), cap entries at
-// most.  ka, va: free buffers of the intersection capacity; kv_tmp: a free one
+// The per-tile depth order of every run of bins[0..num_bins), about `pairs` entries
+// (only a choice depends on that).  ka, va: free buffers of the intersection capacity; kv_tmp: a free one
 // of twice that.  batch: the bins are view << tile_bits | tile, else one view's
 // tiles in the raster kernels' numbering.
 //
@@ -803,33 +803,33 @@ __global__ __launch_bounds__(THREADS, 6) void tile_depth_sort_loop_kernel(
 // goes through global scratch and holds its CU's other waves back.  12 views of
 // 500k Gaussians at 800 x 800 (26M pairs, 85% of them in runs of 1537 to 4467):
 // 422 us in one launch of 256 threads, 64 + 197 in two.  A view takes the second
-// launch where its average run (of the capacity) is long: it costs 7 us where
-// none is (1M Gaussians spread over 1080p, 808 pairs per tile: 46 us alone);
+// launch where its average run (of the expected pairs, or the capacity) is long: it
+// costs 7 us where none is (1M Gaussians spread over 1080p, 808 pairs per tile: 46 us alone);
 // 500k Gaussians in half of an 800 x 800 image, 848 per tile: 53 us in one, 43
 // in two; 1M, 1700: 136 and 92; 1.5M, 2540: 239 and 166.  A batch, many of whose
 // bins are empty, takes it from a sixth of that (535 pairs per bin above; 5 views
 // of 15k at 492 x 383, 37 per bin: 214 us per step in one, 223 in two).
 constexpr int kLongBatchPairs = 256;
-hipError_t tile_depth_order(const int2* bins, int num_bins, int cap, bool batch,
+hipError_t tile_depth_order(const int2* bins, int num_bins, int pairs, bool batch,
                             const uint32_t* dkeys, uint32_t* ids, uint32_t* ka, uint32_t* va,
                             uint2* kv_tmp, hipStream_t s) {
     if (num_bins <= 0) return hipSuccess;
     // two bins per workgroup (A/B at 6 waves per SIMD: multi32 +7%, orbit64 -1%
     // against one; 4 or 8 cost orbit64's long runs more)
-    const int pairs = (num_bins + 1) / 2;
+    const int grid = (num_bins + 1) / 2;
     const int whole = seg_cap(kSegThreads);
     const bool two =
-        cap > whole && cap > (batch ? kLongBatchPairs : whole) * (long long)num_bins;
+        pairs > whole && pairs > (batch ? kLongBatchPairs : whole) * (long long)num_bins;
     const int most = two ? whole : INT32_MAX;
     if (batch)
-        tile_depth_sort_loop_kernel<kSegThreads><<<pairs, kSegThreads, 0, s>>>(
+        tile_depth_sort_loop_kernel<kSegThreads><<<grid, kSegThreads, 0, s>>>(
             bins, num_bins, 0, most, dkeys, ids, ka, va, kv_tmp);
     else
         tile_depth_sort_kernel<<<xcd_grid(num_bins, kXcdChunkView), kSegThreads, 0, s>>>(
             bins, num_bins, most, dkeys, ids, ka, va, kv_tmp);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !two) return e;
-    tile_depth_sort_loop_kernel<kSegThreadsLong><<<pairs, kSegThreadsLong, 0, s>>>(
+    tile_depth_sort_loop_kernel<kSegThreadsLong><<<grid, kSegThreadsLong, 0, s>>>(
         bins, num_bins, whole + 1, INT32_MAX, dkeys, ids, ka, va, kv_tmp);
     return hipGetLastError();
 }
@@ -986,16 +986,16 @@ BinLayout layout(const BinPlan& p) {
         const size_t n4 = align256(4ull * (p.n > 0 ? p.n : 1));
         L.rows = o; o = align256(o + p.rows.scratch_bytes);
         L.runs = o; o += 2 * i4;
+        L.kv = o;
         if (p.by_depth) {
             L.depth_sort = o; o = align256(o + p.depth_sort.scratch_bytes);
             L.keys_out = o; o += n4;
             L.perm = o; o += n4;
             L.dtmp_k = o; o += n4;
             L.dtmp_v = o; o += n4;
-        } else {
-            L.kv = o; o += 2 * i4;
         }
-        L.end = o;
+        // (the depth sort takes far less: more than 16 pairs per Gaussian)
+        L.end = o > L.kv + 2 * i4 ? o : L.kv + 2 * i4;
         return L;
     }
     L.tile_sort = o; o = align256(o + p.tile_sort.scratch_bytes);
@@ -1036,13 +1036,13 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
     stage_mark(kMarkBinned, s);
     if (p.by_depth) return hipSuccess;
     const size_t i4 = align256(4ull * (p.isect_cap > 0 ? p.isect_cap : 1));
-    return tile_depth_order(bins, p.num_tiles, p.isect_cap, false, dkeys, ids, U(L.runs),
+    return tile_depth_order(bins, p.num_tiles, p.order_pairs, false, dkeys, ids, U(L.runs),
                             U(L.runs + i4), reinterpret_cast<uint2*>(b + L.kv), s);
 }
 
 }  // namespace
 
-// Pairs of the capacity per Gaussian and per tile from which the lists are
+// Expected pairs per Gaussian and per tile from which the lists are
 // ordered by one depth sort of the Gaussians and stable placements, instead of
 // tile by tile: the depth sort costs 45 us + 36 us per 1M Gaussians, the order of
 // the tiles 7.6 us per 1M pairs in runs of up to 1536 and two to three times that
@@ -1052,6 +1052,14 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 //                             1M: 18, 2513: 355, 470     25k: 29, 467: 157, 127
 //                             30k: 20, 427: 165, 111     25k: 95, 400: 196, 180
 //                             300k: 10, 1061: 203, 159     2k: 93, 32: 160, 116
+// A capacity is no such number: 2k Gaussians at 500 x 758 (18 pairs per tile) with 38
+// times the room they need took 85 us by depth, 60 tile by tile; 60k at 360 x 640, 8
+// times: 119 and 74; 300k at 719 x 1277, 4 times: 226 and 178; 1M at 1080p, 2.6 times:
+// 342 and 295.  Where the pairs are not known the capacity stands for them from
+// kByDepthUnknown Gaussians: there the depth order costs a fifth at most where the
+// lists are short, and saves most of the time where they are long (3M large ones at
+// 1080p: 785 against 3550).
+constexpr int kByDepthUnknown = 1 << 19;
 constexpr int kByDepthPairs = 16;
 constexpr int kByDepthTilePairs = 640;
 // Grids of up to this many tiles are one radix pass of the emitted pairs,
@@ -1059,16 +1067,19 @@ constexpr int kByDepthTilePairs = 640;
 // (2k Gaussians at 256 x 256: 50 against 61 us of kernels).
 constexpr int kOnePassTiles = 256;
 
-BinPlan bin_plan(const Camera& c, int isect_cap) {
+BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     BinPlan p;
     p.n = c.num_points;
     p.isect_cap = isect_cap;
+    expected = expected < isect_cap ? expected : isect_cap;
+    p.order_pairs = expected > 0 ? expected : isect_cap;
     p.num_tiles = c.tiles_x * c.tiles_y;
     p.tile_bits = bitlen((uint32_t)(p.num_tiles > 1 ? p.num_tiles - 1 : 1));
     p.by_rows = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
                 p.num_tiles > kOnePassTiles;
-    p.by_depth = p.by_rows && (long long)isect_cap > kByDepthPairs * (long long)p.n &&
-                 (long long)isect_cap > kByDepthTilePairs * (long long)p.num_tiles;
+    if (expected <= 0 && p.n >= kByDepthUnknown) expected = isect_cap;
+    p.by_depth = p.by_rows && (long long)expected > kByDepthPairs * (long long)p.n &&
+                 (long long)expected > kByDepthTilePairs * (long long)p.num_tiles;
     p.rows = row_bin_plan(p.n, c.tiles_x, c.tiles_y, isect_cap);
     p.depth_sort = sort_plan(p.n, 0, 32);
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
@@ -1147,7 +1158,7 @@ hipError_t bin_emit(const BinPlan& p, const Camera& c, int num_isect_host,
     stage_mark(kMarkBinned, s);
     // per-tile depth order; the emission's pair buffers and the sort's
     // ping-pong buffers (adjacent) are free again and serve the longer runs
-    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.isect_cap,
+    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.order_pairs,
                             false, dkeys, ids, U(L.tiles), U(L.gids),
                             reinterpret_cast<uint2*>(b + L.ttmp_k), s);
 }
@@ -1207,7 +1218,7 @@ hipError_t bin_rects(const BinPlan& p, const Camera& c, const float* depths,
                                                    reinterpret_cast<int2*>(tile_bins), err);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     stage_mark(kMarkBinned, s);
-    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.isect_cap,
+    return tile_depth_order(reinterpret_cast<const int2*>(tile_bins), p.num_tiles, p.order_pairs,
                             false, reinterpret_cast<const uint32_t*>(depths), ids, U(L.tiles),
                             U(L.gids), reinterpret_cast<uint2*>(b + L.ttmp_k), s);
 }

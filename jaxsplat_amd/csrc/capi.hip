@@ -379,7 +379,7 @@ int jaxsplat_project_backward(const jaxsplat_descriptor* d, const float* means3d
 
 size_t jaxsplat_bin_workspace_size(const jaxsplat_descriptor* d, uint32_t num_intersects) {
     if (!d || validate(d)) return 0;
-    const jsa::BinPlan p = jsa::bin_plan(camera_of(d), (int)num_intersects);
+    const jsa::BinPlan p = jsa::bin_plan(camera_of(d), (int)num_intersects, (int)num_intersects);
     return align256(p.scratch_bytes);
 }
 
@@ -394,7 +394,7 @@ int jaxsplat_bin_and_sort(const jaxsplat_descriptor* d, const float* xys, const 
         return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
     if (!tile_bins) return fail(JAXSPLAT_ERR_INVALID, "bin_and_sort: tile_bins is NULL");
     const jsa::Camera c = camera_of(d);
-    const jsa::BinPlan p = jsa::bin_plan(c, (int)num_intersects);
+    const jsa::BinPlan p = jsa::bin_plan(c, (int)num_intersects, (int)num_intersects);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (num_intersects == 0 || d->num_points == 0) {
         JSA_CHECK_HIP(jsa::fill_zero(tile_bins, 8ull * p.num_tiles, s), "bin_and_sort");
@@ -413,7 +413,7 @@ int jaxsplat_bin_and_sort(const jaxsplat_descriptor* d, const float* xys, const 
 
 size_t jaxsplat_bin_depth_workspace_size(const jaxsplat_descriptor* d) {
     if (!d || validate(d)) return 0;
-    return align256(jsa::bin_plan(camera_of(d), 0).depth_bytes);
+    return align256(jsa::bin_plan(camera_of(d), 0, 0).depth_bytes);
 }
 
 int jaxsplat_bin_depth_sort(const jaxsplat_descriptor* d, const float* xys, const float* depths,
@@ -423,7 +423,7 @@ int jaxsplat_bin_depth_sort(const jaxsplat_descriptor* d, const float* xys, cons
     if (int st = validate(d)) return st;
     if (d->num_points == 0) return JAXSPLAT_OK;
     const jsa::Camera c = camera_of(d);
-    const jsa::BinPlan p = jsa::bin_plan(c, 0);
+    const jsa::BinPlan p = jsa::bin_plan(c, 0, 0);
     if (!xys || !depths || !radii)
         return fail(JAXSPLAT_ERR_INVALID, "bin_depth_sort: NULL required pointer");
     if (!depth_workspace || depth_workspace_bytes < p.depth_bytes)
@@ -443,7 +443,7 @@ int jaxsplat_bin_depth_sort_rects(const jaxsplat_descriptor* d, const float* dep
     if (int st = validate(d)) return st;
     if (d->num_points == 0) return JAXSPLAT_OK;
     const jsa::Camera c = camera_of(d);
-    const jsa::BinPlan p = jsa::bin_plan(c, 0);
+    const jsa::BinPlan p = jsa::bin_plan(c, 0, 0);
     if (!depths || !radii || !tile_rects)
         return fail(JAXSPLAT_ERR_INVALID, "bin_depth_sort_rects: NULL required pointer");
     if (!depth_workspace || depth_workspace_bytes < p.depth_bytes)
@@ -459,20 +459,32 @@ int jaxsplat_bin_depth_sort_rects(const jaxsplat_descriptor* d, const float* dep
 
 size_t jaxsplat_bin_emit_workspace_size(const jaxsplat_descriptor* d, uint32_t num_intersects) {
     if (!d || validate(d)) return 0;
-    return align256(jsa::bin_plan(camera_of(d), (int)num_intersects).emit_bytes);
+    return align256(
+        jsa::bin_plan(camera_of(d), (int)num_intersects, (int)num_intersects).emit_bytes);
 }
 
 int jaxsplat_bin_emit_sort(const jaxsplat_descriptor* d, uint32_t num_intersects,
                            const void* depth_workspace, int32_t* gaussian_ids_sorted,
                            int32_t* tile_ids_sorted, int32_t* tile_bins, void* workspace,
                            size_t workspace_bytes, void* stream) {
+    return jaxsplat_bin_emit_sort_expecting(d, num_intersects, num_intersects, depth_workspace,
+                                            gaussian_ids_sorted, tile_ids_sorted, tile_bins,
+                                            workspace, workspace_bytes, stream);
+}
+
+int jaxsplat_bin_emit_sort_expecting(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                     uint32_t expected, const void* depth_workspace,
+                                     int32_t* gaussian_ids_sorted, int32_t* tile_ids_sorted,
+                                     int32_t* tile_bins, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
     g_err.clear();
     if (int st = validate(d)) return st;
     if (num_intersects >= (1u << 30))
         return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
     if (!tile_bins) return fail(JAXSPLAT_ERR_INVALID, "bin_emit_sort: tile_bins is NULL");
     const jsa::Camera c = camera_of(d);
-    const jsa::BinPlan p = jsa::bin_plan(c, (int)num_intersects);
+    const jsa::BinPlan p =
+        jsa::bin_plan(c, (int)num_intersects, (int)std::min(expected, num_intersects));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (num_intersects == 0 || d->num_points == 0) {
         JSA_CHECK_HIP(jsa::fill_zero(tile_bins, 8ull * p.num_tiles, s), "bin_emit_sort");
@@ -494,13 +506,26 @@ int jaxsplat_bin_rects_sort(const jaxsplat_descriptor* d, const float* depths,
                             uint32_t num_intersects, int32_t* gaussian_ids_sorted,
                             int32_t* tile_ids_sorted, int32_t* tile_bins, void* workspace,
                             size_t workspace_bytes, void* stream) {
+    return jaxsplat_bin_rects_sort_expecting(d, depths, tile_rects, cum_tiles_hit,
+                                             num_intersects, num_intersects,
+                                             gaussian_ids_sorted, tile_ids_sorted, tile_bins,
+                                             workspace, workspace_bytes, stream);
+}
+
+int jaxsplat_bin_rects_sort_expecting(const jaxsplat_descriptor* d, const float* depths,
+                                      const uint32_t* tile_rects, const int32_t* cum_tiles_hit,
+                                      uint32_t num_intersects, uint32_t expected,
+                                      int32_t* gaussian_ids_sorted, int32_t* tile_ids_sorted,
+                                      int32_t* tile_bins, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
     g_err.clear();
     if (int st = validate(d)) return st;
     if (num_intersects >= (1u << 30))
         return fail(JAXSPLAT_ERR_CAPACITY, "num_intersects %u exceeds 2^30", num_intersects);
     if (!tile_bins) return fail(JAXSPLAT_ERR_INVALID, "bin_rects_sort: tile_bins is NULL");
     const jsa::Camera c = camera_of(d);
-    const jsa::BinPlan p = jsa::bin_plan(c, (int)num_intersects);
+    const jsa::BinPlan p =
+        jsa::bin_plan(c, (int)num_intersects, (int)std::min(expected, num_intersects));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (num_intersects == 0 || d->num_points == 0) {
         JSA_CHECK_HIP(jsa::fill_zero(tile_bins, 8ull * p.num_tiles, s), "bin_rects_sort");
@@ -523,7 +548,7 @@ int jaxsplat_bin_check(const jaxsplat_descriptor* d, uint32_t num_intersects,
     g_err.clear();
     if (int st = validate(d)) return st;
     if (num_intersects == 0 || d->num_points == 0 || !workspace) return JAXSPLAT_OK;
-    const jsa::BinPlan p = jsa::bin_plan(camera_of(d), (int)num_intersects);
+    const jsa::BinPlan p = jsa::bin_plan(camera_of(d), (int)num_intersects, (int)num_intersects);
     hipStream_t s = static_cast<hipStream_t>(stream);
     uint32_t err = 0;
     JSA_CHECK_HIP(hipMemcpyAsync(&err, jsa::bin_error_word(p, workspace), 4,
@@ -1158,6 +1183,18 @@ int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects
                            uint32_t channels, void* lists, size_t lists_bytes, void* bin_ws,
                            size_t bin_ws_bytes, float* out_img, int32_t* err, int64_t* total,
                            void* stream) {
+    // (with err, num_intersects is a capacity)
+    return jaxsplat_render_finish_expecting(d, num_intersects, err ? 0u : num_intersects, state,
+                                            state_bytes, background, channels, lists, lists_bytes,
+                                            bin_ws, bin_ws_bytes, out_img, err, total, stream);
+}
+
+int jaxsplat_render_finish_expecting(const jaxsplat_descriptor* d, uint32_t num_intersects,
+                                     uint32_t expected, const void* state, size_t state_bytes,
+                                     const float* background, uint32_t channels, void* lists,
+                                     size_t lists_bytes, void* bin_ws, size_t bin_ws_bytes,
+                                     float* out_img, int32_t* err, int64_t* total,
+                                     void* stream) {
     g_err.clear();
     if (int st = validate(d)) return st;
     if (num_intersects >= (1u << 30))
@@ -1169,10 +1206,10 @@ int jaxsplat_render_finish(const jaxsplat_descriptor* d, uint32_t num_intersects
         return fail(JAXSPLAT_ERR_WORKSPACE, "render_finish: buffer too small or misaligned");
     int32_t* gids = at<int32_t>(lists, l.gids);
     int32_t* bins = at<int32_t>(lists, l.bins);
-    if (int st = jaxsplat_bin_rects_sort(d, at<float>(state, r.depths),
-                                         at<uint32_t>(state, r.rects), at<int32_t>(state, r.cum),
-                                         num_intersects, gids, nullptr, bins, bin_ws,
-                                         bin_ws_bytes, stream))
+    if (int st = jaxsplat_bin_rects_sort_expecting(
+            d, at<float>(state, r.depths), at<uint32_t>(state, r.rects),
+            at<int32_t>(state, r.cum), num_intersects, expected, gids, nullptr, bins, bin_ws,
+            bin_ws_bytes, stream))
         return st;
     if (int st = jaxsplat_rasterize_forward_splats(
             d, gids, bins, num_intersects, at<float>(state, r.splats), background, channels,

@@ -731,6 +731,7 @@ hipError_t batch_row_bin(const BatchRowPlan& p, const ViewRec* views, const uint
 struct BinPlan {
     int n;              // Gaussians
     int isect_cap;      // intersection capacity
+    int order_pairs;    // intersections that the order of the long lists is chosen for
     int num_tiles;
     int tile_bits;
     bool by_rows;           // rowbin.hip (tile grids up to kRowBinAxis per axis)
@@ -742,7 +743,9 @@ struct BinPlan {
     size_t emit_bytes;      // emission stage workspace
     size_t scratch_bytes;   // both, for bin_and_sort: emission region first
 };
-BinPlan bin_plan(const Camera& c, int isect_cap);
+// expected: the number of intersections as far as it is known, at most isect_cap (0:
+// unknown).  The results and the workspace do not depend on it.
+BinPlan bin_plan(const Camera& c, int isect_cap, int expected);
 // Depth stage: per-Gaussian depth keys (depth bits; 0xFFFFFFFF for Gaussians
 // that emit nothing) and packed tile rectangles.  rects (optional, packed as
 // pack_rect) replaces the rectangles computed from xys and radii.
