@@ -261,9 +261,10 @@ __device__ __forceinline__ int place(PlaceShared<V, COLS, CAP, STABLE>& sh, cons
 }
 
 // A partition's intervals in rounds of PER per lane: the stage of a stable
-// placement (whose masks take LDS too) holds half a partition.
+// placement (whose masks take LDS too) holds half a partition.  Returns where the
+// thread's column's values end.
 template <int PER, typename V, int COLS, int CAP, bool STABLE>
-__device__ __forceinline__ void place_all(PlaceShared<V, COLS, CAP, STABLE>& sh,
+__device__ __forceinline__ int place_all(PlaceShared<V, COLS, CAP, STABLE>& sh,
                                           const Interval* iv, const V* val, int ncols,
                                           int column_base, V* out_g, int cap) {
     static_assert(kRbPer % PER == 0, "whole rounds");
@@ -277,6 +278,7 @@ __device__ __forceinline__ void place_all(PlaceShared<V, COLS, CAP, STABLE>& sh,
             column_base,
             (uint32_t)place<PER>(sh, iv + r, val + r, ncols, column_base, out_g, cap), cap);
     }
+    return column_base;
 }
 // Interval k (of kRbPer) of a lane, in rounds of PER: its index within the
 // partition.
@@ -326,16 +328,15 @@ __device__ __forceinline__ Cut emission_cut(const int* __restrict__ cum,
     if (rows == 0) return {id, 0, -1, 0};
     return {id, rows, (int)(rc.x >> 16) + rows - 1, (int)(left - (uint32_t)(rows - 1) * w)};
 }
-// Gaussian id's rectangle up to the cut (its last row whole: run_span).
+// Gaussian id's rectangle up to the cut (its last row whole: cut_run).
 __device__ __forceinline__ uint2 cut_rect(uint2 rc, uint32_t id, const Cut& cut) {
     if (id < (uint32_t)cut.id) return rc;
     const uint32_t rows = id == (uint32_t)cut.id ? (uint32_t)cut.rows : 0u;
     return make_uint2(rc.x, (rc.y & 0xFFFFu) | min(rc.y >> 16, rows) << 16);
 }
-// A run's columns (x0 | w << 16); here: it lies in the cut's last row.
-__device__ __forceinline__ uint32_t run_span(uint2 run, const Cut& cut, bool here) {
-    if (!here || run.x != (uint32_t)cut.id) return run.y;
-    return (run.y & 0xFFFFu) | min(run.y >> 16, (uint32_t)cut.width) << 16;
+// The width of the cut's last row into its run (id, x0 | w << 16).
+__device__ __forceinline__ void cut_run(uint2& run, const Cut& cut) {
+    run.y = (run.y & 0xFFFFu) | min(run.y >> 16, (uint32_t)cut.width) << 16;
 }
 
 // Step 1, counting: partition b holds the Gaussians perm[1024 b ..) (the ids
@@ -353,11 +354,6 @@ __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
     const int tid = threadIdx.x, part = blockIdx.x;
-    const Cut cut = emission_cut(cum, rects, n, cap);
-    if (part == 0 && tid == 0) {
-        *err = 0u;
-        *cut_out = cut;
-    }
     for (int t = part * kRbThreads + tid; t < num_tiles; t += gridDim.x * kRbThreads)
         bins[t] = make_int2(0, 0);
     uint2 rc[kRbPer];
@@ -367,6 +363,11 @@ __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
         const int i = part * kRbPart + k * kRbThreads + tid;
         id[k] = i < n ? (perm ? perm[i] : (uint32_t)i) : 0u;
         rc[k] = i < n ? rects[id[k]] : make_uint2(0u, 0u);
+    }
+    const Cut cut = emission_cut(cum, rects, n, cap);
+    if (part == 0 && tid == 0) {
+        *err = 0u;
+        *cut_out = cut;
     }
     s_d[tid] = 0;
     __syncthreads();
@@ -431,7 +432,18 @@ __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     if (fold && part == 0 && tid < tiles_y) row_len[tid] = own.y;
     const uint64_t at = block_exclusive_scan256((uint64_t)own.y, s_sum) + own.x;
     const int base = (int)min(at, (uint64_t)cap);
-    place_all<PER>(sh, iv, val, tiles_y, base, runs, cap);
+    const int past = place_all<PER>(sh, iv, val, tiles_y, base, runs, cap);
+    if ((unsigned)cut.row < (unsigned)tiles_y) {    // uniform: more pairs than the capacity
+        // the run of the cut's last row, if it is among this partition's, which are
+        // [base, past) of the row's thread
+        if (tid == cut.row) {
+            sh.first[0] = base;
+            sh.first[1] = past;
+        }
+        __syncthreads();
+        for (int i = sh.first[0] + tid; i < sh.first[1]; i += kRbThreads)
+            if (runs[i].x == (uint32_t)cut.id) cut_run(runs[i], cut);
+    }
     if (part != 0) return;
     uint64_t sum = 0;
     for (int i = tid; i < parts; i += kRbThreads) sum += part_tot[i];
@@ -495,16 +507,16 @@ __device__ __forceinline__ void for_partitions(int total, F body) {
 }
 
 // counts[column] = the runs [begin, end) that cover the column, all 256 of them.
-// here: see run_span.  Called by the whole workgroup.
+// Called by the whole workgroup.
 __device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, int begin, int end,
-                                              const Cut& cut, bool here, int* s_d,
-                                              uint32_t* s_tmp, uint32_t* __restrict__ counts) {
+                                              int* s_d, uint32_t* s_tmp,
+                                              uint32_t* __restrict__ counts) {
     const int tid = threadIdx.x;
     uint32_t w[kRbPer];
 #pragma unroll
     for (int k = 0; k < kRbPer; ++k) {
         const int i = k * kRbThreads + tid;
-        w[k] = i < end - begin ? run_span(runs[begin + i], cut, here) : 0u;
+        w[k] = i < end - begin ? runs[begin + i].y : 0u;
     }
     s_d[tid] = 0;
     __syncthreads();
@@ -522,13 +534,12 @@ __device__ __forceinline__ void count_columns(const uint2* __restrict__ runs, in
 // first partition), desc[-1].x the number of partitions.
 __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
     const uint2* __restrict__ runs, const uint32_t* __restrict__ row_len, int tiles_y, int cap,
-    const Cut* __restrict__ cut_in, uint32_t* __restrict__ counts, int4* __restrict__ desc) {
+    uint32_t* __restrict__ counts, int4* __restrict__ desc) {
     __shared__ RowTable rt;
     __shared__ int s_d[kRbThreads];
     __shared__ uint32_t s_tmp[kRbWaves];
     __shared__ uint64_t s_tmp64[kRbWaves];
     const int tid = threadIdx.x;
-    const Cut cut = *cut_in;
     row_table(rt, row_len, tiles_y, cap, s_tmp64);
     if (blockIdx.x == 0 && tid == 0) desc[-1] = make_int4(rt.p0[kRowBinAxis], 0, 0, 0);
     for_partitions(rt.p0[kRowBinAxis], [&](int p) {
@@ -536,8 +547,7 @@ __global__ __launch_bounds__(kRbThreads) void col_count_kernel(
         const int begin = rt.e0[r] + (p - rt.p0[r]) * kRbPart;
         const int end = part_end(begin, rt.e0[r + 1], kRbPart);
         if (tid == 0) desc[p] = make_int4(r, begin, end, p == rt.p0[r] ? 1 : 0);
-        count_columns(runs, begin, end, cut, r == cut.row, s_d, s_tmp,
-                      counts + (size_t)p * kRowBinAxis);
+        count_columns(runs, begin, end, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
     });
 }
 
@@ -649,9 +659,8 @@ __global__ __launch_bounds__(kScanThreads) void col_scan_kernel(
 template <bool STABLE, int COLS>
 __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
     const uint2* __restrict__ runs, const int4* __restrict__ desc, int tiles_x, int tiles_y,
-    int cap, const Cut* __restrict__ cut_in, const uint32_t* __restrict__ counts,
-    const uint32_t* __restrict__ tile_first, uint32_t* __restrict__ ids,
-    int2* __restrict__ bins) {
+    int cap, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ tile_first,
+    uint32_t* __restrict__ ids, int2* __restrict__ bins) {
     constexpr int PER = round_per(STABLE);
     __shared__ PlaceShared<uint32_t, COLS, STABLE ? (COLS == 128 ? 4096 : 3072) : 5120, STABLE> sh;
     __shared__ int s_row0[kRowBinAxis];
@@ -661,19 +670,16 @@ __global__ __launch_bounds__(kRbThreads) void col_place_kernel(
         tid < tiles_y ? tile_first[(size_t)tid * (kRowBinAxis + 1) + kRowBinAxis] : 0u;
     s_row0[tid] = (int)min(block_exclusive_scan256(pairs, s_tmp), (uint64_t)cap);
     const int parts = uniform_i(desc[-1].x);
-    const Cut cut = *cut_in;
     for_partitions(parts, [&](int p) {
         const int4 d = desc[p];
-        const bool here = d.x == cut.row;
         Interval iv[kRbPer];
         uint32_t id[kRbPer];
 #pragma unroll
         for (int k = 0; k < kRbPer; ++k) {
             const int i = interval_index<PER>(k);
             const uint2 run = i < d.z - d.y ? runs[d.y + i] : make_uint2(0u, 0u);
-            const uint32_t span = run_span(run, cut, here);
             id[k] = run.x;
-            iv[k] = {(int)(span & 0xFFFFu), (int)(span >> 16)};
+            iv[k] = {(int)(run.y & 0xFFFFu), (int)(run.y >> 16)};
         }
         clear_place(sh);
         __syncthreads();
@@ -888,8 +894,7 @@ __global__ __launch_bounds__(kRbThreads) void batch_col_count_kernel(
     const int tid = threadIdx.x;
     for_partitions(uniform_i(desc[-1].x), [&](int p) {
         const int4 d = desc[p];
-        count_columns(runs, d.y, d.z, Cut{}, false, s_d, s_tmp,
-                      counts + (size_t)p * kRowBinAxis);
+        count_columns(runs, d.y, d.z, s_d, s_tmp, counts + (size_t)p * kRowBinAxis);
     });
 }
 
@@ -1019,7 +1024,7 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     // persistent: as many workgroups as fit the chip, or one per partition
     const int most = 8 * ((p.max_col_parts + 7) / 8);
     const int grid = most < 2048 ? most : 2048;
-    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_y, p.cap, cut,
+    col_count_kernel<<<grid, kRbThreads, 0, s>>>(runs, U(p.row_len), p.tiles_y, p.cap,
                                                  U(p.col_counts), desc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_LAUNCH(COLS)                                                                      \
@@ -1030,8 +1035,7 @@ hipError_t row_bin(const RowBinPlan& p, const uint32_t* perm, const uint2* rects
     if ((e = hipGetLastError()) != hipSuccess) return e;
 #define JSA_COL(ST, COLS)                                                                     \
     col_place_kernel<ST, COLS><<<grid, kRbThreads, 0, s>>>(                                   \
-        runs, desc, p.tiles_x, p.tiles_y, p.cap, cut, U(p.col_counts), U(p.tile_first), ids,  \
-        bins)
+        runs, desc, p.tiles_x, p.tiles_y, p.cap, U(p.col_counts), U(p.tile_first), ids, bins)
     if (narrow(p.tiles_x)) {
         if (perm) JSA_COL(true, 128); else JSA_COL(false, 128);
     } else {
