@@ -12,7 +12,8 @@
 // Grids of up to 256 tiles per axis are binned by tile rows (rowbin.hip): of a
 // view's Gaussians in depth order where they have many pairs each and the lists
 // are long, else, and in batches, in id order with step 5 below after it.  Views
-// of up to 256 tiles in all (one radix pass) and larger grids:
+// of up to 256 tiles in all (one radix pass) or few pairs (kRowsMany) and larger
+// grids:
 //  1. depth_keys_kernel: per Gaussian its depth bits and packed tile
 //     rectangle;
 //  2. emission in Gaussian id order: a reduce-then-scan of the Gaussians'
@@ -941,7 +942,7 @@ hipError_t emit(int n, const int* n_dev, int tiles_x_plain, const ViewRec* views
     return hipGetLastError();
 }
 
-// Depth stage: per-Gaussian depth keys and rectangles and (by_rows) the inclusive
+// Depth stage: per-Gaussian depth keys and rectangles and (for by_rows) the inclusive
 // counts of the tiles.  It needs no intersection count, so a caller can run it while
 // it reads the count back; its workspace depends on the Gaussian count only.
 struct DepthLayout {
@@ -1042,16 +1043,21 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 
 }  // namespace
 
-// Expected pairs per Gaussian and per tile from which the lists are
+// Expected pairs per Gaussian, per tile and in all from which the lists are
 // ordered by one depth sort of the Gaussians and stable placements, instead of
-// tile by tile: the depth sort costs 45 us + 36 us per 1M Gaussians, the order of
-// the tiles 7.6 us per 1M pairs in runs of up to 1536 and two to three times that
-// beyond.  Many pairs per Gaussian mean large Gaussians, whose overlap makes some
-// runs several times the average.  By depth against tile by tile, forward, us:
+// tile by tile: the depth sort costs 25 to 50 us up to 500k Gaussians (36 us per 1M
+// beyond), the order of the tiles 7.6 us per 1M pairs in runs of up to 1536 and two
+// to three times that beyond.  Many pairs per Gaussian mean large Gaussians, whose
+// overlap makes some runs several times the average.  By depth against tile by tile,
+// forward, us:
 //   per Gaussian, per tile    50k: 95, 804: 219, 263      50k: 29, 939: 167, 176
 //                             1M: 18, 2513: 355, 470     25k: 29, 467: 157, 127
 //                             30k: 20, 427: 165, 111     25k: 95, 400: 196, 180
 //                             300k: 10, 1061: 203, 159     2k: 93, 32: 160, 116
+// Below 1M pairs nothing saves what the sort costs (0.73M: 124, 113; 1.0M of 50k
+// Gaussians in the middle of 400 x 640: 133, 160), and with more than 128 tiles in a
+// row or column, whose stable placements take twice the LDS, below 2.5M (60 x 4000,
+// 0.66M: 145, 101; 1.3M: 130, 100; 1.7M: 191, 153; 3.3M: 150, 160).
 // A capacity is no such number: 2k Gaussians at 500 x 758 (18 pairs per tile) with 38
 // times the room they need took 85 us by depth, 60 tile by tile; 60k at 360 x 640, 8
 // times: 119 and 74; 300k at 719 x 1277, 4 times: 226 and 178; 1M at 1080p, 2.6 times:
@@ -1062,10 +1068,26 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 constexpr int kByDepthUnknown = 1 << 19;
 constexpr int kByDepthPairs = 16;
 constexpr int kByDepthTilePairs = 640;
-// Grids of up to this many tiles are one radix pass of the emitted pairs,
-// whose three launches fewer are worth more than the traffic of few pairs
-// (2k Gaussians at 256 x 256: 50 against 61 us of kernels).
+constexpr int kByDepthLeast = 1000000, kByDepthLeastWide = 2500000;
+// Where the pairs are emitted and sorted instead of binned by tile rows (the
+// capacity stands for their number here in any case: what the pair sort takes grows
+// with it).  Rows cost little per pair, but a wave takes as long as its longest
+// interval and a partition of 1024 has a workgroup, so that few Gaussians leave the
+// chip idle; the pair sort has a launch for each 256 tiles' digit.  Rows against
+// pairs, forward, us:
+//   up to 256 tiles (one radix pass), 256 x 256: 24k Gaussians 57, 49; 200k 169, 164;
+//     1M 424, 423
+//   below 64k Gaussians and 0.4M pairs: 100 at 272 x 272 40, 33; 2k (12 pairs each)
+//     at 1080p 88, 83; 24k, 0.29M 119, 114; but 50k, 0.64M at 600 x 1000 (8-pixel
+//     tiles) 104, 109, and 100k, 0.18M: 83, 84
+//   below 12k Gaussians and 4M pairs: 1k, 2.6M at 1080p 250, 209; 2k, 1.6M at
+//     683 x 1021 147, 129; 8k, 3.5M at 1080p 235, 227; but 4k, 11M: 317, 371
+//   up to 8 tiles high or wide, below 32k Gaussians and 4M pairs: 8k, 3.7M at
+//     60 x 4000 235, 175; 16k, 2.8M 171, 145; but 50k, 3.3M: 150, 164
 constexpr int kOnePassTiles = 256;
+constexpr int kRowsMany = 65536, kRowsFew = 12288, kRowsFewFlat = 32768;    // Gaussians
+constexpr int kRowsPairs = 400000, kRowsPairsFew = 4000000;
+constexpr int kRowsFlat = 8;                            // tiles
 
 BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     BinPlan p;
@@ -1075,11 +1097,17 @@ BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     p.order_pairs = expected > 0 ? expected : isect_cap;
     p.num_tiles = c.tiles_x * c.tiles_y;
     p.tile_bits = bitlen((uint32_t)(p.num_tiles > 1 ? p.num_tiles - 1 : 1));
-    p.by_rows = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
-                p.num_tiles > kOnePassTiles;
+    p.rows_grid = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
+                  p.num_tiles > kOnePassTiles;
+    const bool flat = c.tiles_x <= kRowsFlat || c.tiles_y <= kRowsFlat;
+    const bool few = p.n < (flat ? kRowsFewFlat : kRowsFew);
+    p.by_rows = p.rows_grid &&
+                (p.n >= kRowsMany || isect_cap >= (few ? kRowsPairsFew : kRowsPairs));
     if (expected <= 0 && p.n >= kByDepthUnknown) expected = isect_cap;
+    const bool wide = c.tiles_x > 128 || c.tiles_y > 128;
     p.by_depth = p.by_rows && (long long)expected > kByDepthPairs * (long long)p.n &&
-                 (long long)expected > kByDepthTilePairs * (long long)p.num_tiles;
+                 (long long)expected > kByDepthTilePairs * (long long)p.num_tiles &&
+                 expected > (wide ? kByDepthLeastWide : kByDepthLeast);
     p.rows = row_bin_plan(p.n, c.tiles_x, c.tiles_y, isect_cap);
     p.depth_sort = sort_plan(p.n, 0, 32);
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
@@ -1094,11 +1122,12 @@ const uint32_t* bin_error_word(const BinPlan& p, const void* scratch) {
 }
 
 hipError_t bin_depth(const BinPlan& p, const Camera& c, const float* xys, const float* depths,
-                     const int* radii, const uint2* rects, void* depth_ws, hipStream_t s) {
+                     const int* radii, const uint2* rects, bool counts, void* depth_ws,
+                     hipStream_t s) {
     if (p.n <= 0) return hipSuccess;
     const DepthLayout D = depth_layout(p);
     uint8_t* b = static_cast<uint8_t*>(depth_ws);
-    int* cum = p.by_rows ? reinterpret_cast<int*>(b + D.cum) : nullptr;
+    int* cum = counts ? reinterpret_cast<int*>(b + D.cum) : nullptr;
     uint32_t* part_tot = reinterpret_cast<uint32_t*>(b + D.part_tot);
     depth_keys_kernel<<<(p.n + kCountPart - 1) / kCountPart, kCountPart, 0, s>>>(
         c, depths, radii, reinterpret_cast<const float2*>(xys), rects,
@@ -1230,7 +1259,7 @@ hipError_t bin_and_sort(const BinPlan& p, const Camera& c, const float* xys, con
                         int* gids_sorted, int* tiles_sorted, int* tile_bins, void* scratch,
                         hipStream_t s) {
     uint8_t* depth_ws = static_cast<uint8_t*>(scratch) + p.emit_bytes;
-    hipError_t e = bin_depth(p, c, xys, depths, radii, nullptr, depth_ws, s);
+    hipError_t e = bin_depth(p, c, xys, depths, radii, nullptr, p.by_rows, depth_ws, s);
     if (e != hipSuccess) return e;
     return bin_emit(p, c, num_isect_host, depth_ws, gids_sorted, tiles_sorted,
                     tile_bins, scratch, s);

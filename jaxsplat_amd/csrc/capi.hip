@@ -429,7 +429,7 @@ int jaxsplat_bin_depth_sort(const jaxsplat_descriptor* d, const float* xys, cons
     if (!depth_workspace || depth_workspace_bytes < p.depth_bytes)
         return fail(JAXSPLAT_ERR_WORKSPACE, "bin_depth_sort: workspace too small (%zu < %zu)",
                     depth_workspace_bytes, p.depth_bytes);
-    JSA_CHECK_HIP(jsa::bin_depth(p, c, xys, depths, radii, nullptr, depth_workspace,
+    JSA_CHECK_HIP(jsa::bin_depth(p, c, xys, depths, radii, nullptr, p.rows_grid, depth_workspace,
                                  static_cast<hipStream_t>(stream)),
                   "bin_depth_sort");
     return JAXSPLAT_OK;
@@ -451,7 +451,8 @@ int jaxsplat_bin_depth_sort_rects(const jaxsplat_descriptor* d, const float* dep
                     "bin_depth_sort_rects: workspace too small (%zu < %zu)",
                     depth_workspace_bytes, p.depth_bytes);
     JSA_CHECK_HIP(jsa::bin_depth(p, c, nullptr, depths, radii,
-                                 reinterpret_cast<const uint2*>(tile_rects), depth_workspace,
+                                 reinterpret_cast<const uint2*>(tile_rects), p.rows_grid,
+                                 depth_workspace,
                                  static_cast<hipStream_t>(stream)),
                   "bin_depth_sort_rects");
     return JAXSPLAT_OK;

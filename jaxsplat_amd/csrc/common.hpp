@@ -734,7 +734,8 @@ struct BinPlan {
     int order_pairs;    // intersections that the order of the long lists is chosen for
     int num_tiles;
     int tile_bits;
-    bool by_rows;           // rowbin.hip (tile grids up to kRowBinAxis per axis)
+    bool rows_grid;         // the grid can be binned by rows (up to kRowBinAxis per axis)
+    bool by_rows;           // and is: rowbin.hip
     bool by_depth;          // by_rows, from the Gaussians in depth order
     RowBinPlan rows;
     SortPlan depth_sort;    // by_depth
@@ -748,9 +749,11 @@ struct BinPlan {
 BinPlan bin_plan(const Camera& c, int isect_cap, int expected);
 // Depth stage: per-Gaussian depth keys (depth bits; 0xFFFFFFFF for Gaussians
 // that emit nothing) and packed tile rectangles.  rects (optional, packed as
-// pack_rect) replaces the rectangles computed from xys and radii.
+// pack_rect) replaces the rectangles computed from xys and radii.  counts: also
+// their inclusive tile counts, which bin_emit by rows needs.
 hipError_t bin_depth(const BinPlan& p, const Camera& c, const float* xys, const float* depths,
-                     const int* radii, const uint2* rects, void* depth_ws, hipStream_t s);
+                     const int* radii, const uint2* rects, bool counts, void* depth_ws,
+                     hipStream_t s);
 // Emission stage over the depth stage's workspace: emission in id order, the
 // stable tile sort, edges, and the per-tile depth order.
 // p.isect_cap bounds the slots written; the sort and the edges cover the slots

@@ -59,15 +59,15 @@ PATHS = {"fused": (3, True), "reference tiles": (3, False), "wide": (5, True)}
 def test_headroom_adds_no_depth_sort(path, monkeypatch):
     channels, tight = PATHS[path]
     monkeypatch.setattr(_ops, "TIGHT_TILES", tight)
-    run = _scene(1500, np.log(0.05), (330, 400), channels)     # 525 tiles, short lists
+    run = _scene(70000, np.log(0.01), (330, 400), channels)    # 525 tiles, short lists
     probe = IsectCapacity(1 << 22)
     want = H.host(run(probe))
     total = probe.check()
-    assert total < 100 * 525
+    assert total < 640 * 525
     tight_cap = IsectCapacity(total)
     base, img = _kernels(lambda: run(tight_cap))
     assert np.array_equal(img, want)
-    for cap in (1 << 20, 1 << 24):
+    for cap in (1 << 21, 1 << 24):
         known = IsectCapacity(cap)
         nodes, img = _kernels(lambda: run(known))
         assert np.array_equal(img, want)
@@ -82,16 +82,36 @@ def test_headroom_adds_no_depth_sort(path, monkeypatch):
 def test_checked_total_chooses_the_depth_order(path, monkeypatch):
     channels, tight = PATHS[path]
     monkeypatch.setattr(_ops, "TIGHT_TILES", tight)
-    run = _scene(4000, np.log(0.6), (330, 400), channels)      # large ones: long lists
+    run = _scene(6000, np.log(0.6), (330, 400), channels)      # large ones: long lists
     want = H.host(run())
     cap = IsectCapacity(1 << 23)
     unknown, img = _kernels(lambda: run(cap))
     assert np.array_equal(img, want)
     total = cap.check()
-    assert total > 16 * 4000 and total > 640 * 525
+    assert total > 1_000_000
     nodes, img = _kernels(lambda: run(cap))
     assert np.array_equal(img, want)
     assert nodes > unknown + 3
     cap.check()
     cap.check()                                 # nothing rendered: still known
     assert _kernels(lambda: run(cap))[0] == nodes
+
+
+def test_few_pairs_are_not_sorted_by_depth():
+    """Long lists of few pairs (fewer than 1M): hardly more kernels than short lists of
+    as many Gaussians (a depth sort of them is eight)."""
+    nodes = []
+    for log_scale in (np.log(0.01), np.log(0.6)):
+        run = _scene(3000, log_scale, (272, 272), 3)           # 289 tiles
+        want = H.host(run())
+        cap = IsectCapacity(1 << 22)
+        run(cap)
+        total = cap.check()
+        tight = IsectCapacity(total)
+        run(tight)
+        assert tight.check() == total
+        n, img = _kernels(lambda: run(tight))
+        assert np.array_equal(img, want)
+        nodes.append(n)
+    assert 16 * 3000 < total < 1_000_000 and total > 640 * 289
+    assert nodes[1] <= nodes[0] + 5
