@@ -1467,6 +1467,7 @@ struct jaxsplat_batch {
     int num_scenes = 0, num_views = 0;
     int n_items = 0, n_gauss = 0, max_view_n = 0, max_scene_n = 0;
     int total_tiles = 0, max_view_tiles = 0;
+    int chunk = 1;                        // RasterGrid::chunk
     long long num_pixels = 0;
     float glob_scale = 1.f, clip_thresh = 0.f;
     int block_width = 16;
@@ -1499,6 +1500,7 @@ jsa::RasterGrid batch_grid(const jaxsplat_batch* b, uint8_t* w) {
     g.n_items = b->n_items;
     g.fwd_depth = b->fwd_depth;
     g.bwd_depth = b->bwd_depth;
+    g.chunk = b->chunk;
     g.ch_stride = 3;
     g.ch_off = 0;
     g.ch_n = 3;
@@ -1614,6 +1616,7 @@ int jaxsplat_batch_create(jaxsplat_batch** out, const jaxsplat_scene* scenes, in
     }
     b->n_items = (int)items;
     b->total_tiles = (int)tiles;
+    b->chunk = jsa::batch_chunk(b->views.data(), num_views, b->total_tiles);
     b->num_pixels = pix;
     b->bin = jsa::batch_bin_plan(b->n_items, num_views, b->max_view_tiles, (int)parts,
                                  (int)rows, max_x, max_y, (int)isect_capacity);

@@ -8,6 +8,8 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include "positions.hpp"
+
 namespace jsa {
 
 constexpr int kWave = 64;
@@ -141,24 +143,22 @@ __device__ __forceinline__ T wave_inclusive_sum(T v) {
         return v;
     }
 }
-// Tile of workgroup b in a grid of xcd_grid(num_tiles, log2_chunk) workgroups:
-// workgroups are dealt to the 8 XCDs round robin, so XCD b & 7 gets chunks of
-// 2^log2_chunk consecutive tiles, which share Gaussians in its L2, and the chunks
-// are dealt to the XCDs in turn (indexes past num_tiles are the caller's to
-// skip).  One contiguous band per XCD left the XCDs of a picture's empty borders
-// idle.  One view, chunks of 16: backward records of 50k Gaussians in the middle
-// of 683 x 1021 185 -> 149 us, forward of 50k at 900 x 1600 89 -> 77; evenly
-// filled pictures (1M Gaussians at 1080p) the same within 1%, as with chunks of 8
-// or 32 and blocks of 4 x 4.  A batch, chunks of 64: 12 views of 800 x 800 with
-// 500k Gaussians, records 1040 -> 1024 us (16: 1058).
-constexpr int kXcdChunkView = 4, kXcdChunkBatch = 6;
-inline int xcd_grid(int num_tiles, int log2_chunk) {
-    return ((num_tiles + (8 << log2_chunk) - 1) >> (3 + log2_chunk)) << (3 + log2_chunk);
-}
-__device__ __forceinline__ int xcd_tile(int b, int log2_chunk) {
-    const int j = b >> 3;
-    return ((((j >> log2_chunk) << 3) + (b & 7)) << log2_chunk) + (j & ((1 << log2_chunk) - 1));
-}
+// Chunks in which the raster kernels' tiles are dealt to the XCDs (xcd_tile).
+//
+// One view, chunks of 16: one contiguous band per XCD left the XCDs of a picture's
+// empty borders idle (backward records of 50k Gaussians in the middle of 683 x 1021
+// 185 -> 149 us, forward of 50k at 900 x 1600 89 -> 77); evenly filled pictures (1M
+// Gaussians at 1080p) the same within 1%, as with chunks of 8 or 32 and blocks of
+// 4 x 4.
+constexpr int kXcdChunkView = 16;
+// A batch: a band per XCD, in which a view's Gaussians stay in one L2 and whose ends
+// lie in different views (steps, band against chunks of 64: 64 views of 200 x 200
+// with 100k Gaussians 3188, 3449 us; 8 views of 365 x 529 with 110k 787, 922; 12 of
+// 800 x 800 with 500k 2252, 2274).  Fewer than four views are cut as one is (2 views
+// of 600 x 800 with 50k: 402, 366; 3 of 500 x 700 with 60k: 476, 401), and so are
+// views so uneven that a band has more than twice its share of the Gaussians (64 of
+// 100 x 100 with 200 and 2 of 500 x 500 with 100k: 672, 603).
+constexpr int kXcdChunkFew = 64, kXcdBandViews = 4;
 
 // Mask of the lanes of this wave whose `bits`-bit digit equals this lane's
 // (restricted to lanes in `valid`): one ballot per digit bit.
@@ -534,6 +534,7 @@ struct RasterGrid {
     int n_items;          // sorted entries name items in [0, n_items)
     int fwd_depth;        // Gaussians staged per batch: 64, 128 or 256 (0: workgroup size)
     int bwd_depth;        // likewise for the backward (0: 64)
+    int chunk;            // tiles per chunk dealt to an XCD (xcd_tile)
     // channel pass: channels [ch_off, ch_off + ch_n) (ch_n <= pass_channels) of
     // colors, backgrounds, images and v_colors stored with ch_stride channels per
     // row
@@ -556,6 +557,9 @@ struct RasterGrid {
 // the records stay within the 16 lanes of a row sum, 116 VGPRs (four waves per
 // SIMD, three channels: 80 and six).
 inline int pass_channels(int left) { return left < 8 ? left : 8; }
+
+// RasterGrid::chunk of a batch of these views.
+int batch_chunk(const ViewRec* views, int num_views, int num_tiles);
 
 ViewRec single_view(const Camera& c);
 RasterGrid single_grid(const Camera& c);

@@ -31,6 +31,8 @@
 //  * the tile index is remapped so that each of the 8 XCDs (blocks are issued
 //    round-robin over XCDs) renders chunks of consecutive tiles (xcd_tile),
 //    keeping neighbouring tiles' Gaussians in the same L2.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace jsa {
@@ -50,10 +52,6 @@ inline int bwd_threads(int block_width, int slots) {
 }
 static_assert((kMaxTileThreads + 3) / 4 <= 64 && 128 / 2 <= 64,
               "one wave covers a tile at 4 (more than 128 pixels) or 2 pixels per lane");
-
-__host__ __device__ __forceinline__ int xcd_chunk(const RasterGrid& g) {
-    return g.views ? kXcdChunkBatch : kXcdChunkView;
-}
 
 constexpr float kTEps = 1e-4f;
 // The batches hold the conic scaled to base 2: (a, b, c) * (log2(e)/2,
@@ -512,7 +510,7 @@ __global__ __launch_bounds__(256) void raster_fwd_kernel(
     const float* __restrict__ colors, const float* __restrict__ opac,
     const float* __restrict__ bgs, float* __restrict__ final_Ts, int* __restrict__ final_idx,
     float* __restrict__ out_img) {
-    const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
+    const int gt = xcd_tile(blockIdx.x, rg.chunk);
     if (gt >= rg.total_tiles) return;
     raster_fwd_tile<DEPTH, CH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
                                final_idx, out_img);
@@ -1039,7 +1037,7 @@ __global__ __launch_bounds__(64) void raster_bwd_kernel(
     const float* __restrict__ v_out_alpha, float* __restrict__ v_rgb,
     float* __restrict__ v_opacity, float* __restrict__ v_xy, float* __restrict__ v_xy_abs,
     float* __restrict__ v_conic, StagedOut st) {
-    const int gt = xcd_tile(blockIdx.x, xcd_chunk(rg));
+    const int gt = xcd_tile(blockIdx.x, rg.chunk);
     if (gt >= rg.total_tiles) return;
     raster_bwd_tile<CONSISTENT, ABS, DEPTH, STAGED, NSLOT, CH>(
         rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts, final_idx, v_out_img,
@@ -1251,6 +1249,24 @@ ViewRec single_view(const Camera& c) {
     return v;
 }
 
+int batch_chunk(const ViewRec* views, int num_views, int num_tiles) {
+    if (num_views < kXcdBandViews) return kXcdChunkFew;
+    const int band = num_tiles > 8 ? (num_tiles + 7) / 8 : 1;
+    double share[8] = {}, all = 0;      // Gaussians of the bands' tiles
+    for (int v = 0; v < num_views; ++v) {
+        const int tiles = views[v].tiles_x * views[v].tiles_y;
+        const double per = (double)views[v].n / tiles;
+        for (int t = views[v].tile_off, left = tiles; left > 0;) {
+            const int b = t / band, here = std::min(left, (b + 1) * band - t);
+            share[b < 8 ? b : 7] += per * here;
+            t += here;
+            left -= here;
+        }
+        all += views[v].n;
+    }
+    return *std::max_element(share, share + 8) * 8 > 2 * all ? kXcdChunkFew : band;
+}
+
 RasterGrid single_grid(const Camera& c) {
     RasterGrid g{};
     g.v0 = single_view(c);
@@ -1261,6 +1277,7 @@ RasterGrid single_grid(const Camera& c) {
     g.n_items = c.num_points;
     g.fwd_depth = 0;
     g.bwd_depth = 0;
+    g.chunk = kXcdChunkView;
     g.ch_stride = 3;
     g.ch_off = 0;
     g.ch_n = 3;
@@ -1299,7 +1316,7 @@ hipError_t raster_fwd_grid(const RasterGrid& g, const int* items_sorted, const i
     // default: the smallest batch depth that holds one entry per thread (a
     // 12- or 13-pixel tile has 192 threads: 256, two staging rounds)
     const int depth = g.fwd_depth > 0 ? g.fwd_depth : (nthr <= 64 ? 64 : nthr <= 128 ? 128 : 256);
-    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
+    const int grid = xcd_grid(g.total_tiles, g.chunk);
     const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
     const float2* x2 = reinterpret_cast<const float2*>(xys);
     if (g.order) {
@@ -1383,7 +1400,7 @@ hipError_t raster_bwd_grid(const RasterGrid& g, const int* items_sorted, const i
     if (g.total_tiles <= 0) return hipSuccess;
     const int slots = bwd_slots(g.block_width);
     const int nthr = bwd_threads(g.block_width, slots);
-    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
+    const int grid = xcd_grid(g.total_tiles, g.chunk);
     // 64 Gaussians per batch by default: the LDS partial sums (depth x 9..11 x 4
     // floats) otherwise limit the workgroups per CU (measured fastest on the
     // 1080p, 800x800 and mixed-size workloads)
@@ -1457,7 +1474,7 @@ hipError_t raster_bwd_staged(const Camera& c, int nch, const int* gids_sorted,
     g.splats = splats;
     const int slots = bwd_slots(g.block_width);
     const int nthr = bwd_threads(g.block_width, slots);
-    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
+    const int grid = xcd_grid(g.total_tiles, g.chunk);
     const int blocks = (c.num_points + 255) / 256;
     const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
     const float2* x2 = reinterpret_cast<const float2*>(xys);
@@ -1536,7 +1553,7 @@ hipError_t raster_bwd_batch_staged(const RasterGrid& g, int max_view_n, const in
     if (e != hipSuccess) return e;
     const int slots = bwd_slots(g.block_width);
     const int nthr = bwd_threads(g.block_width, slots);
-    const int grid = xcd_grid(g.total_tiles, xcd_chunk(g));
+    const int grid = xcd_grid(g.total_tiles, g.chunk);
     const int2* b2 = reinterpret_cast<const int2*>(tile_bins);
     const float2* x2 = reinterpret_cast<const float2*>(xys);
     // work queue (g.order): a persistent grid takes the tiles in that order

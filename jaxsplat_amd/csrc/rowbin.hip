@@ -36,7 +36,6 @@
 // stored contiguously; with more values than the stage holds (long intervals,
 // whose columns then hold many values anyway) they are stored directly.
 #include "common.hpp"
-#include "positions.hpp"
 
 namespace jsa {
 namespace {
