@@ -1270,7 +1270,7 @@ hipError_t bin_and_sort(const BinPlan& p, const Camera& c, const float* xys, con
 // ---------------------------------------------------------------------------
 // Items are numbered view by view (ViewRec::item_off), so the item order is
 // the (view, item) order.  Up to 256 tiles per axis: by tile rows (batch_row_bin),
-// then step 5 below.  Larger grids:
+// then step 5 below.  Larger grids and few pairs (see kOnePassSmall):
 //  1. view_keys: every item's view;
 //  2. emission (BATCH) in item order: keys view << tile_bits | tile, values =
 //     item ids, with the total and the clamped count published on the device;
@@ -1319,6 +1319,19 @@ BatchLayout batch_layout(const BatchBinPlan& p) {
 
 }  // namespace
 
+// Where batches take the pair sort for the reasons that views do (kOnePassTiles).
+// Rows against pairs, forward, us:
+//   views of up to 64 tiles: 16 of 64 x 64, 2k items each 137, 124 (0.16M pairs); 64,
+//     40k 1023, 1012 (3.5M)
+//   up to 256 tiles and 1M pairs: 5 of 200 x 200, 2k 109, 100 (0.24M); 16, 2k 151, 147
+//     (0.8M); but 5, 10k, 1.2M 160, 166
+//   fewer than 12k items and 2.5M pairs, more than 64 each in views up to 8 tiles high
+//     or wide: 2 of 60 x 2000, 2k 119, 100; 5, 200 98, 85; or 512 elsewhere: 1 of
+//     1080p, 200 154, 133; but 2 of 1080p, 2k, 5.2M 303, 338
+constexpr int kOnePassSmall = 64;                       // tiles
+constexpr int kBatchRowsOnePass = 1000000, kBatchRowsFew = 2500000;     // pairs
+constexpr int kBatchWideFlat = 64, kBatchWide = 512;    // and per item
+
 BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int parts, int rows,
                             int max_x, int max_y, int isect_cap) {
     BatchBinPlan p{};
@@ -1329,7 +1342,15 @@ BatchBinPlan batch_bin_plan(int n_items, int num_views, int max_view_tiles, int 
     p.view_bits = bitlen((uint32_t)(num_views > 1 ? num_views - 1 : 0));
     p.num_bins = num_views << p.tile_bits;
     p.tile_sort = sort_plan(isect_cap, 0, p.tile_bits);
-    p.by_rows = max_x <= kRowBinAxis && max_y <= kRowBinAxis && num_views <= kMaxBatchViews;
+    // (largest views of) one radix pass: the pair sort up to 64 tiles or 1M pairs
+    const bool pass = max_view_tiles <= kOnePassSmall ||
+                      (max_view_tiles <= kOnePassTiles && isect_cap < kBatchRowsOnePass);
+    // few items that cover many tiles each
+    const bool flat = max_x <= kRowsFlat || max_y <= kRowsFlat;
+    const bool few = n_items < kRowsFew && isect_cap < kBatchRowsFew &&
+                     isect_cap > (flat ? kBatchWideFlat : kBatchWide) * (long long)n_items;
+    p.by_rows = max_x <= kRowBinAxis && max_y <= kRowBinAxis && num_views <= kMaxBatchViews &&
+                !pass && !few;
     if (p.by_rows) p.rows = batch_row_plan(num_views, parts, rows, max_x, max_y, isect_cap);
     p.scratch_bytes = batch_layout(p).end;
     return p;
