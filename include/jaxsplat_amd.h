@@ -223,8 +223,11 @@ int jaxsplat_bin_emit_sort(const jaxsplat_descriptor* d, uint32_t num_intersects
  * jaxsplat_bin_rects_sort expect num_intersects.  The _expecting forms take the
  * number separately, for a num_intersects that is a capacity with headroom: the
  * count of an earlier, similar binning, or 0 where none is known (from 2^19
- * Gaussians the capacity then stands for it).  Same workspace.
+ * Gaussians the capacity then stands for it).  Same workspace
+ * (jaxsplat_bin_emit_workspace_size), or the smaller one for that number.
  */
+size_t jaxsplat_bin_emit_workspace_size_expecting(const jaxsplat_descriptor* d,
+                                                  uint32_t num_intersects, uint32_t expected);
 int jaxsplat_bin_emit_sort_expecting(const jaxsplat_descriptor* d, uint32_t num_intersects,
                                      uint32_t expected, const void* depth_workspace,
                                      int32_t* gaussian_ids_sorted, int32_t* tile_ids_sorted,

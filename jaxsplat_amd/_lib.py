@@ -45,6 +45,7 @@ EXPORTS = (
     "jaxsplat_render_begin", "jaxsplat_render_count", "jaxsplat_render_finish",
     "jaxsplat_render_finish_backward", "jaxsplat_render_finish_expecting",
     "jaxsplat_bin_emit_sort_expecting", "jaxsplat_bin_rects_sort_expecting",
+    "jaxsplat_bin_emit_workspace_size_expecting",
     "jaxsplat_project_forward_splats", "jaxsplat_rasterize_forward_splats",
     "jaxsplat_rasterize_forward_binned", "jaxsplat_rasterize_backward_binned",
     "jaxsplat_rasterize_forward_nd", "jaxsplat_rasterize_backward_nd",
@@ -131,6 +132,7 @@ _SIGS = {
     "jaxsplat_bin_emit_workspace_size": (SZ, [DP, U32]),
     "jaxsplat_bin_emit_sort": (I32, [DP, U32, P, P, P, P, P, SZ, P]),
     "jaxsplat_bin_rects_sort": (I32, [DP, P, P, P, U32, P, P, P, P, SZ, P]),
+    "jaxsplat_bin_emit_workspace_size_expecting": (SZ, [DP, U32, U32]),
     "jaxsplat_bin_emit_sort_expecting": (I32, [DP, U32, U32, P, P, P, P, P, SZ, P]),
     "jaxsplat_bin_rects_sort_expecting": (I32, [DP, P, P, P, U32, U32, P, P, P, P, SZ, P]),
     "jaxsplat_rasterize_backward_staged_workspace_size": (SZ, [DP, U32]),

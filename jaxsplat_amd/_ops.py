@@ -344,10 +344,11 @@ def _emit(d, dws, isect, dev, capacity):
     ntiles = d.grid_dim_2d.x * d.grid_dim_2d.y
     gids = torch.empty(max(isect, 1), dtype=torch.int32, device=dev)
     bins = torch.empty((ntiles, 2), dtype=torch.int32, device=dev)
-    ws_bytes = L.jaxsplat_bin_emit_workspace_size(ctypes.byref(d), isect)
+    expected = _expected(isect, capacity)
+    ws_bytes = L.jaxsplat_bin_emit_workspace_size_expecting(ctypes.byref(d), isect, expected)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     _lib.check(L.jaxsplat_bin_emit_sort_expecting(
-        ctypes.byref(d), isect, _expected(isect, capacity), _p(dws), _p(gids), None, _p(bins),
+        ctypes.byref(d), isect, expected, _p(dws), _p(gids), None, _p(bins),
         _p(ws), ws_bytes, _stream(dev)))
     if capacity is not None:
         capacity._record(ws)
@@ -431,11 +432,12 @@ def _bin_rects(d, depths, rects, cum, dev, capacity=None):
             isect = capacity.capacity
         gids = torch.empty(max(isect, 1), dtype=torch.int32, device=dev)
         bins = torch.empty((ntiles, 2), dtype=torch.int32, device=dev)
-        ws_bytes = L.jaxsplat_bin_emit_workspace_size(ctypes.byref(d), isect)
+        expected = _expected(isect, capacity)
+        ws_bytes = L.jaxsplat_bin_emit_workspace_size_expecting(ctypes.byref(d), isect, expected)
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
         _lib.check(L.jaxsplat_bin_rects_sort_expecting(
-            ctypes.byref(d), _p(depths), _p(rects), _p(cum), isect, _expected(isect, capacity),
-            _p(gids), None, _p(bins), _p(ws), ws_bytes, _stream(dev)))
+            ctypes.byref(d), _p(depths), _p(rects), _p(cum), isect, expected, _p(gids), None,
+            _p(bins), _p(ws), ws_bytes, _stream(dev)))
     if capacity is not None:
         capacity._record(ws)
     return gids[:isect], bins, isect
@@ -625,11 +627,12 @@ class _Render(torch.autograd.Function):
             else:
                 isect = capacity.capacity if N else 0
             lists_bytes = L.jaxsplat_render_lists_size(db, isect)
-            ws_bytes = L.jaxsplat_bin_emit_workspace_size(db, isect)
+            expected = _expected(isect, capacity)
+            ws_bytes = L.jaxsplat_bin_emit_workspace_size_expecting(db, isect, expected)
             lists = torch.empty(lists_bytes // 4, dtype=torch.int32, device=dev)
             ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
             _lib.check(L.jaxsplat_render_finish_expecting(
-                db, isect, _expected(isect, capacity), _p(state), state_bytes, _p(background), nch,
+                db, isect, expected, _p(state), state_bytes, _p(background), nch,
                 _p(lists), lists_bytes, _p(ws), ws_bytes, _p(img), *words, s))
         ctx.d = d
         ctx.isect = isect

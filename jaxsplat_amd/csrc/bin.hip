@@ -987,16 +987,16 @@ BinLayout layout(const BinPlan& p) {
         const size_t n4 = align256(4ull * (p.n > 0 ? p.n : 1));
         L.rows = o; o = align256(o + p.rows.scratch_bytes);
         L.runs = o; o += 2 * i4;
-        L.kv = o;
         if (p.by_depth) {
             L.depth_sort = o; o = align256(o + p.depth_sort.scratch_bytes);
             L.keys_out = o; o += n4;
             L.perm = o; o += n4;
             L.dtmp_k = o; o += n4;
             L.dtmp_v = o; o += n4;
+        } else {
+            L.kv = o; o += 2 * i4;
         }
-        // (the depth sort takes far less: more than 16 pairs per Gaussian)
-        L.end = o > L.kv + 2 * i4 ? o : L.kv + 2 * i4;
+        L.end = o;
         return L;
     }
     L.tile_sort = o; o = align256(o + p.tile_sort.scratch_bytes);

@@ -460,8 +460,17 @@ int jaxsplat_bin_depth_sort_rects(const jaxsplat_descriptor* d, const float* dep
 
 size_t jaxsplat_bin_emit_workspace_size(const jaxsplat_descriptor* d, uint32_t num_intersects) {
     if (!d || validate(d)) return 0;
-    return align256(
-        jsa::bin_plan(camera_of(d), (int)num_intersects, (int)num_intersects).emit_bytes);
+    // (1: the order tile by tile)
+    return std::max(jaxsplat_bin_emit_workspace_size_expecting(d, num_intersects, num_intersects),
+                    jaxsplat_bin_emit_workspace_size_expecting(d, num_intersects, 1));
+}
+
+size_t jaxsplat_bin_emit_workspace_size_expecting(const jaxsplat_descriptor* d,
+                                                  uint32_t num_intersects, uint32_t expected) {
+    if (!d || validate(d)) return 0;
+    return align256(jsa::bin_plan(camera_of(d), (int)num_intersects,
+                                  (int)std::min(expected, num_intersects))
+                        .emit_bytes);
 }
 
 int jaxsplat_bin_emit_sort(const jaxsplat_descriptor* d, uint32_t num_intersects,

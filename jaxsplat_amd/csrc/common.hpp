@@ -750,7 +750,8 @@ struct BinPlan {
     size_t scratch_bytes;   // both, for bin_and_sort: emission region first
 };
 // expected: the number of intersections as far as it is known, at most isect_cap (0:
-// unknown).  The results and the workspace do not depend on it.
+// unknown).  The results do not depend on it; the depth order's workspace is the
+// smaller one.
 BinPlan bin_plan(const Camera& c, int isect_cap, int expected);
 // Depth stage: per-Gaussian depth keys (depth bits; 0xFFFFFFFF for Gaussians
 // that emit nothing) and packed tile rectangles.  rects (optional, packed as
