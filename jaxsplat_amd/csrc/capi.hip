@@ -1031,7 +1031,8 @@ int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, v
     // giving up the processor in between, and after 20 ms asleep for the most part.
     // The stream itself is asked at 2, 4, 8, ... ms: one that failed ends the wait, and
     // where it has ended without the count (another read's late store took the
-    // word) the count is copied.
+    // word) the count is copied.  After a second what is queued by then is waited for,
+    // so that a stream that never ends cannot hold a count that was taken.
     using namespace std::chrono;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const auto begin = steady_clock::now();
@@ -1044,7 +1045,7 @@ int jaxsplat_count_wait(const int32_t* count, uint64_t ticket, int32_t* value, v
         if (waited < milliseconds(2)) continue;
         if (waited >= ask) {
             ask *= 2;
-            const hipError_t q = hipStreamQuery(s);
+            const hipError_t q = waited < seconds(1) ? hipStreamQuery(s) : hipStreamSynchronize(s);
             if (q == hipSuccess) break;
             if (q != hipErrorNotReady) JSA_CHECK_HIP(q, "count_wait");
             (void)hipGetLastError();            // not ready is no error
