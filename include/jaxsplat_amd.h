@@ -345,8 +345,9 @@ int jaxsplat_rasterize_backward_binned(
  * calls.  The blend and its adjoint are those of the 3-channel entry points
  * for every channel, accumulated in fp32 (the reference's dead N-channel code
  * accumulates in fp16 and its backward skips the last contributor); C = 3
- * gives exactly the 3-channel results.  Channels run in passes of up to
- * three.  v_xy_abs must be NULL for C > 3 (it does not add over passes).
+ * gives exactly the 3-channel results.  Channels run in passes, of up to eight
+ * forward and three backward (jaxsplat_rasterize_backward_staged_nd: eight).
+ * v_xy_abs must be NULL for C > 3 (it does not add over passes).
  */
 int jaxsplat_rasterize_forward_nd(const jaxsplat_descriptor* d,
                                   const int32_t* gaussian_ids_sorted, const int32_t* tile_bins,
@@ -466,8 +467,9 @@ int jaxsplat_render_backward(
 /*
  * Host reads of a count (an inclusive count's last entry) without a copy or an
  * event: jaxsplat_count_begin queues a kernel that writes *count with a ticket to
- * a pinned word of the calling thread, and jaxsplat_count_wait (same thread)
- * returns it as soon as it has arrived, whatever else the stream still holds.  A
+ * a pinned word of the calling thread, and jaxsplat_count_wait (same thread, its
+ * last ticket) returns it as soon as it has arrived, whatever else the stream still
+ * holds (a wait of more than a second ends with what the stream holds by then).  A
  * capturing stream is refused.
  */
 int jaxsplat_count_begin(const int32_t* count, uint64_t* ticket, void* stream);

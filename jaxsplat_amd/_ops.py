@@ -420,9 +420,9 @@ def _bin_tight(d, xys, depths, radii, conics, opacities, dev, capacity=None):
 
 def _bin_rects(d, depths, rects, cum, dev, capacity=None):
     """Binning into given tile rectangles with their inclusive counts cum
-    (jaxsplat_bin_rects_sort: emission straight from the rectangles and
-    counts, no depth stage), after a host read of the total, or (with a
-    capacity) no read.  Returns (gaussian_ids_sorted, tile_bins, isect)."""
+    (jaxsplat_bin_rects_sort: straight from the rectangles and counts, no depth
+    stage), after a host read of the total, or (with a capacity) no read.
+    Returns (gaussian_ids_sorted, tile_bins, isect)."""
     L = _lib.lib()
     ntiles = d.grid_dim_2d.x * d.grid_dim_2d.y
     with _on(dev):
@@ -479,9 +479,9 @@ def _rasterize_forward(d, gids, bins, isect, xys, conics, colors, opacities, bac
 
 def _staged_workspace(d, isect, nch, dev):
     """Workspace of the staged rasterize backward (records and bitmap), or
-    None where that backward does not apply or its bytes (52 per intersection,
-    60 beyond four channels) do not fit (the atomic backward is then used).
-    Returns (ws, bytes)."""
+    None where that backward does not apply or its bytes (per intersection 48 up
+    to three channels, 40 for four and 56 beyond, and a bit) do not fit (the atomic
+    backward is then used).  Returns (ws, bytes)."""
     L = _lib.lib()
     if staged_backward_applies(nch, isect):
         wsb = L.jaxsplat_rasterize_backward_staged_workspace_size(ctypes.byref(d), isect)

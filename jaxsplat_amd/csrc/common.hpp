@@ -424,7 +424,8 @@ __device__ __forceinline__ uint64_t slot_window(const uint32_t* __restrict__ bit
 // scheduling.  A longer range of which at most two slots are flagged needs no
 // wave either: zeros change no sum, and two values have one order.  That is
 // most of them where tiles are opaque: the flags of the tiles behind stay
-// clear (3M large Gaussians at 1080p, 33 slots each: tail 300 -> 106 us, 610k with 11: 43 -> 31).
+// clear (3M large Gaussians at 1080p, 33 slots each: tail 300 -> 106 us, 610k with
+// 11: 43 -> 31).
 // Called by every lane of the wave.
 template <int NV>
 __device__ __forceinline__ void sum_records(int off, int end, const float* __restrict__ rec,
@@ -691,8 +692,8 @@ hipError_t sort_pairs(const SortPlan& p, const uint32_t* keys_in, const uint32_t
 hipError_t column_scan(uint32_t* counts, int parts, uint32_t* totals, int columns, hipStream_t s);
 
 // ---- binning by tile rows (rowbin.hip) ----
-constexpr int kRowBinAxis = 256;
-constexpr int kRowBinPart = 1024;       // Gaussians or runs per partition    // tiles per axis, at most
+constexpr int kRowBinAxis = 256;        // tiles per axis, at most
+constexpr int kRowBinPart = 1024;       // Gaussians or runs per partition
 struct RowBinPlan {
     int n, tiles_x, tiles_y, cap;
     int parts;              // partitions of the Gaussians
@@ -857,7 +858,8 @@ hipError_t raster_fwd_grid(const RasterGrid& g, const int* items_sorted, const i
                            int* final_idx, float* out_img, hipStream_t s);
 // Single-view backward with staged gradients instead of float atomics (see
 // StagedOut in raster.hip): nch channels in passes of up to eight (v_xy_abs and
-// splats: nch <= 3), workspace raster_bwd_staged_bytes; radii and cum_tiles_hit are the projection's.  Writes every gradient row.
+// splats: nch <= 3), workspace raster_bwd_staged_bytes; radii and cum_tiles_hit are
+// the projection's.  Writes every gradient row.
 // Workspace for nch channels: records of the widest channel pass and bitmap.
 size_t raster_bwd_staged_bytes(int num_isect, int nch = 3);
 // rects (optional, packed as pack_rect) replaces the rectangles computed from

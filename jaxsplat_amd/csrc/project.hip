@@ -304,7 +304,7 @@ __device__ __forceinline__ Camera view_camera(const ViewRec& v, float glob_scale
 
 // Batched forward: blockIdx.y = view, kBatchPer Gaussians per lane of the
 // view's scene.  Writes the item rows the binning and rasterizer read, and the
-// depth sort key; no scan (the emission scans in depth order itself).
+// depth key; no scan (the binning finds the items' first slots itself).
 __global__ __launch_bounds__(256) void project_batch_fwd_kernel(
     const ViewRec* __restrict__ views, float glob_scale, float clip_thresh, int block_width,
     const float* __restrict__ means3d, const float* __restrict__ scales,
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256) void project_bwd_kernel(
 // Antialiased (AA): the blend took opacity times compensation; both get their
 // part of its gradient, and the projection that of the compensation.  (As separate
 // nodes, with three products, their sums and a second pass over the Gaussians,
-// a step of 300k at 719 x 1279 took 485 us instead of 460.)
+// a step of 300k at 719 x 1277 took 485 us instead of 460.)
 template <bool AA>
 __global__ __launch_bounds__(256) void render_bwd_tail_kernel(
     Camera c, int num_isect, const float* __restrict__ means3d, const float* __restrict__ scales,

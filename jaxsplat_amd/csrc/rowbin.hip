@@ -17,8 +17,9 @@
 // took 126 us and these take 62; at 3M large Gaussians 1540 us, and 445 in the
 // stable form, after a depth sort of 150, which also replaces 3440 us of
 // ordering the tiles' runs.  What bounds the placements is LDS (the
-// per-pair accesses and their bank conflicts) and its latency: the arrays are
-// sized for six workgroups per CU.
+// per-pair accesses and their bank conflicts) and its latency: the arrays leave
+// room for five workgroups per CU, six of the column placements of up to 128
+// columns, four of the stable row placement of more.
 //
 // Stable form (STABLE): the intervals of a partition are placed in their
 // order, by 64-lane column masks in LDS (an interval's rank in a column is the
@@ -391,9 +392,10 @@ __global__ __launch_bounds__(kRbThreads) void row_count_kernel(
 }
 
 // Step 1, placement: the runs of partition b into the row segments, which lie
-// end to end in runs[0 .. sum of row_len).  rects in perm's order; counts: exclusive over the
-// partitions of a row (column_scan), row_len their totals, or with fold the
-// counts themselves, and workgroup 0 writes row_len.  Workgroup 0 also writes the exact pair total and bit 8 of err where it exceeds cap.
+// end to end in runs[0 .. sum of row_len).  rects in perm's order; counts: exclusive
+// over the partitions of a row (column_scan), row_len their totals, or with fold the
+// counts themselves, and workgroup 0 writes row_len.  Workgroup 0 also writes the
+// exact pair total and bit 8 of err where it exceeds cap.
 template <bool STABLE, int COLS>
 __global__ __launch_bounds__(kRbThreads) void row_place_kernel(
     int n, const uint32_t* __restrict__ perm, const uint2* __restrict__ rects, int tiles_x,
