@@ -465,13 +465,14 @@ def stage_breakdown(torch, sc, cam, params, target, iters):
     # "tile_sort" reads the runs twice and writes an id per pair; with many pairs
     # per Gaussian and per tile (csrc/bin.hip), "emission" is led by a depth sort
     # of the Gaussians (four passes of 20 B) and the lists are then in order.
-    # Small grids, few pairs and more than 256 tiles per axis emit and sort the pairs.
+    # Small grids, few large Gaussians and more than 256 tiles per axis emit and sort
+    # the pairs.
     gx, gy = d.grid_dim_2d.x, d.grid_dim_2d.y
-    few = N < (32768 if min(gx, gy) <= 8 else 12288)
+    few, each = (32768, 4) if min(gx, gy) <= 8 else (12288, 24)
     by_rows = T > 256 and max(gx, gy) <= 256 and \
-        (N >= 65536 or isect >= (4_000_000 if few else 400_000))
+        not (N < few and each * N < isect < 4_000_000)
     by_depth = by_rows and isect > 16 * N and isect > 640 * T and \
-        isect > (2_500_000 if max(gx, gy) > 128 else 1_000_000)
+        isect > (2_500_000 if max(gx, gy) > 128 else 750_000)
     runs = int((rects[:, 1] >> 16).sum().item())
     stage_bytes = {
         "project_fwd": 144 * N,

@@ -12,8 +12,8 @@
 // Grids of up to 256 tiles per axis are binned by tile rows (rowbin.hip): of a
 // view's Gaussians in depth order where they have many pairs each and the lists
 // are long, else, and in batches, in id order with step 5 below after it.  Views
-// of up to 256 tiles in all (one radix pass) or few pairs (kRowsMany) and larger
-// grids:
+// of up to 256 tiles in all (one radix pass) or few large Gaussians (kRowsFew) and
+// larger grids:
 //  1. depth_keys_kernel: per Gaussian its depth bits and packed tile
 //     rectangle;
 //  2. emission in Gaussian id order: a reduce-then-scan of the Gaussians'
@@ -1054,7 +1054,7 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 //                             1M: 18, 2513: 355, 470     25k: 29, 467: 157, 127
 //                             30k: 20, 427: 165, 111     25k: 95, 400: 196, 180
 //                             300k: 10, 1061: 203, 159     2k: 93, 32: 160, 116
-// Below 1M pairs nothing saves what the sort costs (0.73M: 124, 113; 1.0M of 50k
+// Below 0.75M pairs nothing saves what the sort costs (0.73M: 124, 113; but 1.0M of 50k
 // Gaussians in the middle of 400 x 640: 133, 160), and with more than 128 tiles in a
 // row or column, whose stable placements take twice the LDS, below 2.5M (60 x 4000,
 // 0.66M: 145, 101; 1.3M: 130, 100; 1.7M: 191, 153; 3.3M: 150, 160).
@@ -1068,26 +1068,25 @@ hipError_t bin_by_rows(const BinPlan& p, const uint32_t* dkeys, const uint2* rec
 constexpr int kByDepthUnknown = 1 << 19;
 constexpr int kByDepthPairs = 16;
 constexpr int kByDepthTilePairs = 640;
-constexpr int kByDepthLeast = 1000000, kByDepthLeastWide = 2500000;
+constexpr int kByDepthLeast = 750000, kByDepthLeastWide = 2500000;
 // Where the pairs are emitted and sorted instead of binned by tile rows (the
 // capacity stands for their number here in any case: what the pair sort takes grows
 // with it).  Rows cost little per pair, but a wave takes as long as its longest
-// interval and a partition of 1024 has a workgroup, so that few Gaussians leave the
-// chip idle; the pair sort has a launch for each 256 tiles' digit.  Rows against
-// pairs, forward, us:
+// interval and a partition of 1024 has a workgroup, so that few Gaussians that cover
+// many tiles each leave the chip idle.  Rows against pairs, forward, us:
 //   up to 256 tiles (one radix pass), 256 x 256: 24k Gaussians 57, 49; 200k 169, 164;
 //     1M 424, 423
-//   below 64k Gaussians and 0.4M pairs: 100 at 272 x 272 40, 33; 2k (12 pairs each)
-//     at 1080p 88, 83; 24k, 0.29M 119, 114; but 50k, 0.64M at 600 x 1000 (8-pixel
-//     tiles) 104, 109, and 100k, 0.18M: 83, 84
-//   below 12k Gaussians and 4M pairs: 1k, 2.6M at 1080p 250, 209; 2k, 1.6M at
-//     683 x 1021 147, 129; 8k, 3.5M at 1080p 235, 227; but 4k, 11M: 317, 371
-//   up to 8 tiles high or wide, below 32k Gaussians and 4M pairs: 8k, 3.7M at
-//     60 x 4000 235, 175; 16k, 2.8M 171, 145; but 50k, 3.3M: 150, 164
+//   below 12k Gaussians and 4M pairs, more than 24 each: 1k, 2.6M at 1080p 250, 209;
+//     2k, 1.6M at 683 x 1021 147, 129; 8k, 3.5M at 1080p 235, 227; but 4k, 11M: 317,
+//     371.  With fewer each rows take up to 8 us more, but four launches less: steps
+//     of 12.5k, 0.1M at 581 x 1008 174, 183
+//   up to 8 tiles high or wide, below 32k Gaussians and 4M pairs, more than 4 each: 8k,
+//     3.7M at 60 x 4000 235, 175; 16k, 2.8M 171, 145; but 50k, 3.3M: 150, 164
 constexpr int kOnePassTiles = 256;
-constexpr int kRowsMany = 65536, kRowsFew = 12288, kRowsFewFlat = 32768;    // Gaussians
-constexpr int kRowsPairs = 400000, kRowsPairsFew = 4000000;
-constexpr int kRowsFlat = 8;                            // tiles
+constexpr int kRowsFlat = 8;                                    // tiles
+constexpr int kRowsFew = 12288, kRowsFewFlat = 32768;           // Gaussians
+constexpr int kRowsPairsFew = 4000000;                          // pairs
+constexpr int kRowsEach = 24, kRowsEachFlat = 4;                // per Gaussian
 
 BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     BinPlan p;
@@ -1100,9 +1099,9 @@ BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     p.rows_grid = c.tiles_x <= kRowBinAxis && c.tiles_y <= kRowBinAxis &&
                   p.num_tiles > kOnePassTiles;
     const bool flat = c.tiles_x <= kRowsFlat || c.tiles_y <= kRowsFlat;
-    const bool few = p.n < (flat ? kRowsFewFlat : kRowsFew);
-    p.by_rows = p.rows_grid &&
-                (p.n >= kRowsMany || isect_cap >= (few ? kRowsPairsFew : kRowsPairs));
+    const bool few = p.n < (flat ? kRowsFewFlat : kRowsFew) && isect_cap < kRowsPairsFew &&
+                     isect_cap > (flat ? kRowsEachFlat : kRowsEach) * (long long)p.n;
+    p.by_rows = p.rows_grid && !few;
     if (expected <= 0 && p.n >= kByDepthUnknown) expected = isect_cap;
     const bool wide = c.tiles_x > 128 || c.tiles_y > 128;
     p.by_depth = p.by_rows && (long long)expected > kByDepthPairs * (long long)p.n &&

@@ -98,7 +98,7 @@ def test_checked_total_chooses_the_depth_order(path, monkeypatch):
 
 
 def test_few_pairs_are_not_sorted_by_depth():
-    """Long lists of few pairs (fewer than 1M): hardly more kernels than short lists of
+    """Long lists of few pairs (fewer than 0.75M): hardly more kernels than short lists of
     as many Gaussians (a depth sort of them is eight)."""
     nodes = []
     for log_scale in (np.log(0.01), np.log(0.6)):
@@ -113,5 +113,5 @@ def test_few_pairs_are_not_sorted_by_depth():
         n, img = _kernels(lambda: run(tight))
         assert np.array_equal(img, want)
         nodes.append(n)
-    assert 16 * 3000 < total < 1_000_000 and total > 640 * 289
+    assert 16 * 3000 < total < 750_000 and total > 640 * 289
     assert nodes[1] <= nodes[0] + 5

@@ -5,8 +5,8 @@ always, with bit 8 of the error word and the exact total in the workspace's head
 
 Sorted ids, tile ids and bins must equal the oracle's order of those pairs exactly,
 at capacities that end between two Gaussians, after a whole row of a rectangle and
-inside one: for the pair sort (few Gaussians), by rows in id order and in depth order
-(65600 Gaussians, 0.06 of them over the whole grid), and where 128 and 256 tiles per
+inside one: for the pair sort (few Gaussians over many tiles), by rows in id order and
+in depth order (65600 Gaussians, 0.06 of them over the whole grid), and where 128 and 256 tiles per
 axis change the kernels.
 """
 

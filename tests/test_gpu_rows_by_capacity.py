@@ -1,6 +1,7 @@
-"""Which binning a view takes depends on its Gaussians and its capacity: by tile rows
-from 65536 Gaussians or 400k (few Gaussians: 4M) pairs, else the pair sort.  With a capacity of 4M the scenes of ``test_gpu_row_bin`` are binned by rows
-whatever their size, and at the limits of the rule the scenes here take either.
+"""Which binning a view takes depends on its Gaussians and its capacity: few Gaussians
+with many pairs each take the pair sort up to 4M pairs, others tile rows.  With a
+capacity of 4M the scenes of ``test_gpu_row_bin`` are binned by rows whatever their
+size, and at the limits of the rule the scenes here take either.
 
 Sorted ids, tile ids and bins must equal the oracle's stable (tile, depth bits, id)
 order exactly, on the edges of partitions (1023, 1025 Gaussians), of the LDS widths
@@ -72,9 +73,10 @@ def test_rows_by_capacity(tiles, n, expected, path):
 
 @pytest.mark.parametrize("path", ["split", "rects"])
 @pytest.mark.parametrize("n,tiles,cap", [
-    (65535, (17, 20), 399_999), (65536, (17, 20), 399_999), (65535, (17, 20), 400_000),
-    (32767, (8, 40), 3_999_999), (32768, (40, 8), 400_000), (32767, (8, 40), 4_000_000),
-    (12287, (20, 20), 3_999_999), (12288, (20, 20), 400_000), (12287, (20, 20), 4_000_000)],
+    (12287, (20, 20), 24 * 12287), (12287, (20, 20), 24 * 12287 + 1),
+    (12287, (20, 20), 3_999_999), (12287, (20, 20), 4_000_000), (12288, (20, 20), 400_000),
+    (32767, (8, 40), 3_999_999), (32767, (40, 8), 4_000_000), (32768, (8, 40), 400_000),
+    (32767, (9, 40), 400_000)],
     ids=str)
 def test_limits_of_the_rule(n, tiles, cap, path):
     _check(R._scene(n, tiles, 12, seed=n), tiles, cap, 0, path)
