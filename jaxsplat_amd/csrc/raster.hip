@@ -53,6 +53,11 @@ inline int bwd_threads(int block_width, int slots) {
 static_assert((kMaxTileThreads + 3) / 4 <= 64 && 128 / 2 <= 64,
               "one wave covers a tile at 4 (more than 128 pixels) or 2 pixels per lane");
 
+// The tile of this workgroup (a view's chunk is a constant: no division).
+__device__ __forceinline__ int grid_tile(const RasterGrid& rg) {
+    return rg.views ? xcd_tile(blockIdx.x, rg.chunk) : xcd_tile(blockIdx.x, kXcdChunkView);
+}
+
 constexpr float kTEps = 1e-4f;
 // The batches hold the conic scaled to base 2: (a, b, c) * (log2(e)/2,
 // log2(e), log2(e)/2), so that sigma2 = sigma * log2(e) =
@@ -510,7 +515,7 @@ __global__ __launch_bounds__(256) void raster_fwd_kernel(
     const float* __restrict__ colors, const float* __restrict__ opac,
     const float* __restrict__ bgs, float* __restrict__ final_Ts, int* __restrict__ final_idx,
     float* __restrict__ out_img) {
-    const int gt = xcd_tile(blockIdx.x, rg.chunk);
+    const int gt = grid_tile(rg);
     if (gt >= rg.total_tiles) return;
     raster_fwd_tile<DEPTH, CH>(rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts,
                                final_idx, out_img);
@@ -1037,7 +1042,7 @@ __global__ __launch_bounds__(64) void raster_bwd_kernel(
     const float* __restrict__ v_out_alpha, float* __restrict__ v_rgb,
     float* __restrict__ v_opacity, float* __restrict__ v_xy, float* __restrict__ v_xy_abs,
     float* __restrict__ v_conic, StagedOut st) {
-    const int gt = xcd_tile(blockIdx.x, rg.chunk);
+    const int gt = grid_tile(rg);
     if (gt >= rg.total_tiles) return;
     raster_bwd_tile<CONSISTENT, ABS, DEPTH, STAGED, NSLOT, CH>(
         rg, gt, gids, bins, xys, conics, colors, opac, bgs, final_Ts, final_idx, v_out_img,
