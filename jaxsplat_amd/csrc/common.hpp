@@ -151,15 +151,19 @@ __device__ __forceinline__ T wave_inclusive_sum(T v) {
 // Gaussians at 1080p) the same within 1%, as with chunks of 8 or 32 and blocks of
 // 4 x 4.
 constexpr int kXcdChunkView = 16;
-// A batch of at least as many views: a band per XCD, in which a view's Gaussians stay
-// in one L2 (steps, band against chunks of 64: 64 views of 200 x 200 with 100k
-// Gaussians 3188, 3449 us; 8 views of 365 x 529 with 110k 787, 922; 12 of 800 x 800
-// with 500k 2252, 2274; 8 draws of 8 views 9% faster, 17 of 9 to 12 the same).  Fewer
-// views are cut as one is, since a band is a part of one (2 views of 600 x 800 with
-// 50k: 402, 366; 3 of 500 x 700 with 60k: 476, 401; 24 draws of 5 to 7 views the
-// same), and so are views so uneven that a band has more than twice its share of the
-// Gaussians (64 of 100 x 100 with 200 and 2 of 500 x 500 with 100k: 672, 603).
-constexpr int kXcdChunkFew = 64, kXcdBandViews = 8;
+// A batch of as many views as XCDs or of at least kXcdBandViews: a band per XCD, in
+// which a view's Gaussians stay in one L2 (steps, band against chunks of 64: 64 views
+// of 200 x 200 with 100k Gaussians 3188, 3449 us; 8 views of 365 x 529 with 110k 787,
+// 922; 12 of 800 x 800 with 500k 2252, 2274; fourteen draws of 8 views 6% faster, six
+// each of 12 10%, of 13 to 64 2%, with single ones whose rows the chunks dealt to the
+// same XCDs again and again up to 41%).  Of 9 to 11 views a band holds the full middle
+// of one view or of two (9: 3% slower than chunks, 10: 1% faster, but 10 of 771 x 587
+// with 26k in two scenes 445, 414 us, 11: 7% slower).  Fewer views are cut as one is,
+// since a band is a part of one (2 views of 600 x 800 with 50k: 402, 366; 3 of
+// 500 x 700 with 60k: 476, 401; 24 draws of 5 to 7 views the same), and so are views so
+// uneven that a band has more than twice its share of the Gaussians (64 of 100 x 100
+// with 200 and 2 of 500 x 500 with 100k: 672, 603).
+constexpr int kXcdChunkFew = 64, kXcdBandViews = 12, kXcds = 8;
 
 // Mask of the lanes of this wave whose `bits`-bit digit equals this lane's
 // (restricted to lanes in `valid`): one ballot per digit bit.

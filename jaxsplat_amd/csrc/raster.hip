@@ -1255,7 +1255,7 @@ ViewRec single_view(const Camera& c) {
 }
 
 int batch_chunk(const ViewRec* views, int num_views, int num_tiles) {
-    if (num_views < kXcdBandViews) return kXcdChunkFew;
+    if (num_views < kXcdBandViews && num_views != kXcds) return kXcdChunkFew;
     const int band = num_tiles > 8 ? (num_tiles + 7) / 8 : 1;
     double share[8] = {}, all = 0;      // Gaussians of the bands' tiles
     for (int v = 0; v < num_views; ++v) {
