@@ -468,7 +468,7 @@ def stage_breakdown(torch, sc, cam, params, target, iters):
     # Small grids, few large Gaussians and more than 256 tiles per axis emit and sort
     # the pairs.
     gx, gy = d.grid_dim_2d.x, d.grid_dim_2d.y
-    few, each = (32768, 4) if min(gx, gy) <= 8 else (12288, 24)
+    few, each = (32768, 16) if min(gx, gy) <= 8 else (12288, 48)
     by_rows = T > 256 and max(gx, gy) <= 256 and \
         not (N < few and each * N < isect < 4_000_000)
     by_depth = by_rows and isect > 16 * N and isect > 640 * T and \

@@ -1076,17 +1076,20 @@ constexpr int kByDepthLeast = 750000, kByDepthLeastWide = 2500000;
 // many tiles each leave the chip idle.  Rows against pairs, forward, us:
 //   up to 256 tiles (one radix pass), 256 x 256: 24k Gaussians 57, 49; 200k 169, 164;
 //     1M 424, 423
-//   below 12k Gaussians and 4M pairs, more than 24 each: 1k, 2.6M at 1080p 250, 209;
-//     2k, 1.6M at 683 x 1021 147, 129; 8k, 3.5M at 1080p 235, 227; but 4k, 11M: 317,
-//     371.  With fewer each rows take up to 8 us more, but four launches less: steps
-//     of 12.5k, 0.1M at 581 x 1008 174, 183
-//   up to 8 tiles high or wide, below 32k Gaussians and 4M pairs, more than 4 each: 8k,
-//     3.7M at 60 x 4000 235, 175; 16k, 2.8M 171, 145; but 50k, 3.3M: 150, 164
+//   below 12k Gaussians and 4M pairs, more than 48 each: 1k, 2.6M at 1080p 250, 209;
+//     2k, 1.6M at 683 x 1021 147, 129; 2k, 0.14M at 1080p 112, 97; 8k, 3.5M 235, 227;
+//     2k, 0.11M at 400 x 640 87, 80; but 4k, 11M: 317, 371.  With fewer each rows take
+//     5 to 9 us more (10k, 0.33M at 1080p 128, 118), but four launches less, which
+//     steps that wait for the host notice (4k, 0.1M at 428 x 757 220, 227; 12.5k, 0.1M
+//     at 581 x 1008 174, 183)
+//   up to 8 tiles high or wide, below 32k Gaussians and 4M pairs, more than 16 each: 8k,
+//     3.7M at 60 x 4000 235, 175; 10k, 0.31M 86, 71 (steps 169, 177); 16k, 2.8M 171,
+//     145; 10k, 0.18M at 4000 x 64 109, 98; but 50k, 3.3M: 150, 164
 constexpr int kOnePassTiles = 256;
 constexpr int kRowsFlat = 8;                                    // tiles
 constexpr int kRowsFew = 12288, kRowsFewFlat = 32768;           // Gaussians
 constexpr int kRowsPairsFew = 4000000;                          // pairs
-constexpr int kRowsEach = 24, kRowsEachFlat = 4;                // per Gaussian
+constexpr int kRowsEach = 48, kRowsEachFlat = 16;               // per Gaussian
 
 BinPlan bin_plan(const Camera& c, int isect_cap, int expected) {
     BinPlan p;

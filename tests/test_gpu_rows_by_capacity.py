@@ -73,7 +73,8 @@ def test_rows_by_capacity(tiles, n, expected, path):
 
 @pytest.mark.parametrize("path", ["split", "rects"])
 @pytest.mark.parametrize("n,tiles,cap", [
-    (12287, (20, 20), 24 * 12287), (12287, (20, 20), 24 * 12287 + 1),
+    (12287, (20, 20), 48 * 12287), (12287, (20, 20), 48 * 12287 + 1),
+    (32767, (8, 40), 16 * 32767), (32767, (8, 40), 16 * 32767 + 1),
     (12287, (20, 20), 3_999_999), (12287, (20, 20), 4_000_000), (12288, (20, 20), 400_000),
     (32767, (8, 40), 3_999_999), (32767, (40, 8), 4_000_000), (32768, (8, 40), 400_000),
     (32767, (9, 40), 400_000)],
